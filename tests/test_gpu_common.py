@@ -304,6 +304,20 @@ def test_label_helpers(cuda):
     assert int(drivers.get_nb_distinct_clusters(_dev(a, cuda), 50)) == len(np.unique(a))
 
 
+# either side of the clusters whose flags a workgroup keeps in LDS, vector loads with and without a
+# remainder, a start off their alignment
+@pytest.mark.parametrize("n,k,offset", [(1, 1, 0), (7, 3, 0), (4096 * 5 + 3, 10, 0), (100_001, 5, 1), (300_000, 32768, 0),
+                                        (300_000, 32769, 0)])
+def test_distinct_labels_are_counted(cuda, n, k, offset):
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + k)
+    kept = np.flatnonzero(rng.random(k) < 0.7) if k > 1 else np.zeros(1, dtype=np.int64)
+    labels = rng.choice(kept, n + offset).astype(np.int32)
+    got = drivers.get_nb_distinct_clusters(_dev(labels, cuda)[offset:], k)
+    assert int(got) == len(np.unique(labels[offset:]))
+
+
 # every instantiation of the distance and inertia kernels (register / tiled distances,
 # centroids in LDS or not, 128-bit or scalar accesses) against numpy in fp64
 @pytest.mark.parametrize("shape", [(1003, 14, 127, np.float32), (4096, 32, 7, np.float32), (777, 33, 5, np.float32),
