@@ -16,7 +16,7 @@
  *   - Outputs and workspaces are allocated by the caller; `*_workspace_bytes` give sizes.
  *     No entry point allocates or frees device memory.
  *   - `stream` is a hipStream_t (NULL = default stream).  Calls only enqueue work; none
- *     synchronises except kmx_lloyd_status_read.
+ *     waits except kmx_lloyd_status_read and kmx_lloyd_run.
  *   - Return value: 0 on success, a negative KMX_ERR_* for rejected arguments, or a positive
  *     hipError_t reported by the runtime.  Nothing throws or exits.
  *   - Calls that share a workspace must be issued on one stream (or otherwise ordered).
@@ -70,7 +70,7 @@ typedef struct kmx_lloyd_status {
     double tol;           /* loop runs while shift_sum > tol                               */
     int32_t max_iter;
     uint32_t ticket;      /* internal: block counter of the reduction kernel               */
-    double max_sq_dist;   /* scratch for the relocation guard                              */
+    uint64_t reserved0;
     int64_t reserved[2];
 } kmx_lloyd_status;       /* 64 bytes */
 
@@ -193,6 +193,22 @@ int32_t kmx_lloyd_iter_traced(const kmx_lloyd_plan* plan, const void* X_t, const
                               void* cluster_sizes, uint32_t* empty_clusters, void* workspace,
                               size_t workspace_bytes, void* stream);
 int32_t kmx_lloyd_trace_collect(float* kernel_ms_mean, float* kernel_ms_min, int32_t* n_launches);
+
+/* Iterations n_done, n_done + 1, ... until the state is no longer KMX_RUNNING or max_iter (the value
+ * given to kmx_lloyd_init) is reached: enqueues kmx_lloyd_iter a few ahead of the last one that has
+ * announced itself to the host and returns with what it learned in status_host (n_iter, state,
+ * n_empty, shift_sum).  Iteration j reads the centroids and previous labels of its parity and
+ * writes those of the other one: centroids_even holds the initial centroids, and iteration 0 writes
+ * centroids_odd and labels_odd.  After KMX_NEED_RELOCATION the caller relocates, calls
+ * kmx_lloyd_finalize and comes back with n_done = status.n_iter + 1 if the run goes on.  Waits for
+ * the end of the run on the host (without synchronising the stream: launches that find the run over
+ * may still be queued).  Safe to call from several threads on workspaces and streams of their own.
+ * Replaces the loop of lloyd(), kmeans/drivers.py:188-343. */
+int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X_rowmajor,
+                      const void* sample_weight, void* centroids_even, void* centroids_odd,
+                      uint32_t* labels_even, uint32_t* labels_odd, void* cluster_sizes,
+                      uint32_t* empty_clusters, void* workspace, size_t workspace_bytes,
+                      int32_t n_done, int32_t max_iter, kmx_lloyd_status* status_host, void* stream);
 
 /* Second half of (2) alone, for the iteration that stopped with KMX_NEED_RELOCATION after
  * the host has relocated the empty clusters: sums / sizes, shift, convergence test, state

@@ -14,6 +14,7 @@
 #include "kmx_common.h"
 #include "lloyd_layout.h"
 
+#include <cstring>
 #include <mutex>
 #include <vector>
 #include "lloyd_tail.h"
@@ -316,7 +317,8 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
     T* __restrict__ partial, int n_partials, int clear_partials, T* __restrict__ sums_t,
     T* __restrict__ sizes, uint32_t* __restrict__ empty_clusters,
     kmx_lloyd_status* __restrict__ status, int d, int k,
-    unsigned long long* __restrict__ gsum, const int* __restrict__ q_exp, int with_tail) {
+    unsigned long long* __restrict__ gsum, const int* __restrict__ q_exp, int with_tail,
+    unsigned long long* __restrict__ progress) {
     if (status->state != KMX_RUNNING) return;
     const int items = (d + 1) * k;
     if (gsum != nullptr) {
@@ -439,7 +441,10 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
         status->reserved[0] = bidx;
         status->n_empty = base;
         status->ticket = 0;
-        if (base > 0) status->state = KMX_NEED_RELOCATION;
+        if (base > 0) {
+            status->state = KMX_NEED_RELOCATION;
+            lloyd_publish(progress, status->n_iter, KMX_NEED_RELOCATION, base, status->shift_sum);
+        }
     }
 }
 
@@ -459,7 +464,7 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
     const T* __restrict__ old_centroids_t, T* __restrict__ new_centroids_t,
     const T* __restrict__ sizes, T* __restrict__ cpack, T* __restrict__ half_norms,
     double* __restrict__ shift_partial, kmx_lloyd_status* __restrict__ status, int d, int k,
-    int dpad, int force) {
+    int dpad, int force, unsigned long long* __restrict__ progress) {
     const int state = status->state;
     if (force ? (state != KMX_NEED_RELOCATION && state != KMX_RUNNING) : (state != KMX_RUNNING))
         return;
@@ -535,21 +540,8 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
         double total = parked_shift;
         for (unsigned int b = 0; b < gridDim.x; ++b)
             total += __builtin_nontemporal_load(shift_partial + b);
-        const int n_iter = status->n_iter + 1;
-        const unsigned int changed = status->n_changed;
-        status->n_iter = n_iter;
-        status->shift_sum = total;
-        status->n_changed = 0;
         status->ticket = 0;
-        int next = KMX_RUNNING;
-        if (n_iter > 1 && changed == 0)
-            next = KMX_CONVERGED_STRICT;
-        else if (!(total > status->tol))
-            next = KMX_CONVERGED_TOL;
-        else if (n_iter >= status->max_iter)
-            next = KMX_MAX_ITER;
-        status->state = next;
-        status->reserved[1] = (int64_t)changed;
+        lloyd_update_status(status, total, status->n_changed, progress);
     }
 }
 
@@ -604,7 +596,7 @@ __global__ __launch_bounds__(256) void lloyd_pack_kernel(const T* __restrict__ c
         status->tol = tol;
         status->max_iter = max_iter;
         status->ticket = 0;
-        status->max_sq_dist = 0.0;
+        status->reserved0 = 0;
         status->reserved[0] = 0;
         status->reserved[1] = 0;
     }
@@ -810,6 +802,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
             tail.d = d;
             tail.k = k;
             tail.dpad = L.dpad;
+            tail.progress = L.progress;
             hipLaunchKernelGGL((lloyd_small_finalize_kernel<float, true>), dim3(1), dim3(256),
                                (size_t)items * sizeof(float), stream, gsum, q_exp, tail);
             KMX_LAUNCH_CHECK();
@@ -826,7 +819,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
                        stream, partial, n_partials_used,
                        ((L.acc_mode == ACC_GLOBAL || L.acc_mode == KMX_ACC_BUCKET) && gsum == nullptr) ? 1 : 0,
                        (T*)new_centroids_t, (T*)sizes, empty_clusters, status, d, k, gsum, q_exp,
-                       small_tail ? 0 : 1);
+                       small_tail ? 0 : 1, L.progress);
     KMX_LAUNCH_CHECK();
     if (events) (void)hipEventRecord(events[2], stream);
     if (small_tail) {
@@ -841,17 +834,18 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         tail.d = d;
         tail.k = k;
         tail.dpad = L.dpad;
+        tail.progress = L.progress;
         hipLaunchKernelGGL((lloyd_small_finalize_kernel<T, false>), dim3(1), dim3(256),
                            (size_t)items * sizeof(T), stream, nullptr, nullptr, tail);
     } else {
         if (fin_lanes(d, k) == 64)
             hipLaunchKernelGGL((lloyd_finalize_kernel<T, 64>), dim3((unsigned)fin_grid(d, k)), dim3(256), 0,
                                stream, (const T*)centroids_t, (T*)new_centroids_t, (const T*)sizes, cpack,
-                               half_norms, shift_partial, status, d, k, L.dpad, 0);
+                               half_norms, shift_partial, status, d, k, L.dpad, 0, L.progress);
         else
             hipLaunchKernelGGL((lloyd_finalize_kernel<T, 8>), dim3((unsigned)fin_grid(d, k)), dim3(256), 0,
                                stream, (const T*)centroids_t, (T*)new_centroids_t, (const T*)sizes, cpack,
-                               half_norms, shift_partial, status, d, k, L.dpad, 0);
+                               half_norms, shift_partial, status, d, k, L.dpad, 0, L.progress);
     }
     KMX_LAUNCH_CHECK();
     if (events) (void)hipEventRecord(events[3], stream);
@@ -1032,7 +1026,8 @@ static int32_t lloyd_iter_dispatch(const kmx_lloyd_plan* plan, const void* X_t, 
                                    void* new_centroids_t,
                                    const uint32_t* labels_prev, uint32_t* labels,
                                    void* cluster_sizes, uint32_t* empty_clusters, void* workspace,
-                                   size_t workspace_bytes, void* stream_, hipEvent_t* events) {
+                                   size_t workspace_bytes, void* stream_, hipEvent_t* events,
+                                   unsigned long long* progress = nullptr) {
     KMX_REQUIRE_PLAN(plan);
     KMX_REQUIRE_PTR(X_t);
     KMX_REQUIRE_PTR(sample_weight);
@@ -1045,8 +1040,9 @@ static int32_t lloyd_iter_dispatch(const kmx_lloyd_plan* plan, const void* X_t, 
     KMX_REQUIRE_PTR(workspace);
     const int64_t n = plan->n;
     const int32_t d = plan->d, k = plan->k, dtype = plan->dtype;
-    const LloydLayout L = lloyd_layout(n, d, k, dtype, plan->flags);
+    LloydLayout L = lloyd_layout(n, d, k, dtype, plan->flags);
     if (workspace_bytes < L.total) return KMX_ERR_WORKSPACE;
+    L.progress = progress;
     hipStream_t stream = (hipStream_t)stream_;
     if (dtype == KMX_F32) {
         if (L.variant == KMX_VARIANT_MFMA)
@@ -1079,6 +1075,127 @@ int32_t kmx_lloyd_iter(const kmx_lloyd_plan* plan, const void* X_t, const void* 
     return lloyd_iter_dispatch(plan, X_t, X_rowmajor, sample_weight, centroids_t, new_centroids_t, labels_prev,
                                labels, cluster_sizes, empty_clusters, workspace, workspace_bytes, stream_,
                                nullptr);
+}
+
+// Pinned words for the runs that are under way (lloyd_publish): one page, allocated once, a slot
+// of a cache line each.  A run that finds none free reads the status the slow way.
+static std::mutex progress_mutex;
+static unsigned long long* progress_page = nullptr;
+static uint64_t progress_free = 0;  // bit i: slot i is free
+static bool progress_tried = false;
+constexpr int KMX_PROGRESS_SLOTS = 64, KMX_PROGRESS_STRIDE = 16;  // (in words: 128 bytes apart)
+
+static unsigned long long* progress_take() {
+    std::lock_guard<std::mutex> guard(progress_mutex);
+    if (!progress_tried) {
+        progress_tried = true;
+        void* p = nullptr;
+        if (hipHostMalloc(&p, KMX_PROGRESS_SLOTS * KMX_PROGRESS_STRIDE * 8, hipHostMallocPortable | hipHostMallocMapped) ==
+            hipSuccess) {
+            progress_page = (unsigned long long*)p;
+            progress_free = ~0ull;
+        } else {
+            (void)hipGetLastError();
+        }
+    }
+    if (progress_free == 0) return nullptr;
+    const int i = __builtin_ctzll(progress_free);
+    progress_free &= progress_free - 1;
+    unsigned long long* slot = progress_page + i * KMX_PROGRESS_STRIDE;
+    for (int j = 0; j < KMX_PROGRESS_WORDS; ++j) __atomic_store_n(&slot[j], 0ull, __ATOMIC_SEQ_CST);
+    return slot;
+}
+static void progress_give_back(unsigned long long* slot) {
+    if (slot == nullptr) return;
+    std::lock_guard<std::mutex> guard(progress_mutex);
+    progress_free |= 1ull << ((slot - progress_page) / KMX_PROGRESS_STRIDE);
+}
+static bool progress_look(const unsigned long long* slot, kmx_lloyd_status* out) {
+    const unsigned long long a = __atomic_load_n(&slot[0], __ATOMIC_RELAXED), b = __atomic_load_n(&slot[1], __ATOMIC_RELAXED),
+                             c = __atomic_load_n(&slot[2], __ATOMIC_RELAXED);
+    if (__atomic_load_n(&slot[3], __ATOMIC_RELAXED) != lloyd_progress_check(a, b, c)) return false;
+    out->n_iter = (int32_t)(uint32_t)a;
+    out->state = (int32_t)(a >> 32);
+    std::memcpy(&out->shift_sum, &b, sizeof(b));
+    out->n_empty = (int32_t)c;
+    return true;
+}
+
+int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X_rowmajor,
+                      const void* sample_weight, void* centroids_even, void* centroids_odd,
+                      uint32_t* labels_even, uint32_t* labels_odd, void* cluster_sizes,
+                      uint32_t* empty_clusters, void* workspace, size_t workspace_bytes,
+                      int32_t n_done, int32_t max_iter, kmx_lloyd_status* status_host, void* stream_) {
+    KMX_ENTRY();
+    KMX_REQUIRE_PTR(centroids_even);
+    KMX_REQUIRE_PTR(centroids_odd);
+    KMX_REQUIRE_PTR(labels_even);
+    KMX_REQUIRE_PTR(labels_odd);
+    KMX_REQUIRE_PTR(status_host);
+    if (n_done < 0 || max_iter < 0) return KMX_ERR_BAD_ARGUMENT;
+    void* cent[2] = {centroids_even, centroids_odd};
+    uint32_t* labels[2] = {labels_even, labels_odd};
+    hipStream_t stream = (hipStream_t)stream_;
+    // Iterations in flight beyond the last one the host knows of.  Three cover the host's round trip
+    // for the shortest iterations; those behind the end of the run do nothing, but cost their
+    // launches (4.5 us each).
+    constexpr int AHEAD = 3;
+    int enqueued = n_done;
+    auto enqueue = [&](unsigned long long* progress) {
+        const int a = enqueued & 1;
+        const int32_t rc = lloyd_iter_dispatch(plan, X_t, X_rowmajor, sample_weight, cent[a], cent[a ^ 1], labels[a],
+                                               labels[a ^ 1], cluster_sizes, empty_clusters, workspace, workspace_bytes,
+                                               stream_, nullptr, progress);
+        ++enqueued;
+        return rc;
+    };
+    unsigned long long* slot = n_done < max_iter ? progress_take() : nullptr;
+    if (slot == nullptr) {
+        // (nothing to run, or no slot: a look at the status per batch of iterations)
+        for (int batch = 1;; batch = batch < 16 ? 2 * batch : 16) {
+            for (int i = 0; i < batch && enqueued < max_iter; ++i) {
+                const int32_t rc = enqueue(nullptr);
+                if (rc != KMX_OK) return rc;
+            }
+            const int32_t rc = kmx_lloyd_status_read(workspace, status_host, stream_);
+            if (rc != KMX_OK) return rc;
+            if (status_host->state != KMX_RUNNING || enqueued >= max_iter) return KMX_OK;
+        }
+    }
+    kmx_lloyd_status seen;
+    std::memset(&seen, 0, sizeof(seen));
+    seen.n_iter = n_done;
+    seen.state = KMX_RUNNING;
+    unsigned int spins = 0;
+    while (true) {
+        while (enqueued < max_iter && enqueued < seen.n_iter + AHEAD) {
+            const int32_t rc = enqueue(slot);
+            if (rc != KMX_OK) return rc;  // (the slot stays taken: launches before this one may still write to it)
+        }
+        kmx_lloyd_status now = seen;
+        if (progress_look(slot, &now) && (now.n_iter != seen.n_iter || now.state != KMX_RUNNING)) {
+            seen = now;
+            spins = 0;
+            if (seen.state != KMX_RUNNING || seen.n_iter >= max_iter) break;
+            continue;
+        }
+        // Not there yet.  Now and then ask whether the stream is done without a word from it (a
+        // launch that failed, a state that was terminal to begin with).
+        if (++spins % 20000u == 0u) {
+            const hipError_t e = hipStreamQuery(stream);
+            if (e != hipSuccess && e != hipErrorNotReady) return (int32_t)e;
+            if (e == hipSuccess && !(progress_look(slot, &now) && (now.n_iter != seen.n_iter || now.state != KMX_RUNNING))) {
+                const int32_t rc = kmx_lloyd_status_read(workspace, status_host, stream_);
+                progress_give_back(slot);
+                return rc;
+            }
+        }
+        __builtin_ia32_pause();
+    }
+    progress_give_back(slot);
+    seen.max_iter = max_iter;
+    *status_host = seen;
+    return KMX_OK;
 }
 
 int32_t kmx_lloyd_iter_timed(const kmx_lloyd_plan* plan, const void* X_t, const void* X_rowmajor,
@@ -1191,7 +1308,7 @@ int32_t kmx_lloyd_finalize(const kmx_lloyd_plan* plan, const void* centroids_t,
     hipLaunchKernelGGL((lloyd_finalize_kernel<T, LANES>), dim3(grid), dim3(256), 0, stream,           \
                        (const T*)centroids_t, (T*)new_centroids_t, (const T*)cluster_sizes,           \
                        (T*)(ws + L.off_cpack), (T*)(ws + L.off_half), shift_partial, status, d, k,    \
-                       L.dpad, 1)
+                       L.dpad, 1, (unsigned long long*)nullptr)
     if (dtype == KMX_F32) {
         if (fin_lanes(d, k) == 64) KMX_FINALIZE(float, 64); else KMX_FINALIZE(float, 8);
     } else {

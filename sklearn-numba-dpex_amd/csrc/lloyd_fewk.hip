@@ -1092,6 +1092,7 @@ int32_t kmx_lloyd_iter_fewk(const LloydLayout& L, const void* X_t, const void* X
     tail.d = d;
     tail.k = k;
     tail.dpad = L.dpad;
+    tail.progress = L.progress;
     const int* q_exp = reinterpret_cast<const int*>(ws + L.off_scales) + (d + 1);
     unsigned long long* gsum = reinterpret_cast<unsigned long long*>(ws + L.off_gsum);
     kmx_lloyd_status* status = tail.status;

@@ -117,6 +117,7 @@ struct LloydLayout {
     bool screen_labels;  // KMX_VARIANT_GEMM (fp32, d <= 64): labels by the screened kernel of variant 61 without its sums
     bool direct_sums;    // with screen_labels: sums straight from the labels (fixed point in LDS) instead of per bucket
     uint32_t flags;      // the caller's KMX_FLAG_* selection
+    unsigned long long* progress = nullptr;  // where the iterations of a run announce themselves (lloyd_publish), or null
     int wgs_per_cu;      // workgroups per compute unit asked for (0: the kernel's default)
     int cols;            // sample columns per lane asked for (0: the kernel's default)
     size_t off_status, off_scales, off_gsum, off_cpack, off_half, off_shift, off_bucket, off_wscreen, off_partial;

@@ -606,6 +606,7 @@ int32_t kmx_lloyd_iter_mfma_f32(const LloydLayout& L, const void* X_t, const voi
     tail.d = d;
     tail.k = k;
     tail.dpad = L.dpad;
+    tail.progress = L.progress;
     const int* q_exp = reinterpret_cast<const int*>(ws + L.off_scales) + (d + 1);
     unsigned long long* gsum = reinterpret_cast<unsigned long long*>(ws + L.off_gsum);
     if (events) (void)hipEventRecord(events[0], stream);
@@ -673,6 +674,7 @@ int32_t kmx_lloyd_iter_mfma_screen_f64(const LloydLayout& L, const void* X_t, co
     tail.d = d;
     tail.k = k;
     tail.dpad = L.dpad;
+    tail.progress = L.progress;
     const int* q_exp = reinterpret_cast<const int*>(ws + L.off_scales) + (d + 1);
     unsigned long long* gsum = reinterpret_cast<unsigned long long*>(ws + L.off_gsum);
     uint32_t* uncertain = reinterpret_cast<uint32_t*>(ws + L.off_bucket);

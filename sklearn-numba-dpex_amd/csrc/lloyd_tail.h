@@ -6,6 +6,27 @@
 
 #include "kmx_common.h"
 
+// Where a run of iterations tells the host how far it is: four words of pinned host memory, written
+// at the end of an iteration by the thread that sets the state, so that the host can follow a run
+// without a copy and a wait per look (a 64-byte copy and the wait for it take 25 us of an idle
+// GPU, more than many an iteration).  The words reach the host in any order; the last one is the
+// exclusive or of the others, and the host takes no notice of words that do not fit together.
+constexpr int KMX_PROGRESS_WORDS = 4;
+constexpr unsigned long long KMX_PROGRESS_MARK = 0x6b6d78206c6c6f79ull;
+__host__ __device__ inline unsigned long long lloyd_progress_check(unsigned long long a, unsigned long long b,
+                                                                   unsigned long long c) {
+    return a ^ (b << 1 | b >> 63) ^ (c << 2 | c >> 62) ^ KMX_PROGRESS_MARK;
+}
+__device__ inline void lloyd_publish(unsigned long long* progress, int n_iter, int state, int n_empty, double shift) {
+    if (progress == nullptr) return;
+    const unsigned long long w[3] = {(unsigned long long)(unsigned int)n_iter | (unsigned long long)state << 32,
+                                     (unsigned long long)__double_as_longlong(shift),
+                                     (unsigned long long)(unsigned int)n_empty};
+    for (int i = 0; i < 3; ++i) __hip_atomic_store(&progress[i], w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&progress[3], lloyd_progress_check(w[0], w[1], w[2]), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <typename T>
 struct LloydTail {
     T* sums_t;               // (d, k): sums on entry, the new centroids on exit
@@ -16,6 +37,7 @@ struct LloydTail {
     T* half_norms;
     kmx_lloyd_status* status;
     int d, k, dpad;
+    unsigned long long* progress = nullptr;  // see lloyd_publish
     uint32_t* clear_word = nullptr;  // a counter to copy to the next word and zero, or null
     // Screened fused step only: word clear_word[2] tells the next step whether it may correct the
     // fixed-point sums for the samples that change cluster instead of rebuilding them; the sums
@@ -130,7 +152,8 @@ __device__ inline int lloyd_list_empty_one_wave(const T* sizes, uint32_t* empty_
 
 // End of an iteration, by one thread: iteration count, shift, and the next state (strict
 // convergence from the second iteration on, then the tolerance, then the iteration limit).
-__device__ inline void lloyd_update_status(kmx_lloyd_status* st, double total_shift, unsigned int changed) {
+__device__ inline void lloyd_update_status(kmx_lloyd_status* st, double total_shift, unsigned int changed,
+                                           unsigned long long* progress) {
     const int n_iter = st->n_iter + 1;
     st->n_iter = n_iter;
     st->shift_sum = total_shift;
@@ -144,6 +167,7 @@ __device__ inline void lloyd_update_status(kmx_lloyd_status* st, double total_sh
         next = KMX_MAX_ITER;
     st->state = next;
     st->reserved[1] = (int64_t)changed;
+    lloyd_publish(progress, n_iter, next, 0, total_shift);
 }
 
 // Division, packed copy, half norms, shift and convergence test by ONE workgroup of 256
@@ -192,7 +216,7 @@ __device__ inline void lloyd_finalize_block(const LloydTail<T>& a, int n_empty, 
         }
     }
     const double total = kmx_block_sum<double>(shift, scratch);
-    if (threadIdx.x == 0) lloyd_update_status(a.status, total, a.status->n_changed);
+    if (threadIdx.x == 0) lloyd_update_status(a.status, total, a.status->n_changed, a.progress);
 }
 
 
@@ -361,6 +385,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         }
         if (threadIdx.x == 0) {
             a.status->state = KMX_NEED_RELOCATION;
+            lloyd_publish(a.progress, a.status->n_iter, KMX_NEED_RELOCATION, n_empty, a.status->shift_sum);
             if (a.clear_word != nullptr) a.clear_word[2] = 0u;
         }
         return;
@@ -449,7 +474,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         }
     }
     const double total = kmx_block_sum<double>(shift, scratch);
-    if (threadIdx.x == 0) lloyd_update_status(a.status, total, n_changed);
+    if (threadIdx.x == 0) lloyd_update_status(a.status, total, n_changed, a.progress);
 }
 
 // The same as a launch of its own: ordered after the producers of the sums by the kernel boundary.

@@ -18,10 +18,6 @@ from ..common.random import create_xoroshiro128pp_states, get_random_raw, raw_to
 from ..common.reductions import sum_reduction
 from ..common.topk import topk_idx
 
-# How many Lloyd iterations may be enqueued before the host next reads the status.
-_MAX_LOOKAHEAD = 16
-
-
 
 def lloyd(
     X_t,
@@ -39,9 +35,9 @@ def lloyd(
     Returns (assignments_idx (n,), inertia numpy scalar, centroids_t (d, k), n_iteration).
 
     The loop state (iteration count, convergence, empty clusters) lives on the device, and
-    every kernel of an iteration is a no-op once the state is terminal, so iterations are
-    enqueued ahead and the host reads the status once per batch instead of three times per
-    iteration.
+    every kernel of an iteration is a no-op once the state is terminal, so the library enqueues
+    iterations a few ahead of the one that last announced itself to the host, where the
+    reference's loop reads three scalars back per iteration.
 
     relocation: which centroids the distances that rank samples for empty-cluster relocation
     are measured to: "sklearn" = the centroids the labels were computed from (what
@@ -84,16 +80,13 @@ def lloyd(
           "kmx_lloyd_init")
 
     status = LloydStatus()
-    enqueued = 0
-    lookahead = 1
+    n_done, max_iter = 0, int(max_iter)
     while True:
-        for _ in range(lookahead):
-            a, b = enqueued % 2, (enqueued + 1) % 2
-            check(lib.kmx_lloyd_iter(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(cent[a]), ptr(cent[b]),
-                                     ptr(labels[a]), ptr(labels[b]), ptr(sizes), ptr(empty_list),
-                                     ptr(ws), ws_bytes, stream), "kmx_lloyd_iter")
-            enqueued += 1
-        check(lib.kmx_lloyd_status_read(ptr(ws), status, stream), "kmx_lloyd_status_read")
+        # (verbose: an iteration at a time)
+        until = min(n_done + 1, max_iter) if verbose else max_iter
+        check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(cent[0]), ptr(cent[1]),
+                                ptr(labels[0]), ptr(labels[1]), ptr(sizes), ptr(empty_list), ptr(ws), ws_bytes,
+                                n_done, until, status, stream), "kmx_lloyd_run")
 
         if status.state == _capi.KMX_NEED_RELOCATION:
             j = status.n_iter  # the iteration that stopped: reads cent[j % 2], wrote sums to the other
@@ -104,8 +97,6 @@ def lloyd(
             )
             check(lib.kmx_lloyd_finalize(plan, ptr(cent[a]), ptr(cent[b]), ptr(sizes), ptr(ws), ws_bytes,
                                          stream), "kmx_lloyd_finalize")
-            enqueued = j + 1
-            lookahead = 1
             check(lib.kmx_lloyd_status_read(ptr(ws), status, stream), "kmx_lloyd_status_read")
 
         if verbose:
@@ -116,8 +107,7 @@ def lloyd(
 
         if status.state != _capi.KMX_RUNNING:
             break
-        enqueued = status.n_iter
-        lookahead = 1 if verbose else min(2 * lookahead, _MAX_LOOKAHEAD)
+        n_done = status.n_iter
 
     n_iteration = status.n_iter
     if verbose:

@@ -19,6 +19,64 @@ def _dev(a, cuda):
     return torch.as_tensor(np.ascontiguousarray(a), device=cuda)
 
 
+# a step per kernel family; more runs at once than there are words to announce iterations in (64), so
+# that some of them read the status instead
+@pytest.mark.parametrize("n,d,k,dtype,runs", [(3_001, 14, 20, np.float32, 70), (3_001, 10, 5, np.float64, 3),
+                                              (5_000, 70, 6, np.float32, 3), (5_003, 100, 40, np.float64, 3)])
+def test_runs_in_several_threads_equal_iterations_one_by_one(cuda, n, d, k, dtype, runs):
+    import threading
+
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib, ptr
+
+    rng = np.random.default_rng(n + d)
+    X_t, w = _dev(rng.standard_normal((d, n)).astype(dtype), cuda), _dev(rng.uniform(0.5, 1.5, n).astype(dtype), cuda)
+    max_iter = 7
+
+    def run(out, in_one_call):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            plan = _capi.lloyd_plan(n, d, k, _capi.dtype_code(X_t.dtype))
+            cent = [X_t[:, :k].contiguous(), torch.empty(d, k, dtype=X_t.dtype, device=cuda)]
+            labels = [torch.empty(n, dtype=torch.int32, device=cuda) for _ in range(2)]
+            sizes, empty = torch.empty(k, dtype=X_t.dtype, device=cuda), torch.empty(k, dtype=torch.int32, device=cuda)
+            ws, status = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=cuda), _capi.LloydStatus()
+            _capi.check(lib.kmx_lloyd_init(plan, ptr(ws), plan.workspace_bytes, ptr(X_t), ptr(w), ptr(cent[0]),
+                                           max_iter, 0.0, stream.cuda_stream), "init")
+            if in_one_call:
+                _capi.check(lib.kmx_lloyd_run(plan, ptr(X_t), None, ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]),
+                                              ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes, 0,
+                                              max_iter, status, stream.cuda_stream), "run")
+            else:
+                for it in range(max_iter):
+                    a, b = it % 2, (it + 1) % 2
+                    _capi.check(lib.kmx_lloyd_iter(plan, ptr(X_t), None, ptr(w), ptr(cent[a]), ptr(cent[b]),
+                                                   ptr(labels[a]), ptr(labels[b]), ptr(sizes), ptr(empty), ptr(ws),
+                                                   plan.workspace_bytes, stream.cuda_stream), "iter")
+                _capi.check(lib.kmx_lloyd_status_read(ptr(ws), status, stream.cuda_stream), "status")
+            stream.synchronize()
+            b = status.n_iter % 2
+            out.append((status.n_iter, status.state, status.shift_sum, cent[b].cpu().numpy(), labels[b].cpu().numpy()))
+
+    expected, got = [], []
+    torch.cuda.synchronize()
+    run(expected, False)
+    threads = [threading.Thread(target=run, args=(got, True)) for _ in range(runs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == runs
+    tol = 1e-6 if dtype == np.float32 else 1e-13  # (fp64 sums by floating-point atomics: order of additions)
+    for r in got:
+        assert r[:2] == expected[0][:2]
+        np.testing.assert_allclose(r[2], expected[0][2], rtol=10 * tol)
+        np.testing.assert_allclose(r[3], expected[0][3], rtol=tol, atol=tol)
+        np.testing.assert_array_equal(r[4], expected[0][4])
+
+
 def _small_configs():
     return {
         "C1": lambda: datasets.config1(n=100_000),
