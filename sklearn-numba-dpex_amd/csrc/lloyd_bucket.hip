@@ -78,7 +78,9 @@ __global__ __launch_bounds__(256) void bucket_count_kernel(
 }
 
 __global__ __launch_bounds__(1024) void bucket_offsets_kernel(const int* __restrict__ counts,
-                                                             int* __restrict__ offsets, int k) {
+                                                             int* __restrict__ offsets, int k,
+                                                             const kmx_lloyd_status* __restrict__ status) {
+    if (status->state != KMX_RUNNING) return;
     __shared__ int wave_tot[16];
     __shared__ int carry_s;
     if (threadIdx.x == 0) carry_s = 0;
@@ -108,7 +110,10 @@ __global__ __launch_bounds__(1024) void bucket_offsets_kernel(const int* __restr
 __global__ __launch_bounds__(256) void bucket_scatter_kernel(const uint32_t* __restrict__ labels,
                                                              const int* __restrict__ offsets,
                                                              const int* __restrict__ ranks,
-                                                             int* __restrict__ order, int64_t n) {
+                                                             int* __restrict__ order, int64_t n,
+                                                             const kmx_lloyd_status* __restrict__ status) {
+    // (an iteration behind the end of the run: its labels may never have been written)
+    if (status->state != KMX_RUNNING) return;
     const int64_t stride = (int64_t)gridDim.x * 256;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
         order[offsets[labels[i]] + ranks[i]] = (int)i;
@@ -304,12 +309,12 @@ size_t kmx_bucket_bytes(int64_t n, int k) { return ((size_t)2 * k + 1 + 2 * (siz
 
 // offsets and order from counts and ranks (also used by the wide fp32 path)
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,
-                         int* order, int64_t n, int k, hipStream_t stream) {
-    hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, k);
+                         int* order, const kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream) {
+    hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, k, status);
     int64_t sg = kmx_cdiv(n, 256 * 4);
     if (sg > 2048) sg = 2048;
     hipLaunchKernelGGL(bucket_scatter_kernel, dim3((unsigned)sg), dim3(256), 0, stream, labels, offsets, ranks,
-                       order, n);
+                       order, n, status);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
@@ -332,7 +337,7 @@ int32_t kmx_lloyd_bucket_sums(const void* X_t, const void* X_rowmajor, const voi
     hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)cg), dim3(256), 0, stream, labels, labels_prev,
                        counts, ranks, status, n, k);
     KMX_LAUNCH_CHECK();
-    const int32_t rc = kmx_bucket_order(labels, counts, offsets, ranks, order, n, k, stream);
+    const int32_t rc = kmx_bucket_order(labels, counts, offsets, ranks, order, status, n, k, stream);
     if (rc != KMX_OK) return rc;
     // With few samples a chunk of 1024 positions per workgroup leaves most compute units without
     // one (10^5 samples: 98 workgroups): smaller chunks, down to 128 positions, and the passes over

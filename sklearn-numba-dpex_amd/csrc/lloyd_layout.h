@@ -74,7 +74,7 @@ int32_t kmx_lloyd_gemm_screen_labels(const void* X_t, const void* centroids_t, c
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,
-                         int* order, int64_t n, int k, hipStream_t stream);
+                         int* order, const kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream);
 int32_t kmx_lloyd_bucket_sums(const void* X_t, const void* X_rowmajor, const void* w,
                               const uint32_t* labels_prev, const uint32_t* labels, void* sums,
                               kmx_lloyd_status* status, char* bucket, int64_t n, int d, int k,

@@ -261,7 +261,9 @@ template <bool VEC>
 __global__ __launch_bounds__(256) void bucket_accumulate_kernel(
     const float* __restrict__ X_rm, const float* __restrict__ sample_weight,
     const int* __restrict__ order, const int* __restrict__ offsets, int* __restrict__ counts,
-    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum, int n, int d, int k) {
+    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum,
+    const kmx_lloyd_status* __restrict__ status, int n, int d, int k) {
+    if (status->state != KMX_RUNNING) return;
     __shared__ long long red[4][WIDE_D_MAX + 1];
     __shared__ int c_first;
     const int P0 = blockIdx.x * ACC_CHUNK;
@@ -466,17 +468,17 @@ int32_t kmx_lloyd_step_mfma_wide_f32(const LloydLayout& L, const void* X_t, cons
         rc = launch_wide<MODE_COUNT>(L, X_t, w, centroids_t, half_norms, labels_prev, labels, status,
                                      q_exp, gsum, counts, ranks, n, d, k, stream);
     if (rc != KMX_OK) return rc;
-    rc = kmx_bucket_order(labels, counts, offsets, ranks, order, n, k, stream);
+    rc = kmx_bucket_order(labels, counts, offsets, ranks, order, status, n, k, stream);
     if (rc != KMX_OK) return rc;
     const unsigned ag = (unsigned)kmx_cdiv(n, ACC_CHUNK);
     if (d % 4 == 0 && ((((uintptr_t)X_rowmajor) & 15) == 0))
         hipLaunchKernelGGL((bucket_accumulate_kernel<true>), dim3(ag), dim3(256), 0, stream,
                            (const float*)X_rowmajor, (const float*)w, order, offsets, counts, q_exp,
-                           gsum, (int)n, d, k);
+                           gsum, status, (int)n, d, k);
     else
         hipLaunchKernelGGL((bucket_accumulate_kernel<false>), dim3(ag), dim3(256), 0, stream,
                            (const float*)X_rowmajor, (const float*)w, order, offsets, counts, q_exp,
-                           gsum, (int)n, d, k);
+                           gsum, status, (int)n, d, k);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }

@@ -77,6 +77,42 @@ def test_runs_in_several_threads_equal_iterations_one_by_one(cuda, n, d, k, dtyp
         np.testing.assert_array_equal(r[4], expected[0][4])
 
 
+# a kernel family each; the iterations enqueued behind one that stops for a relocation find label
+# buffers that no iteration has written
+@pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
+                                         (5_000, 70, 6, np.float32), (5_003, 100, 40, np.float64), (5_003, 100, 40, np.float32),
+                                         (4_001, 128, 300, np.float32), (4_001, 14, 700, np.float32)])
+def test_iterations_behind_a_stop_leave_everything_alone(cuda, n, d, k, dtype):
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib, ptr
+
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(dtype)
+    init = X[:k].copy()
+    init[1] = 1e3  # empty at once
+    X_t, w = _dev(X.T, cuda), _dev(np.ones(n, dtype=dtype), cuda)
+    plan = _capi.lloyd_plan(n, d, k, _capi.dtype_code(X_t.dtype))
+    X_rm = _dev(X, cuda) if lib.kmx_lloyd_plan_reads_rowmajor(plan) else None
+    cent = [_dev(init.T, cuda), torch.empty(d, k, dtype=X_t.dtype, device=cuda)]
+    labels = [torch.full((n,), -16, dtype=torch.int32, device=cuda) for _ in range(2)]
+    sizes, empty = torch.empty(k, dtype=X_t.dtype, device=cuda), torch.empty(k, dtype=torch.int32, device=cuda)
+    ws, status = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=cuda), _capi.LloydStatus()
+    stream = _capi.current_stream()
+    _capi.check(lib.kmx_lloyd_init(plan, ptr(ws), plan.workspace_bytes, ptr(X_t), ptr(w), ptr(cent[0]), 9, 0.0, stream),
+                "init")
+    _capi.check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]),
+                                  ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes, 0, 9, status,
+                                  stream), "run")
+    torch.cuda.synchronize()
+    assert (status.state, status.n_iter, status.n_empty) == (_capi.KMX_NEED_RELOCATION, 0, 1)
+    assert int(empty[0]) == 1
+    assert bool((labels[0] == -16).all())
+    got = labels[1].cpu().numpy().astype(np.int64)
+    np.testing.assert_array_equal(sizes.cpu().numpy(), np.bincount(got, minlength=k))
+
+
 def _small_configs():
     return {
         "C1": lambda: datasets.config1(n=100_000),
