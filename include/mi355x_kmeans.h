@@ -208,7 +208,35 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
                       const void* sample_weight, void* centroids_even, void* centroids_odd,
                       uint32_t* labels_even, uint32_t* labels_odd, void* cluster_sizes,
                       uint32_t* empty_clusters, void* workspace, size_t workspace_bytes,
-                      int32_t n_done, int32_t max_iter, kmx_lloyd_status* status_host, void* stream);
+                      void* resident, size_t resident_bytes, int32_t n_done, int32_t max_iter,
+                      kmx_lloyd_status* status_host, void* stream);
+
+/* Samples of many features: a run that the caller gives memory for it takes its labels from a
+ * half-precision copy of X in the layout of the matrix instructions, certified per sample and
+ * resolved from the exact rows where that fails (same labels, a fraction of the bytes and of the matrix work).
+ * kmx_lloyd_resident_bytes: how much (0: the plan's kernels have no use for it).
+ * kmx_lloyd_init_resident is kmx_lloyd_init and fills, in the same pass over X_t, `resident` and the
+ * row-major copy X_rowmajor (OUT, n x d).  Both are then handed to kmx_lloyd_run, whose
+ * `resident` may be NULL (labels from X_t).  kmx_lloyd_labels_inertia ends such a run: the labels for
+ * the final centroids (centroids_t and the workspace as the run of n_iter iterations left them) and
+ * their inertia; inertia_workspace as for kmx_inertia.
+ * They have no counterpart in the reference, which computes from one layout of X in its own type
+ * (kmeans/drivers.py:146-391). */
+size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan);
+/* Squared distance of every sample to the centroid of its label among those an iteration started
+ * from (their packed copy in the workspace), for the relocation: out (n).  X_rowmajor: (n, d).
+ * Replaces the distance pass of kmeans/drivers.py:239-259. */
+int32_t kmx_lloyd_sample_distances(const kmx_lloyd_plan* plan, const void* X_rowmajor, const uint32_t* labels,
+                                   const void* workspace, void* out, void* stream);
+int32_t kmx_lloyd_init_resident(const kmx_lloyd_plan* plan, void* workspace, size_t workspace_bytes,
+                                const void* X_t, const void* sample_weight, const void* centroids_t,
+                                int32_t max_iter, double tol, void* X_rowmajor, void* resident,
+                                size_t resident_bytes, void* stream);
+int32_t kmx_lloyd_labels_inertia(const kmx_lloyd_plan* plan, const void* X_t, const void* X_rowmajor,
+                                 const void* sample_weight, const void* centroids_t, uint32_t* labels,
+                                 void* out_total, void* workspace, size_t workspace_bytes,
+                                 void* resident, size_t resident_bytes, int32_t n_iter,
+                                 void* inertia_workspace, size_t inertia_workspace_bytes, void* stream);
 
 /* Second half of (2) alone, for the iteration that stopped with KMX_NEED_RELOCATION after
  * the host has relocated the empty clusters: sums / sizes, shift, convergence test, state

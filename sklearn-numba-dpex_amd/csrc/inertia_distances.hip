@@ -109,6 +109,71 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
     }
 }
 
+// The same from the rows of a row-major copy of X and of the packed centroids: 16 lanes per sample and
+// 128-bit loads (VEC: rows of whole 16-byte groups), so that the gathered centroid is whole cache
+// lines too; lanes sum in T, the sample and the total in fp64.  Bound by reading X once.
+// per-sample values to `out` (SUM false) or the workgroup's total to `partial`.
+template <typename T, bool VEC, bool SUM>
+__global__ __launch_bounds__(256) void rows_inertia_kernel(
+    const T* __restrict__ X_rm, const T* __restrict__ sample_weight, const T* __restrict__ cpack,
+    const uint32_t* __restrict__ labels, T* __restrict__ out, double* __restrict__ partial, int64_t n, int d, int dpad) {
+    constexpr int W = VEC ? 16 / (int)sizeof(T) : 1;
+    const int e = threadIdx.x & 15;
+    const int64_t per_pass = (int64_t)gridDim.x * 32;  // two samples per group of lanes
+    double total = 0.0;
+    for (int64_t base = (int64_t)blockIdx.x * 32; base < n; base += per_pass) {
+        const int64_t i0 = base + 2 * (threadIdx.x >> 4);
+        const T* __restrict__ row[2];
+        const T* __restrict__ cen[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int64_t i = i0 + u < n ? i0 + u : n - 1;
+            row[u] = X_rm + (size_t)i * d;
+            cen[u] = cpack + (size_t)labels[i] * dpad;
+        }
+        T acc[2] = {T(0), T(0)};
+#pragma unroll 2
+        for (int f = e * W; f < d; f += 16 * W) {
+            T x[2][W], c[2][W];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                if constexpr (VEC) {
+                    using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
+                    const V xv = *reinterpret_cast<const V*>(row[u] + f), cv = *reinterpret_cast<const V*>(cen[u] + f);
+                    __builtin_memcpy(x[u], &xv, 16);
+                    __builtin_memcpy(c[u], &cv, 16);
+                } else {
+                    x[u][0] = row[u][f];
+                    c[u][0] = cen[u][f];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    const T diff = x[u][j] - c[u][j];
+                    acc[u] += diff * diff;
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            double v = (double)acc[u];
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+            if (e == 0 && i0 + u < n) {
+                if (sample_weight != nullptr) v *= (double)sample_weight[i0 + u];
+                if constexpr (SUM) total += v;
+                else out[i0 + u] = (T)v;
+            }
+        }
+    }
+    if constexpr (SUM) {
+        __shared__ double wave_part[4];
+        total = kmx_block_sum<double>(total, wave_part);
+        if (threadIdx.x == 0) partial[blockIdx.x] = total;
+    }
+}
+
 // out[0] = sum of the workgroup partials, in order.
 template <typename T>
 __global__ __launch_bounds__(256) void inertia_total_kernel(const double* __restrict__ partial, int count,
@@ -457,6 +522,46 @@ int32_t kmx_inertia(const void* X_t, const void* sample_weight, const void* cent
     return inertia_launch(X_t, sample_weight, centroids_t, labels, out_total, (double*)workspace, n, d, k, dtype,
                           (hipStream_t)stream_);
 }
+
+}  // extern "C"
+
+// (the feature-major kernel keeps its stretch of the centroids in LDS if that takes up to 48 KB)
+bool kmx_inertia_in_lds(int64_t n, int d, int k, int dtype) {
+    const int grid = stream_grid(kmx_cdiv(n, 4));
+    int64_t gy = kmx_cdiv((int64_t)kmx_num_cus() * 4, grid);
+    if (gy > d / 16) gy = d / 16;
+    if (gy < 1) gy = 1;
+    return (size_t)kmx_cdiv(d, gy) * k * kmx_dtype_size(dtype) <= 48 * 1024;
+}
+
+int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, const void* cpack, const uint32_t* labels,
+                         void* out, double* workspace, int64_t n, int d, int dpad, int dtype, hipStream_t stream) {
+    int64_t grid = kmx_cdiv(n, 32);
+    const int64_t cap = workspace != nullptr ? inertia_partial_slots(n) : 65536;
+    if (grid > 8 * (int64_t)kmx_num_cus()) grid = 8 * (int64_t)kmx_num_cus();
+    if (grid > cap) grid = cap;
+    const size_t es = kmx_dtype_size(dtype);
+    const bool vec = (size_t)d * es % 16 == 0 && (((uintptr_t)X_rowmajor) & 15) == 0 && (((uintptr_t)cpack) & 15) == 0 &&
+                     (size_t)dpad * es % 16 == 0;
+#define KMX_ROWS_INERTIA(T, V, S)                                                                                     \
+    hipLaunchKernelGGL((rows_inertia_kernel<T, V, S>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor, \
+                       (const T*)sample_weight, (const T*)cpack, labels, (S) ? nullptr : (T*)out, workspace, n, d, dpad)
+#define KMX_ROWS_INERTIA_T(T)                                                  \
+    do {                                                                       \
+        if (vec && workspace) KMX_ROWS_INERTIA(T, true, true);                 \
+        else if (vec) KMX_ROWS_INERTIA(T, true, false);                        \
+        else if (workspace) KMX_ROWS_INERTIA(T, false, true);                  \
+        else KMX_ROWS_INERTIA(T, false, false);                                \
+    } while (0)
+    if (dtype == KMX_F32) KMX_ROWS_INERTIA_T(float); else KMX_ROWS_INERTIA_T(double);
+#undef KMX_ROWS_INERTIA_T
+#undef KMX_ROWS_INERTIA
+    if (workspace != nullptr) return kmx_inertia_total_launch(workspace, (int)grid, out, dtype, stream);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
+extern "C" {
 
 int32_t kmx_euclidean_distances(const void* X_t, const void* centroids_t, void* distances_t,
                                 int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream_) {

@@ -319,6 +319,18 @@ int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets
     return KMX_OK;
 }
 
+// counts (zero on entry), ranks, and the number of changed labels
+int32_t kmx_bucket_count(const uint32_t* labels_prev, const uint32_t* labels, int* counts, int* ranks,
+                         kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream) {
+    int64_t cg = kmx_cdiv(n, BUCKET_COUNT_TILE);
+    const int64_t cap = (int64_t)8 * kmx_num_cus();
+    if (cg > cap) cg = cap;
+    hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)cg), dim3(256), 0, stream, labels, labels_prev,
+                       counts, ranks, status, n, k);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
 // After a labels-only kernel: sums[(d + 1) * k] += the weighted rows per cluster, and
 // status->n_changed.  `bucket` holds kmx_bucket_bytes; its first k words (the counts) are zero on
 // entry and on return.
@@ -331,13 +343,9 @@ int32_t kmx_lloyd_bucket_sums(const void* X_t, const void* X_rowmajor, const voi
     int* offsets = counts + k;
     int* order = offsets + (k + 1);
     int* ranks = order + n;
-    int64_t cg = kmx_cdiv(n, BUCKET_COUNT_TILE);
-    const int64_t cap = (int64_t)8 * kmx_num_cus();
-    if (cg > cap) cg = cap;
-    hipLaunchKernelGGL(bucket_count_kernel, dim3((unsigned)cg), dim3(256), 0, stream, labels, labels_prev,
-                       counts, ranks, status, n, k);
-    KMX_LAUNCH_CHECK();
-    const int32_t rc = kmx_bucket_order(labels, counts, offsets, ranks, order, status, n, k, stream);
+    int32_t rc = kmx_bucket_count(labels_prev, labels, counts, ranks, status, n, k, stream);
+    if (rc != KMX_OK) return rc;
+    rc = kmx_bucket_order(labels, counts, offsets, ranks, order, status, n, k, stream);
     if (rc != KMX_OK) return rc;
     // With few samples a chunk of 1024 positions per workgroup leaves most compute units without
     // one (10^5 samples: 98 workgroups): smaller chunks, down to 128 positions, and the passes over

@@ -97,6 +97,14 @@ __device__ __forceinline__ void stage_load_listed_f32(float4 (&r)[L], const floa
     }
 }
 
+// Number of listed samples: one word, or (count_parity >= 0) two words of which the parity of the
+// iteration says which, the given one where there is no run.
+__device__ __forceinline__ int64_t listed_count(const unsigned int* __restrict__ list_count,
+                                                const kmx_lloyd_status* __restrict__ status, int count_parity) {
+    if (count_parity < 0) return (int64_t)list_count[0];
+    return (int64_t)list_count[status != nullptr ? status->n_iter & 1 : count_parity];
+}
+
 // NA: 32-centroid row tiles per pass over the features (4: tiles of 128 centroids; 1 or 2 for
 // up to 32 / 64 clusters, where wider tiles would multiply padding).  A stage copies the 32 NA
 // centroid columns in use.  With one row tile a stage is 32 features instead of 16: the small
@@ -109,9 +117,10 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t,
     const float* __restrict__ half_norms, uint32_t* __restrict__ labels,
     const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
-    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
+    int count_parity = -1) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int64_t n_work = LISTED ? (int64_t)*list_count : n;
+    const int64_t n_work = LISTED ? listed_count(list_count, status, count_parity) : n;
     constexpr int GK = NA == 1 ? 2 * GK32 : GK32;           // features per stage
     constexpr int XL = GK / 8;                              // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                              // groups of four columns per centroid row
@@ -242,15 +251,39 @@ __device__ __forceinline__ void stage_store_f64(double (*tile)[LD], const double
     }
 }
 
+template <int L>
+__device__ __forceinline__ void stage_load_listed_f64(double2 (&r)[L], const double* __restrict__ X_t, int64_t n,
+                                                      const int (&cols)[2], int d, int f0) {
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+        const int g = threadIdx.x + 256 * l;
+        const int f = f0 + (g >> 6);
+        const bool row_ok = f < d;
+        const double* __restrict__ row = X_t + (size_t)(row_ok ? f : 0) * (size_t)n;
+        double v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const bool ok = row_ok && cols[e] >= 0;
+            const double x = row[ok ? cols[e] : 0];
+            v[e] = ok ? x : 0.0;
+        }
+        r[l] = make_double2(v[0], v[1]);
+    }
+}
+
 // NA: 16-centroid row tiles per pass (8: tiles of 128 centroids; 2 or 4 for up to 32 / 64 clusters).
 // A stage copies the 16 NA centroid columns in use; with two row tiles it is 16 features instead
 // of 8 (see the fp32 kernel).
-template <int NA>
+// LISTED: as in the fp32 kernel.
+template <int NA, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
     const double* __restrict__ X_t, const double* __restrict__ centroids_t,
     const double* __restrict__ half_norms, uint32_t* __restrict__ labels,
-    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec) {
+    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
+    int count_parity = -1) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
+    const int64_t n_work = LISTED ? listed_count(list_count, status, count_parity) : n;
     constexpr int GK = NA == 2 ? 2 * GK64 : GK64;  // features per stage
     constexpr int XL = GK / 4;                     // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                     // pairs of columns per centroid row
@@ -263,18 +296,30 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, j = lane & 15;
     const int n_stages = (d + GK - 1) / GK;
-    const int64_t n_tiles = (n + GT - 1) / GT;
+    const int64_t n_tiles = (n_work + GT - 1) / GT;
 
     for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
         const int64_t i0 = tile * GT;
         double best[2] = {-kmx_inf<double>(), -kmx_inf<double>()};
         int bidx[2] = {0, 0};
+        int cols[2];  // LISTED: the samples behind the thread's columns of a stage
+        if constexpr (LISTED) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int64_t slot = i0 + 2 * (threadIdx.x & 63) + e;
+                cols[e] = slot < n_work ? list[slot] : -1;
+            }
+        }
+        auto load_x = [&](double2(&r)[XL], const int f0) {
+            if constexpr (LISTED) stage_load_listed_f64<XL>(r, X_t, n, cols, d, f0);
+            else stage_load_f64<XL>(r, X_t, n, i0, d, f0, x_vec != 0);
+        };
         for (int c0 = 0; c0 < k; c0 += 16 * NA) {
             __syncthreads();
             if (threadIdx.x < GT)
                 hn[threadIdx.x] = c0 + (int)threadIdx.x < k ? -half_norms[c0 + threadIdx.x] : -kmx_inf<double>();
             double2 rx[XL], rc[CL];
-            stage_load_f64<XL>(rx, X_t, n, i0, d, 0, x_vec != 0);
+            load_x(rx, 0);
             stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, 0, c_vec != 0);
             stage_store_f64<XL, GLD64>(xs[0], rx);
             stage_store_f64<CL, CLD, CG>(cs[0], rc);
@@ -295,7 +340,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
             for (int st = 0; st < n_stages; ++st) {
                 const int cur = st & 1;
                 if (st + 1 < n_stages) {
-                    stage_load_f64<XL>(rx, X_t, n, i0, d, (st + 1) * GK, x_vec != 0);
+                    load_x(rx, (st + 1) * GK);
                     stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, (st + 1) * GK, c_vec != 0);
                 }
 #pragma unroll
@@ -346,8 +391,8 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
                     bidx[b] = oi;
                 }
             }
-            const int64_t i = i0 + 32 * wave + 16 * b + j;
-            if (g == 0 && i < n) labels[i] = (uint32_t)bidx[b];
+            const int64_t slot = i0 + 32 * wave + 16 * b + j;
+            if (g == 0 && slot < n_work) labels[LISTED ? (int64_t)list[slot] : slot] = (uint32_t)bidx[b];
         }
     }
 }
@@ -387,24 +432,29 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
     return KMX_OK;
 }
 
-// The fp32 kernel on the samples list[0 .. *list_count) (both on the device): what a screened
-// label kernel could not certify.  The grid covers the worst case; workgroups without a tile
-// of the list leave at once.
+// The same kernels on the samples list[0 .. count) (list and count on the device): what a screened
+// label kernel could not certify; count_parity: see listed_count.  The grid covers the worst
+// case; workgroups without a tile of the list leave at once.
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
-                                     const unsigned int* list_count, int64_t n, int d, int k,
-                                     hipStream_t stream) {
-    const int c_vec = (k % 4 == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
+                                     const unsigned int* list_count, int count_parity, int64_t n, int d, int k,
+                                     int32_t dtype, hipStream_t stream) {
+    const int c_vec = (k % (dtype == KMX_F32 ? 4 : 2) == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
     int64_t grid = kmx_cdiv(n, GT);
-    const int64_t cap = (int64_t)3 * kmx_num_cus();
+    const int64_t cap = (int64_t)(dtype == KMX_F32 ? 3 : 2) * kmx_num_cus();
     if (grid > cap) grid = cap;
-#define KMX_GEMM_LISTED(NA_)                                                                                   \
-    hipLaunchKernelGGL((lloyd_gemm_labels_f32_kernel<NA_, true>), dim3((unsigned)grid), dim3(256), 0, stream,   \
-                       (const float*)X_t, (const float*)centroids_t, (const float*)half_norms, labels, status, \
-                       n, d, k, 0, c_vec, list, list_count)
-    if (k <= 32) KMX_GEMM_LISTED(1);
-    else if (k <= 64) KMX_GEMM_LISTED(2);
-    else KMX_GEMM_LISTED(4);
+#define KMX_GEMM_LISTED(KERNEL, T)                                                                             \
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t, (const T*)centroids_t, \
+                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count, count_parity)
+    if (dtype == KMX_F32) {
+        if (k <= 32) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<1, true>), float);
+        else if (k <= 64) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<2, true>), float);
+        else KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<4, true>), float);
+    } else {
+        if (k <= 32) KMX_GEMM_LISTED((lloyd_gemm_labels_f64_kernel<2, true>), double);
+        else if (k <= 64) KMX_GEMM_LISTED((lloyd_gemm_labels_f64_kernel<4, true>), double);
+        else KMX_GEMM_LISTED((lloyd_gemm_labels_f64_kernel<8, true>), double);
+    }
 #undef KMX_GEMM_LISTED
     KMX_LAUNCH_CHECK();
     return KMX_OK;

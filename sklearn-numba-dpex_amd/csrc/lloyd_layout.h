@@ -61,8 +61,8 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
                               int32_t dtype, hipStream_t stream);
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
-                                     const unsigned int* list_count, int64_t n, int d, int k,
-                                     hipStream_t stream);
+                                     const unsigned int* list_count, int count_parity, int64_t n, int d, int k,
+                                     int32_t dtype, hipStream_t stream);
 // the same product screened on the fp16 matrix cores (lloyd_gemm_screen.hip), fp32 only
 size_t kmx_gemm_screen_bytes(int64_t n);
 bool kmx_gemm_screen_enabled(int64_t n, int d, int k, uint32_t flags);
@@ -71,10 +71,25 @@ int32_t kmx_lloyd_gemm_screen_labels(const void* X_t, const void* centroids_t, c
                                      const unsigned int* absmax, char* area, uint32_t* labels,
                                      const kmx_lloyd_status* status, int64_t n, int d, int k,
                                      hipStream_t stream);
+// labels from a half-precision copy of X kept for the run (lloyd_tiles.hip)
+bool kmx_tiles_fit(int64_t n, int d, int k);
+size_t kmx_tiles_bytes(int64_t n, int d, int k);
+int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
+                          int64_t n, int d, int k, int dtype, hipStream_t stream);
+// weighted squared distances to the own centroid from the rows of X and of the packed centroids: their
+// sum (out: one value), or per sample (out: n values, workspace null); inertia_distances.hip
+bool kmx_inertia_in_lds(int64_t n, int d, int k, int dtype);  // whether kmx_inertia has the centroids in LDS
+int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, const void* cpack, const uint32_t* labels,
+                         void* out, double* workspace, int64_t n, int d, int dpad, int dtype, hipStream_t stream);
+int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
+                         const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
+                         int d, int dpad, int k, int dtype, int parity, hipStream_t stream);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,
                          int* order, const kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream);
+int32_t kmx_bucket_count(const uint32_t* labels_prev, const uint32_t* labels, int* counts, int* ranks,
+                         kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream);
 int32_t kmx_lloyd_bucket_sums(const void* X_t, const void* X_rowmajor, const void* w,
                               const uint32_t* labels_prev, const uint32_t* labels, void* sums,
                               kmx_lloyd_status* status, char* bucket, int64_t n, int d, int k,
@@ -117,6 +132,7 @@ struct LloydLayout {
     bool screen_labels;  // KMX_VARIANT_GEMM (fp32, d <= 64): labels by the screened kernel of variant 61 without its sums
     bool direct_sums;    // with screen_labels: sums straight from the labels (fixed point in LDS) instead of per bucket
     uint32_t flags;      // the caller's KMX_FLAG_* selection
+    char* tiles = nullptr;  // the run's half-precision copy of X (lloyd_tiles.hip), or null
     unsigned long long* progress = nullptr;  // where the iterations of a run announce themselves (lloyd_publish), or null
     int wgs_per_cu;      // workgroups per compute unit asked for (0: the kernel's default)
     int cols;            // sample columns per lane asked for (0: the kernel's default)
@@ -272,8 +288,27 @@ static inline LloydLayout lloyd_layout(int64_t n, int d, int k, int dtype, uint3
     return L;
 }
 
+// Whether a run of the plan's kernels takes its labels from a half-precision copy of X where the
+// caller has memory for one (lloyd_tiles.hip): instead of the tiled product, the wide fp32 step, and
+// the fp64 step whose sums are bucketed.  The path costs two launches more per iteration (15 us) and
+// saves matrix work, so the line is drawn in products n d k.  Measured, ten iterations, without / with:
+//   fp32 tiled product: 1e5 x 200, k = 24 (4.8e8) 1.15 / 1.16 ms; 1e6 x 70, k = 30 (2.1e9) 2.64 / 2.47;
+//     4e5 x 100, k = 64 (2.6e9) 1.81 / 1.57
+//   fp32 wide step (k > 256): 2e4 x 100, k = 300 (6e8) 1.90 / 1.32; 3e5 x 256, k = 300 (2.3e10) 6.5 / 3.6
+//   fp64: 2e5 x 70, k = 20 (2.8e8) 1.15 / 1.09; 5e4 x 130, k = 40 (2.6e8) 0.97 / 0.96; 2e4 x 100, k = 300
+//     (6e8) 1.28 / 0.91; 3e5 x 256, k = 300 15.2 / 3.9
+static inline bool lloyd_tiles_wanted(const LloydLayout& L, int64_t n, int d, int k, int dtype) {
+    if ((L.flags & (KMX_FLAG_PATH_MASK | KMX_FLAG_LABELS_MASK)) != 0) return false;
+    if (L.variant != KMX_VARIANT_MFMA_WIDE && (L.acc_mode != KMX_ACC_BUCKET || L.screen_labels)) return false;
+    const double products = (double)n * d * k;
+    const double least = L.variant == KMX_VARIANT_MFMA_WIDE ? 3e8 : dtype == KMX_F32 ? 1.5e9 : 4e8;
+    return products >= least && kmx_tiles_fit(n, d, k);
+}
+
 // fp32 matrix-core implementations (lloyd_mfma.hip)
 // Fixed-point exponents from max|X_t row|, max|w| and n; clears the fixed-point sums.
+// X_t null: the words of max|X_t row| are there already (cleared by kmx_lloyd_absmax_clear, then filled)
+void kmx_lloyd_absmax_clear(const LloydLayout& L, char* ws, int d, hipStream_t stream);
 int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void* w, char* ws,
                                int64_t n, int d, int dtype, hipStream_t stream);
 int32_t kmx_lloyd_iter_mfma_f32(const LloydLayout& L, const void* X_t, const void* w,

@@ -562,21 +562,29 @@ bool kmx_mfma_supported(int d, int k) {
     return d <= 64 && k >= 16 && mfma_lds_bytes(d, k, true) <= 64 * 1024;
 }
 
+void kmx_lloyd_absmax_clear(const LloydLayout& L, char* ws, int d, hipStream_t stream) {
+    hipLaunchKernelGGL(absmax_zero_kernel, dim3(1), dim3(256), 0, stream,
+                       reinterpret_cast<unsigned int*>(ws + L.off_scales), d + 1);
+}
+
 int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void* w, char* ws,
                                int64_t n, int d, int dtype, hipStream_t stream) {
     unsigned int* absmax = reinterpret_cast<unsigned int*>(ws + L.off_scales);
     int* q_exp = reinterpret_cast<int*>(absmax + (d + 1));
-    hipLaunchKernelGGL(absmax_zero_kernel, dim3(1), dim3(256), 0, stream, absmax, d + 1);
+    if (X_t != nullptr) kmx_lloyd_absmax_clear(L, ws, d, stream);
+    // (without X_t: one row, the weights)
+    const int rows = X_t != nullptr ? d : 0;
+    unsigned int* first = absmax + (d - rows);
     int64_t gx = kmx_cdiv(n, 256 * 64);
     if (gx > 64) gx = 64;
-    if (gx * (d + 1) < 1024) gx = kmx_cdiv(1024, d + 1) < kmx_cdiv(n, 1024) ? kmx_cdiv(1024, d + 1) : kmx_cdiv(n, 1024);
+    if (gx * (rows + 1) < 1024) gx = kmx_cdiv(1024, rows + 1) < kmx_cdiv(n, 1024) ? kmx_cdiv(1024, rows + 1) : kmx_cdiv(n, 1024);
     const int vec_ok = (n % 4 == 0) && ((((uintptr_t)X_t) & 15) == 0) && ((((uintptr_t)w) & 15) == 0);
     if (dtype == KMX_F64)
-        hipLaunchKernelGGL(absmax_rows_kernel<double>, dim3((unsigned)gx, (unsigned)(d + 1)), dim3(256), 0,
-                           stream, (const double*)X_t, (const double*)w, absmax, n, d, vec_ok);
+        hipLaunchKernelGGL(absmax_rows_kernel<double>, dim3((unsigned)gx, (unsigned)(rows + 1)), dim3(256), 0,
+                           stream, (const double*)X_t, (const double*)w, first, n, rows, vec_ok);
     else
-        hipLaunchKernelGGL(absmax_rows_kernel<float>, dim3((unsigned)gx, (unsigned)(d + 1)), dim3(256), 0,
-                           stream, (const float*)X_t, (const float*)w, absmax, n, d, vec_ok);
+        hipLaunchKernelGGL(absmax_rows_kernel<float>, dim3((unsigned)gx, (unsigned)(rows + 1)), dim3(256), 0,
+                           stream, (const float*)X_t, (const float*)w, first, n, rows, vec_ok);
     hipLaunchKernelGGL(fixed_point_exponents_kernel, dim3((unsigned)kmx_cdiv(d + 1, 128)), dim3(128), 0,
                        stream, absmax, q_exp, n, d);
     const size_t words = (size_t)(d + 1) * L.k_for_gsum * 2;

@@ -65,19 +65,33 @@ def lloyd(
 
     # the wide fp32 path and the bucketed sums add up each cluster's rows from a row-major copy
     # of X (one transpose per run, n * d extra elements of HBM): whole cache lines per sample
-    X_rm = None
+    X_rm = resident = None
+    resident_bytes = lib.kmx_lloyd_resident_bytes(plan)
     reads_rowmajor = lib.kmx_lloyd_plan_reads_rowmajor(plan)
     if reads_rowmajor < 0:
         check(reads_rowmajor, "kmx_lloyd_plan_reads_rowmajor")
     if reads_rowmajor == 1:
         try:
-            X_rm = transposed_copy(X_t)
+            # ... and, for many features, a half-precision copy that the labels are screened with
+            if resident_bytes:
+                resident = torch.empty(resident_bytes, dtype=torch.uint8, device=dev)
+                X_rm = torch.empty((n, d), dtype=dt, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            X_rm = resident = None  # labels from the feature-major array (slower, same results)
+        try:
+            if X_rm is None:
+                X_rm = transposed_copy(X_t)
         except torch.cuda.OutOfMemoryError:
             X_rm = None  # the kernels then gather the feature-major array (slower, same results)
 
-    check(lib.kmx_lloyd_init(plan, ptr(ws), ws_bytes, ptr(X_t), ptr(sample_weight), ptr(cent[0]), int(max_iter),
-                             float(tol), stream),
-          "kmx_lloyd_init")
+    if resident is not None:
+        check(lib.kmx_lloyd_init_resident(plan, ptr(ws), ws_bytes, ptr(X_t), ptr(sample_weight), ptr(cent[0]),
+                                          int(max_iter), float(tol), ptr(X_rm), ptr(resident), resident_bytes, stream),
+              "kmx_lloyd_init_resident")
+    else:
+        check(lib.kmx_lloyd_init(plan, ptr(ws), ws_bytes, ptr(X_t), ptr(sample_weight), ptr(cent[0]), int(max_iter),
+                                 float(tol), stream),
+              "kmx_lloyd_init")
 
     status = LloydStatus()
     n_done, max_iter = 0, int(max_iter)
@@ -86,14 +100,20 @@ def lloyd(
         until = min(n_done + 1, max_iter) if verbose else max_iter
         check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(cent[0]), ptr(cent[1]),
                                 ptr(labels[0]), ptr(labels[1]), ptr(sizes), ptr(empty_list), ptr(ws), ws_bytes,
-                                n_done, until, status, stream), "kmx_lloyd_run")
+                                ptr(resident), resident_bytes, n_done, until, status, stream), "kmx_lloyd_run")
 
         if status.state == _capi.KMX_NEED_RELOCATION:
             j = status.n_iter  # the iteration that stopped: reads cent[j % 2], wrote sums to the other
             a, b = j % 2, (j + 1) % 2
+            sq_dist = None
+            if resident is not None and relocation == "sklearn":
+                # (from the rows, whole cache lines of sample and centroid)
+                sq_dist = torch.empty(n, dtype=dt, device=dev)
+                check(lib.kmx_lloyd_sample_distances(plan, ptr(X_rm), ptr(labels[b]), ptr(ws), ptr(sq_dist), stream),
+                      "kmx_lloyd_sample_distances")
             _relocate_empty_clusters(
                 status.n_empty, X_t, sample_weight, cent[b], sizes, labels[b], empty_list,
-                cent[a] if relocation == "sklearn" else cent[b],
+                cent[a] if relocation == "sklearn" else cent[b], sq_dist,
             )
             check(lib.kmx_lloyd_finalize(plan, ptr(cent[a]), ptr(cent[b]), ptr(sizes), ptr(ws), ws_bytes,
                                          stream), "kmx_lloyd_finalize")
@@ -121,7 +141,17 @@ def lloyd(
     # labels for the final centroids and the exact inertia (kmeans/drivers.py:356-391)
     best = cent[n_iteration % 2]
     assignments_idx = labels[0]
-    inertia = _assign_with_inertia(X_t, sample_weight, best, assignments_idx, flags)[0]
+    if resident is None:
+        inertia = _assign_with_inertia(X_t, sample_weight, best, assignments_idx, flags)[0]
+    else:
+        inertia_ws_bytes = lib.kmx_inertia_workspace_bytes(n)
+        out = torch.empty(1, dtype=dt, device=dev)
+        check(lib.kmx_lloyd_labels_inertia(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(best),
+                                           ptr(assignments_idx), ptr(out), ptr(ws), ws_bytes, ptr(resident),
+                                           resident_bytes, n_iteration,
+                                           ptr(workspace(inertia_ws_bytes, dev, tag="inertia")), inertia_ws_bytes,
+                                           stream), "kmx_lloyd_labels_inertia")
+        inertia = out.cpu().numpy()[0]
     return assignments_idx, inertia, best, n_iteration
 
 
@@ -188,6 +218,7 @@ def _relocate_empty_clusters(
     assignments_idx,
     empty_clusters_list,
     distance_centroids_t,
+    sq_dist=None,
 ):
     """Moves every empty cluster onto one of the samples farthest from its centroid
     (reference: kmeans/drivers.py:396-433 and the distance pass at :239-259).
@@ -200,7 +231,8 @@ def _relocate_empty_clusters(
     d, n = X_t.shape
     k = centroids_t.shape[1]
     # unit weights: the unweighted squared distance to the assigned centroid
-    sq_dist = _per_sample_inertia(X_t, None, distance_centroids_t, assignments_idx)
+    if sq_dist is None:
+        sq_dist = _per_sample_inertia(X_t, None, distance_centroids_t, assignments_idx)
     far = topk_idx(sq_dist, int(n_empty_clusters))
     if not float(sq_dist[far[0]]) > 0.0:
         # more clusters than distinct samples: nothing to relocate; the finalisation parks

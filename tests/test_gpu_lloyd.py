@@ -47,8 +47,8 @@ def test_runs_in_several_threads_equal_iterations_one_by_one(cuda, n, d, k, dtyp
                                            max_iter, 0.0, stream.cuda_stream), "init")
             if in_one_call:
                 _capi.check(lib.kmx_lloyd_run(plan, ptr(X_t), None, ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]),
-                                              ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes, 0,
-                                              max_iter, status, stream.cuda_stream), "run")
+                                              ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes,
+                                              None, 0, 0, max_iter, status, stream.cuda_stream), "run")
             else:
                 for it in range(max_iter):
                     a, b = it % 2, (it + 1) % 2
@@ -77,6 +77,74 @@ def test_runs_in_several_threads_equal_iterations_one_by_one(cuda, n, d, k, dtyp
         np.testing.assert_array_equal(r[4], expected[0][4])
 
 
+# every number of 16-feature steps (fp64 up to 64 features, both types beyond), one and two columns of samples per
+# wave (from 65 536 samples on), centroid tiles resident in LDS and streamed, sample counts at the edges of tiles
+# and of 128-bit loads, clusters at the edges of blocks of 32
+@pytest.mark.parametrize("n,d,k,dtype,data", [
+    (20_001, 16, 1300, np.float64, "blobs"), (20_032, 17, 1250, np.float64, "blobs"), (16_385, 48, 640, np.float64, "blobs"),
+    (16_383, 64, 513, np.float64, "blobs"), (20_001, 65, 300, np.float32, "blobs"), (20_000, 96, 257, np.float32, "blobs"),
+    (65_600, 100, 100, np.float64, "blobs"), (65_600, 112, 272, np.float32, "blobs"), (65_537, 128, 65, np.float64, "blobs"),
+    (20_063, 129, 288, np.float32, "blobs"), (20_031, 160, 1000, np.float32, "blobs"), (66_049, 161, 320, np.float32, "blobs"),
+    (20_001, 177, 200, np.float64, "blobs"), (66_001, 192, 1025, np.float32, "blobs"), (20_001, 208, 300, np.float32, "blobs"),
+    (20_001, 224, 300, np.float32, "blobs"), (65_999, 240, 500, np.float32, "blobs"), (65_543, 256, 1100, np.float32, "blobs"),
+    (20_001, 256, 130, np.float64, "blobs"), (20_001, 100, 300, np.float32, "integers"), (20_001, 100, 300, np.float64, "integers"),
+    (20_001, 100, 300, np.float32, "far"), (20_001, 100, 300, np.float64, "outliers"), (20_001, 100, 300, np.float64, "few values"),
+])
+def test_labels_from_the_half_precision_copy(cuda, n, d, k, dtype, data):
+    """Labels of a run and of its end against fp64 distances: the exact arg-min, or one whose distance is the same to
+    the rounding of one score in the input type (2 (d + 2) ulp of |x| |c|)."""
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d + k)
+    X = (rng.uniform(-2, 2, (k, d))[rng.integers(0, k, n)] + rng.standard_normal((n, d)))
+    if data == "integers":
+        X = np.round(X)
+    elif data == "few values":
+        X = X[rng.integers(0, 500, n)]  # every centroid among the samples, most of them more than once
+    elif data == "outliers":
+        X[::97] *= 1e5
+    X = X.astype(dtype)
+    init = X[rng.choice(n, k, replace=False)].copy()
+    if data == "far":
+        init[3] = 1e4
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    plan = _capi.lloyd_plan(n, d, k, _capi.dtype_code(np.dtype(dtype)), 0)
+    assert lib.kmx_lloyd_resident_bytes(plan) > 0
+    labels, inertia, centroids_t, n_iter = drivers.lloyd(_dev(X.T, cuda), _dev(w, cuda), _dev(init.T, cuda), False,
+                                                         max_iter=2, tol=0.0, flags=0)
+    x, c = _dev(X, cuda).double(), centroids_t.double()
+    half = (c * c).sum(0) / 2
+    lab = labels.long()
+    assert int(lab.min()) >= 0 and int(lab.max()) < k
+    ulp = float(np.finfo(dtype).eps)
+    own, total = torch.empty(n, dtype=torch.float64, device=cuda), 0.0
+    for lo in range(0, n, 8192):
+        hi = min(n, lo + 8192)
+        scores = half[None] - x[lo:hi] @ c.contiguous()
+        mine = scores.gather(1, lab[lo:hi, None])[:, 0]
+        allowed = 2 * (d + 2) * ulp * (x[lo:hi].norm(dim=1) * c.norm(dim=0).max() + half.max())
+        assert bool((mine - scores.min(1).values <= allowed).all())
+        own[lo:hi] = ((x[lo:hi] - c.T[lab[lo:hi]]) ** 2).sum(1)
+    expected = float((own * _dev(w, cuda).double()).sum())
+    np.testing.assert_allclose(float(inertia), expected, rtol=1e-5 if dtype == np.float32 else 1e-12)
+    # the first iteration's labels and sums, through the centroids of a run of one iteration
+    labels1, _, first_t, n_iter = drivers.lloyd(_dev(X.T, cuda), _dev(w, cuda), _dev(init.T, cuda), False, max_iter=1,
+                                                tol=0.0, flags=0)
+    if data in ("blobs", "outliers"):
+        d2 = [((x[lo:lo + 8192] @ _dev(init.T, cuda).double()) - (_dev(init, cuda).double() ** 2).sum(1) / 2).argmax(1)
+              for lo in range(0, n, 8192)]
+        start = torch.cat(d2)
+        weights = torch.zeros(k, dtype=torch.float64, device=cuda).index_add_(0, start, _dev(w, cuda).double())
+        sums = torch.zeros(k, d, dtype=torch.float64, device=cuda).index_add_(0, start, x * _dev(w, cuda).double()[:, None])
+        full = weights > 0
+        err = (first_t.T.double() - sums / weights[:, None])[full].abs().max() / sums[full].div(weights[full, None]).abs().max()
+        assert float(err) <= (2e-5 if dtype == np.float32 else 1e-11)
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
@@ -103,8 +171,8 @@ def test_iterations_behind_a_stop_leave_everything_alone(cuda, n, d, k, dtype):
     _capi.check(lib.kmx_lloyd_init(plan, ptr(ws), plan.workspace_bytes, ptr(X_t), ptr(w), ptr(cent[0]), 9, 0.0, stream),
                 "init")
     _capi.check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]),
-                                  ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes, 0, 9, status,
-                                  stream), "run")
+                                  ptr(labels[1]), ptr(sizes), ptr(empty), ptr(ws), plan.workspace_bytes, None, 0, 0, 9,
+                                  status, stream), "run")
     torch.cuda.synchronize()
     assert (status.state, status.n_iter, status.n_empty) == (_capi.KMX_NEED_RELOCATION, 0, 1)
     assert int(empty[0]) == 1
