@@ -484,6 +484,16 @@ int32_t kmx_broadcast_div_cols(void* a, const void* v, int64_t rows, int64_t col
 int32_t kmx_transpose(const void* src, void* dst, int64_t rows, int64_t cols, int32_t dtype,
                       void* stream);
 
+/* kmx_transpose, and *not_finite (device) = 1 if src holds a NaN or an infinity, else 0.  The check
+ * of the input that the reference leaves to scikit-learn's check_array on the host
+ * (kmeans/engine.py:293-302), taken while the values pass through. */
+int32_t kmx_transpose_finite(const void* src, void* dst, int64_t rows, int64_t cols,
+                             int32_t* not_finite, int32_t dtype, void* stream);
+
+/* *not_finite (device) = 1 if one of the n_items values is a NaN or an infinity, else 0. */
+int32_t kmx_all_finite(const void* data, int64_t n_items, int32_t* not_finite, int32_t dtype,
+                       void* stream);
+
 /* data[i] = data[i] / divisor.  make_apply_elementwise_func with _divide_by,
  * common/kernels.py:11-36, common/_utils.py:17-33. */
 int32_t kmx_divide_by(void* data, int64_t n_items, double divisor, int32_t dtype, void* stream);

@@ -47,15 +47,28 @@ def divide_by(data, divisor):
           "kmx_divide_by")
 
 
-def transposed_copy(array):
+def transposed_copy(array, not_finite=None):
     """A C-contiguous copy of array.T for a C-contiguous 2-d fp32 / fp64 array (the reference
-    leaves these copies to the array library: kmeans/engine.py:88-98)."""
+    leaves these copies to the array library: kmeans/engine.py:88-98).  `not_finite`, an int32
+    tensor of one element, is set to whether the array holds a NaN or an infinity."""
     _require_contiguous(array)
     rows, cols = array.shape
     out = torch.empty((cols, rows), dtype=array.dtype, device=array.device)
-    check(lib.kmx_transpose(ptr(array), ptr(out), rows, cols, dcode(array), _capi.current_stream()),
-          "kmx_transpose")
+    if not_finite is None:
+        check(lib.kmx_transpose(ptr(array), ptr(out), rows, cols, dcode(array), _capi.current_stream()),
+              "kmx_transpose")
+    else:
+        check(lib.kmx_transpose_finite(ptr(array), ptr(out), rows, cols, ptr(not_finite), dcode(array),
+                                       _capi.current_stream()), "kmx_transpose_finite")
     return out
+
+
+def all_finite(array, not_finite):
+    """Sets `not_finite`, an int32 tensor of one element, to whether the array holds a NaN or an
+    infinity."""
+    _require_contiguous(array)
+    check(lib.kmx_all_finite(ptr(array), array.numel(), ptr(not_finite), dcode(array), _capi.current_stream()),
+          "kmx_all_finite")
 
 
 def initialize_to_zeros(data):

@@ -369,35 +369,147 @@ int sum_blocks_per_row(int64_t cols) {
 }
 
 
-// dst (cols x rows) = transpose of src (rows x cols), 64 x 64 tiles through LDS (rows padded
-// by one word: the transposed reads fall on distinct banks); both sides move whole segments.
-// One workgroup per tile, tiles numbered along the columns first.
+// Whether a value is a NaN or an infinity: all bits of the exponent set.
+__device__ __forceinline__ bool kmx_not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+__device__ __forceinline__ bool kmx_not_finite(double v) {
+    return ((unsigned)(__double_as_longlong(v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
+}
+
+// The elements of a transposed tile that fit its LDS (33 KB: four workgroups' tiles and their
+// loads are in flight on a compute unit).
 template <typename T>
+constexpr int TRANSPOSE_LDS = 33792 / (int)sizeof(T);
+constexpr int TRANSPOSE_XCDS = 8;
+
+// dst (cols x rows) = transpose of src (rows x cols), through LDS.  Bound by memory.  A tile is
+// tall (up to 1 KB of a row of dst) and narrow (about 32 columns): dst's rows start at any
+// address, and long runs leave few cache lines that two tiles share.  Tiles are numbered along
+// the columns and handed out to the XCDs in contiguous ranges, so the lines that neighbours share
+// meet in one L2.  Both sides walk the tile flat, every lane with an element, eight loads in flight
+// per lane; an odd pitch spreads the transposed stores over the banks.
+// 70 000 x 784 fp32 106 -> 87 us (5.0 TB/s); 300 007 x 100 fp32 82 -> 59 us (4.0 TB/s), both with the
+// check, from tiles of 64 x 64 without it.
+// CHECK: *not_finite = 1 if an element is a NaN or an infinity (any number of equal stores).
+template <typename T, bool CHECK>
 __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                        int64_t rows, int64_t cols, int64_t tiles_c) {
-    __shared__ T tile[64][65];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int64_t r0 = ((int64_t)blockIdx.x / tiles_c) * 64, c0 = ((int64_t)blockIdx.x % tiles_c) * 64;
-    const int nr = rows - r0 < 64 ? (int)(rows - r0) : 64, nc = cols - c0 < 64 ? (int)(cols - c0) : 64;
-    if (cols <= 64) {
-        // narrow source: the tile's rows are one contiguous run of nr * cols elements
-        const T* __restrict__ run = src + (size_t)r0 * cols;
-        for (int e = threadIdx.x; e < nr * (int)cols; e += 256) tile[e / (int)cols][e % (int)cols] = run[e];
-    } else {
-#pragma unroll 4
-        for (int i = ty; i < 64; i += 4)
-            if (i < nr && tx < nc) tile[i][tx] = src[(size_t)(r0 + i) * cols + c0 + tx];
+                                                        int64_t rows, int64_t cols, int tile_r, int tile_c,
+                                                        int64_t tiles_c, int64_t tiles, int64_t per_xcd,
+                                                        int32_t* __restrict__ not_finite) {
+    __shared__ T tile[TRANSPOSE_LDS<T>];
+    const int64_t t = (int64_t)(blockIdx.x % TRANSPOSE_XCDS) * per_xcd + blockIdx.x / TRANSPOSE_XCDS;
+    if (t >= tiles) return;
+    const int64_t r0 = t / tiles_c * tile_r, c0 = t % tiles_c * tile_c;
+    const int nr = rows - r0 < tile_r ? (int)(rows - r0) : tile_r;
+    const int nc = cols - c0 < tile_c ? (int)(cols - c0) : tile_c;
+    const int pitch = tile_r | 1;
+    constexpr int B = 8;
+    bool bad = false;
+    {
+        const T* __restrict__ from = src + (size_t)r0 * cols + c0;
+        const int step_r = 256 / nc, step_c = 256 % nc;
+        int r = (int)threadIdx.x / nc, c = (int)threadIdx.x % nc;
+        for (int e0 = 0; e0 < nr * nc; e0 += 256 * B) {
+            T v[B];
+            int at[B];
+#pragma unroll
+            for (int i = 0; i < B; ++i) {
+                const int rc = r < nr ? r : nr - 1;  // past the end: a valid element, not kept
+                v[i] = from[(size_t)rc * cols + c];
+                at[i] = r < nr ? c * pitch + r : -1;
+                r += step_r;
+                c += step_c;
+                if (c >= nc) {
+                    c -= nc;
+                    ++r;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < B; ++i) {
+                if (CHECK) bad |= kmx_not_finite(v[i]);
+                if (at[i] >= 0) tile[at[i]] = v[i];
+            }
+        }
     }
+    if (CHECK && bad) *not_finite = 1;
     __syncthreads();
-    if (rows <= 64) {
-        // narrow result: the tile's columns are one contiguous run of nc * rows elements
-        T* __restrict__ run = dst + (size_t)c0 * rows;
-        for (int e = threadIdx.x; e < nc * (int)rows; e += 256) run[e] = tile[e % (int)rows][e / (int)rows];
-    } else {
+    T* __restrict__ to = dst + (size_t)c0 * rows + r0;
+    const int step_c = 256 / nr, step_r = 256 % nr;
+    int c = (int)threadIdx.x / nr, r = (int)threadIdx.x % nr;
 #pragma unroll 4
-        for (int i = ty; i < 64; i += 4)
-            if (i < nc && tx < nr) dst[(size_t)(c0 + i) * rows + r0 + tx] = tile[tx][i];
+    for (int e = threadIdx.x; e < nr * nc; e += 256) {
+        to[(size_t)c * rows + r] = tile[c * pitch + r];
+        c += step_c;
+        r += step_r;
+        if (r >= nr) {
+            r -= nr;
+            ++c;
+        }
     }
+}
+
+// *not_finite = 1 if one of the n values is a NaN or an infinity.  One read at memory speed;
+// VEC: 16 bytes a load (aligned arrays).
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void all_finite_kernel(const T* __restrict__ a, int64_t n,
+                                                         int32_t* __restrict__ not_finite) {
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    bool bad = false;
+    int64_t done = 0;
+    if constexpr (VEC) {
+        constexpr int V = 16 / sizeof(T);
+        struct alignas(16) Quad { T v[V]; };
+        const Quad* __restrict__ q = reinterpret_cast<const Quad*>(a);
+        const int64_t nq = n / V;
+#pragma unroll 4
+        for (int64_t i = id; i < nq; i += stride) {
+            const Quad x = q[i];
+#pragma unroll
+            for (int j = 0; j < V; ++j) bad |= kmx_not_finite(x.v[j]);
+        }
+        done = nq * V;
+    }
+    for (int64_t i = done + id; i < n; i += stride) bad |= kmx_not_finite(a[i]);
+    if (bad) *not_finite = 1;
+}
+
+// Tile of the transposed copy: up to 1 KB of a dst row (2 KB where src has at most 16 columns, or a
+// tile would be a few elements per lane), and the columns that then fit the LDS, evenly split.
+template <typename T>
+void launch_transpose(const void* src, void* dst, int64_t rows, int64_t cols, int32_t* not_finite, hipStream_t s) {
+    const int64_t most_r = (cols <= 16 ? 2048 : 1024) / (int64_t)sizeof(T);
+    const int tile_r = (int)(rows < most_r ? rows : most_r);
+    const int64_t fit_c = TRANSPOSE_LDS<T> / (tile_r | 1);
+    const int64_t tiles_c = kmx_cdiv(cols, fit_c);
+    const int tile_c = (int)kmx_cdiv(cols, tiles_c);
+    const int64_t used_c = kmx_cdiv(cols, tile_c);
+    const int64_t tiles = used_c * kmx_cdiv(rows, tile_r), per_xcd = kmx_cdiv(tiles, TRANSPOSE_XCDS);
+    const dim3 grid((unsigned)(per_xcd * TRANSPOSE_XCDS));
+    if (not_finite)
+        hipLaunchKernelGGL((transpose_kernel<T, true>), grid, dim3(256), 0, s, (const T*)src, (T*)dst, rows, cols,
+                           tile_r, tile_c, used_c, tiles, per_xcd, not_finite);
+    else
+        hipLaunchKernelGGL((transpose_kernel<T, false>), grid, dim3(256), 0, s, (const T*)src, (T*)dst, rows, cols,
+                           tile_r, tile_c, used_c, tiles, per_xcd, not_finite);
+}
+
+int32_t transpose_copy(const void* src, void* dst, int64_t rows, int64_t cols, int32_t* not_finite, int32_t dtype,
+                       hipStream_t stream) {
+    KMX_REQUIRE_PTR(src);
+    KMX_REQUIRE_PTR(dst);
+    if (rows <= 0 || cols <= 0) return KMX_ERR_BAD_SHAPE;
+    KMX_REQUIRE_DTYPE(dtype);
+    if (src == dst) return KMX_ERR_BAD_ARGUMENT;
+    if (kmx_cdiv(cols, 64) * kmx_cdiv(rows, 64) > INT32_MAX) return KMX_ERR_BAD_SHAPE;
+    if (not_finite)
+        hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(256), 0, stream, not_finite, (int64_t)1, 0,
+                           (int32_t*)nullptr, 0);
+    if (dtype == KMX_F32)
+        launch_transpose<float>(src, dst, rows, cols, not_finite, stream);
+    else
+        launch_transpose<double>(src, dst, rows, cols, not_finite, stream);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
 }
 
 }  // namespace
@@ -572,22 +684,39 @@ int32_t kmx_half_sq_norms(const void* a_t, void* out, int32_t rows, int32_t cols
     return KMX_OK;
 }
 
-int32_t kmx_transpose(const void* src, void* dst, int64_t rows, int64_t cols, int32_t dtype, void* stream_) {
+int32_t kmx_transpose(const void* src, void* dst, int64_t rows, int64_t cols, int32_t dtype, void* stream) {
     KMX_ENTRY();
-    KMX_REQUIRE_PTR(src);
-    KMX_REQUIRE_PTR(dst);
-    if (rows <= 0 || cols <= 0) return KMX_ERR_BAD_SHAPE;
+    return transpose_copy(src, dst, rows, cols, nullptr, dtype, (hipStream_t)stream);
+}
+
+int32_t kmx_transpose_finite(const void* src, void* dst, int64_t rows, int64_t cols, int32_t* not_finite,
+                             int32_t dtype, void* stream) {
+    KMX_ENTRY();
+    KMX_REQUIRE_PTR(not_finite);
+    return transpose_copy(src, dst, rows, cols, not_finite, dtype, (hipStream_t)stream);
+}
+
+int32_t kmx_all_finite(const void* data, int64_t n_items, int32_t* not_finite, int32_t dtype, void* stream_) {
+    KMX_ENTRY();
+    KMX_REQUIRE_PTR(data);
+    KMX_REQUIRE_PTR(not_finite);
+    if (n_items <= 0) return KMX_ERR_BAD_SHAPE;
     KMX_REQUIRE_DTYPE(dtype);
-    if (src == dst) return KMX_ERR_BAD_ARGUMENT;
-    const int64_t tiles_c = kmx_cdiv(cols, 64), tiles = tiles_c * kmx_cdiv(rows, 64);
-    if (tiles > INT32_MAX) return KMX_ERR_BAD_SHAPE;
     hipStream_t stream = (hipStream_t)stream_;
-    if (dtype == KMX_F32)
-        hipLaunchKernelGGL((transpose_kernel<float>), dim3((unsigned)tiles), dim3(256), 0, stream,
-                           (const float*)src, (float*)dst, rows, cols, tiles_c);
-    else
-        hipLaunchKernelGGL((transpose_kernel<double>), dim3((unsigned)tiles), dim3(256), 0, stream,
-                           (const double*)src, (double*)dst, rows, cols, tiles_c);
+    hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(256), 0, stream, not_finite, (int64_t)1, 0, (int32_t*)nullptr, 0);
+    // (four loads of 16 bytes per thread, at most eight workgroups a compute unit)
+    int64_t blocks = kmx_cdiv(n_items * (int64_t)kmx_dtype_size(dtype), 256 * 64);
+    if (blocks > 8 * kmx_num_cus()) blocks = 8 * kmx_num_cus();
+    const bool vec = (uintptr_t)data % 16 == 0;
+#define KMX_FINITE(T, VEC)                                                                               \
+    hipLaunchKernelGGL((all_finite_kernel<T, VEC>), dim3((unsigned)blocks), dim3(256), 0, stream, (const T*)data, \
+                       n_items, not_finite)
+    if (dtype == KMX_F32) {
+        if (vec) KMX_FINITE(float, true); else KMX_FINITE(float, false);
+    } else {
+        if (vec) KMX_FINITE(double, true); else KMX_FINITE(double, false);
+    }
+#undef KMX_FINITE
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }

@@ -37,7 +37,7 @@ except ImportError:  # stock scikit-learn
 
 
 from ..common._buffers import require_cuda, upload
-from ..common.kernels import transposed_copy
+from ..common.kernels import all_finite, transposed_copy
 from .drivers import (
     get_euclidean_distances,
     get_labels_inertia,
@@ -236,15 +236,13 @@ class KMeansEngine(_EngineBase):
             return array.to(device=self.device, dtype=dtype)
         return torch.as_tensor(np.asarray(array), device=self.device).to(dtype)
 
-    def _assert_all_finite(self, X_t, X_host):
+    def _assert_all_finite(self, not_finite, X_t, X_host):
         """scikit-learn's check of the input (check_array(ensure_all_finite=True), as the
-        reference's engine runs it: kmeans/engine.py:293-302), taken on the device: one pass at
-        memory speed instead of a single-threaded host pass that costs more than the upload.
-        Non-finite data then get scikit-learn's own error from the host copy.  As in
-        scikit-learn, the sum goes first (one read, nothing written): a NaN or an infinity
-        anywhere makes it non-finite, and so may an overflow of finite values, which the
-        element-wise test then clears."""
-        if bool(torch.isfinite(X_t.sum())) or bool(torch.isfinite(X_t).all()):
+        reference's engine runs it: kmeans/engine.py:293-302), taken on the device: the values
+        were looked at when they were transposed (or in one read of their own) instead of in a
+        single-threaded host pass that costs more than the upload.  Non-finite data then get
+        scikit-learn's own error from the host copy."""
+        if not int(not_finite):
             return
         from sklearn.utils.validation import _assert_all_finite
 
@@ -276,10 +274,15 @@ class KMeansEngine(_EngineBase):
             # (d, n) contiguous; already the case for an F-ordered tensor
             X_t = X_dev.T
             owns_copy = X_dev.data_ptr() != X.data_ptr()
-            if not X_t.is_contiguous():
-                X_t = transposed_copy(X_dev) if X_dev.is_contiguous() else X_t.contiguous()
+            not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
+            if X_dev.is_contiguous() and not X_t.is_contiguous():
+                X_t = transposed_copy(X_dev, not_finite)
                 owns_copy = True
-            self._assert_all_finite(X_t, None)
+            else:
+                owns_copy = owns_copy or not X_t.is_contiguous()
+                X_t = X_t.contiguous()
+                all_finite(X_t, not_finite)
+            self._assert_all_finite(not_finite, X_t, None)
         else:
             owns_copy = True  # the upload below is this engine's own device copy
             X_np = check_array(
@@ -296,8 +299,12 @@ class KMeansEngine(_EngineBase):
             # upload, then transpose on the device: (d, n) contiguous
             # (through pinned staging buffers when the array is large)
             X_t = upload(np.ascontiguousarray(X_np.T) if X_np.flags.f_contiguous else X_np, self.device)
-            X_t = X_t if X_np.flags.f_contiguous else transposed_copy(X_t)
-            self._assert_all_finite(X_t, X_np)
+            not_finite = torch.empty(1, dtype=torch.int32, device=X_t.device)
+            if X_np.flags.f_contiguous:
+                all_finite(X_t, not_finite)
+            else:
+                X_t = transposed_copy(X_t, not_finite)
+            self._assert_all_finite(not_finite, X_t, X_np)
 
         # prepare_fit centres the data in place when this buffer is not the caller's (or copy_x is off)
         self._owns_X = owns_copy

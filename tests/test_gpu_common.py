@@ -392,3 +392,28 @@ def test_transposed_copy(cuda, shape, dtype):
     got = transposed_copy(_dev(a, cuda))
     assert got.is_contiguous() and tuple(got.shape) == (shape[1], shape[0])
     np.testing.assert_array_equal(got.cpu().numpy(), a.T)
+
+
+# (one value, one tile, tiles with remainders on both sides, few long rows, few columns, a start
+# that is not aligned to 16 bytes)
+@pytest.mark.parametrize("shape, skip", [((1, 1), 0), ((256, 32), 0), ((257, 33), 1), ((3, 20_001), 0), ((5_003, 14), 1),
+                                         ((1_025, 129), 0)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_not_finite_values_are_seen(cuda, shape, skip, dtype):
+    import torch
+
+    from sklearn_numba_dpex_amd.common.kernels import all_finite, transposed_copy
+
+    n = shape[0] * shape[1]
+    a = _dev(np.full(n + skip, np.finfo(dtype).max, dtype), cuda)[skip:].reshape(shape)
+    a.view(-1)[::2] = -float(np.finfo(dtype).max)
+    flag = torch.full((1,), 7, dtype=torch.int32, device=cuda)
+    for at in sorted({0, n // 2, n - 1}):
+        for value, expected in [(np.nan, 1), (np.inf, 1), (-np.inf, 1), (0.0, 0)]:
+            a.view(-1)[at] = value
+            all_finite(a, flag)
+            assert int(flag) == expected
+            flag.fill_(7)
+            got = transposed_copy(a, flag)
+            assert int(flag) == expected
+            np.testing.assert_array_equal(got.cpu().numpy(), a.cpu().numpy().T)
