@@ -372,6 +372,10 @@ int32_t kmx_rng_next_raw(uint64_t* states, int32_t n_states, int32_t n_steps, ui
 
 size_t kmx_kpp_workspace_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials, int32_t dtype);
 
+/* Bytes beyond kmx_kpp_workspace_bytes that kmx_kpp_run makes use of where the workspace has them (0:
+ * none): copies of X that its later steps read in place of X itself.  The results are the same. */
+size_t kmx_kpp_screen_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials, int32_t dtype);
+
 /* closest[i] = w_i ||x_i - x_start||^2, centers_t[:, 0] = x_start, center_indices[0] = start,
  * and the per-block partial potentials.  Replaces make_kmeansplusplus_init_kernel
  * (kmeans/kernels/kmeans_plusplus.py:16-58) + the potential reduction (kmeans/drivers.py:844). */

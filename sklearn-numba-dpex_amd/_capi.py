@@ -139,6 +139,7 @@ SIGNATURES = {
     "kmx_rng_init_states": (_I32, [ctypes.c_uint64, _I32, _I32, _P]),
     "kmx_rng_next_raw": (_I32, [_P, _I32, _I32, _P]),
     "kmx_kpp_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32]),
+    "kmx_kpp_screen_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32]),
     "kmx_kpp_init": (_I32, [_P, _P, _I32, _P, _P, _P, _SZ, _I64, _I32, _I32, _I32, _I32, _U32, _P]),
     "kmx_kpp_sample_candidates": (_I32, [_P, _P, _P, _P, _SZ, _I64, _I32, _I32, _I32, _I32, _U32, _P]),
     "kmx_kpp_step": (_I32, [_P, _P, _I32, _P, _P, _P, _SZ, _I64, _I32, _I32, _I32, _I32, _U32, _P]),

@@ -17,7 +17,7 @@
 // Per new centre: [select previous best + sample candidates] then [step].  The sampler is a
 // search in the fp64 inclusive scan of `closest`: coarse over the block sums, fine inside one
 // block of 1024 samples, so it never re-reads the whole array.
-#include "kmx_common.h"
+#include "lloyd_layout.h"
 
 #include <type_traits>
 
@@ -25,6 +25,14 @@ namespace {
 
 constexpr int TN_MAX = 16;      // n_local_trials = 2 + floor(ln k) <= 16 for k < 1.2e6
 constexpr int CHUNK = 1024;     // samples per workgroup (256 threads x 4)
+// Screened steps (kpp_screen_step_kernel): from these sizes on.  The copies they read cost about two
+// plain steps, and a step still writes all its rows: with few features there is little to save.
+// Measured, whole seedings, plain / screened steps: fp32 1e6 x 32, 128 centres 5.3 / 6.1 ms; 3e5 x 64,
+// 32 centres 1.35 / 1.22; 1e6 x 64, 256 centres 15.9 / 15.4; 1 000 003 x 64 (unaligned rows) 23.6 / 16.1;
+// 4e5 x 255, 100 centres 10.9 / 8.1; fp64 1e6 x 16, 128 centres 5.5 / 7.2; 5e5 x 50, 100 centres 5.0 / 5.0;
+// 5e5 x 64, 200 centres 11.5 / 9.4; 3e5 x 128, 64 centres 6.0 / 5.1.
+constexpr int64_t SCREEN_MIN_N = 1 << 17;
+constexpr int SCREEN_MIN_K = 32, SCREEN_MIN_D = 64;
 constexpr int SPLIT_MIN_D = 64; // from this many features on, few samples are stepped with the
                                 // features split over the four waves of a workgroup
 
@@ -155,6 +163,43 @@ struct KppCandBatch {
     __device__ __forceinline__ T get(int t, int j) const { return kpp_readlane<T>(v[t / TPL], (t % TPL) * FB + j); }
 };
 
+// The end of a step for a workgroup's 1 024 samples: `value` yields the new closest distances of four
+// samples (4 q .. 4 q + 3, q = thread % 256) for a trial; they go to its row, and their sum over the
+// workgroup to the block sums.  HALVES = 2: 512 threads, whose halves take every other trial.
+template <typename T, int TN, int HALVES, bool full, typename V>
+__device__ __forceinline__ void kpp_finish_block(T* __restrict__ rows, double* __restrict__ block_pot,
+                                                 double (*wave_pot)[TN], int64_t i0, int64_t n, int n_trials,
+                                                 V&& value) {
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+    const int half = HALVES == 1 ? 0 : (int)(threadIdx.x >> 8);
+    double pot[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        pot[t] = 0.0;
+        if (t < n_trials && t % HALVES == half) {
+            T v[4];
+            value(t, v);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (i0 + r < n) pot[t] += (double)v[r];
+            store4<T>(rows + (size_t)t * n, i0, n, full, v);
+        }
+    }
+    // all row sums of the workgroup with one barrier: waves first, then one thread per trial
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        if (t < n_trials && t % HALVES == half) {
+            const double ws = kmx_wave_sum<double>(pot[t]);
+            if (lane == 0) wave_pot[wave][t] = ws;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < n_trials)
+        block_pot[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
+            (wave_pot[0][threadIdx.x] + wave_pot[1][threadIdx.x]) +
+            (wave_pot[2][threadIdx.x] + wave_pot[3][threadIdx.x]);
+}
+
 // rows[t, i] = min(w_i * ||x_i - x_cand_t||^2, closest_i) and per-block row sums.
 // Candidate rows come from a small (TN, d) buffer, a batch of features at a time spread over
 // the lanes and read back as scalars (no LDS, no barriers in the feature loop); every thread
@@ -168,9 +213,9 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
     int64_t n, int d, int k, int n_trials, int vec_ok, int32_t start, T* __restrict__ centers_t,
     int32_t* __restrict__ center_indices) {
     __shared__ double wave_pot[4][TN];
-    const int64_t i0 = (int64_t)blockIdx.x * CHUNK + threadIdx.x * 4;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int best = INIT ? 0 : header->best_row;
+    const int64_t i0 = (int64_t)blockIdx.x * CHUNK + threadIdx.x * 4;
+    const int lane = threadIdx.x & 63;
     // Whether the 128-bit accesses are legal is decided once per workgroup and known at compile
     // time inside the body: with a test per access every load sat in a branch of its own and
     // was waited for before the next one was issued.
@@ -234,34 +279,13 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
             accumulate(std::false_type{});
     }
 
-    double pot[TN];
+    kpp_finish_block<T, TN, 1, full>(rows, block_pot, wave_pot, i0, n, n_trials, [&](int t, T (&v)[4]) {
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        pot[t] = 0.0;
-        if (t < n_trials) {
-            T v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                v[r] = acc[t][r] * w[r];
-                if constexpr (!INIT) v[r] = fmin(v[r], cl[r]);
-                if (i0 + r < n) pot[t] += (double)v[r];
-            }
-            store4<T>(rows + (size_t)t * n, i0, n, full, v);
+        for (int r = 0; r < 4; ++r) {
+            v[r] = acc[t][r] * w[r];
+            if constexpr (!INIT) v[r] = fmin(v[r], cl[r]);
         }
-    }
-    // all row sums of the workgroup with one barrier: waves first, then one thread per trial
-#pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        if (t < n_trials) {
-            const double ws = kmx_wave_sum<double>(pot[t]);
-            if (lane == 0) wave_pot[wave][t] = ws;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < n_trials)
-        block_pot[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
-            (wave_pot[0][threadIdx.x] + wave_pot[1][threadIdx.x]) +
-            (wave_pot[2][threadIdx.x] + wave_pot[3][threadIdx.x]);
+    });
     };
     if (vec_ok && (int64_t)(blockIdx.x + 1) * CHUNK <= n)
         body(std::true_type{});
@@ -275,6 +299,243 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
             header->total = 0.0;
         }
     }
+}
+
+
+// ---------------------------------------------------------------- screened step
+//
+// Most candidates are nearer than the closest centre so far for few samples: one in c + 1 for c
+// centres already there, and fewer where the data have clusters.  For the rest the new closest
+// distance is the old one, and a lower bound of the candidate's distance shows it: the samples'
+// half-precision tiles (lloyd_tiles.hip; a candidate's row is read from them as well) give all of a
+// workgroup's distances with matrix instructions at 2 bytes per value,
+//     D >= sqrt(|x'|^2 + |c'|^2 - 2 <x', c'> - slack) - |e_x| - |e_c|
+// (primes: rounded, e: what rounding took, known per sample; slack: fp32 accumulation).  The pairs
+// that it does not settle are gathered and their distances taken from the row-major copy exactly
+// as the plain step takes them (features in order, one fused multiply-add each): rows, block sums
+// and therefore candidates are those of the plain step, bit for bit.  A workgroup with more than
+// SCREEN_QUEUE of its 1 024 x trials pairs unsettled takes all of them from X.
+constexpr int SCREEN_TN = 8;         // trials: accumulator registers 0 .. 3 of both halves of a wave
+constexpr int SCREEN_FROM = 8;       // centres before the first screened step
+constexpr int SCREEN_QUEUE = 1792;
+constexpr int SCREEN_PITCH = CHUNK + 16;
+constexpr float SCREEN_ULP = 1.1920929e-7f;  // 2^-23
+
+typedef float kpp_v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 kpp_v8h __attribute__((ext_vector_type(8)));
+
+template <typename T>
+size_t screen_lds(int d, int S) {
+    return (size_t)S * 1024 + SCREEN_TN * (SCREEN_PITCH + (size_t)((d + 3) & ~3)) * sizeof(T) +
+           SCREEN_QUEUE * sizeof(uint16_t);
+}
+
+// Eight waves, four tiles of 32 samples each: a wave's tiles travel as items of four steps of 16
+// features, four items in flight from the first instruction on (nothing they need depends on the
+// candidates).  Bound by memory and, with one or two rounds of workgroups, by the phases that a
+// workgroup goes through one after the other: 49 us at 1e6 x 64 (168 MB) where the plain step
+// takes 52 (284 MB at 5.5 TB/s); registers for four waves per SIMD, LDS for two workgroups.
+template <typename T>
+__global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
+    const T* __restrict__ X_t, const T* __restrict__ X_rm, KmxTiles tiles, const T* __restrict__ sample_weight,
+    const int32_t* __restrict__ cand, const T* __restrict__ cand_rows, T* __restrict__ rows,
+    double* __restrict__ block_pot, const KppHeader* __restrict__ header, int64_t n, int d, int n_trials, int vec_ok,
+    int row_vec) {
+    extern __shared__ __align__(16) unsigned char screen_smem[];
+    __shared__ double wave_pot[4][SCREEN_TN];
+    __shared__ int queued_s;
+    const int S = tiles.S, dp = (d + 3) & ~3;
+    uint4* a_s = reinterpret_cast<uint4*>(screen_smem);       // the candidates' fragments, S x 64
+    T* v_s = reinterpret_cast<T*>(a_s + S * 64);              // new closest distances, trials x SCREEN_PITCH
+    T* cand_s = v_s + SCREEN_TN * SCREEN_PITCH;               // the candidates' rows, trials x dp
+    uint16_t* queue = reinterpret_cast<uint16_t*>(cand_s + SCREEN_TN * dp);  // unsettled pairs: trial, sample
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int h = lane >> 5, j = lane & 31;
+    const int64_t base = (int64_t)blockIdx.x * CHUNK;
+
+    // the wave's tiles (those past the end, there are none in the copy, repeat the last one)
+    const int64_t tile0 = base / 32 + wave * 4, last_tile = (n - 1) / 32;
+    const int per_tile = (S + 3) / 4, n_items = 4 * per_tile;
+    auto load_item = [&](int item, uint4 (&x)[4]) {
+        const int u = item / per_tile, s0 = (item - u * per_tile) * 4;
+        const int64_t tile = tile0 + u < last_tile ? tile0 + u : last_tile;
+        const uint4* __restrict__ src = tiles.xt + (size_t)tile * S * 64 + lane;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = src[(s0 + q < S ? s0 + q : S - 1) * 64];
+    };
+    uint4 x[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) load_item(b, x[b]);  // (n_items >= 4)
+
+    if (threadIdx.x == 0) queued_s = 0;
+    // (rows past the last trial repeat it; nothing reads their scores)
+    const int64_t cj = cand[j < n_trials ? j : n_trials - 1];
+    for (int s = wave; s < S; s += 8)
+        a_s[s * 64 + lane] = tiles.xt[((size_t)(cj >> 5) * S + s) * 64 + h * 32 + (cj & 31)];
+    for (int e = threadIdx.x; e < n_trials * d; e += 512) cand_s[e / d * dp + e % d] = cand_rows[e];
+    const int best = header->best_row;
+    float xn[4], xe[4];
+    T w[4], cl[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int64_t i = (tile0 + u) * 32 + j, ic = i < n ? i : n - 1;
+        xn[u] = tiles.norm[ic];
+        xe[u] = tiles.err[ic];
+        w[u] = sample_weight[ic];
+        cl[u] = rows[(size_t)best * n + ic];
+    }
+    // norm, root and rounding of this lane's four candidates: trials 4 h .. 4 h + 3
+    float cn[4], cr[4], ce[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int64_t c = cand[4 * h + r < n_trials ? 4 * h + r : n_trials - 1];
+        cn[r] = tiles.norm[c];
+        ce[r] = tiles.err[c];
+        cr[r] = sqrtf(cn[r]);
+    }
+    const T inv_scale = T(1) / (T)tiles.scale[0];
+    const float rho = SCREEN_ULP * (17.0f * (float)S + 8.0f);
+    const T keep = T(1) - T((d + 32) * 2.0 * SCREEN_ULP);  // the roundings of a distance in T, and of the bound
+    const T least = sizeof(T) == 4 ? T(1e-30) : T(1e-290); // below: rounding to zero would count
+    __syncthreads();
+
+    kpp_v16f acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    auto settle = [&](int u, float xn_u, float xe_u, T w_u, T cl_u) {
+        const int sl = (wave * 4 + u) * 32 + j;
+        const bool live = base + sl < n;
+        const float xr = sqrtf(xn_u);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 4 * h + r;
+            const float both = xn_u + cn[r];
+            const float d2 = both - 2.0f * acc[r] - rho * (2.0f * xr * cr[r] + both);
+            const float root = sqrtf(fmaxf(d2, 0.0f));  // (a NaN: zero, nothing settled)
+            const float lb = root * (1.0f - 8.0f * SCREEN_ULP) - (xe_u + ce[r]) * (1.0f + 8.0f * SCREEN_ULP);
+            const T true_lb = (T)lb * inv_scale;
+            const T lb2 = true_lb * true_lb;
+            const bool settled = lb > 1e-6f && lb2 > least && w_u >= T(0) && w_u * lb2 * keep >= cl_u;
+            const bool open = live && t < n_trials && !settled;
+            if (live && t < n_trials) v_s[t * SCREEN_PITCH + sl] = cl_u;
+            const unsigned long long mask = __ballot(open);
+            if (mask != 0) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&queued_s, (int)__popcll(mask));
+                at = __builtin_amdgcn_readfirstlane(at);
+                at += (int)__popcll(mask & ((1ull << lane) - 1));
+                if (open && at < SCREEN_QUEUE) queue[at] = (uint16_t)(t << 10 | sl);
+            }
+        }
+    };
+    int u = 0, part = 0;  // tile and part of the current item
+    for (int item0 = 0; item0 < n_items; item0 += 4) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int s = part * 4 + q;
+                if (s < S)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(kpp_v8h, a_s[s * 64 + lane]),
+                                                                 __builtin_bit_cast(kpp_v8h, x[b][q]), acc, 0, 0, 0);
+            }
+            if (item0 + b + 4 < n_items) load_item(item0 + b + 4, x[b]);
+            if (++part == per_tile) {
+                settle(u, u == 0 ? xn[0] : u == 1 ? xn[1] : u == 2 ? xn[2] : xn[3],
+                       u == 0 ? xe[0] : u == 1 ? xe[1] : u == 2 ? xe[2] : xe[3],
+                       u == 0 ? w[0] : u == 1 ? w[1] : u == 2 ? w[2] : w[3],
+                       u == 0 ? cl[0] : u == 1 ? cl[1] : u == 2 ? cl[2] : cl[3]);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+                part = 0;
+                ++u;
+            }
+        }
+    }
+    __syncthreads();
+    const int queued = queued_s;
+    if (queued > SCREEN_QUEUE) {
+        // (the same for the whole workgroup) every pair, two samples per thread from X itself
+        const int sl = threadIdx.x * 2;
+        const bool pair = vec_ok && base + CHUNK <= n;
+        T dist[SCREEN_TN][2];
+#pragma unroll
+        for (int t = 0; t < SCREEN_TN; ++t) dist[t][0] = dist[t][1] = T(0);
+        constexpr int FB = 8;
+        for (int f0 = 0; f0 < d; f0 += FB) {
+            T xv[FB][2];
+#pragma unroll
+            for (int q = 0; q < FB; ++q) {
+                const T* __restrict__ row = X_t + (size_t)(f0 + q < d ? f0 + q : d - 1) * n;
+                if (pair) {
+                    using V2 = std::conditional_t<sizeof(T) == 4, float2, double2>;
+                    const V2 v = *reinterpret_cast<const V2*>(row + base + sl);
+                    xv[q][0] = v.x; xv[q][1] = v.y;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) xv[q][r] = row[base + sl + r < n ? base + sl + r : n - 1];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < FB; ++q) {
+                if (f0 + q < d) {
+#pragma unroll
+                    for (int t = 0; t < SCREEN_TN; ++t) {
+                        const T cv = cand_s[t * dp + f0 + q];  // (past n_trials: not used)
+#pragma unroll
+                        for (int r = 0; r < 2; ++r) dist[t][r] = kpp_sq_acc<true>(xv[q][r] - cv, dist[t][r]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (base + sl + r < n) {
+                const T wv = sample_weight[base + sl + r];
+                for (int t = 0; t < n_trials; ++t) {
+                    T* at = v_s + t * SCREEN_PITCH + sl + r;
+                    T dt = dist[0][r];
+#pragma unroll
+                    for (int q = 1; q < SCREEN_TN; ++q) dt = t == q ? dist[q][r] : dt;
+                    *at = fmin(dt * wv, *at);
+                }
+            }
+        }
+    } else {
+        for (int e = threadIdx.x; e < queued; e += 512) {
+            const int t = queue[e] >> 10, sl = queue[e] & (CHUNK - 1);
+            const T* __restrict__ row = X_rm + (size_t)(base + sl) * d;
+            const T* __restrict__ c = cand_s + t * dp;
+            T dist = T(0);
+            if (row_vec) {
+#pragma unroll 8
+                for (int f = 0; f < d; f += 4) {
+                    T v[4];
+                    load4<T>(row, f, d, true, v);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) dist = kpp_sq_acc<true>(v[q] - c[f + q], dist);
+                }
+            } else {
+#pragma unroll 16
+                for (int f = 0; f < d; ++f) dist = kpp_sq_acc<true>(row[f] - c[f], dist);
+            }
+            T* at = v_s + t * SCREEN_PITCH + sl;
+            *at = fmin(dist * sample_weight[base + sl], *at);
+        }
+    }
+    __syncthreads();
+    const int q4 = (threadIdx.x & 255) * 4;
+    auto finish = [&](auto full_tag) {
+        kpp_finish_block<T, SCREEN_TN, 2, decltype(full_tag)::value>(
+            rows, block_pot, wave_pot, base + q4, n, n_trials, [&](int t, T (&v)[4]) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v_s[t * SCREEN_PITCH + q4 + r];
+            });
+    };
+    if (vec_ok && base + CHUNK <= n)
+        finish(std::true_type{});
+    else
+        finish(std::false_type{});
 }
 
 // SPT consecutive values of a row at i0: one access of SPT elements when `full`, else element
@@ -869,6 +1130,35 @@ void launch_step(const void* X_t, const void* w, const int32_t* cand, const KppP
 #undef KMX_KPP_STEP
 }
 
+// Whether kmx_kpp_run screens its steps where the workspace has room for the copies of X they read,
+// and that room: the row-major copy, then the samples' tiles.
+bool screen_wanted(const KppLayout& L, int64_t n, int d, int k, int n_trials) {
+    return !L.split && n_trials <= SCREEN_TN && n >= SCREEN_MIN_N && k >= SCREEN_MIN_K && d >= SCREEN_MIN_D &&
+           kmx_tiles_fit(n, d, k);
+}
+
+size_t screen_bytes(const KppLayout& L, int64_t n, int d, int k, int n_trials, int dtype) {
+    if (!screen_wanted(L, n, d, k, n_trials)) return 0;
+    return kmx_align256((size_t)n * d * kmx_dtype_size(dtype)) + kmx_align256(kmx_tiles_samples_bytes(n, d));
+}
+
+template <typename T>
+int32_t launch_screen_step(const void* X_t, const void* X_rm, const KmxTiles& tiles, const void* w, const int32_t* cand,
+                           const KppPtrs& p, const KppLayout& L, int64_t n, int d, int n_trials, hipStream_t s) {
+    const int vec_ok = (n % 4 == 0) && (((uintptr_t)X_t) % 16 == 0) && (((uintptr_t)w) % 16 == 0) &&
+                       (((uintptr_t)p.rows) % 16 == 0);
+    const size_t lds = screen_lds<T>(d, tiles.S);
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&kpp_screen_step_kernel<T>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int32_t)e;
+    }
+    hipLaunchKernelGGL((kpp_screen_step_kernel<T>), dim3((unsigned)L.n_blocks), dim3(512), lds, s, (const T*)X_t,
+                       (const T*)X_rm, tiles, (const T*)w, cand, (const T*)p.cand_rows, (T*)p.rows, p.block_pot,
+                       p.header, n, d, n_trials, vec_ok, d % 4 == 0 ? 1 : 0);
+    return KMX_OK;
+}
+
 template <typename T>
 void launch_select_sample(const void* X_t, const double* uniforms, const int32_t* cand_prev,
                           int32_t* cand_next, int32_t* cand_out, void* centers_t, int32_t* idx,
@@ -913,6 +1203,12 @@ size_t kmx_kpp_workspace_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials
     if (n <= 0 || n_trials <= 0 || n_trials > TN_MAX || (dtype != KMX_F32 && dtype != KMX_F64))
         return 0;
     return kpp_layout(n, d, n_trials, dtype).total;
+}
+
+size_t kmx_kpp_screen_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials, int32_t dtype) {
+    if (n <= 0 || d <= 0 || k <= 0 || n_trials <= 0 || n_trials > TN_MAX || (dtype != KMX_F32 && dtype != KMX_F64))
+        return 0;
+    return screen_bytes(kpp_layout(n, d, n_trials, dtype), n, d, k, n_trials, dtype);
 }
 
 int32_t kmx_kpp_init(const void* X_t, const void* sample_weight, int32_t start_index,
@@ -1004,7 +1300,19 @@ int32_t kmx_kpp_run(const void* X_t, const void* sample_weight, const double* un
     const KppLayout L = kpp_layout(n, d, n_trials, dtype);
     const KppPtrs p = kpp_ptrs((char*)workspace, L);
     hipStream_t s = (hipStream_t)stream_;
+    const size_t extra = literal ? 0 : screen_bytes(L, n, d, k, n_trials, dtype);
+    const bool screened = extra != 0 && workspace_bytes >= L.total + extra && ((uintptr_t)workspace & 15) == 0;
+    void* X_rm = nullptr;
+    KmxTiles tiles = {};
+    if (screened) {
+        X_rm = (char*)workspace + L.total;
+        char* area = (char*)X_rm + kmx_align256((size_t)n * d * kmx_dtype_size(dtype));
+        rc = kmx_tiles_prepare_samples(X_t, X_rm, area, n, d, dtype, s);
+        if (rc != KMX_OK) return rc;
+        tiles = kmx_tiles_view(area, n, d);
+    }
     for (int c = 1; c < k; ++c) {
+        const bool screen = screened && c >= SCREEN_FROM;
         // candidates alternate between two buffers: the fused launch reads the previous
         // step's candidates (to record its winner) while it writes the next ones
         int32_t* cand_prev = p.cand + ((c - 1) & 1) * TN_MAX;
@@ -1014,12 +1322,19 @@ int32_t kmx_kpp_run(const void* X_t, const void* sample_weight, const double* un
         if (dtype == KMX_F32) {
             launch_select_sample<float>(X_t, u, cand_prev, cand_next, nullptr, centers_t,
                                         center_indices, p, L, n, d, k, n_trials, c - 1, do_select, 1, s, literal);
-            launch_step<float>(X_t, sample_weight, cand_next, p, L, n, d, n_trials, s, literal);
+            if (screen)
+                rc = launch_screen_step<float>(X_t, X_rm, tiles, sample_weight, cand_next, p, L, n, d, n_trials, s);
+            else
+                launch_step<float>(X_t, sample_weight, cand_next, p, L, n, d, n_trials, s, literal);
         } else {
             launch_select_sample<double>(X_t, u, cand_prev, cand_next, nullptr, centers_t,
                                          center_indices, p, L, n, d, k, n_trials, c - 1, do_select, 1, s, literal);
-            launch_step<double>(X_t, sample_weight, cand_next, p, L, n, d, n_trials, s, literal);
+            if (screen)
+                rc = launch_screen_step<double>(X_t, X_rm, tiles, sample_weight, cand_next, p, L, n, d, n_trials, s);
+            else
+                launch_step<double>(X_t, sample_weight, cand_next, p, L, n, d, n_trials, s, literal);
         }
+        if (rc != KMX_OK) return rc;
         KMX_LAUNCH_CHECK();
     }
     int32_t* cand_last = p.cand + ((k - 1) & 1) * TN_MAX;

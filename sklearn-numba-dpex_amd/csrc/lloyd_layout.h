@@ -76,6 +76,18 @@ bool kmx_tiles_fit(int64_t n, int d, int k);
 size_t kmx_tiles_bytes(int64_t n, int d, int k);
 int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
                           int64_t n, int d, int k, int dtype, hipStream_t stream);
+// the samples' tiles alone, for kmeans++: fragments, |x'|^2 and |e_x| per sample (scaled), the scale
+struct KmxTiles {
+    const uint4* xt;
+    const float* norm;
+    const float* err;
+    const float* scale;
+    int S;  // steps of 16 features
+};
+size_t kmx_tiles_samples_bytes(int64_t n, int d);
+int32_t kmx_tiles_prepare_samples(const void* X_t, void* X_rowmajor, char* area, int64_t n, int d, int dtype,
+                                  hipStream_t stream);
+KmxTiles kmx_tiles_view(char* area, int64_t n, int d);
 // weighted squared distances to the own centroid from the rows of X and of the packed centroids: their
 // sum (out: one value), or per sample (out: n values, workspace null); inertia_distances.hip
 bool kmx_inertia_in_lds(int64_t n, int d, int k, int dtype);  // whether kmx_inertia has the centroids in LDS

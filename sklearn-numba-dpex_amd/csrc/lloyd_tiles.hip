@@ -81,18 +81,8 @@ __device__ __forceinline__ _Float16 to_half(float v) {
 // The scale: a power of two that brings the largest centroid coordinate into [2^10, 2^11), which
 // leaves samples 32 times further out inside fp16 (beyond it they become infinite and get no
 // certificate).  One workgroup.
-template <typename T>
-__global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__ centroids_t, unsigned int* __restrict__ header,
-                                                           int items) {
-    __shared__ float m_s[16];
-    float m = 0.0f;
-    for (int i0 = threadIdx.x; i0 < items; i0 += 16 * 1024) {
-        float v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = i0 + u * 1024 < items ? fabsf((float)centroids_t[i0 + u * 1024]) : 0.0f;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
-    }
+// (`m`: the largest magnitude a thread has seen)
+__device__ __forceinline__ void tiles_write_scale(float m, float* m_s, unsigned int* __restrict__ header) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0) m_s[threadIdx.x >> 6] = m;
@@ -110,6 +100,38 @@ __global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__
         }
         header[TH_SCALE] = __float_as_uint(xs);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__ centroids_t, unsigned int* __restrict__ header,
+                                                           int items) {
+    __shared__ float m_s[16];
+    float m = 0.0f;
+    for (int i0 = threadIdx.x; i0 < items; i0 += 16 * 1024) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = i0 + u * 1024 < items ? fabsf((float)centroids_t[i0 + u * 1024]) : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
+    }
+    tiles_write_scale(m, m_s, header);
+}
+
+// The same from 256 samples spread over X, where there are no centroids yet.  One workgroup.
+template <typename T>
+__global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __restrict__ X_t, unsigned int* __restrict__ header,
+                                                                  int64_t n, int d) {
+    __shared__ float m_s[16];
+    const int64_t i = (int64_t)(threadIdx.x & 255) * n / 256;
+    float m = 0.0f;
+    for (int f0 = threadIdx.x >> 8; f0 < d; f0 += 4 * 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = fabsf((float)X_t[(size_t)(f0 + 4 * u < d ? f0 + 4 * u : f0) * n + i]);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
+    }
+    tiles_write_scale(m, m_s, header);
 }
 
 // The tiles, |x'|^2 and |e_x| per sample, the row-major copy of X and (absmax not null) the bits of
@@ -714,27 +736,57 @@ bool kmx_tiles_fit(int64_t n, int d, int k) {
 
 size_t kmx_tiles_bytes(int64_t n, int d, int k) { return tile_area(n, d, k).total; }
 
-// Scale, tiles and norms of X, and its row-major copy; `centroids_t`: the initial centroids.
-int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
-                          int64_t n, int d, int k, int dtype, hipStream_t stream) {
-    const TileArea a = tile_area(n, d, k);
-    unsigned int* header = (unsigned int*)area;
+static void tiles_copy(const void* X_t, void* X_rowmajor, char* area, unsigned int* absmax, int64_t n, int d, int dtype,
+                       hipStream_t stream) {
+    const TileArea a = tile_area(n, d, 0);  // (the samples' part depends on n and d alone)
+    const unsigned int* header = (const unsigned int*)area;
     const int64_t n_pad = a.n_tiles * 32;
     int64_t grid = kmx_cdiv(n_pad, 128);
     const int64_t cap = (int64_t)(dtype == KMX_F32 ? 8 : 4) * kmx_num_cus();
     if (grid > cap) grid = cap;
-#define KMX_TILES_PREPARE(T)                                                                                              \
+#define KMX_TILES_COPY(T)                                                                                                 \
     do {                                                                                                                  \
-        hipLaunchKernelGGL((tiles_scale_kernel<T>), dim3(1), dim3(1024), 0, stream, (const T*)centroids_t, header, d* k);  \
         const int x_vec = n % (16 / (int)sizeof(T)) == 0 && (((uintptr_t)X_t) & 15) == 0;                                 \
         hipLaunchKernelGGL((tiles_prepare_kernel<T>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t,          \
                            (T*)X_rowmajor, (uint4*)(area + a.off_xt), (float*)(area + a.off_norm),                        \
                            (float*)(area + a.off_err), header, absmax, n, d, a.S, n_pad, x_vec);                          \
     } while (0)
-    if (dtype == KMX_F32) KMX_TILES_PREPARE(float); else KMX_TILES_PREPARE(double);
-#undef KMX_TILES_PREPARE
+    if (dtype == KMX_F32) KMX_TILES_COPY(float); else KMX_TILES_COPY(double);
+#undef KMX_TILES_COPY
+}
+
+// Scale, tiles and norms of X, and its row-major copy; `centroids_t`: the initial centroids.
+int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
+                          int64_t n, int d, int k, int dtype, hipStream_t stream) {
+    unsigned int* header = (unsigned int*)area;
+    if (dtype == KMX_F32)
+        hipLaunchKernelGGL((tiles_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)centroids_t, header, d * k);
+    else
+        hipLaunchKernelGGL((tiles_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)centroids_t, header, d * k);
+    tiles_copy(X_t, X_rowmajor, area, absmax, n, d, dtype, stream);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
+}
+
+// The same without centroids (kmeans++, kmeanspp.hip): the area ends where the centroid tiles would begin.
+size_t kmx_tiles_samples_bytes(int64_t n, int d) { return tile_area(n, d, 0).off_ct; }
+
+int32_t kmx_tiles_prepare_samples(const void* X_t, void* X_rowmajor, char* area, int64_t n, int d, int dtype,
+                                  hipStream_t stream) {
+    unsigned int* header = (unsigned int*)area;
+    if (dtype == KMX_F32)
+        hipLaunchKernelGGL((tiles_sample_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)X_t, header, n, d);
+    else
+        hipLaunchKernelGGL((tiles_sample_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)X_t, header, n, d);
+    tiles_copy(X_t, X_rowmajor, area, nullptr, n, d, dtype, stream);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
+KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
+    const TileArea a = tile_area(n, d, 0);
+    return {(const uint4*)(area + a.off_xt), (const float*)(area + a.off_norm), (const float*)(area + a.off_err),
+            (const float*)area + TH_SCALE, a.S};
 }
 
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace

@@ -379,7 +379,15 @@ def kmeans_plusplus(X_t, sample_weight, n_clusters, random_state, sampler="scan"
     ws_bytes = lib.kmx_kpp_workspace_bytes(n, d, n_clusters, n_local_trials, dc)
     if ws_bytes == 0:
         raise ValueError(f"kmeans++ does not support n_local_trials={n_local_trials}")
-    ws = workspace(ws_bytes, dev)
+    # copies of X that the later steps read instead (kmx_kpp_run looks for them behind its workspace)
+    screen_bytes = lib.kmx_kpp_screen_bytes(n, d, n_clusters, n_local_trials, dc) if sampler == "scan" else 0
+    try:
+        ws = workspace(ws_bytes + screen_bytes, dev)
+        ws_bytes += screen_bytes
+    except torch.cuda.OutOfMemoryError:
+        if not screen_bytes:
+            raise
+        ws = workspace(ws_bytes, dev)  # steps that read X (slower, same results)
     check(lib.kmx_kpp_run(ptr(X_t), ptr(sample_weight), ptr(uniforms), starting_center_id, ptr(centers_t),
                           ptr(center_indices), ptr(ws), ws_bytes, n, d, n_clusters, n_local_trials, dc,
                           _capi.KMX_KPP_SAMPLER_LITERAL if sampler == "literal" else _capi.KMX_KPP_SAMPLER_SCAN,

@@ -215,3 +215,48 @@ def test_output_sanity_and_data_order(cuda):
     Xp, _, sw = engine.prepare_fit(np.asfortranarray(X_sk))
     centers_f = engine.init_centroids(Xp, sw).T.cpu().numpy()
     np.testing.assert_allclose(centers_c, centers_f)
+
+
+# (a million samples' worth of blocks is not needed: the last block ragged or whole, features that fill
+# the steps of 16 or not, one or two fragments' worth, data that leave every pair open, far outliers,
+# weights of zero)
+@pytest.mark.parametrize("n, d, k, dtype, kind", [
+    (262_145, 64, 40, np.float32, "blobs"), (263_168, 65, 32, np.float32, "blobs"), (262_300, 96, 33, np.float32, "equal"),
+    (131_073, 64, 64, np.float64, "blobs"), (132_096, 250, 32, np.float64, "outliers"), (140_001, 71, 40, np.float64, "equal"),
+    (270_000, 100, 50, np.float32, "outliers"),
+])
+def test_screened_seeding_is_the_plain_one(cuda, n, d, k, dtype, kind):
+    """kmx_kpp_run with room for the copies of X against the same call without: the same picks and the
+    same closest distances, bit for bit."""
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import check, lib, ptr
+
+    gen = torch.Generator(device=cuda).manual_seed(9)
+    T = torch.float32 if dtype == np.float32 else torch.float64
+    X_t = torch.randn(d, n, generator=gen, device=cuda, dtype=T)
+    if kind == "blobs":
+        centres = 10 * torch.randn(d, k, generator=gen, device=cuda, dtype=T)
+        X_t += centres[:, torch.randint(0, k, (n,), generator=gen, device=cuda)]
+    elif kind == "equal":
+        X_t = (X_t > 1.5).to(T)
+    else:
+        X_t *= torch.exp(4 * torch.randn(n, generator=gen, device=cuda, dtype=T))
+    w = torch.rand(n, generator=gen, device=cuda, dtype=T)
+    w[::7] = 0
+    trials, dc = 2 + int(np.log(k)), _capi.dtype_code(T)
+    u = torch.rand(k - 1, trials, generator=gen, device=cuda, dtype=torch.float64)
+    plain = lib.kmx_kpp_workspace_bytes(n, d, k, trials, dc)
+    extra = lib.kmx_kpp_screen_bytes(n, d, k, trials, dc)
+    assert extra > 0
+    results = []
+    for size in (plain, plain + extra):
+        ws = torch.zeros(size, dtype=torch.uint8, device=cuda)
+        centers = torch.empty(d, k, dtype=T, device=cuda)
+        picks = torch.empty(k, dtype=torch.int32, device=cuda)
+        check(lib.kmx_kpp_run(ptr(X_t), ptr(w), ptr(u), 5, ptr(centers), ptr(picks), ptr(ws), size, n, d, k, trials, dc,
+                              _capi.KMX_KPP_SAMPLER_SCAN, _capi.current_stream()), "kmx_kpp_run")
+        results.append((picks.cpu().numpy(), centers.cpu().numpy(), ws[:plain][512:].cpu().numpy()))
+    for a, b in zip(*results):
+        np.testing.assert_array_equal(a, b)
