@@ -373,7 +373,8 @@ int32_t kmx_rng_next_raw(uint64_t* states, int32_t n_states, int32_t n_steps, ui
 size_t kmx_kpp_workspace_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials, int32_t dtype);
 
 /* Bytes beyond kmx_kpp_workspace_bytes that kmx_kpp_run makes use of where the workspace has them (0:
- * none): copies of X that its later steps read in place of X itself.  The results are the same. */
+ * none): copies of X that its later steps read in place of X itself.  The results are the same.  No
+ * counterpart in the reference, whose steps read X (kmeans/drivers.py:856-919). */
 size_t kmx_kpp_screen_bytes(int64_t n, int32_t d, int32_t k, int32_t n_trials, int32_t dtype);
 
 /* closest[i] = w_i ||x_i - x_start||^2, centers_t[:, 0] = x_start, center_indices[0] = start,
@@ -494,7 +495,8 @@ int32_t kmx_transpose(const void* src, void* dst, int64_t rows, int64_t cols, in
 int32_t kmx_transpose_finite(const void* src, void* dst, int64_t rows, int64_t cols,
                              int32_t* not_finite, int32_t dtype, void* stream);
 
-/* *not_finite (device) = 1 if one of the n_items values is a NaN or an infinity, else 0. */
+/* *not_finite (device) = 1 if one of the n_items values is a NaN or an infinity, else 0: the same
+ * check (kmeans/engine.py:293-302) for an array that is already in place. */
 int32_t kmx_all_finite(const void* data, int64_t n_items, int32_t* not_finite, int32_t dtype,
                        void* stream);
 
