@@ -1538,8 +1538,15 @@ int32_t kmx_assign_labels(const void* X_t, const void* centroids_t, uint32_t* la
                                                          nullptr, n, d, k, stream, absmax, area);
         if (rc != KMX_OK) return rc;
     } else {
-        // fp64 inputs of the screened step: the same kernel without the update
-        if (L.screen64)
+        // fp64 inputs: the screened step's kernel without the update, also where its sums would
+        // not fit the LDS beside the operands.  Against fp64 products, labels of 1e6 samples: 14 features,
+        // 500 clusters 340 -> 77 us; 4, 1 200 356 -> 130; 50, 150 317 -> 147; 64, 128 (rows at no fixed
+        // alignment) 338 both; 20 000 x 14, 500 63 -> 20.  Not below four features, where the margins of many
+        // clusters are too narrow for the certificate: 1, 1 500 468 -> 1 202.
+        const bool labels_only = d >= 4 && (L.variant == KMX_VARIANT_MFMA_F64 || L.variant == KMX_VARIANT_GEMM) &&
+                                 (flags & (KMX_FLAG_PATH_MASK | KMX_FLAG_LABELS_MASK)) == 0 &&
+                                 kmx_mfma_screen_labels_fits(n, d, k, 8);
+        if (L.screen64 || labels_only)
             return kmx_assign_labels_mfma_screen_f64(X_t, centroids_t, labels, n, d, k, L.wgs_per_cu, stream);
         launch_pack<double>(centroids_t, ws + L.off_cpack, ws + L.off_half, nullptr, d, k, L.dpad, 0, 0.0, stream);
         KMX_LAUNCH_CHECK();

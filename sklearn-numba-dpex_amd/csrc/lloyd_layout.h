@@ -118,7 +118,7 @@ bool kmx_mfma_screen_fits(int64_t n, int d, int k);
 bool kmx_mfma_screen_supported(int64_t n, int d, int k, uint32_t flags);
 bool kmx_mfma_screen_f64_supported(int64_t n, int d, int k, uint32_t flags);  // fp64 inputs
 // the same kernel without the sums (labels only): needs less LDS
-bool kmx_mfma_screen_labels_fits(int64_t n, int d, int k);
+bool kmx_mfma_screen_labels_fits(int64_t n, int d, int k, int esize = 4);  // (esize 8: fp64 inputs)
 // few clusters on wide samples, X read once (lloyd_fewk.hip)
 bool kmx_fewk_supported(int d, int k);
 int kmx_fewk_grid(int64_t n, int d, int k, int wgs_per_cu);

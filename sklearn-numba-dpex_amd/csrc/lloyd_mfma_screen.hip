@@ -1793,10 +1793,10 @@ bool kmx_mfma_screen_f64_supported(int64_t n, int d, int k, uint32_t flags) {
 
 // The labels-only kernel needs no accumulators: shapes whose fused step does not fit the LDS
 // can still have their labels screened (the sums are then taken per bucket of samples).
-bool kmx_mfma_screen_labels_fits(int64_t n, int d, int k) {
+bool kmx_mfma_screen_labels_fits(int64_t n, int d, int k, int esize) {
     if (d < 1 || d > 64 || k < 16 || n >= ((int64_t)1 << 29)) return false;
-    const int nk = screen_k_steps(d, k, false);
-    return screen_lds(d, k, nk, false).off_queue <= scr_lds_max(nk);
+    const int nk = screen_k_steps(d, k, false, esize);
+    return screen_lds(d, k, nk, false, esize).off_queue <= scr_lds_max(nk);
 }
 
 // Left to the library it is chosen where it is the faster one: the all-fp32 step pays d / 2 fp32
@@ -1822,8 +1822,8 @@ int32_t launch_screen(const void* X_t, const void* w, const void* centroids_t, c
                       const LloydTail<TX>* tail = nullptr) {
     constexpr int ES = (int)sizeof(TX);
     static_assert(ES == 4 || !INERTIA, "fp64 inputs: labels and inertia are two calls");
-    if (!(ES == 8 ? screen_fits_f64(n, d, k)
-                  : (UPDATE ? kmx_mfma_screen_fits(n, d, k) : kmx_mfma_screen_labels_fits(n, d, k))))
+    if (!(UPDATE ? (ES == 8 ? screen_fits_f64(n, d, k) : kmx_mfma_screen_fits(n, d, k))
+                 : kmx_mfma_screen_labels_fits(n, d, k, ES)))
         return KMX_ERR_UNSUPPORTED;
     const int nk = screen_k_steps(d, k, UPDATE, ES);
     const int waves = scr_waves(nk);
@@ -1907,7 +1907,7 @@ int32_t kmx_assign_labels_mfma_screen(const void* X_t, const void* centroids_t, 
                                 nullptr, nullptr, nullptr, n, d, k, wgs_per_cu, stream);
 }
 
-// Labels only on fp64 inputs (the shapes of the fused fp64 step).
+// Labels only on fp64 inputs.
 int32_t kmx_assign_labels_mfma_screen_f64(const void* X_t, const void* centroids_t, uint32_t* labels,
                                           int64_t n, int d, int k, int wgs_per_cu, hipStream_t stream) {
     return launch_screen<false, false, double>(X_t, nullptr, centroids_t, nullptr, labels, nullptr, nullptr, nullptr,

@@ -693,3 +693,33 @@ def test_labels_and_score_paths_on_every_label_kernel(cuda, name):
     dist = drivers.get_euclidean_distances(X_t[:, :512].contiguous(), C_t).cpu().numpy()
     exact = np.sqrt(((X[:512].astype(np.float64)[:, None, :] - init.astype(np.float64)[None, :, :]) ** 2).sum(axis=2))
     np.testing.assert_allclose(dist, exact, rtol=RTOL[X.dtype] * 2, atol=RTOL[X.dtype])
+
+
+@pytest.mark.parametrize("n,d,k", [
+    (3_001, 4, 300),    # the fewest features that are screened; accumulators of the step beyond LDS
+    (3_001, 3, 1_000),  # one feature fewer: fp64 products
+    (2_000, 16, 700),   # no spare feature slot for the half norms
+    (2_003, 17, 250), (2_004, 33, 230), (1_999, 50, 150),
+    (130, 64, 128),     # two tiles of samples and a remainder
+    (63, 63, 40),       # less than a tile
+    (2_000, 64, 190),   # operands beyond LDS
+])
+def test_fp64_labels_where_only_the_labels_fit_the_lds(cuda, n, d, k):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d)
+    C = rng.uniform(-5, 5, (k, d))
+    C[k // 2] = C[3]  # of equal centroids the first
+    X = C[rng.integers(0, k, n)] + 0.5 * rng.standard_normal((n, d))
+    labels = torch.full((n,), -1, dtype=torch.int32, device=cuda)
+    X_t, C_t = _dev(X.T, cuda), _dev(C.T, cuda)
+    drivers._assign(X_t, C_t, labels)
+    got = labels.cpu().numpy().astype(np.int64)
+    assert_labels_match(got, ok.assign_labels(X, C), X, C)
+    assert not (got == k // 2).any()
+    w = rng.uniform(0.5, 1.5, n)
+    labels2, inertia = drivers.get_labels_inertia(X_t, C_t, _dev(w, cuda), True)
+    np.testing.assert_array_equal(labels2.cpu().numpy(), got)
+    assert float(inertia[0]) == pytest.approx(float(ok.inertia(X, w, C, got)), rel=RTOL[X.dtype] * 5)
