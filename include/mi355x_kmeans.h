@@ -217,9 +217,10 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
  * kmx_lloyd_resident_bytes: how much (0: the plan's kernels have no use for it).
  * kmx_lloyd_init_resident is kmx_lloyd_init and fills, in the same pass over X_t, `resident` and the
  * row-major copy X_rowmajor (OUT, n x d).  Both are then handed to kmx_lloyd_run, whose
- * `resident` may be NULL (labels from X_t).  kmx_lloyd_labels_inertia ends such a run: the labels for
- * the final centroids (centroids_t and the workspace as the run of n_iter iterations left them) and
- * their inertia; inertia_workspace as for kmx_inertia.
+ * `resident` may be NULL (labels from X_t).  kmx_lloyd_labels_inertia gives the labels for the
+ * centroids such a run has come to (centroids_t and the workspace as the run left them; n_iter is not
+ * read) and their inertia; inertia_workspace as for kmx_inertia.  It leaves the run's state alone: it may
+ * be called again, and the run may go on after it.
  * They have no counterpart in the reference, which computes from one layout of X in its own type
  * (kmeans/drivers.py:146-391). */
 size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan);

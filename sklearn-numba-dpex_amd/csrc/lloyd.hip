@@ -756,7 +756,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         const int32_t rc_labels =
             L.tiles != nullptr
                 ? kmx_tiles_labels(X_t, X_rowmajor, centroids_t, cpack, half_norms, L.tiles, status, labels, n, d, L.dpad, k,
-                                   sizeof(T) == 8 ? KMX_F64 : KMX_F32, 0, stream)
+                                   sizeof(T) == 8 ? KMX_F64 : KMX_F32, stream)
                 : launch_fused<T, ACC_NONE>(L, X_t, w, centroids_t, cpack, half_norms, labels_prev, labels,
                                       partial, status, n, d, k, stream,
                                       reinterpret_cast<const unsigned int*>(ws + L.off_scales), ws + L.off_wscreen);
@@ -992,7 +992,7 @@ int32_t kmx_lloyd_sample_distances(const kmx_lloyd_plan* plan, const void* X_row
 int32_t kmx_lloyd_labels_inertia(const kmx_lloyd_plan* plan, const void* X_t, const void* X_rowmajor,
                                  const void* sample_weight, const void* centroids_t, uint32_t* labels, void* out_total,
                                  void* workspace, size_t workspace_bytes, void* resident, size_t resident_bytes,
-                                 int32_t n_iter, void* inertia_workspace, size_t inertia_workspace_bytes, void* stream_) {
+                                 int32_t /*n_iter*/, void* inertia_workspace, size_t inertia_workspace_bytes, void* stream_) {
     KMX_ENTRY();
     KMX_REQUIRE_PLAN(plan);
     KMX_REQUIRE_PTR(X_t);
@@ -1010,7 +1010,7 @@ int32_t kmx_lloyd_labels_inertia(const kmx_lloyd_plan* plan, const void* X_t, co
         return KMX_ERR_WORKSPACE;
     char* ws = (char*)workspace;
     const int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, ws + L.off_cpack, ws + L.off_half, (char*)resident,
-                                        nullptr, labels, plan->n, plan->d, L.dpad, plan->k, plan->dtype, n_iter & 1,
+                                        nullptr, labels, plan->n, plan->d, L.dpad, plan->k, plan->dtype,
                                         (hipStream_t)stream_);
     if (rc != KMX_OK) return rc;
     // From the feature-major array while its kernel holds the centroids in LDS (1e6 x 100 fp64 with 100

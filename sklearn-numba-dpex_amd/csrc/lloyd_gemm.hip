@@ -97,14 +97,6 @@ __device__ __forceinline__ void stage_load_listed_f32(float4 (&r)[L], const floa
     }
 }
 
-// Number of listed samples: one word, or (count_parity >= 0) two words of which the parity of the
-// iteration says which, the given one where there is no run.
-__device__ __forceinline__ int64_t listed_count(const unsigned int* __restrict__ list_count,
-                                                const kmx_lloyd_status* __restrict__ status, int count_parity) {
-    if (count_parity < 0) return (int64_t)list_count[0];
-    return (int64_t)list_count[status != nullptr ? status->n_iter & 1 : count_parity];
-}
-
 // NA: 32-centroid row tiles per pass over the features (4: tiles of 128 centroids; 1 or 2 for
 // up to 32 / 64 clusters, where wider tiles would multiply padding).  A stage copies the 32 NA
 // centroid columns in use.  With one row tile a stage is 32 features instead of 16: the small
@@ -117,10 +109,9 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t,
     const float* __restrict__ half_norms, uint32_t* __restrict__ labels,
     const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
-    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
-    int count_parity = -1) {
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int64_t n_work = LISTED ? listed_count(list_count, status, count_parity) : n;
+    const int64_t n_work = LISTED ? (int64_t)*list_count : n;
     constexpr int GK = NA == 1 ? 2 * GK32 : GK32;           // features per stage
     constexpr int XL = GK / 8;                              // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                              // groups of four columns per centroid row
@@ -280,10 +271,9 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
     const double* __restrict__ X_t, const double* __restrict__ centroids_t,
     const double* __restrict__ half_norms, uint32_t* __restrict__ labels,
     const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
-    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
-    int count_parity = -1) {
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int64_t n_work = LISTED ? listed_count(list_count, status, count_parity) : n;
+    const int64_t n_work = LISTED ? (int64_t)*list_count : n;
     constexpr int GK = NA == 2 ? 2 * GK64 : GK64;  // features per stage
     constexpr int XL = GK / 4;                     // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                     // pairs of columns per centroid row
@@ -433,11 +423,11 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
 }
 
 // The same kernels on the samples list[0 .. count) (list and count on the device): what a screened
-// label kernel could not certify; count_parity: see listed_count.  The grid covers the worst
-// case; workgroups without a tile of the list leave at once.
+// label kernel could not certify.  The grid covers the worst case; workgroups without a tile of the
+// list leave at once.
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
-                                     const unsigned int* list_count, int count_parity, int64_t n, int d, int k,
+                                     const unsigned int* list_count, int64_t n, int d, int k,
                                      int32_t dtype, hipStream_t stream) {
     const int c_vec = (k % (dtype == KMX_F32 ? 4 : 2) == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
     int64_t grid = kmx_cdiv(n, GT);
@@ -445,7 +435,7 @@ int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, c
     if (grid > cap) grid = cap;
 #define KMX_GEMM_LISTED(KERNEL, T)                                                                             \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t, (const T*)centroids_t, \
-                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count, count_parity)
+                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count)
     if (dtype == KMX_F32) {
         if (k <= 32) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<1, true>), float);
         else if (k <= 64) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<2, true>), float);

@@ -289,5 +289,5 @@ int32_t kmx_lloyd_gemm_screen_labels(const void* X_t, const void* centroids_t, c
 #undef KMX_GS_LAUNCH
     KMX_LAUNCH_CHECK();
     return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, list,
-                                        header + GS_UNCERTAIN, -1, n, d, k, KMX_F32, stream);
+                                        header + GS_UNCERTAIN, n, d, k, KMX_F32, stream);
 }

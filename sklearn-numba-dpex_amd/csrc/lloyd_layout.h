@@ -61,7 +61,7 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
                               int32_t dtype, hipStream_t stream);
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
-                                     const unsigned int* list_count, int count_parity, int64_t n, int d, int k,
+                                     const unsigned int* list_count, int64_t n, int d, int k,
                                      int32_t dtype, hipStream_t stream);
 // the same product screened on the fp16 matrix cores (lloyd_gemm_screen.hip), fp32 only
 size_t kmx_gemm_screen_bytes(int64_t n);
@@ -95,7 +95,7 @@ int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, cons
                          void* out, double* workspace, int64_t n, int d, int dpad, int dtype, hipStream_t stream);
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, int parity, hipStream_t stream);
+                         int d, int dpad, int k, int dtype, hipStream_t stream);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,

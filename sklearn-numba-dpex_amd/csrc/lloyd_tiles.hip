@@ -41,20 +41,19 @@ constexpr int GRP = 8;               // accumulator registers per arg-max group
 constexpr float ULP = 1.1920929e-7f; // 2^-23
 constexpr float HALF_MIN = 6.1035156e-5f;  // 2^-14: smaller magnitudes are rounded to zero (no fp16 subnormals)
 
-// Header words.  Maxima over the centroids are kept twice, by the parity of the iteration: the kernel
-// that takes them for one iteration clears those of the next.
+// Header words.  The two counts belong to one labelling and are cleared by its first kernel: whatever
+// was labelled before (a run that goes on, a call repeated, another run on the same copy) leaves
+// nothing behind that could run the lists past their n entries.
 constexpr int TH_SCALE = 0;      // bits of the scale
-constexpr int TH_LISTED = 1;     // [2] samples without a certificate
-constexpr int TH_REST = 3;       // [2] samples left to the tiled product
-constexpr int TH_HMAX = 5;       // [2] bits of max 0.5 |c'|^2
-constexpr int TH_EMAX = 7;       // [2] bits of max |e_c|
+constexpr int TH_LISTED = 1;     // samples without a certificate
+constexpr int TH_REST = 2;       // samples left to the tiled product
 constexpr int TH_WORDS = 64;
 
 struct TileArea {
     int S;              // steps of 16 features
     int n_blocks;       // blocks of 32 centroids
     int64_t n_tiles;    // tiles of 32 samples (even)
-    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_list, off_thr, off_rest, total;
+    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_list, off_thr, off_rest, total;
 };
 
 inline TileArea tile_area(int64_t n, int d, int k) {
@@ -67,7 +66,8 @@ inline TileArea tile_area(int64_t n, int d, int k) {
     a.off_err = a.off_norm + kmx_align256((size_t)a.n_tiles * 32 * sizeof(float));
     a.off_ct = a.off_err + kmx_align256((size_t)a.n_tiles * 32 * sizeof(float));
     a.off_hneg = a.off_ct + (size_t)a.n_blocks * a.S * 1024;
-    a.off_list = a.off_hneg + kmx_align256((size_t)a.n_blocks * 32 * sizeof(float));
+    a.off_cmax = a.off_hneg + kmx_align256((size_t)a.n_blocks * 32 * sizeof(float));
+    a.off_list = a.off_cmax + kmx_align256((size_t)a.n_blocks * sizeof(float2));
     a.off_thr = a.off_list + kmx_align256((size_t)n * sizeof(int));
     a.off_rest = a.off_thr + kmx_align256((size_t)n * sizeof(float));
     a.total = a.off_rest + kmx_align256((size_t)n * sizeof(int));
@@ -243,16 +243,15 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
     }
 }
 
-// The centroids of an iteration: their tiles (32 centroids x 16 features, laid out like those of
-// the samples), -0.5 |c'|^2 (-inf past the last one), and the maxima of 0.5 |c'|^2 and |e_c|.  A
-// workgroup per block of 32 centroids; four waves share the steps.
+// The centroids of a labelling: their tiles (32 centroids x 16 features, laid out like those of
+// the samples), -0.5 |c'|^2 (-inf past the last one), and per block of 32 the maxima of 0.5 |c'|^2 and
+// |e_c|.  A workgroup per block; four waves share the steps.  The first one clears the counts.
 template <typename T>
 __global__ __launch_bounds__(256) void tiles_centroids_kernel(const T* __restrict__ centroids_t, uint4* __restrict__ ct,
-                                                              float* __restrict__ hneg, unsigned int* __restrict__ header,
-                                                              const kmx_lloyd_status* __restrict__ status, int d, int k, int S,
-                                                              int fixed_parity) {
+                                                              float* __restrict__ hneg, float2* __restrict__ cmax,
+                                                              unsigned int* __restrict__ header,
+                                                              const kmx_lloyd_status* __restrict__ status, int d, int k, int S) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int par = status != nullptr ? status->n_iter & 1 : fixed_parity;
     __shared__ double part[2][4][64];
     const float xs = __uint_as_float(header[TH_SCALE]);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -298,13 +297,10 @@ __global__ __launch_bounds__(256) void tiles_centroids_kernel(const T* __restric
             em = fmaxf(em, __shfl_xor(em, off, 64));
         }
         if (threadIdx.x == 0) {
-            atomicMax(header + TH_HMAX + par, __float_as_uint(hm));
-            atomicMax(header + TH_EMAX + par, __float_as_uint(em));
+            cmax[blockIdx.x] = make_float2(hm, em);
             if (blockIdx.x == 0) {
-                header[TH_HMAX + (par ^ 1)] = 0u;
-                header[TH_EMAX + (par ^ 1)] = 0u;
-                header[TH_LISTED + (par ^ 1)] = 0u;
-                header[TH_REST + (par ^ 1)] = 0u;
+                header[TH_LISTED] = 0u;
+                header[TH_REST] = 0u;
             }
         }
     }
@@ -324,7 +320,7 @@ __device__ __forceinline__ void lds_wait(v4f& a, v4f& b, v4f& c, v4f& d) {
     asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "n"(N));
 }
 
-// LDS buffers of centroid tiles in STREAM mode: three of CHUNK_KB each
+// Blocks of centroid tiles in each of the three LDS buffers of STREAM mode (S kilobytes a block)
 constexpr int stream_blocks(int S) { return S >= 8 ? 2 : S >= 4 ? 4 : 8; }
 
 constexpr int PEND = 128;  // entries a wave gathers before it adds them to the list
@@ -335,11 +331,10 @@ constexpr int PEND = 128;  // entries a wave gathers before it adds them to the 
 template <int S, int NCOL, bool STREAM>
 __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     const uint4* __restrict__ xt, const float* __restrict__ norm, const float* __restrict__ err,
-    const uint4* __restrict__ ct, const float* __restrict__ hneg, unsigned int* __restrict__ header,
-    const kmx_lloyd_status* __restrict__ status, uint32_t* __restrict__ labels, int* __restrict__ list,
-    float* __restrict__ list_thr, int64_t n, int n_blocks, int fixed_parity) {
+    const uint4* __restrict__ ct, const float* __restrict__ hneg, const float2* __restrict__ block_max,
+    unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status, uint32_t* __restrict__ labels,
+    int* __restrict__ list, float* __restrict__ list_thr, int64_t n, int n_blocks) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int par = status != nullptr ? status->n_iter & 1 : fixed_parity;
     extern __shared__ __align__(16) unsigned char tiles_lds[];
     constexpr int CB = STREAM ? stream_blocks(S) : 1;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -356,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     int pending = 0;  // (the same in all lanes)
     auto flush = [&]() __attribute__((always_inline)) {
         unsigned int base = 0;
-        if (lane == 0) base = atomicAdd(header + TH_LISTED + par, (unsigned int)pending);
+        if (lane == 0) base = atomicAdd(header + TH_LISTED, (unsigned int)pending);
         base = (unsigned int)__builtin_amdgcn_readfirstlane((int)base);
         for (int e = lane; e < pending; e += 64) {
             list[base + e] = pend_i[wave][e];
@@ -375,8 +370,19 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     };
     if constexpr (!STREAM) copy_tiles(ct, 0, n_blocks * S);
 
-    const float hmax = __uint_as_float(header[TH_HMAX + par]);
-    const float emax = __uint_as_float(header[TH_EMAX + par]);
+    float hmax = 0.0f, emax = 0.0f;  // over all blocks of centroids
+    for (int b = lane; b < n_blocks; b += 64) {
+        const float2 m = block_max[b];
+        hmax = fmaxf(hmax, m.x);
+        emax = fmaxf(emax, m.y);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        hmax = fmaxf(hmax, __shfl_xor(hmax, off, 64));
+        emax = fmaxf(emax, __shfl_xor(emax, off, 64));
+    }
+    hmax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(hmax)));
+    emax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(emax)));
     const float cmax = sqrtf(2.0f * hmax) * 1.0001f;
     const float rho = ULP * (17.0f * (float)S + 4.0f);
     float pos_inf = kmx_inf<float>();
@@ -584,14 +590,13 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const T* __restrict__ X_rm, const T* __restrict__ cpack, const uint4* __restrict__ xt, const uint4* __restrict__ ct,
     const float* __restrict__ hneg, unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status,
     uint32_t* __restrict__ labels, const int* __restrict__ list, const float* __restrict__ list_thr, int* __restrict__ rest,
-    int64_t n, int d, int dpad, int k, int n_blocks, int fixed_parity) {
+    int64_t n, int d, int dpad, int k, int n_blocks) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int par = status != nullptr ? status->n_iter & 1 : fixed_parity;
     __shared__ int cand_n[32];
     __shared__ int cand[32][CAND];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, j = lane & 31;
-    const int64_t n_listed = (int64_t)header[TH_LISTED + par];
+    const int64_t n_listed = (int64_t)header[TH_LISTED];
     const bool too_many = n_listed > (n >> 3);  // the tiled product takes them all
     for (int64_t t0 = (int64_t)blockIdx.x * 32; t0 < n_listed; t0 += (int64_t)gridDim.x * 32) {
         const int64_t slot = t0 + j;
@@ -684,7 +689,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
             if (fine && arg < k)
                 labels[is] = (uint32_t)arg;
             else
-                rest[atomicAdd(header + TH_REST + par, 1u)] = is;
+                rest[atomicAdd(header + TH_REST, 1u)] = is;
         }
         __syncthreads();
     }
@@ -692,7 +697,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
 
 template <int S, int NCOL, bool STREAM>
 int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                      int parity, hipStream_t stream) {
+                      hipStream_t stream) {
     const size_t hneg_bytes = ((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023;
     const size_t lds = hneg_bytes + (STREAM ? (size_t)3 * stream_blocks(S) * S * 1024 : (size_t)a.n_blocks * S * 1024);
     if (lds > 64 * 1024) {
@@ -704,8 +709,9 @@ int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* sta
     if (grid > kmx_num_cus()) grid = kmx_num_cus();
     hipLaunchKernelGGL((tiles_label_kernel<S, NCOL, STREAM>), dim3((unsigned)grid), dim3(512), lds, stream,
                        (const uint4*)(area + a.off_xt), (const float*)(area + a.off_norm), (const float*)(area + a.off_err),
-                       (const uint4*)(area + a.off_ct), (const float*)(area + a.off_hneg), (unsigned int*)area, status, labels,
-                       (int*)(area + a.off_list), (float*)(area + a.off_thr), n, a.n_blocks, parity);
+                       (const uint4*)(area + a.off_ct), (const float*)(area + a.off_hneg),
+                       (const float2*)(area + a.off_cmax), (unsigned int*)area, status, labels,
+                       (int*)(area + a.off_list), (float*)(area + a.off_thr), n, a.n_blocks);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
@@ -714,17 +720,17 @@ constexpr size_t TILES_LDS_MAX = 148 * 1024;  // (beside the 8 KB of the waves' 
 
 template <int S>
 int32_t launch_labels_s(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                        int parity, hipStream_t stream) {
+                        hipStream_t stream) {
     const size_t resident = (((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023) + (size_t)a.n_blocks * S * 1024;
     const bool in_lds = resident <= TILES_LDS_MAX;
     // two columns per wave (a centroid fragment read from LDS serves two products) unless that leaves
     // compute units without a wave
     const bool two = n >= (int64_t)64 * 8 * kmx_num_cus() / 2;
     if (in_lds)
-        return two ? launch_labels<S, 2, false>(a, area, status, labels, n, parity, stream)
-                   : launch_labels<S, 1, false>(a, area, status, labels, n, parity, stream);
-    return two ? launch_labels<S, 2, true>(a, area, status, labels, n, parity, stream)
-               : launch_labels<S, 1, true>(a, area, status, labels, n, parity, stream);
+        return two ? launch_labels<S, 2, false>(a, area, status, labels, n, stream)
+                   : launch_labels<S, 1, false>(a, area, status, labels, n, stream);
+    return two ? launch_labels<S, 2, true>(a, area, status, labels, n, stream)
+               : launch_labels<S, 1, true>(a, area, status, labels, n, stream);
 }
 
 }  // namespace
@@ -790,23 +796,24 @@ KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
 }
 
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace
-// holds them).  `status` null: labels whatever the state, with the words of `parity`.
+// holds them).  `status` null: labels whatever the state.
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, int parity, hipStream_t stream) {
+                         int d, int dpad, int k, int dtype, hipStream_t stream) {
     const TileArea a = tile_area(n, d, k);
     unsigned int* header = (unsigned int*)area;
     uint4* ct = (uint4*)(area + a.off_ct);
     float* hneg = (float*)(area + a.off_hneg);
+    float2* cmax = (float2*)(area + a.off_cmax);
     if (dtype == KMX_F32)
         hipLaunchKernelGGL((tiles_centroids_kernel<float>), dim3((unsigned)a.n_blocks), dim3(256), 0, stream,
-                           (const float*)centroids_t, ct, hneg, header, status, d, k, a.S, parity);
+                           (const float*)centroids_t, ct, hneg, cmax, header, status, d, k, a.S);
     else
         hipLaunchKernelGGL((tiles_centroids_kernel<double>), dim3((unsigned)a.n_blocks), dim3(256), 0, stream,
-                           (const double*)centroids_t, ct, hneg, header, status, d, k, a.S, parity);
+                           (const double*)centroids_t, ct, hneg, cmax, header, status, d, k, a.S);
     int32_t rc = KMX_ERR_UNSUPPORTED;
     switch (a.S) {
-#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, n, parity, stream); break
+#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, n, stream); break
         KMX_TILES_CASE(1); KMX_TILES_CASE(2); KMX_TILES_CASE(3); KMX_TILES_CASE(4);
         KMX_TILES_CASE(5); KMX_TILES_CASE(6); KMX_TILES_CASE(7); KMX_TILES_CASE(8);
         KMX_TILES_CASE(9); KMX_TILES_CASE(10); KMX_TILES_CASE(11); KMX_TILES_CASE(12);
@@ -822,7 +829,7 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
 #define KMX_TILES_RESOLVE(T, S_)                                                                                         \
     hipLaunchKernelGGL((tiles_resolve_kernel<T, S_>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor,   \
                        (const T*)cpack, (const uint4*)(area + a.off_xt), ct, hneg, header, status, labels, list, thr,    \
-                       rest, n, d, dpad, k, a.n_blocks, parity)
+                       rest, n, d, dpad, k, a.n_blocks)
     switch (a.S) {
 #define KMX_TILES_CASE(S_)                                                                         \
     case S_:                                                                                       \
@@ -836,10 +843,9 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
     }
 #undef KMX_TILES_RESOLVE
     KMX_LAUNCH_CHECK();
-    // (the words of both parities: the kernel takes the one of the iteration)
-    return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + TH_REST, parity, n, d, k,
-                                        dtype, stream);
+    return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + TH_REST, n, d, k, dtype,
+                                        stream);
 }
 
 // samples of the last labelling that had no certificate
-const uint32_t* kmx_tiles_counter(const char* area, int parity) { return (const uint32_t*)area + TH_LISTED + parity; }
+const uint32_t* kmx_tiles_counter(const char* area) { return (const uint32_t*)area + TH_LISTED; }

@@ -145,6 +145,107 @@ def test_labels_from_the_half_precision_copy(cuda, n, d, k, dtype, data):
         assert float(err) <= (2e-5 if dtype == np.float32 else 1e-11)
 
 
+class _ResidentRun:
+    """A run with the half-precision copy, through the C ABI."""
+
+    def __init__(self, cuda, X, w, init, max_iter):
+        import torch
+
+        from sklearn_numba_dpex_amd import _capi
+        from sklearn_numba_dpex_amd._capi import lib, ptr
+
+        n, d = X.shape
+        k = len(init)
+        dtype = _dev(X[:1], cuda).dtype
+        self.lib, self.ptr, self.check, self.stream = lib, ptr, _capi.check, _capi.current_stream()
+        self.n, self.max_iter, self.n_done = n, max_iter, 0
+        self.plan = _capi.lloyd_plan(n, d, k, _capi.dtype_code(dtype), 0)
+        self.X_t, self.w = _dev(X.T, cuda), _dev(w, cuda)
+        self.X_rm = torch.empty(n, d, dtype=dtype, device=cuda)
+        self.cent = [_dev(init.T, cuda), torch.empty(d, k, dtype=dtype, device=cuda)]
+        self.labels = [torch.empty(n, dtype=torch.int32, device=cuda) for _ in range(2)]
+        self.sizes, self.empty = torch.empty(k, dtype=dtype, device=cuda), torch.empty(k, dtype=torch.int32, device=cuda)
+        self.ws_bytes, self.res_bytes = self.plan.workspace_bytes, lib.kmx_lloyd_resident_bytes(self.plan)
+        assert self.res_bytes > 0
+        self.ws = torch.empty(self.ws_bytes, dtype=torch.uint8, device=cuda)
+        self.resident = torch.empty(self.res_bytes, dtype=torch.uint8, device=cuda)
+        self.status = _capi.LloydStatus()
+        self.init()
+
+    def init(self):
+        ptr = self.ptr
+        self.check(self.lib.kmx_lloyd_init_resident(
+            self.plan, ptr(self.ws), self.ws_bytes, ptr(self.X_t), ptr(self.w), ptr(self.cent[0]), self.max_iter, 0.0,
+            ptr(self.X_rm), ptr(self.resident), self.res_bytes, self.stream), "kmx_lloyd_init_resident")
+
+    def run(self, until):
+        ptr = self.ptr
+        self.check(self.lib.kmx_lloyd_run(
+            self.plan, ptr(self.X_t), ptr(self.X_rm), ptr(self.w), ptr(self.cent[0]), ptr(self.cent[1]),
+            ptr(self.labels[0]), ptr(self.labels[1]), ptr(self.sizes), ptr(self.empty), ptr(self.ws), self.ws_bytes,
+            ptr(self.resident), self.res_bytes, self.n_done, until, self.status, self.stream), "kmx_lloyd_run")
+        self.n_done = self.status.n_iter
+        return self.cent[self.n_done % 2]
+
+    def labels_inertia(self):
+        import torch
+
+        ptr, centroids_t = self.ptr, self.cent[self.n_done % 2]
+        labels, out = torch.full_like(self.labels[0], -1), torch.empty(1, dtype=centroids_t.dtype, device=centroids_t.device)
+        area_bytes = self.lib.kmx_inertia_workspace_bytes(self.n)
+        area = torch.empty(area_bytes, dtype=torch.uint8, device=centroids_t.device)
+        self.check(self.lib.kmx_lloyd_labels_inertia(
+            self.plan, ptr(self.X_t), ptr(self.X_rm), ptr(self.w), ptr(centroids_t), ptr(labels), ptr(out), ptr(self.ws),
+            self.ws_bytes, ptr(self.resident), self.res_bytes, self.n_done, ptr(area), area_bytes, self.stream),
+            "kmx_lloyd_labels_inertia")
+        return labels.cpu().numpy(), out.cpu().numpy()
+
+    def listed(self):
+        """Samples of the last labelling without a certificate: the second word of the copy's header."""
+        import torch
+
+        return int(self.resident[:8].view(torch.int32)[1])
+
+
+@pytest.mark.parametrize("n,d,k,data", [(20_003, 128, 260, "offset"), (5_003, 128, 500, "blobs")])
+def test_labels_of_a_resident_run_taken_twice_and_midway(cuda, n, d, k, data):
+    """kmx_lloyd_labels_inertia again and between two halves of a run: each labelling starts its lists anew (three that
+    list nearly all samples would run past their n entries otherwise), and the run goes on as if not interrupted."""
+    rng = np.random.default_rng(d)
+    X = rng.standard_normal((n, d))
+    if data == "offset":
+        X[:, 0] += 300  # no clusters, and a rounding to half precision of the order of the margins: little is certified
+    else:
+        X += rng.uniform(-2, 2, (k, d))[rng.integers(0, k, n)]
+    X = X.astype(np.float32)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    init = X[rng.choice(n, k, replace=False)]
+    whole = _ResidentRun(cuda, X, w, init, 6)
+    expected = whole.run(6).cpu().numpy()
+    parts = _ResidentRun(cuda, X, w, init, 6)
+    parts.run(3)
+    first, first_inertia = parts.labels_inertia()
+    if data == "offset":
+        assert parts.listed() > n // 2
+    for _ in range(3):
+        again, inertia = parts.labels_inertia()
+        np.testing.assert_array_equal(again, first)
+        np.testing.assert_array_equal(inertia, first_inertia)
+    np.testing.assert_array_equal(parts.run(6).cpu().numpy(), expected)  # (sums in fixed point: whatever the order)
+    assert parts.n_done == whole.n_done == 6
+    for a, b in zip(parts.labels_inertia(), whole.labels_inertia()):
+        np.testing.assert_array_equal(a, b)
+    # another run on the same copy, begun with the plain initialisation
+    again = _ResidentRun(cuda, X, w, init, 6)
+    again.run(3)
+    again.cent[0].copy_(_dev(init.T, cuda))
+    ptr = again.ptr
+    again.check(again.lib.kmx_lloyd_init(again.plan, ptr(again.ws), again.ws_bytes, ptr(again.X_t), ptr(again.w),
+                                         ptr(again.cent[0]), 6, 0.0, again.stream), "kmx_lloyd_init")
+    again.n_done = 0
+    np.testing.assert_array_equal(again.run(6).cpu().numpy(), expected)
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
