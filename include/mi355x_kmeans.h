@@ -219,8 +219,8 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
  * row-major copy X_rowmajor (OUT, n x d).  Both are then handed to kmx_lloyd_run, whose
  * `resident` may be NULL (labels from X_t).  kmx_lloyd_labels_inertia gives the labels for the
  * centroids such a run has come to (centroids_t and the workspace as the run left them; n_iter is not
- * read) and their inertia; inertia_workspace as for kmx_inertia.  It leaves the run's state alone: it may
- * be called again, and the run may go on after it.
+ * read), the same as kmx_assign_labels gives for them, and their inertia; inertia_workspace as for
+ * kmx_inertia.  It leaves the run's state alone: it may be called again, and the run may go on after it.
  * They have no counterpart in the reference, which computes from one layout of X in its own type
  * (kmeans/drivers.py:146-391). */
 size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan);

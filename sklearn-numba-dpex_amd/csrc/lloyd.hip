@@ -1009,9 +1009,16 @@ int32_t kmx_lloyd_labels_inertia(const kmx_lloyd_plan* plan, const void* X_t, co
     if (resident_bytes < need || workspace_bytes < L.total || inertia_workspace_bytes < kmx_inertia_workspace_bytes(plan->n))
         return KMX_ERR_WORKSPACE;
     char* ws = (char*)workspace;
-    const int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, ws + L.off_cpack, ws + L.off_half, (char*)resident,
-                                        nullptr, labels, plan->n, plan->d, L.dpad, plan->k, plan->dtype,
-                                        (hipStream_t)stream_);
+    // (the half norms as kmx_assign_labels takes them; the workspace keeps those of the run, the last
+    // update's, which round differently)
+    char* half = kmx_tiles_half_norms((char*)resident, plan->n, plan->d, plan->k);
+    hipStream_t s = (hipStream_t)stream_;
+    if (plan->dtype == KMX_F32)
+        launch_pack<float>(centroids_t, ws + L.off_cpack, half, nullptr, plan->d, plan->k, L.dpad, 0, 0.0, s);
+    else
+        launch_pack<double>(centroids_t, ws + L.off_cpack, half, nullptr, plan->d, plan->k, L.dpad, 0, 0.0, s);
+    const int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, ws + L.off_cpack, half, (char*)resident, nullptr,
+                                        labels, plan->n, plan->d, L.dpad, plan->k, plan->dtype, s);
     if (rc != KMX_OK) return rc;
     // From the feature-major array while its kernel holds the centroids in LDS (1e6 x 100 fp64 with 100
     // clusters: 141 us against 218 from the rows), else from the rows (1e6 x 256 with 1 024 clusters: 193

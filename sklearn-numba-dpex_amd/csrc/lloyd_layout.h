@@ -93,6 +93,7 @@ KmxTiles kmx_tiles_view(char* area, int64_t n, int d);
 bool kmx_inertia_in_lds(int64_t n, int d, int k, int dtype);  // whether kmx_inertia has the centroids in LDS
 int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, const void* cpack, const uint32_t* labels,
                          void* out, double* workspace, int64_t n, int d, int dpad, int dtype, hipStream_t stream);
+char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k);  // room for k half norms
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream);

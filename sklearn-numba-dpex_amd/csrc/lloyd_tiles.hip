@@ -21,6 +21,13 @@
 // more such centroids than that kernel holds, or all of them if the list is long, go through
 // the tiled product of lloyd_gemm.hip.
 //
+// The labels that a run ends with are those that kmx_assign_labels gives for its centroids, which for
+// fp32 inputs is the arg-max of fp32 scores: there the thresholds also leave room for the errors E of two
+// such scores (MATCH in the code below; E = prod_rho (|x| C + C^2 / 2), C = max |c|).  A score gap of 2 E is
+// a gap of 4 E between squared distances, and D_j^2 - D_b^2 >= (D'_j - eps)^2 - (D'_b + eps)^2 asks of the
+// scores s a further 2 E (D'_b + 2 eps) / (D'_b + eps).  Candidates closer than that are decided by the
+// scores themselves, from the instruction that the product uses, pair by pair on a diagonal.
+//
 // Measured, labels of one iteration: 1e6 x 256 fp32, 1 024 clusters 1.60 -> 0.54 ms (three fp16 products
 // per pair and the listed samples in fp32 before), 1e6 x 100 fp64, 100 clusters 0.54 -> 0.10 ms (fp64 products
 // before).  Bound by the matrix cores for many clusters (1.07e15 operations per second, where a large
@@ -53,7 +60,7 @@ struct TileArea {
     int S;              // steps of 16 features
     int n_blocks;       // blocks of 32 centroids
     int64_t n_tiles;    // tiles of 32 samples (even)
-    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_list, off_thr, off_rest, total;
+    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_half, off_list, off_thr, off_rest, total;
 };
 
 inline TileArea tile_area(int64_t n, int d, int k) {
@@ -67,7 +74,8 @@ inline TileArea tile_area(int64_t n, int d, int k) {
     a.off_ct = a.off_err + kmx_align256((size_t)a.n_tiles * 32 * sizeof(float));
     a.off_hneg = a.off_ct + (size_t)a.n_blocks * a.S * 1024;
     a.off_cmax = a.off_hneg + kmx_align256((size_t)a.n_blocks * 32 * sizeof(float));
-    a.off_list = a.off_cmax + kmx_align256((size_t)a.n_blocks * sizeof(float2));
+    a.off_half = a.off_cmax + kmx_align256((size_t)a.n_blocks * sizeof(float2));
+    a.off_list = a.off_half + kmx_align256((size_t)k * sizeof(double));
     a.off_thr = a.off_list + kmx_align256((size_t)n * sizeof(int));
     a.off_rest = a.off_thr + kmx_align256((size_t)n * sizeof(float));
     a.total = a.off_rest + kmx_align256((size_t)n * sizeof(int));
@@ -323,6 +331,24 @@ __device__ __forceinline__ void lds_wait(v4f& a, v4f& b, v4f& c, v4f& d) {
 // Blocks of centroid tiles in each of the three LDS buffers of STREAM mode (S kilobytes a block)
 constexpr int stream_blocks(int S) { return S >= 8 ? 2 : S >= 4 ? 4 : 8; }
 
+// over all blocks of centroids: max 0.5 |c'|^2 and max |e_c| (uniform)
+__device__ __forceinline__ float2 reduce_block_max(const float2* __restrict__ block_max, int n_blocks) {
+    float2 v = make_float2(0.0f, 0.0f);
+    for (int b = threadIdx.x & 63; b < n_blocks; b += 64) {
+        const float2 m = block_max[b];
+        v.x = fmaxf(v.x, m.x);
+        v.y = fmaxf(v.y, m.y);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        v.x = fmaxf(v.x, __shfl_xor(v.x, off, 64));
+        v.y = fmaxf(v.y, __shfl_xor(v.y, off, 64));
+    }
+    v.x = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v.x)));
+    v.y = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v.y)));
+    return v;
+}
+
 constexpr int PEND = 128;  // entries a wave gathers before it adds them to the list
 
 // NCOL: tiles of 32 samples per wave.  STREAM: the centroid tiles do not fit the LDS and travel
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     const uint4* __restrict__ xt, const float* __restrict__ norm, const float* __restrict__ err,
     const uint4* __restrict__ ct, const float* __restrict__ hneg, const float2* __restrict__ block_max,
     unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status, uint32_t* __restrict__ labels,
-    int* __restrict__ list, float* __restrict__ list_thr, int64_t n, int n_blocks) {
+    int* __restrict__ list, float* __restrict__ list_thr, int64_t n, int n_blocks, float prod_rho) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
     extern __shared__ __align__(16) unsigned char tiles_lds[];
     constexpr int CB = STREAM ? stream_blocks(S) : 1;
@@ -370,19 +396,8 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     };
     if constexpr (!STREAM) copy_tiles(ct, 0, n_blocks * S);
 
-    float hmax = 0.0f, emax = 0.0f;  // over all blocks of centroids
-    for (int b = lane; b < n_blocks; b += 64) {
-        const float2 m = block_max[b];
-        hmax = fmaxf(hmax, m.x);
-        emax = fmaxf(emax, m.y);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        hmax = fmaxf(hmax, __shfl_xor(hmax, off, 64));
-        emax = fmaxf(emax, __shfl_xor(emax, off, 64));
-    }
-    hmax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(hmax)));
-    emax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(emax)));
+    const float2 most = reduce_block_max(block_max, n_blocks);
+    const float hmax = most.x, emax = most.y;
     const float cmax = sqrtf(2.0f * hmax) * 1.0001f;
     const float rho = ULP * (17.0f * (float)S + 4.0f);
     float pos_inf = kmx_inf<float>();
@@ -558,7 +573,14 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
             const float delta = rho * fmaf(sqrtf(nx2) * 1.0001f, cmax, hmax);
             const float eps = (ex + emax) * 1.0001f;
             const float d2 = fmaxf(nx2 * 1.00005f - 2.0f * bb + 2.0f * delta, 0.0f);
-            const float thr = (2.0f * delta + 2.0f * eps * (sqrtf(d2) + eps)) * 1.0001f;
+            float thr = (2.0f * delta + 2.0f * eps * (sqrtf(d2) + eps)) * 1.0001f;
+            if (prod_rho > 0.0f) {  // MATCH
+                const float cfull = cmax + emax;
+                const float e_prod = prod_rho * fmaf(sqrtf(nx2) * 1.0001f + ex, cfull, 0.5f * cfull * cfull);
+                const float near = sqrtf(fmaxf(nx2 * 0.99995f - 2.0f * bb - 2.0f * delta, 0.0f));
+                const float ratio = near + eps > 0.0f ? (near + 2.0f * eps) / (near + eps) : 2.0f;
+                thr += 2.0f * e_prod * ratio * 1.0001f;
+            }
             // (a NaN anywhere makes the sample uncertain)
             const bool unsure = mine && !(bb - sec > thr);
             const unsigned long long um = __ballot(unsure);
@@ -566,7 +588,7 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
                 if (unsure) {
                     const int at = pending + __popcll(um & ((1ull << lane) - 1ull));
                     pend_i[wave][at] = (int)i;
-                    pend_thr[wave][at] = bb - thr;
+                    pend_thr[wave][at] = bb - thr - ULP * fabsf(bb);  // (rounded down)
                 }
                 pending += __popcll(um);
                 if (pending > PEND - 32) flush();
@@ -584,16 +606,30 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
 // centroids dealt out to the four waves, the next block's tiles in flight), then their squared distances
 // are taken in fp64 from the exact rows, eight lanes per sample; the lowest index wins a tie.  Bound
 // by trips to memory: a few percent of the samples are listed in the usual run.
+// MATCH (fp32 inputs): candidates whose squared distances are not 4 E apart are decided by the scores of
+// the product: pair p of a sample and a candidate is row and column p of 32 x 32 blocks of
+// v_mfma_f32_32x32x2_f32, features in order from -0.5 |c|^2 (`half_norms`), of which the diagonal counts.
 constexpr int CAND = 8;
-template <typename T, int S>
+template <typename T, int S, bool MATCH>
 __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const T* __restrict__ X_rm, const T* __restrict__ cpack, const uint4* __restrict__ xt, const uint4* __restrict__ ct,
     const float* __restrict__ hneg, unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status,
     uint32_t* __restrict__ labels, const int* __restrict__ list, const float* __restrict__ list_thr, int* __restrict__ rest,
-    int64_t n, int d, int dpad, int k, int n_blocks) {
+    int64_t n, int d, int dpad, int k, int n_blocks, const float2* __restrict__ block_max,
+    const float* __restrict__ half_norms, float prod_rho) {
+    static_assert(!MATCH || sizeof(T) == 4, "fp64 inputs: labels by fp64 distances");
     if (status != nullptr && status->state != KMX_RUNNING) return;
     __shared__ int cand_n[32];
     __shared__ int cand[32][CAND];
+    __shared__ int n_pairs;                                     // MATCH: pairs to be decided by scores
+    __shared__ uint16_t pair_s[MATCH ? 32 * CAND : 1];          // sample * CAND + candidate
+    __shared__ float score_s[MATCH ? 32 : 1][CAND];
+    __shared__ bool close_s[32];
+    double c_most = 0.0;  // max |c|, unscaled
+    if constexpr (MATCH) {
+        const float2 most = reduce_block_max(block_max, n_blocks);
+        c_most = (sqrt(2.0 * (double)most.x) * 1.0001 + (double)most.y) / (double)__uint_as_float(header[TH_SCALE]);
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, j = lane & 31;
     const int64_t n_listed = (int64_t)header[TH_LISTED];
@@ -603,7 +639,11 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
         const bool live = slot < n_listed;
         const int i = list[live ? slot : t0];
         const float thr = live ? list_thr[slot] : kmx_inf<float>();
-        if (threadIdx.x < 32) cand_n[j] = (live && !too_many) ? 0 : CAND + 1;
+        if (threadIdx.x < 32) {
+            cand_n[j] = (live && !too_many) ? 0 : CAND + 1;
+            close_s[j] = false;
+        }
+        if (MATCH && threadIdx.x == 0) n_pairs = 0;
         __syncthreads();
         if (!too_many && wave < n_blocks) {
             const uint4* __restrict__ xs = xt + (size_t)(i >> 5) * S * 64 + h * 32 + (i & 31);
@@ -649,7 +689,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
         const bool here = sl < n_listed;
         const int is = list[here ? sl : t0];
         const bool fine = here && nc >= 1 && nc <= CAND;
-        double best = __builtin_huge_val();
+        double best = __builtin_huge_val(), next = __builtin_huge_val(), x_sq = 0.0;
         int arg = 0x7fffffff;
         const T* __restrict__ row = X_rm + (size_t)is * d;
         int most = fine ? nc : 0;
@@ -666,6 +706,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
 #pragma unroll 8
             for (int f = e; f < d; f += 8) {
                 const double xv = (double)row[f];
+                if (MATCH && m == 0) x_sq = fma(xv, xv, x_sq);
                 const double da = xv - (double)ra[f], db = xv - (double)rb[f];
                 sa = fma(da, da, sa);
                 sb = fma(db, db, sb);
@@ -675,16 +716,34 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
                 sa += __shfl_xor(sa, off, 64);
                 sb += __shfl_xor(sb, off, 64);
             }
-            if (fine && m < nc && (sa < best || (sa == best && ca < arg))) {
-                best = sa;
-                arg = ca;
+            if (fine && m < nc) {
+                next = fmin(next, fmax(sa, best));
+                if (sa < best || (sa == best && ca < arg)) {
+                    best = sa;
+                    arg = ca;
+                }
             }
-            if (fine && m + 1 < nc && (sb < best || (sb == best && cb < arg))) {
-                best = sb;
-                arg = cb;
+            if (fine && m + 1 < nc) {
+                next = fmin(next, fmax(sb, best));
+                if (sb < best || (sb == best && cb < arg)) {
+                    best = sb;
+                    arg = cb;
+                }
             }
         }
-        if (e == 0 && here) {
+        bool close = false;
+        if constexpr (MATCH) {
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) x_sq += __shfl_xor(x_sq, off, 64);
+            const double e_prod = (double)prod_rho * (sqrt(x_sq) + 0.5 * c_most) * c_most;
+            close = fine && nc > 1 && !(next - best > 4.001 * e_prod + (d + 8) * 2.3e-16 * (next + best));
+            if (close && e == 0) {
+                const int at = atomicAdd(&n_pairs, nc);
+                for (int m = 0; m < nc; ++m) pair_s[at + m] = (uint16_t)(js * CAND + m);
+                close_s[js] = true;
+            }
+        }
+        if (e == 0 && here && !close) {
             // (no candidate at all, or a distance that is not a number: left to the tiled product too)
             if (fine && arg < k)
                 labels[is] = (uint32_t)arg;
@@ -692,12 +751,58 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
                 rest[atomicAdd(header + TH_REST, 1u)] = is;
         }
         __syncthreads();
+        if constexpr (MATCH) {
+            for (int b = wave; 32 * b < n_pairs; b += 4) {
+                const int p = 32 * b + j;
+                const int pair = pair_s[p < n_pairs ? p : 0], c = cand[pair / CAND][pair % CAND];
+                const float* __restrict__ xr = X_rm + (size_t)list[t0 + pair / CAND] * d;
+                const float* __restrict__ cr = cpack + (size_t)c * dpad;
+                const float start = -half_norms[c];
+                v16f acc;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[r] = start;
+                for (int f0 = 0; f0 < d; f0 += 16) {
+                    float xv[8], cv[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const int f = f0 + 2 * u + h;
+                        xv[u] = f < d ? xr[f] : 0.0f;
+                        cv[u] = f < d ? cr[f] : 0.0f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(cv[u], xv[u], acc, 0, 0, 0);
+                }
+                // the diagonal: row j is register 4 (j / 8) + j % 4 of half (j / 4) % 2
+                float v = acc[0];
+#pragma unroll
+                for (int r = 1; r < 16; ++r) v = r == 4 * (j >> 3) + (j & 3) ? acc[r] : v;
+                if (p < n_pairs && h == ((j >> 2) & 1)) score_s[pair / CAND][pair % CAND] = v;
+            }
+            __syncthreads();
+            if (threadIdx.x < 32 && close_s[j]) {
+                float top = -kmx_inf<float>();
+                int lab = 0x7fffffff;
+                bool finite = true;
+                for (int m = 0; m < cand_n[j]; ++m) {
+                    const float v = score_s[j][m];
+                    finite &= fabsf(v) < kmx_inf<float>();
+                    if (v > top || (v == top && cand[j][m] < lab)) {
+                        top = v;
+                        lab = cand[j][m];
+                    }
+                }
+                const int ic = list[t0 + j];
+                if (finite) labels[ic] = (uint32_t)lab;
+                else rest[atomicAdd(header + TH_REST, 1u)] = ic;
+            }
+            __syncthreads();
+        }
     }
 }
 
 template <int S, int NCOL, bool STREAM>
 int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                      hipStream_t stream) {
+                      float prod_rho, hipStream_t stream) {
     const size_t hneg_bytes = ((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023;
     const size_t lds = hneg_bytes + (STREAM ? (size_t)3 * stream_blocks(S) * S * 1024 : (size_t)a.n_blocks * S * 1024);
     if (lds > 64 * 1024) {
@@ -711,7 +816,7 @@ int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* sta
                        (const uint4*)(area + a.off_xt), (const float*)(area + a.off_norm), (const float*)(area + a.off_err),
                        (const uint4*)(area + a.off_ct), (const float*)(area + a.off_hneg),
                        (const float2*)(area + a.off_cmax), (unsigned int*)area, status, labels,
-                       (int*)(area + a.off_list), (float*)(area + a.off_thr), n, a.n_blocks);
+                       (int*)(area + a.off_list), (float*)(area + a.off_thr), n, a.n_blocks, prod_rho);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
@@ -720,17 +825,17 @@ constexpr size_t TILES_LDS_MAX = 148 * 1024;  // (beside the 8 KB of the waves' 
 
 template <int S>
 int32_t launch_labels_s(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                        hipStream_t stream) {
+                        float prod_rho, hipStream_t stream) {
     const size_t resident = (((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023) + (size_t)a.n_blocks * S * 1024;
     const bool in_lds = resident <= TILES_LDS_MAX;
     // two columns per wave (a centroid fragment read from LDS serves two products) unless that leaves
     // compute units without a wave
     const bool two = n >= (int64_t)64 * 8 * kmx_num_cus() / 2;
     if (in_lds)
-        return two ? launch_labels<S, 2, false>(a, area, status, labels, n, stream)
-                   : launch_labels<S, 1, false>(a, area, status, labels, n, stream);
-    return two ? launch_labels<S, 2, true>(a, area, status, labels, n, stream)
-               : launch_labels<S, 1, true>(a, area, status, labels, n, stream);
+        return two ? launch_labels<S, 2, false>(a, area, status, labels, n, prod_rho, stream)
+                   : launch_labels<S, 1, false>(a, area, status, labels, n, prod_rho, stream);
+    return two ? launch_labels<S, 2, true>(a, area, status, labels, n, prod_rho, stream)
+               : launch_labels<S, 1, true>(a, area, status, labels, n, prod_rho, stream);
 }
 
 }  // namespace
@@ -795,8 +900,11 @@ KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
             (const float*)area + TH_SCALE, a.S};
 }
 
+char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k) { return area + tile_area(n, d, k).off_half; }
+
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace
-// holds them).  `status` null: labels whatever the state.
+// holds them).  `status` null: labels whatever the state, those of kmx_assign_labels, whose half norms
+// `half_norms` are then.
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream) {
@@ -811,9 +919,12 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
     else
         hipLaunchKernelGGL((tiles_centroids_kernel<double>), dim3((unsigned)a.n_blocks), dim3(256), 0, stream,
                            (const double*)centroids_t, ct, hneg, cmax, header, status, d, k, a.S);
+    // (an fp32 score: d + 1 roundings of partial sums, as many of the half norm)
+    const bool match = status == nullptr && dtype == KMX_F32;
+    const float prod_rho = match ? ULP * (float)(d + 8) : 0.0f;
     int32_t rc = KMX_ERR_UNSUPPORTED;
     switch (a.S) {
-#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, n, stream); break
+#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, n, prod_rho, stream); break
         KMX_TILES_CASE(1); KMX_TILES_CASE(2); KMX_TILES_CASE(3); KMX_TILES_CASE(4);
         KMX_TILES_CASE(5); KMX_TILES_CASE(6); KMX_TILES_CASE(7); KMX_TILES_CASE(8);
         KMX_TILES_CASE(9); KMX_TILES_CASE(10); KMX_TILES_CASE(11); KMX_TILES_CASE(12);
@@ -826,14 +937,16 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
     int* rest = (int*)(area + a.off_rest);
     int64_t grid = kmx_cdiv(n, 32);
     if (grid > 4 * (int64_t)kmx_num_cus()) grid = 4 * (int64_t)kmx_num_cus();
-#define KMX_TILES_RESOLVE(T, S_)                                                                                         \
-    hipLaunchKernelGGL((tiles_resolve_kernel<T, S_>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor,   \
+#define KMX_TILES_RESOLVE(T, S_, M_)                                                                                     \
+    hipLaunchKernelGGL((tiles_resolve_kernel<T, S_, M_>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor,   \
                        (const T*)cpack, (const uint4*)(area + a.off_xt), ct, hneg, header, status, labels, list, thr,    \
-                       rest, n, d, dpad, k, a.n_blocks)
+                       rest, n, d, dpad, k, a.n_blocks, cmax, (const float*)half_norms, prod_rho)
     switch (a.S) {
 #define KMX_TILES_CASE(S_)                                                                         \
     case S_:                                                                                       \
-        if (dtype == KMX_F32) KMX_TILES_RESOLVE(float, S_); else KMX_TILES_RESOLVE(double, S_);    \
+        if (match) KMX_TILES_RESOLVE(float, S_, true);                                             \
+        else if (dtype == KMX_F32) KMX_TILES_RESOLVE(float, S_, false);                            \
+        else KMX_TILES_RESOLVE(double, S_, false);                                                 \
         break
         KMX_TILES_CASE(1); KMX_TILES_CASE(2); KMX_TILES_CASE(3); KMX_TILES_CASE(4);
         KMX_TILES_CASE(5); KMX_TILES_CASE(6); KMX_TILES_CASE(7); KMX_TILES_CASE(8);

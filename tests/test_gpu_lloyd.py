@@ -246,6 +246,31 @@ def test_labels_of_a_resident_run_taken_twice_and_midway(cuda, n, d, k, data):
     np.testing.assert_array_equal(again.run(6).cpu().numpy(), expected)
 
 
+# whole-numbered features, many samples nearly as far from two centroids; the wide fp32 step, the tiled product, an
+# odd number of features, the largest number of 16-feature steps, and data where the screen settles next to nothing
+@pytest.mark.parametrize("n,d,k,values,offset", [(1_000_000, 100, 300, 3, 0), (400_000, 101, 64, 2, 0), (300_000, 256, 1000, 2, 0),
+                                                 (200_003, 70, 300, 2, 0), (60_000, 100, 300, 3, 2000), (200_000, 129, 65, 3, 300)])
+@pytest.mark.parametrize("seed", [1, 2])
+def test_labels_of_a_run_are_those_of_its_centroids(cuda, n, d, k, values, offset, seed):
+    """labels_ of a fit and predict() on the same data: equal, near ties included."""
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    gen = torch.Generator(device=cuda).manual_seed(seed)
+    X = torch.randint(0, values, (n, d), generator=gen, device=cuda).float()
+    X[:, 0] += offset
+    w = torch.ones(n, device=cuda)
+    assert lib.kmx_lloyd_resident_bytes(_capi.lloyd_plan(n, d, k, _capi.KMX_F32, 0)) > 0
+    X_t = X.T.contiguous()
+    for iters in (1, 3):
+        labels, _, centroids_t, _ = drivers.lloyd(X_t, w, X[:k].T.contiguous(), True, iters, False, 0.0, flags=0)
+        expected, _ = drivers.get_labels_inertia(X_t, centroids_t, w, True)
+        assert int((labels != expected).sum()) == 0
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
