@@ -88,48 +88,46 @@ __device__ __forceinline__ _Float16 to_half(float v) {
 
 // The scale: a power of two that brings the largest centroid coordinate into [2^10, 2^11), which
 // leaves samples 32 times further out inside fp16 (beyond it they become infinite and get no
-// certificate).  One workgroup.
-// (`m`: the largest magnitude a thread has seen)
-__device__ __forceinline__ void tiles_write_scale(float m, float* m_s, unsigned int* __restrict__ header) {
+// certificate), but not the largest coordinate of 256 samples spread over X below 1: initial
+// centroids far from all samples would round the samples away for the whole run, though the first
+// relocation removes them (1e6 x 100 fp64, 100 clusters of which 3 start at 1e8: 27.5 -> 6.6 ms for
+// ten iterations).  One workgroup.
+// The exponent that brings m into [2^at, 2^(at + 1)), within what a float holds after scaling either
+// way; none: lower than any.
+constexpr int NO_EXPONENT = -1000;
+__device__ __forceinline__ int scale_exponent(float m, int at) {
+    if (!(m > 0.0f && m < kmx_inf<float>())) return NO_EXPONENT;
+    const int e = at - ilogbf(m);
+    return e > 100 ? 100 : e < -100 ? -100 : e;
+}
+
+// (`high`, `low`: the largest magnitudes a thread has seen of what goes to 2^10 and of what stays above 1)
+__device__ __forceinline__ void tiles_write_scale(float high, float low, float (*m_s)[16], unsigned int* __restrict__ header) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) m_s[threadIdx.x >> 6] = m;
+    for (int off = 32; off > 0; off >>= 1) {
+        high = fmaxf(high, __shfl_xor(high, off, 64));
+        low = fmaxf(low, __shfl_xor(low, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        m_s[0][threadIdx.x >> 6] = high;
+        m_s[1][threadIdx.x >> 6] = low;
+    }
     __syncthreads();
     if (threadIdx.x < TH_WORDS) header[threadIdx.x] = 0u;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int i = 1; i < 16; ++i) m = fmaxf(m, m_s[i]);
-        // (the exponent within what a float holds after scaling either way)
-        float xs = 1.0f;
-        if (m > 0.0f && m < kmx_inf<float>()) {
-            int e = 10 - ilogbf(m);
-            e = e > 100 ? 100 : e < -100 ? -100 : e;
-            xs = ldexpf(1.0f, e);
+        for (int i = 1; i < 16; ++i) {
+            high = fmaxf(high, m_s[0][i]);
+            low = fmaxf(low, m_s[1][i]);
         }
-        header[TH_SCALE] = __float_as_uint(xs);
+        const int eh = scale_exponent(high, 10), el = scale_exponent(low, 0), e = eh > el ? eh : el;
+        header[TH_SCALE] = __float_as_uint(e == NO_EXPONENT ? 1.0f : ldexpf(1.0f, e));
     }
 }
 
+// largest magnitude in this thread's share of 256 samples spread over X
 template <typename T>
-__global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__ centroids_t, unsigned int* __restrict__ header,
-                                                           int items) {
-    __shared__ float m_s[16];
-    float m = 0.0f;
-    for (int i0 = threadIdx.x; i0 < items; i0 += 16 * 1024) {
-        float v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = i0 + u * 1024 < items ? fabsf((float)centroids_t[i0 + u * 1024]) : 0.0f;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
-    }
-    tiles_write_scale(m, m_s, header);
-}
-
-// The same from 256 samples spread over X, where there are no centroids yet.  One workgroup.
-template <typename T>
-__global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __restrict__ X_t, unsigned int* __restrict__ header,
-                                                                  int64_t n, int d) {
-    __shared__ float m_s[16];
+__device__ __forceinline__ float sampled_max(const T* __restrict__ X_t, int64_t n, int d) {
     const int64_t i = (int64_t)(threadIdx.x & 255) * n / 256;
     float m = 0.0f;
     for (int f0 = threadIdx.x >> 8; f0 < d; f0 += 4 * 16) {
@@ -139,7 +137,30 @@ __global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __res
 #pragma unroll
         for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
     }
-    tiles_write_scale(m, m_s, header);
+    return m;
+}
+
+template <typename T>
+__global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__ centroids_t, const T* __restrict__ X_t,
+                                                           unsigned int* __restrict__ header, int items, int64_t n, int d) {
+    __shared__ float m_s[2][16];
+    float m = 0.0f;
+    for (int i0 = threadIdx.x; i0 < items; i0 += 16 * 1024) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = i0 + u * 1024 < items ? fabsf((float)centroids_t[i0 + u * 1024]) : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
+    }
+    tiles_write_scale(m, sampled_max(X_t, n, d), m_s, header);
+}
+
+// The same where there are no centroids yet: from the samples alone.  One workgroup.
+template <typename T>
+__global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __restrict__ X_t, unsigned int* __restrict__ header,
+                                                                  int64_t n, int d) {
+    __shared__ float m_s[2][16];
+    tiles_write_scale(sampled_max(X_t, n, d), 0.0f, m_s, header);
 }
 
 // The tiles, |x'|^2 and |e_x| per sample, the row-major copy of X and (absmax not null) the bits of
@@ -871,9 +892,11 @@ int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroi
                           int64_t n, int d, int k, int dtype, hipStream_t stream) {
     unsigned int* header = (unsigned int*)area;
     if (dtype == KMX_F32)
-        hipLaunchKernelGGL((tiles_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)centroids_t, header, d * k);
+        hipLaunchKernelGGL((tiles_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)centroids_t,
+                           (const float*)X_t, header, d * k, n, d);
     else
-        hipLaunchKernelGGL((tiles_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)centroids_t, header, d * k);
+        hipLaunchKernelGGL((tiles_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)centroids_t,
+                           (const double*)X_t, header, d * k, n, d);
     tiles_copy(X_t, X_rowmajor, area, absmax, n, d, dtype, stream);
     KMX_LAUNCH_CHECK();
     return KMX_OK;

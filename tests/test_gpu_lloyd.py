@@ -246,6 +246,35 @@ def test_labels_of_a_resident_run_taken_twice_and_midway(cuda, n, d, k, data):
     np.testing.assert_array_equal(again.run(6).cpu().numpy(), expected)
 
 
+@pytest.mark.parametrize("n,d,k,dtype,far", [(20_001, 100, 300, np.float32, 1e8), (65_600, 100, 100, np.float64, 1e8),
+                                             (20_001, 129, 300, np.float32, -3e4), (20_001, 129, 300, np.float64, 1e200)])
+def test_initial_centroids_far_from_all_samples(cuda, n, d, k, dtype, far):
+    """The half-precision copy keeps the samples' digits whatever the initial centroids are: as soon as those have been
+    relocated, the labelling certifies samples again."""
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d)
+    X = (rng.uniform(-2, 2, (k, d))[rng.integers(0, k, n)] + rng.standard_normal((n, d))).astype(dtype)
+    init = X[:k].copy()
+    init[1:4] = far
+    run = _ResidentRun(cuda, X, np.ones(n, dtype=dtype), init, 6)
+    run.run(6)
+    assert (run.status.state, run.status.n_iter, run.status.n_empty) == (_capi.KMX_NEED_RELOCATION, 0, 3)
+    run.cent[1] /= run.sizes.clamp(min=1)  # (the sums of the first iteration), and samples for the empty clusters
+    run.cent[1][:, 1:4] = _dev(X[k:k + 3].T, cuda)
+    centroids_t = run.cent[1].clone()
+    run.sizes.fill_(1)
+    run.check(run.lib.kmx_lloyd_finalize(run.plan, run.ptr(run.cent[0]), run.ptr(run.cent[1]), run.ptr(run.sizes),
+                                         run.ptr(run.ws), run.ws_bytes, run.stream), "kmx_lloyd_finalize")
+    np.testing.assert_array_equal(run.cent[1].cpu().numpy(), centroids_t.cpu().numpy())
+    run.n_done = 1
+    labels, _ = run.labels_inertia()
+    assert run.listed() < n // 8
+    expected, _ = drivers.get_labels_inertia(run.X_t, centroids_t, run.w, True)
+    np.testing.assert_array_equal(labels, expected.cpu().numpy())
+
+
 # whole-numbered features, many samples nearly as far from two centroids; the wide fp32 step, the tiled product, an
 # odd number of features, the largest number of 16-feature steps, and data where the screen settles next to nothing
 @pytest.mark.parametrize("n,d,k,values,offset", [(1_000_000, 100, 300, 3, 0), (400_000, 101, 64, 2, 0), (300_000, 256, 1000, 2, 0),
