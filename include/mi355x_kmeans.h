@@ -70,7 +70,10 @@ typedef struct kmx_lloyd_status {
     double tol;           /* loop runs while shift_sum > tol                               */
     int32_t max_iter;
     uint32_t ticket;      /* internal: block counter of the reduction kernel               */
-    uint64_t reserved0;
+    int32_t uncertified_iter;  /* 1 + the first iteration whose labels the half-precision copy
+                                  (kmx_lloyd_init_resident) left mostly unsettled; 0: none since
+                                  the start or the last relocation                         */
+    int32_t reserved0;
     int64_t reserved[2];
 } kmx_lloyd_status;       /* 64 bytes */
 
@@ -197,7 +200,7 @@ int32_t kmx_lloyd_trace_collect(float* kernel_ms_mean, float* kernel_ms_min, int
 /* Iterations n_done, n_done + 1, ... until the state is no longer KMX_RUNNING or max_iter (the value
  * given to kmx_lloyd_init) is reached: enqueues kmx_lloyd_iter a few ahead of the last one that has
  * announced itself to the host and returns with what it learned in status_host (n_iter, state,
- * n_empty, shift_sum).  Iteration j reads the centroids and previous labels of its parity and
+ * n_empty, shift_sum, uncertified_iter).  Iteration j reads the centroids and previous labels of its parity and
  * writes those of the other one: centroids_even holds the initial centroids, and iteration 0 writes
  * centroids_odd and labels_odd.  After KMX_NEED_RELOCATION the caller relocates, calls
  * kmx_lloyd_finalize and comes back with n_done = status.n_iter + 1 if the run goes on.  Waits for
@@ -217,7 +220,10 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
  * kmx_lloyd_resident_bytes: how much (0: the plan's kernels have no use for it).
  * kmx_lloyd_init_resident is kmx_lloyd_init and fills, in the same pass over X_t, `resident` and the
  * row-major copy X_rowmajor (OUT, n x d).  Both are then handed to kmx_lloyd_run, whose
- * `resident` may be NULL (labels from X_t).  kmx_lloyd_labels_inertia gives the labels for the
+ * `resident` may be NULL (labels from X_t).  Data that half precision cannot tell apart (one feature
+ * much wider than the others, say) go back to X_t within the run: from iteration 1 on if iteration 0 left
+ * more than an eighth of the samples without a certificate, else three iterations behind the first that
+ * does; after a relocation the copy is tried again.  kmx_lloyd_labels_inertia gives the labels for the
  * centroids such a run has come to (centroids_t and the workspace as the run left them; n_iter is not
  * read), the same as kmx_assign_labels gives for them, and their inertia; inertia_workspace as for
  * kmx_inertia.  It leaves the run's state alone: it may be called again, and the run may go on after it.

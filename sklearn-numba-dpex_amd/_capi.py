@@ -67,7 +67,8 @@ class LloydStatus(ctypes.Structure):
         ("tol", c_double),
         ("max_iter", c_int32),
         ("ticket", ctypes.c_uint32),
-        ("reserved0", ctypes.c_uint64),
+        ("uncertified_iter", c_int32),
+        ("reserved0", c_int32),
         ("reserved", c_int64 * 2),
     ]
 

@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
         status->ticket = 0;
         if (base > 0) {
             status->state = KMX_NEED_RELOCATION;
-            lloyd_publish(progress, status->n_iter, KMX_NEED_RELOCATION, base, status->shift_sum);
+            lloyd_publish(progress, status, status->n_iter, KMX_NEED_RELOCATION, base, status->shift_sum);
         }
     }
 }
@@ -541,6 +541,7 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
         for (unsigned int b = 0; b < gridDim.x; ++b)
             total += __builtin_nontemporal_load(shift_partial + b);
         status->ticket = 0;
+        if (force) status->uncertified_iter = 0;  // (other centroids: the half-precision copy is tried again)
         lloyd_update_status(status, total, status->n_changed, progress);
     }
 }
@@ -596,6 +597,7 @@ __global__ __launch_bounds__(256) void lloyd_pack_kernel(const T* __restrict__ c
         status->tol = tol;
         status->max_iter = max_iter;
         status->ticket = 0;
+        status->uncertified_iter = 0;
         status->reserved0 = 0;
         status->reserved[0] = 0;
         status->reserved[1] = 0;
@@ -1213,7 +1215,8 @@ static bool progress_look(const unsigned long long* slot, kmx_lloyd_status* out)
     out->n_iter = (int32_t)(uint32_t)a;
     out->state = (int32_t)(a >> 32);
     std::memcpy(&out->shift_sum, &b, sizeof(b));
-    out->n_empty = (int32_t)c;
+    out->n_empty = (int32_t)(uint32_t)c;
+    out->uncertified_iter = (int32_t)(c >> 32);
     return true;
 }
 
@@ -1226,7 +1229,7 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
     KMX_ENTRY();
     KMX_REQUIRE_PLAN(plan);
     if (resident != nullptr && resident_bytes < kmx_lloyd_resident_bytes(plan)) return KMX_ERR_WORKSPACE;
-    if (resident != nullptr && kmx_lloyd_resident_bytes(plan) == 0) resident = nullptr;
+    if (X_rowmajor == nullptr || (resident != nullptr && kmx_lloyd_resident_bytes(plan) == 0)) resident = nullptr;
     KMX_REQUIRE_PTR(centroids_even);
     KMX_REQUIRE_PTR(centroids_odd);
     KMX_REQUIRE_PTR(labels_even);
@@ -1241,18 +1244,36 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
     // launches (4.5 us each).
     constexpr int AHEAD = 3;
     int enqueued = n_done;
+    kmx_lloyd_status seen;
+    std::memset(&seen, 0, sizeof(seen));
+    if (resident != nullptr && n_done > 0) {
+        // (what an earlier call found about the copy)
+        const int32_t rc = kmx_lloyd_status_read(workspace, &seen, stream_);
+        if (rc != KMX_OK) return rc;
+    }
+    seen.n_iter = n_done;
+    seen.state = KMX_RUNNING;
+    // Whether iteration `it` takes its labels from the copy.  What decides is known whenever an iteration is
+    // enqueued (the first one of a run is waited for), so the answer does not depend on how far the host
+    // happens to see: a run gives the same results each time.
+    auto copy_serves = [&](int it) {
+        const int bad = seen.uncertified_iter - 1;
+        return bad < 0 || !((bad == 0 && it > 0) || bad <= it - AHEAD);
+    };
     auto enqueue = [&](unsigned long long* progress) {
         const int a = enqueued & 1;
+        char* tiles = resident != nullptr && copy_serves(enqueued) ? (char*)resident : nullptr;
         const int32_t rc = lloyd_iter_dispatch(plan, X_t, X_rowmajor, sample_weight, cent[a], cent[a ^ 1], labels[a],
                                                labels[a ^ 1], cluster_sizes, empty_clusters, workspace, workspace_bytes,
-                                               stream_, nullptr, progress, (char*)resident);
+                                               stream_, nullptr, progress, tiles);
         ++enqueued;
         return rc;
     };
     unsigned long long* slot = n_done < max_iter ? progress_take() : nullptr;
     if (slot == nullptr) {
         // (nothing to run, or no slot: a look at the status per batch of iterations)
-        for (int batch = 1;; batch = batch < 16 ? 2 * batch : 16) {
+        const int most = resident != nullptr ? AHEAD - 1 : 16;
+        for (int batch = 1;; batch = 2 * batch < most ? 2 * batch : most) {
             for (int i = 0; i < batch && enqueued < max_iter; ++i) {
                 const int32_t rc = enqueue(nullptr);
                 if (rc != KMX_OK) return rc;
@@ -1260,15 +1281,12 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
             const int32_t rc = kmx_lloyd_status_read(workspace, status_host, stream_);
             if (rc != KMX_OK) return rc;
             if (status_host->state != KMX_RUNNING || enqueued >= max_iter) return KMX_OK;
+            seen.uncertified_iter = status_host->uncertified_iter;
         }
     }
-    kmx_lloyd_status seen;
-    std::memset(&seen, 0, sizeof(seen));
-    seen.n_iter = n_done;
-    seen.state = KMX_RUNNING;
     unsigned int spins = 0;
     while (true) {
-        while (enqueued < max_iter && enqueued < seen.n_iter + AHEAD) {
+        while (enqueued < max_iter && enqueued < seen.n_iter + (resident != nullptr && seen.n_iter == 0 ? 1 : AHEAD)) {
             const int32_t rc = enqueue(slot);
             if (rc != KMX_OK) return rc;  // (the slot stays taken: launches before this one may still write to it)
         }

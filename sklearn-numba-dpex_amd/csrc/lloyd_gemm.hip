@@ -109,9 +109,12 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t,
     const float* __restrict__ half_norms, uint32_t* __restrict__ labels,
     const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
-    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
+    const unsigned int* __restrict__ all_count = nullptr, int64_t all_from = 0) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int64_t n_work = LISTED ? (int64_t)*list_count : n;
+    // (LISTED: every sample, in order, if *all_count >= all_from)
+    if (LISTED && all_count != nullptr && (int64_t)*all_count >= all_from) list = nullptr;
+    const int64_t n_work = LISTED && list != nullptr ? (int64_t)*list_count : n;
     constexpr int GK = NA == 1 ? 2 * GK32 : GK32;           // features per stage
     constexpr int XL = GK / 8;                              // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                              // groups of four columns per centroid row
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int64_t slot = i0 + 4 * (threadIdx.x & 31) + e;
-                cols[e] = slot < n_work ? list[slot] : -1;
+                cols[e] = slot < n_work ? (list != nullptr ? list[slot] : (int)slot) : -1;
             }
         }
         auto load_x = [&](float4(&r)[XL], const int f0) {
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
         const int oi = __shfl_xor(bidx, 32, 64);
         if (ob > best || (ob == best && oi < bidx)) bidx = oi;
         const int64_t slot = i0 + 32 * wave + j;
-        if (h == 0 && slot < n_work) labels[LISTED ? (int64_t)list[slot] : slot] = (uint32_t)bidx;
+        if (h == 0 && slot < n_work) labels[LISTED && list != nullptr ? (int64_t)list[slot] : slot] = (uint32_t)bidx;
     }
 }
 
@@ -271,9 +274,12 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
     const double* __restrict__ X_t, const double* __restrict__ centroids_t,
     const double* __restrict__ half_norms, uint32_t* __restrict__ labels,
     const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
-    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
+    const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
+    const unsigned int* __restrict__ all_count = nullptr, int64_t all_from = 0) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    const int64_t n_work = LISTED ? (int64_t)*list_count : n;
+    // (LISTED: every sample, in order, if *all_count >= all_from)
+    if (LISTED && all_count != nullptr && (int64_t)*all_count >= all_from) list = nullptr;
+    const int64_t n_work = LISTED && list != nullptr ? (int64_t)*list_count : n;
     constexpr int GK = NA == 2 ? 2 * GK64 : GK64;  // features per stage
     constexpr int XL = GK / 4;                     // 128-bit loads per thread and stage, samples
     constexpr int CG = 8 * NA;                     // pairs of columns per centroid row
@@ -297,7 +303,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const int64_t slot = i0 + 2 * (threadIdx.x & 63) + e;
-                cols[e] = slot < n_work ? list[slot] : -1;
+                cols[e] = slot < n_work ? (list != nullptr ? list[slot] : (int)slot) : -1;
             }
         }
         auto load_x = [&](double2(&r)[XL], const int f0) {
@@ -382,7 +388,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
                 }
             }
             const int64_t slot = i0 + 32 * wave + 16 * b + j;
-            if (g == 0 && slot < n_work) labels[LISTED ? (int64_t)list[slot] : slot] = (uint32_t)bidx[b];
+            if (g == 0 && slot < n_work) labels[LISTED && list != nullptr ? (int64_t)list[slot] : slot] = (uint32_t)bidx[b];
         }
     }
 }
@@ -423,19 +429,20 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
 }
 
 // The same kernels on the samples list[0 .. count) (list and count on the device): what a screened
-// label kernel could not certify.  The grid covers the worst case; workgroups without a tile of the
-// list leave at once.
+// label kernel could not certify; on all samples if there is an `all_count` and it has come to all_from.
+// The grid covers the worst case; workgroups without a tile of the list leave at once.
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
                                      const unsigned int* list_count, int64_t n, int d, int k,
-                                     int32_t dtype, hipStream_t stream) {
+                                     int32_t dtype, hipStream_t stream, const unsigned int* all_count,
+                                     int64_t all_from) {
     const int c_vec = (k % (dtype == KMX_F32 ? 4 : 2) == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
     int64_t grid = kmx_cdiv(n, GT);
     const int64_t cap = (int64_t)(dtype == KMX_F32 ? 3 : 2) * kmx_num_cus();
     if (grid > cap) grid = cap;
 #define KMX_GEMM_LISTED(KERNEL, T)                                                                             \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t, (const T*)centroids_t, \
-                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count)
+                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count, all_count, all_from)
     if (dtype == KMX_F32) {
         if (k <= 32) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<1, true>), float);
         else if (k <= 64) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<2, true>), float);

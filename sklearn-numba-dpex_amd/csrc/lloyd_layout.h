@@ -62,7 +62,8 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
 int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, const void* half_norms,
                                      uint32_t* labels, const kmx_lloyd_status* status, const int* list,
                                      const unsigned int* list_count, int64_t n, int d, int k,
-                                     int32_t dtype, hipStream_t stream);
+                                     int32_t dtype, hipStream_t stream, const unsigned int* all_count = nullptr,
+                                     int64_t all_from = 0);
 // the same product screened on the fp16 matrix cores (lloyd_gemm_screen.hip), fp32 only
 size_t kmx_gemm_screen_bytes(int64_t n);
 bool kmx_gemm_screen_enabled(int64_t n, int d, int k, uint32_t flags);
@@ -95,7 +96,7 @@ int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, cons
                          void* out, double* workspace, int64_t n, int d, int dpad, int dtype, hipStream_t stream);
 char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k);  // room for k half norms
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
-                         const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
+                         const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);

@@ -17,11 +17,13 @@ __host__ __device__ inline unsigned long long lloyd_progress_check(unsigned long
                                                                    unsigned long long c) {
     return a ^ (b << 1 | b >> 63) ^ (c << 2 | c >> 62) ^ KMX_PROGRESS_MARK;
 }
-__device__ inline void lloyd_publish(unsigned long long* progress, int n_iter, int state, int n_empty, double shift) {
+__device__ inline void lloyd_publish(unsigned long long* progress, const kmx_lloyd_status* st, int n_iter, int state,
+                                     int n_empty, double shift) {
     if (progress == nullptr) return;
     const unsigned long long w[3] = {(unsigned long long)(unsigned int)n_iter | (unsigned long long)state << 32,
                                      (unsigned long long)__double_as_longlong(shift),
-                                     (unsigned long long)(unsigned int)n_empty};
+                                     (unsigned long long)(unsigned int)n_empty |
+                                         (unsigned long long)(unsigned int)st->uncertified_iter << 32};
     for (int i = 0; i < 3; ++i) __hip_atomic_store(&progress[i], w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&progress[3], lloyd_progress_check(w[0], w[1], w[2]), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
@@ -167,7 +169,7 @@ __device__ inline void lloyd_update_status(kmx_lloyd_status* st, double total_sh
         next = KMX_MAX_ITER;
     st->state = next;
     st->reserved[1] = (int64_t)changed;
-    lloyd_publish(progress, n_iter, next, 0, total_shift);
+    lloyd_publish(progress, st, n_iter, next, 0, total_shift);
 }
 
 // Division, packed copy, half norms, shift and convergence test by ONE workgroup of 256
@@ -385,7 +387,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         }
         if (threadIdx.x == 0) {
             a.status->state = KMX_NEED_RELOCATION;
-            lloyd_publish(a.progress, a.status->n_iter, KMX_NEED_RELOCATION, n_empty, a.status->shift_sum);
+            lloyd_publish(a.progress, a.status, a.status->n_iter, KMX_NEED_RELOCATION, n_empty, a.status->shift_sum);
             if (a.clear_word != nullptr) a.clear_word[2] = 0u;
         }
         return;

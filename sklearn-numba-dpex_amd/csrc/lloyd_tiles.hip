@@ -18,8 +18,11 @@
 // to the nearest centroid and certify far fewer samples.)  Samples without a certificate are
 // listed together with the score below which no centroid can be theirs; a second kernel looks
 // up the few centroids above it and takes their distances in fp64 from the exact rows.  A sample with
-// more such centroids than that kernel holds, or all of them if the list is long, go through
-// the tiled product of lloyd_gemm.hip.
+// more such centroids than that kernel holds goes through the tiled product of lloyd_gemm.hip.  If more than
+// an eighth of the samples are listed, all samples do, and the run takes its labels from X again
+// soon after (kmx_lloyd_run): the copy cannot tell such data apart, one feature being much wider than the
+// others for instance.  1e6 x 100 with one feature 1e5 times wider, ten iterations, before this copy / with it
+// alone / with the way back: fp32, 300 clusters 18.4 / 28.3 / 17.7 ms; fp64, 100 clusters 8.8 / 14.6 / 9.0.
 //
 // The labels that a run ends with are those that kmx_assign_labels gives for its centroids, which for
 // fp32 inputs is the arg-max of fp32 scores: there the thresholds also leave room for the errors E of two
@@ -90,7 +93,7 @@ __device__ __forceinline__ _Float16 to_half(float v) {
 // leaves samples 32 times further out inside fp16 (beyond it they become infinite and get no
 // certificate), but not the largest coordinate of 256 samples spread over X below 1: initial
 // centroids far from all samples would round the samples away for the whole run, though the first
-// relocation removes them (1e6 x 100 fp64, 100 clusters of which 3 start at 1e8: 27.5 -> 6.6 ms for
+// relocation removes them (1e6 x 100 fp64, 100 clusters of which 3 start at 1e8: 27.5 -> 5.2 ms for
 // ten iterations).  One workgroup.
 // The exponent that brings m into [2^at, 2^(at + 1)), within what a float holds after scaling either
 // way; none: lower than any.
@@ -634,7 +637,7 @@ constexpr int CAND = 8;
 template <typename T, int S, bool MATCH>
 __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const T* __restrict__ X_rm, const T* __restrict__ cpack, const uint4* __restrict__ xt, const uint4* __restrict__ ct,
-    const float* __restrict__ hneg, unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status,
+    const float* __restrict__ hneg, unsigned int* __restrict__ header, kmx_lloyd_status* __restrict__ status,
     uint32_t* __restrict__ labels, const int* __restrict__ list, const float* __restrict__ list_thr, int* __restrict__ rest,
     int64_t n, int d, int dpad, int k, int n_blocks, const float2* __restrict__ block_max,
     const float* __restrict__ half_norms, float prod_rho) {
@@ -654,19 +657,23 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, j = lane & 31;
     const int64_t n_listed = (int64_t)header[TH_LISTED];
-    const bool too_many = n_listed > (n >> 3);  // the tiled product takes them all
+    if (n_listed > (n >> 3)) {  // the tiled product takes all samples
+        if (status != nullptr && blockIdx.x == 0 && threadIdx.x == 0 && status->uncertified_iter == 0)
+            status->uncertified_iter = status->n_iter + 1;
+        return;
+    }
     for (int64_t t0 = (int64_t)blockIdx.x * 32; t0 < n_listed; t0 += (int64_t)gridDim.x * 32) {
         const int64_t slot = t0 + j;
         const bool live = slot < n_listed;
         const int i = list[live ? slot : t0];
         const float thr = live ? list_thr[slot] : kmx_inf<float>();
         if (threadIdx.x < 32) {
-            cand_n[j] = (live && !too_many) ? 0 : CAND + 1;
+            cand_n[j] = live ? 0 : CAND + 1;
             close_s[j] = false;
         }
         if (MATCH && threadIdx.x == 0) n_pairs = 0;
         __syncthreads();
-        if (!too_many && wave < n_blocks) {
+        if (wave < n_blocks) {
             const uint4* __restrict__ xs = xt + (size_t)(i >> 5) * S * 64 + h * 32 + (i & 31);
             v8h x[S];
 #pragma unroll
@@ -929,7 +936,7 @@ char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k) { return area + 
 // holds them).  `status` null: labels whatever the state, those of kmx_assign_labels, whose half norms
 // `half_norms` are then.
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
-                         const void* half_norms, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
+                         const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream) {
     const TileArea a = tile_area(n, d, k);
     unsigned int* header = (unsigned int*)area;
@@ -980,7 +987,7 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
 #undef KMX_TILES_RESOLVE
     KMX_LAUNCH_CHECK();
     return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + TH_REST, n, d, k, dtype,
-                                        stream);
+                                        stream, header + TH_LISTED, (n >> 3) + 1);
 }
 
 // samples of the last labelling that had no certificate

@@ -141,7 +141,8 @@ def lloyd(
     # labels for the final centroids and the exact inertia (kmeans/drivers.py:356-391)
     best = cent[n_iteration % 2]
     assignments_idx = labels[0]
-    if resident is None:
+    if resident is None or status.uncertified_iter:
+        # (the run has gone back from the half-precision copy to X: same labels)
         inertia = _assign_with_inertia(X_t, sample_weight, best, assignments_idx, flags)[0]
     else:
         inertia_ws_bytes = lib.kmx_inertia_workspace_bytes(n)

@@ -178,12 +178,13 @@ class _ResidentRun:
             self.plan, ptr(self.ws), self.ws_bytes, ptr(self.X_t), ptr(self.w), ptr(self.cent[0]), self.max_iter, 0.0,
             ptr(self.X_rm), ptr(self.resident), self.res_bytes, self.stream), "kmx_lloyd_init_resident")
 
-    def run(self, until):
+    def run(self, until, resident=True):
         ptr = self.ptr
         self.check(self.lib.kmx_lloyd_run(
             self.plan, ptr(self.X_t), ptr(self.X_rm), ptr(self.w), ptr(self.cent[0]), ptr(self.cent[1]),
             ptr(self.labels[0]), ptr(self.labels[1]), ptr(self.sizes), ptr(self.empty), ptr(self.ws), self.ws_bytes,
-            ptr(self.resident), self.res_bytes, self.n_done, until, self.status, self.stream), "kmx_lloyd_run")
+            ptr(self.resident) if resident else None, self.res_bytes, self.n_done, until, self.status, self.stream),
+            "kmx_lloyd_run")
         self.n_done = self.status.n_iter
         return self.cent[self.n_done % 2]
 
@@ -273,6 +274,38 @@ def test_initial_centroids_far_from_all_samples(cuda, n, d, k, dtype, far):
     assert run.listed() < n // 8
     expected, _ = drivers.get_labels_inertia(run.X_t, centroids_t, run.w, True)
     np.testing.assert_array_equal(labels, expected.cpu().numpy())
+
+
+@pytest.mark.parametrize("n,d,k,dtype", [(20_001, 100, 300, np.float32), (20_003, 129, 300, np.float32),
+                                         (65_601, 101, 100, np.float64)])
+def test_data_that_half_precision_cannot_tell_apart(cuda, n, d, k, dtype):
+    """One feature far wider than the others: the run leaves the copy after its first iteration, whatever pieces it is
+    asked for in, and comes to what a run without the copy comes to."""
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d))
+    X[:, 0] *= 100
+    X = X.astype(dtype)
+    w, init = rng.uniform(0.5, 1.5, n).astype(dtype), X[rng.choice(n, k, replace=False)]
+    plain = _ResidentRun(cuda, X, w, init, 8)
+    expected = plain.run(8, resident=False).cpu().numpy()
+    assert (plain.n_done, plain.status.uncertified_iter) == (8, 0)
+    rtol = 0 if dtype == np.float32 else 1e-12  # (fp64 sums by floating-point atomics: order of additions)
+    for stops in ([8], [1, 2, 5, 8]):
+        run = _ResidentRun(cuda, X, w, init, 8)
+        for until in stops:
+            got = run.run(until)
+            assert run.status.uncertified_iter == 1
+        assert (run.n_done, run.status.state) == (plain.n_done, plain.status.state)
+        np.testing.assert_allclose(got.cpu().numpy(), expected, rtol=rtol, atol=100 * rtol)
+        last = run.n_done % 2
+        np.testing.assert_array_equal(run.labels[last].cpu().numpy(), plain.labels[last].cpu().numpy())
+    labels, inertia, centroids_t, _ = drivers.lloyd(run.X_t, run.w, _dev(init.T, cuda), False, 8, False, 0.0, flags=0)
+    np.testing.assert_allclose(centroids_t.cpu().numpy(), expected, rtol=rtol, atol=100 * rtol)
+    assigned, score = drivers.get_labels_inertia(run.X_t, centroids_t, run.w, True)
+    np.testing.assert_array_equal(labels.cpu().numpy(), assigned.cpu().numpy())
+    assert float(inertia) == float(score[0])
 
 
 # whole-numbered features, many samples nearly as far from two centroids; the wide fp32 step, the tiled product, an
