@@ -1511,6 +1511,26 @@ size_t kmx_assign_workspace_bytes_for(int64_t n, int32_t d, int32_t k, int32_t d
     return extra ? kmx_align256(base) + extra : base;
 }
 
+// fp64 labels of up to 64 features: the screen, or the fp64 product.  The screen saves matrix work; its
+// operands take longer to prepare, which few samples do not pay back, and features past a multiple of 16
+// are padding.  Rows that 128-bit loads cannot take (any n not divisible by 4) go through its loop of
+// scalar loads, where wide samples lose.  Measured, product -> screen, us (clusters as many as fit):
+//   128-bit loads: 1e6 x 14 311 -> 77, 50 333 -> 173, 64 307 -> 180; 128 000 x 50 57 -> 43, 64 49 -> 38;
+//     64 000 x 48 30 -> 28, 50 32 -> 36, 64 29 -> 32; 8 000 x 6 48 -> 37, 4 39 -> 41; 200 000 x 4 72 -> 51
+//   scalar loads: 300 001 x 17 96 -> 66, 36 100 -> 66, 56 102 -> 94, 64 89 -> 105; 128 001 x 16 39 -> 34,
+//     20 38 -> 41, 24 40 -> 43, 36 55 -> 38, 56 57 -> 49; 64 001 x 24 42 -> 39, 36 30 -> 34, 56 33 -> 46
+// Not below four features, where the margins of many clusters are too narrow for the certificate:
+// 1e6 x 1, 1 500 clusters 468 -> 1 202.
+static bool f64_labels_screened(const void* X_t, const void* labels, int64_t n, int d) {
+    if (d < 6) return d >= 4 && n >= 200000;
+    const bool wide_loads = n % 4 == 0 && (uint64_t)n * (uint64_t)d < ((uint64_t)1 << 29) &&
+                            (((uintptr_t)X_t | (uintptr_t)labels) & 15) == 0;
+    if (wide_loads) return d <= 48 || n >= 100000;
+    if (d <= 16) return true;
+    if (d <= 32) return n >= 200000 || (d >= 24 && n <= 65536);
+    return d <= 56 && n >= 100000;
+}
+
 int32_t kmx_assign_labels(const void* X_t, const void* centroids_t, uint32_t* labels,
                           void* workspace, size_t workspace_bytes, int64_t n, int32_t d, int32_t k,
                           int32_t dtype, uint32_t flags, void* stream_) {
@@ -1564,11 +1584,8 @@ int32_t kmx_assign_labels(const void* X_t, const void* centroids_t, uint32_t* la
         if (rc != KMX_OK) return rc;
     } else {
         // fp64 inputs: the screened step's kernel without the update, also where its sums would
-        // not fit the LDS beside the operands.  Against fp64 products, labels of 1e6 samples: 14 features,
-        // 500 clusters 340 -> 77 us; 4, 1 200 356 -> 130; 50, 150 317 -> 147; 64, 128 (rows at no fixed
-        // alignment) 338 both; 20 000 x 14, 500 63 -> 20.  Not below four features, where the margins of many
-        // clusters are too narrow for the certificate: 1, 1 500 468 -> 1 202.
-        const bool labels_only = d >= 4 && (L.variant == KMX_VARIANT_MFMA_F64 || L.variant == KMX_VARIANT_GEMM) &&
+        // not fit the LDS beside the operands.
+        const bool labels_only = f64_labels_screened(X_t, labels, n, d) && (L.variant == KMX_VARIANT_MFMA_F64 || L.variant == KMX_VARIANT_GEMM) &&
                                  (flags & (KMX_FLAG_PATH_MASK | KMX_FLAG_LABELS_MASK)) == 0 &&
                                  kmx_mfma_screen_labels_fits(n, d, k, 8);
         if (L.screen64 || labels_only)

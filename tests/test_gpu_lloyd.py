@@ -891,6 +891,10 @@ def test_labels_and_score_paths_on_every_label_kernel(cuda, name):
     (130, 64, 128),     # two tiles of samples and a remainder
     (63, 63, 40),       # less than a tile
     (2_000, 64, 190),   # operands beyond LDS
+    # either side of the lines between the screen and the product: few features, wide samples, odd sample counts
+    (200_001, 4, 600), (199_999, 4, 600), (3_001, 6, 800), (2_001, 24, 260), (2_001, 23, 260), (65_537, 24, 260),
+    (200_001, 17, 300), (100_001, 33, 230), (100_001, 56, 120), (100_001, 57, 115), (100_000, 64, 100), (99_996, 49, 140),
+    (2_004, 48, 160),
 ])
 def test_fp64_labels_where_only_the_labels_fit_the_lds(cuda, n, d, k):
     import torch
