@@ -1284,11 +1284,17 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
             seen.uncertified_iter = status_host->uncertified_iter;
         }
     }
+    // A run that ends early gives its slot back once nothing that is queued can write to it any more.
+    auto give_up = [&](int32_t rc) {
+        if (hipStreamSynchronize(stream) == hipSuccess) progress_give_back(slot);
+        else (void)hipGetLastError();
+        return rc;
+    };
     unsigned int spins = 0;
     while (true) {
         while (enqueued < max_iter && enqueued < seen.n_iter + (resident != nullptr && seen.n_iter == 0 ? 1 : AHEAD)) {
             const int32_t rc = enqueue(slot);
-            if (rc != KMX_OK) return rc;  // (the slot stays taken: launches before this one may still write to it)
+            if (rc != KMX_OK) return give_up(rc);
         }
         kmx_lloyd_status now = seen;
         if (progress_look(slot, &now) && (now.n_iter != seen.n_iter || now.state != KMX_RUNNING)) {
@@ -1301,7 +1307,7 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
         // launch that failed, a state that was terminal to begin with).
         if (++spins % 20000u == 0u) {
             const hipError_t e = hipStreamQuery(stream);
-            if (e != hipSuccess && e != hipErrorNotReady) return (int32_t)e;
+            if (e != hipSuccess && e != hipErrorNotReady) return give_up((int32_t)e);
             if (e == hipSuccess && !(progress_look(slot, &now) && (now.n_iter != seen.n_iter || now.state != KMX_RUNNING))) {
                 const int32_t rc = kmx_lloyd_status_read(workspace, status_host, stream_);
                 progress_give_back(slot);

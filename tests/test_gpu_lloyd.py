@@ -333,6 +333,28 @@ def test_labels_of_a_run_are_those_of_its_centroids(cuda, n, d, k, values, offse
         assert int((labels != expected).sum()) == 0
 
 
+def test_runs_that_are_refused_leave_the_words_of_others_free(cuda):
+    """More runs that end with an error than there are words to announce iterations in (64): a run after them still
+    announces itself (it then returns what it announced alone, and not the whole status)."""
+    from sklearn_numba_dpex_amd import _capi
+
+    rng = np.random.default_rng(0)
+    X = rng.standard_normal((20_001, 100)).astype(np.float32)
+    run = _ResidentRun(cuda, X, np.ones(len(X), dtype=np.float32), X[:300], 4)
+    ptr, enough = run.ptr, run.ws_bytes
+    for _ in range(70):
+        rc = run.lib.kmx_lloyd_run(run.plan, ptr(run.X_t), ptr(run.X_rm), ptr(run.w), ptr(run.cent[0]), ptr(run.cent[1]),
+                                   ptr(run.labels[0]), ptr(run.labels[1]), ptr(run.sizes), ptr(run.empty), ptr(run.ws),
+                                   enough - 1, None, 0, 0, 4, run.status, run.stream)
+        assert rc == -4  # KMX_ERR_WORKSPACE
+    run.run(4)
+    assert (run.status.n_iter, run.status.state) == (4, _capi.KMX_MAX_ITER)
+    whole = _capi.LloydStatus()
+    run.check(run.lib.kmx_lloyd_status_read(ptr(run.ws), whole, run.stream), "kmx_lloyd_status_read")
+    assert whole.max_iter == 4 and whole.reserved[1] > 0  # (labels that the last iteration changed)
+    assert run.status.reserved[1] == 0
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
