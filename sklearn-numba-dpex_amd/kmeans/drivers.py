@@ -19,6 +19,13 @@ from ..common.reductions import sum_reduction
 from ..common.topk import topk_idx
 
 
+def _iterations_per_call(n, d, k, itemsize):
+    """Lloyd iterations that one library call runs: about a tenth of a second of them, at least 16.  The
+    interpreter handles signals (Ctrl-C) between the calls only; ending one costs about 20 us."""
+    seconds = max(n * d * itemsize / 4e12, 2.0 * n * d * k / 1e14, 1e-5)
+    return max(16, int(0.1 / seconds))
+
+
 def lloyd(
     X_t,
     sample_weight,
@@ -95,9 +102,10 @@ def lloyd(
 
     status = LloydStatus()
     n_done, max_iter = 0, int(max_iter)
+    per_call = _iterations_per_call(n, d, k, X_t.element_size())
     while True:
         # (verbose: an iteration at a time)
-        until = min(n_done + 1, max_iter) if verbose else max_iter
+        until = min(n_done + (1 if verbose else per_call), max_iter)
         check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(cent[0]), ptr(cent[1]),
                                 ptr(labels[0]), ptr(labels[1]), ptr(sizes), ptr(empty_list), ptr(ws), ws_bytes,
                                 ptr(resident), resident_bytes, n_done, until, status, stream), "kmx_lloyd_run")

@@ -355,6 +355,32 @@ def test_runs_that_are_refused_leave_the_words_of_others_free(cuda):
     assert run.status.reserved[1] == 0
 
 
+@pytest.mark.parametrize("n,d,k,dtype", [(30_001, 14, 40, np.float32), (20_001, 100, 300, np.float32)])
+def test_long_runs_come_back_to_the_interpreter(cuda, monkeypatch, n, d, k, dtype):
+    """A run is several library calls of a bounded length, with Ctrl-C handled between them, and the same run."""
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    assert drivers._iterations_per_call(100_000_000, 64, 1_000, 4) == 16
+    assert drivers._iterations_per_call(1_000_000, 256, 1_024, 4) * 5e-3 <= 0.11
+    X = np.random.default_rng(n).standard_normal((n, d)).astype(dtype)
+    X_t, w, init = _dev(X.T, cuda), _dev(np.ones(n, dtype=dtype), cuda), _dev(X[:k].T, cuda)
+    whole = drivers.lloyd(X_t, w, init, True, 50, False, 0.0, flags=0)
+    assert whole[3] > 16
+    asked, run = [], drivers.lib.kmx_lloyd_run
+
+    def counted(*args):
+        asked.append(args[15] - args[14])
+        return run(*args)
+
+    monkeypatch.setattr(drivers.lib, "kmx_lloyd_run", counted)
+    monkeypatch.setattr(drivers, "_iterations_per_call", lambda *a: 8)
+    pieces = drivers.lloyd(X_t, w, init, True, 50, False, 0.0, flags=0)
+    assert len(asked) >= 3 and max(asked) == 8
+    assert pieces[3] == whole[3]
+    for a, b in zip(pieces[:3:2], whole[:3:2]):
+        np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
