@@ -54,6 +54,21 @@ def release_workspaces():
         _workspaces.clear()
 
 
+# copies up to this size are made without a look at the memory (asking takes longer than they do)
+_ROOM_ASK_BYTES = 1 << 30
+
+
+def room_for(n_bytes, device):
+    """Whether a copy of n_bytes that a call can do without leaves as much memory free again: what the
+    program allocates next must not fail for the sake of a faster call."""
+    if n_bytes <= _ROOM_ASK_BYTES:
+        return True
+    free = torch.cuda.mem_get_info(device)[0]
+    if 2 * n_bytes > free:  # (the allocator's counters take 100 us to read)
+        free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return 2 * n_bytes <= free
+
+
 def dcode(t):
     return _capi.dtype_code(t.dtype)
 

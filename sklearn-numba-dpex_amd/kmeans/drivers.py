@@ -12,7 +12,7 @@ import torch
 
 from .. import _capi
 from .._capi import LloydStatus, check, lib, ptr
-from ..common._buffers import contiguous, dcode, require_cuda, workspace
+from ..common._buffers import contiguous, dcode, require_cuda, room_for, workspace
 from ..common.kernels import broadcast_rows, divide_by, transposed_copy
 from ..common.random import create_xoroshiro128pp_states, get_random_raw, raw_to_uniform
 from ..common.reductions import sum_reduction
@@ -80,11 +80,11 @@ def lloyd(
     if reads_rowmajor == 1:
         try:
             # ... and, for many features, a half-precision copy that the labels are screened with
-            if resident_bytes:
+            if resident_bytes and room_for(resident_bytes + n * d * X_t.element_size(), dev):
                 resident = torch.empty(resident_bytes, dtype=torch.uint8, device=dev)
                 X_rm = torch.empty((n, d), dtype=dt, device=dev)
         except torch.cuda.OutOfMemoryError:
-            X_rm = resident = None  # labels from the feature-major array (slower, same results)
+            X_rm = resident = None  # labels from the feature-major array (slower)
         try:
             if X_rm is None:
                 X_rm = transposed_copy(X_t)
@@ -390,6 +390,8 @@ def kmeans_plusplus(X_t, sample_weight, n_clusters, random_state, sampler="scan"
         raise ValueError(f"kmeans++ does not support n_local_trials={n_local_trials}")
     # copies of X that the later steps read instead (kmx_kpp_run looks for them behind its workspace)
     screen_bytes = lib.kmx_kpp_screen_bytes(n, d, n_clusters, n_local_trials, dc) if sampler == "scan" else 0
+    if screen_bytes and not room_for(screen_bytes, dev):
+        screen_bytes = 0
     try:
         ws = workspace(ws_bytes + screen_bytes, dev)
         ws_bytes += screen_bytes

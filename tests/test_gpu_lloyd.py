@@ -381,6 +381,66 @@ def test_long_runs_come_back_to_the_interpreter(cuda, monkeypatch, n, d, k, dtyp
         np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
 
 
+@pytest.mark.parametrize("short_of", ["room", "the half-precision copy", "the row-major copy", "seeding"])
+def test_runs_and_seedings_without_memory_for_copies(cuda, monkeypatch, short_of):
+    """Copies of X are made where they leave as much memory again; without them the results are the same
+    (up to near ties of the labels, which these data do not have)."""
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    n, d, k = 400_001, 100, 300
+    rng = np.random.default_rng(5)
+    which = rng.integers(0, k, n)
+    X = (rng.uniform(-5, 5, (k, d))[which] + rng.standard_normal((n, d))).astype(np.float32)
+    X_t, w = _dev(X.T, cuda), _dev(np.ones(n, dtype=np.float32), cuda)
+    init = _dev(X[np.unique(which, return_index=True)[1]].T, cuda)  # a sample of every blob: no near ties
+    resident = _capi.lib.kmx_lloyd_resident_bytes(_capi.lloyd_plan(n, d, k, _capi.KMX_F32, 0))
+    screen = _capi.lib.kmx_kpp_screen_bytes(n, d, 40, 5, _capi.KMX_F32)
+    assert resident > 0 and screen > 0
+    expected_seeds = drivers.kmeans_plusplus(X_t, w, 40, np.random.RandomState(0))
+    expected = drivers.lloyd(X_t, w, init, True, 3, False, 0.0, flags=0)
+    empty, refused = torch.empty, []
+
+    def scarce(*size, **kwargs):
+        want = size[0] if len(size) == 1 else size
+        n_bytes = want if isinstance(want, int) and kwargs.get("dtype") == torch.uint8 else 0
+        if (short_of == "the half-precision copy" and n_bytes == resident or short_of == "seeding" and n_bytes > screen or
+                short_of == "the row-major copy" and want == (n, d)):
+            refused.append(want)
+            raise torch.cuda.OutOfMemoryError("as asked")
+        return empty(*size, **kwargs)
+
+    if short_of == "room":
+        monkeypatch.setattr(drivers, "room_for", lambda n_bytes, device: refused.append(n_bytes) or False)
+    else:
+        monkeypatch.setattr(torch, "empty", scarce)
+    seeds = drivers.kmeans_plusplus(X_t, w, 40, np.random.RandomState(0))
+    got = drivers.lloyd(X_t, w, init, True, 3, False, 0.0, flags=0)
+    monkeypatch.undo()
+    assert refused
+    np.testing.assert_array_equal(seeds[1].cpu().numpy(), expected_seeds[1].cpu().numpy())
+    np.testing.assert_array_equal(got[0].cpu().numpy(), expected[0].cpu().numpy())
+    np.testing.assert_allclose(got[2].cpu().numpy(), expected[2].cpu().numpy(), rtol=1e-6, atol=1e-6)
+    np.testing.assert_allclose(float(got[1]), float(expected[1]), rtol=1e-6)
+
+
+def test_copies_of_x_leave_as_much_memory_again(cuda, monkeypatch):
+    import torch
+
+    from sklearn_numba_dpex_amd.common import _buffers
+
+    gib = 1 << 30
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (10 * gib, 300 * gib))
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda device=None: 7 * gib)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda device=None: 5 * gib)
+    assert _buffers.room_for(6 * gib, cuda) and not _buffers.room_for(6 * gib + 1, cuda)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (0, 300 * gib))
+    assert not _buffers.room_for(gib + 1, cuda)
+    assert _buffers.room_for(gib, cuda)  # (small ones are simply asked for)
+
+
 # a kernel family each; the iterations enqueued behind one that stops for a relocation find label
 # buffers that no iteration has written
 @pytest.mark.parametrize("n,d,k,dtype", [(3_001, 14, 20, np.float32), (3_001, 40, 20, np.float64), (3_001, 10, 5, np.float64),
