@@ -91,7 +91,7 @@ __device__ __forceinline__ _Float16 to_half(float v) {
 
 // The scale: a power of two that brings the largest centroid coordinate into [2^10, 2^11), which
 // leaves samples 32 times further out inside fp16 (beyond it they become infinite and get no
-// certificate), but not the largest coordinate of 256 samples spread over X below 1: initial
+// certificate), but not the largest coordinate of 256 samples below 1: initial
 // centroids far from all samples would round the samples away for the whole run, though the first
 // relocation removes them (1e6 x 100 fp64, 100 clusters of which 3 start at 1e8: 27.5 -> 5.2 ms for
 // ten iterations).  One workgroup.
@@ -128,10 +128,13 @@ __device__ __forceinline__ void tiles_write_scale(float high, float low, float (
     }
 }
 
-// largest magnitude in this thread's share of 256 samples spread over X
-template <typename T>
+// largest magnitude in this thread's share of 256 samples: spread evenly over X, or STRETCHES: 64 in a row
+// at four places (whole cache lines: 1e6 x 256, where a line per value takes 145 us, 10)
+template <typename T, bool STRETCHES>
 __device__ __forceinline__ float sampled_max(const T* __restrict__ X_t, int64_t n, int d) {
-    const int64_t i = (int64_t)(threadIdx.x & 255) * n / 256;
+    const int t = threadIdx.x & 255;
+    int64_t i = STRETCHES ? (int64_t)(t >> 6) * n / 4 + (t & 63) : (int64_t)t * n / 256;
+    i = i < n ? i : n - 1;
     float m = 0.0f;
     for (int f0 = threadIdx.x >> 8; f0 < d; f0 += 4 * 16) {
         float v[16];
@@ -155,7 +158,7 @@ __global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__
 #pragma unroll
         for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
     }
-    tiles_write_scale(m, sampled_max(X_t, n, d), m_s, header);
+    tiles_write_scale(m, sampled_max<T, true>(X_t, n, d), m_s, header);
 }
 
 // The same where there are no centroids yet: from the samples alone.  One workgroup.
@@ -163,7 +166,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __restrict__ X_t, unsigned int* __restrict__ header,
                                                                   int64_t n, int d) {
     __shared__ float m_s[2][16];
-    tiles_write_scale(sampled_max(X_t, n, d), 0.0f, m_s, header);
+    tiles_write_scale(sampled_max<T, false>(X_t, n, d), 0.0f, m_s, header);
 }
 
 // The tiles, |x'|^2 and |e_x| per sample, the row-major copy of X and (absmax not null) the bits of
