@@ -255,9 +255,10 @@ int32_t kmx_lloyd_finalize(const kmx_lloyd_plan* plan, const void* centroids_t,
 /* Copies the status to host memory and waits for it (the only synchronising call). */
 int32_t kmx_lloyd_status_read(const void* workspace, kmx_lloyd_status* status_host, void* stream);
 
-/* Kernel variants 61 and 71 only (labels screened on the fp16 matrix cores): number of samples
- * whose label the screen of the last completed iteration could not certify and that were
- * evaluated in the input type instead; 0 for the other variants.  Synchronises the stream.
+/* Where labels are screened on the fp16 matrix cores (kernel variants 61, 71 and 42, the last also in a
+ * run with a half-precision copy): number of samples whose label the screen of the last completed
+ * iteration could not certify and that were evaluated more precisely instead; 0 for the other
+ * variants.  Synchronises the stream.
  * It has no counterpart in the reference (diagnostics). */
 int32_t kmx_lloyd_recheck_count(const kmx_lloyd_plan* plan, const void* workspace,
                                 uint32_t* count_host, void* stream);

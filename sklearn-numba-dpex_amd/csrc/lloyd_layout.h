@@ -97,7 +97,7 @@ int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, cons
 char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k);  // room for k half norms
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, hipStream_t stream);
+                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out = nullptr);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,

@@ -455,7 +455,8 @@ int32_t kmx_lloyd_step_mfma_wide_f32(const LloydLayout& L, const void* X_t, cons
     int32_t rc;
     if (L.tiles != nullptr) {
         rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, ws + L.off_cpack, half_norms, L.tiles, status, labels, n, d,
-                              L.dpad, k, KMX_F32, stream);
+                              L.dpad, k, KMX_F32, stream,
+                              const_cast<unsigned int*>(kmx_wide_screen_counter(ws + L.off_wscreen)));
         if (rc != KMX_OK) return rc;
         rc = kmx_bucket_count(labels_prev, labels, counts, ranks, status, n, k, stream);
     } else if (kmx_wide_screen_enabled(n, d, k, L.flags)) {

@@ -643,7 +643,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const float* __restrict__ hneg, unsigned int* __restrict__ header, kmx_lloyd_status* __restrict__ status,
     uint32_t* __restrict__ labels, const int* __restrict__ list, const float* __restrict__ list_thr, int* __restrict__ rest,
     int64_t n, int d, int dpad, int k, int n_blocks, const float2* __restrict__ block_max,
-    const float* __restrict__ half_norms, float prod_rho) {
+    const float* __restrict__ half_norms, float prod_rho, unsigned int* __restrict__ listed_out) {
     static_assert(!MATCH || sizeof(T) == 4, "fp64 inputs: labels by fp64 distances");
     if (status != nullptr && status->state != KMX_RUNNING) return;
     __shared__ int cand_n[32];
@@ -660,6 +660,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, j = lane & 31;
     const int64_t n_listed = (int64_t)header[TH_LISTED];
+    if (listed_out != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *listed_out = (unsigned int)n_listed;
     if (n_listed > (n >> 3)) {  // the tiled product takes all samples
         if (status != nullptr && blockIdx.x == 0 && threadIdx.x == 0 && status->uncertified_iter == 0)
             status->uncertified_iter = status->n_iter + 1;
@@ -937,10 +938,10 @@ char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k) { return area + 
 
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace
 // holds them).  `status` null: labels whatever the state, those of kmx_assign_labels, whose half norms
-// `half_norms` are then.
+// `half_norms` are then.  listed_out (or null): the number of samples without a certificate.
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, hipStream_t stream) {
+                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out) {
     const TileArea a = tile_area(n, d, k);
     unsigned int* header = (unsigned int*)area;
     uint4* ct = (uint4*)(area + a.off_ct);
@@ -973,7 +974,7 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
 #define KMX_TILES_RESOLVE(T, S_, M_)                                                                                     \
     hipLaunchKernelGGL((tiles_resolve_kernel<T, S_, M_>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor,   \
                        (const T*)cpack, (const uint4*)(area + a.off_xt), ct, hneg, header, status, labels, list, thr,    \
-                       rest, n, d, dpad, k, a.n_blocks, cmax, (const float*)half_norms, prod_rho)
+                       rest, n, d, dpad, k, a.n_blocks, cmax, (const float*)half_norms, prod_rho, listed_out)
     switch (a.S) {
 #define KMX_TILES_CASE(S_)                                                                         \
     case S_:                                                                                       \
@@ -992,6 +993,3 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
     return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + TH_REST, n, d, k, dtype,
                                         stream, header + TH_LISTED, (n >> 3) + 1);
 }
-
-// samples of the last labelling that had no certificate
-const uint32_t* kmx_tiles_counter(const char* area) { return (const uint32_t*)area + TH_LISTED; }

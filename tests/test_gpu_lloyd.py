@@ -247,6 +247,20 @@ def test_labels_of_a_resident_run_taken_twice_and_midway(cuda, n, d, k, data):
     np.testing.assert_array_equal(again.run(6).cpu().numpy(), expected)
 
 
+def test_recheck_count_of_a_resident_run(cuda):
+    """The count of uncertified samples is that of the copy's labelling, where a run takes its labels from it."""
+    import ctypes
+
+    rng = np.random.default_rng(3)
+    X = rng.standard_normal((20_003, 128)).astype(np.float32)
+    run = _ResidentRun(cuda, X, np.ones(len(X), dtype=np.float32), X[:260], 2)
+    run.run(2)
+    assert run.status.uncertified_iter == 0
+    count = ctypes.c_uint32(12345)
+    run.check(run.lib.kmx_lloyd_recheck_count(run.plan, run.ptr(run.ws), ctypes.byref(count), run.stream), "recheck")
+    assert 0 < count.value == run.listed() < len(X) // 8
+
+
 @pytest.mark.parametrize("n,d,k,dtype,far", [(20_001, 100, 300, np.float32, 1e8), (65_600, 100, 100, np.float64, 1e8),
                                              (20_001, 129, 300, np.float32, -3e4), (20_001, 129, 300, np.float64, 1e200)])
 def test_initial_centroids_far_from_all_samples(cuda, n, d, k, dtype, far):
