@@ -203,9 +203,16 @@ class _ResidentRun:
 
     def listed(self):
         """Samples of the last labelling without a certificate: the second word of the copy's header."""
+        return self._header()[1]
+
+    def left(self):
+        """... of which so many had more candidates than are looked at one by one: the third word."""
+        return self._header()[2]
+
+    def _header(self):
         import torch
 
-        return int(self.resident[:8].view(torch.int32)[1])
+        return self.resident[:12].view(torch.int32).tolist()
 
 
 @pytest.mark.parametrize("n,d,k,data", [(20_003, 128, 260, "offset"), (5_003, 128, 500, "blobs")])
@@ -320,6 +327,67 @@ def test_data_that_half_precision_cannot_tell_apart(cuda, n, d, k, dtype):
     assigned, score = drivers.get_labels_inertia(run.X_t, centroids_t, run.w, True)
     np.testing.assert_array_equal(labels.cpu().numpy(), assigned.cpu().numpy())
     assert float(inertia) == float(score[0])
+
+
+@pytest.mark.parametrize("n,d,k,dtype", [(20_003, 128, 260, np.float32), (65_601, 101, 100, np.float64)])
+@pytest.mark.parametrize("branch", ["candidates", "too many candidates", "too many samples"])
+def test_samples_without_a_certificate_take_each_way(cuda, n, d, k, dtype, branch):
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(d)
+    X = rng.standard_normal((n, d))
+    if branch == "too many samples":
+        X[:, 0] *= 100
+    elif branch == "too many candidates":
+        X += rng.uniform(-2, 2, (k, d))[np.arange(n) % k]
+    X = X.astype(dtype)
+    init = X[:k].copy()
+    if branch == "too many candidates":
+        init[k // 2:k // 2 + 12] = init[k // 2]  # a dozen equal ones
+    run = _ResidentRun(cuda, X, np.ones(n, dtype=dtype), init, 1)
+    labels, _ = run.labels_inertia()
+    if branch == "candidates":
+        assert 0 < run.listed() <= n // 8 and run.left() == 0
+    elif branch == "too many candidates":
+        assert 0 < run.left() <= run.listed() <= n // 8
+        assert (labels == k // 2).any() and not np.isin(labels, np.arange(k // 2 + 1, k // 2 + 12)).any()
+    else:
+        assert run.listed() > n // 8
+    expected, _ = drivers.get_labels_inertia(run.X_t, run.cent[0], run.w, True)
+    np.testing.assert_array_equal(labels, expected.cpu().numpy())
+
+
+# rows that 128-bit loads take and rows that they do not
+@pytest.mark.parametrize("n,d,k,dtype", [(20_001, 100, 300, np.float32), (20_003, 129, 300, np.float32),
+                                         (65_601, 100, 100, np.float64), (65_537, 65, 101, np.float64)])
+def test_relocation_in_a_run_with_the_half_precision_copy(cuda, n, d, k, dtype):
+    """The distances that rank the samples against fp64, and the centroids of an iteration that relocates three empty
+    clusters against the oracle."""
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d)
+    X = (rng.uniform(-2, 2, (k, d))[rng.integers(0, k, n)] + rng.standard_normal((n, d))).astype(dtype)
+    for i, stretch in ((7, 3), (n // 2, 4), (n - 1, 5)):  # the samples that are to be picked, far apart in rank
+        X[i] *= stretch
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    init = X[rng.choice(n // 2 - 8, k, replace=False) + 8].copy()
+    init[[2, k // 2, k - 1]] = 1e4
+    run = _ResidentRun(cuda, X, w, init, 1)
+    labels = torch.as_tensor(rng.integers(0, k, n).astype(np.int32), device=cuda)
+    got = torch.full((n,), -1.0, dtype=run.w.dtype, device=cuda)
+    run.check(run.lib.kmx_lloyd_sample_distances(run.plan, run.ptr(run.X_rm), run.ptr(labels), run.ptr(run.ws),
+                                                 run.ptr(got), run.stream), "kmx_lloyd_sample_distances")
+    exact = ((_dev(X, cuda).double() - _dev(init, cuda).double()[labels.long()]) ** 2).sum(1)
+    # a difference, its square and d / 16 + 4 additions, each within an ulp of terms of one sign
+    np.testing.assert_allclose(got.cpu().numpy(), exact.cpu().numpy(), rtol=(d / 16 + 8) * np.finfo(dtype).eps)
+    for relocation in ("sklearn", "literal"):
+        _, _, centroids_t, n_iter = drivers.lloyd(run.X_t, run.w, _dev(init.T, cuda), False, 1, False, 0.0,
+                                                  relocation=relocation, flags=0)
+        it = next(ok.lloyd_iterations(X, w, init, max_iter=1, tol=0.0, relocation=relocation))
+        assert it["n_empty"] == 3 and n_iter == 1
+        assert_centers_close(centroids_t.cpu().numpy().T, it["centers"], dtype, scale_rtol=2e-5 if dtype == np.float32 else 1e-11)
 
 
 # whole-numbered features, many samples nearly as far from two centroids; the wide fp32 step, the tiled product, an
