@@ -308,7 +308,8 @@ static inline LloydLayout lloyd_layout(int64_t n, int d, int k, int dtype, uint3
 // saves matrix work, so the line is drawn in products n d k.  Measured, ten iterations, without / with:
 //   fp32 tiled product: 1e5 x 200, k = 24 (4.8e8) 1.15 / 1.16 ms; 1e6 x 70, k = 30 (2.1e9) 2.64 / 2.47;
 //     4e5 x 100, k = 64 (2.6e9) 1.81 / 1.57
-//   fp32 wide step (k > 256): 2e4 x 100, k = 300 (6e8) 1.90 / 1.32; 3e5 x 256, k = 300 (2.3e10) 6.5 / 3.6
+//   fp32 wide step (k > 256): 4 600 x 256, k = 260 (3.1e8) 3.75 / 2.55; 15 000 x 70, k = 300 (3.2e8) 3.07 / 2.42;
+//     6 000 x 66, k = 1 000 (4e8) 8.3 / 7.2; 2e4 x 100, k = 300 (6e8) 1.90 / 1.32; 3e5 x 256, k = 300 (2.3e10) 6.5 / 3.6
 //   fp64: 2e5 x 70, k = 20 (2.8e8) 1.15 / 1.09; 5e4 x 130, k = 40 (2.6e8) 0.97 / 0.96; 2e4 x 100, k = 300
 //     (6e8) 1.28 / 0.91; 3e5 x 256, k = 300 15.2 / 3.9
 static inline bool lloyd_tiles_wanted(const LloydLayout& L, int64_t n, int d, int k, int dtype) {

@@ -174,7 +174,7 @@ def test_kmeanspp_first_centres_match_oracle_at_full_n(cuda, sampler):
 
 
 def test_score_path_and_topk_at_full_size(cuda):
-    """configs[1] at full size: labels and inertia in one pass equal the two-pass results (labels
+    """5 000 000 x 14, 127 clusters: labels and inertia in one pass equal the two-pass results (labels
     bit for bit, inertia to 1e-5 and to an exact fp64 sum on a slice-free formula), and the
     top-k of the 5e6 per-sample values - unique values, then heavy ties - equals a host sort."""
     import torch

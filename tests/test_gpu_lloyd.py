@@ -910,10 +910,10 @@ def _converging_configs():
     - 43 instead of 39 on C1 with 4 threads - because its per-thread partial sums round
     differently and a Lloyd trajectory at tol = 0 amplifies every flipped near-tie)."""
     return {
-        # BASELINE configs[0] at full size (fused screened step, sums corrected per moved sample)
+        # 100 000 x 14, 127 clusters at full size (fused screened step, sums corrected per moved sample)
         "C1": (lambda: datasets.config1(), 61, 39),
-        # configs[1] (weighted, unequal blobs, one cluster empties and is relocated) and
-        # configs[4] (fp64, sixteen clusters that empty on the first iteration) on fewer samples
+        # 14 features, 127 clusters (weighted, unequal blobs, one cluster empties and is relocated) and
+        # 32 features, 64 clusters (fp64, sixteen clusters that empty on the first iteration) on fewer samples
         "C2_30k": (lambda: datasets.config2(n=30_000), 61, 38),
         "C5_100k": (lambda: datasets.config5(n=100_000), 71, 67),
         # screened labels with the sums taken straight from the labels, and with sums per bucket
