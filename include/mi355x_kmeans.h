@@ -200,9 +200,10 @@ int32_t kmx_lloyd_trace_collect(float* kernel_ms_mean, float* kernel_ms_min, int
 /* Iterations n_done, n_done + 1, ... until the state is no longer KMX_RUNNING or max_iter (the value
  * given to kmx_lloyd_init) is reached: enqueues kmx_lloyd_iter a few ahead of the last one that has
  * announced itself to the host and returns with what it learned in status_host (n_iter, state,
- * n_empty, shift_sum, uncertified_iter).  Iteration j reads the centroids and previous labels of its parity and
- * writes those of the other one: centroids_even holds the initial centroids, and iteration 0 writes
- * centroids_odd and labels_odd.  After KMX_NEED_RELOCATION the caller relocates, calls
+ * n_empty, shift_sum, uncertified_iter).  For a run that goes on (n_done > 0) status_host holds, on entry,
+ * what the call before returned, or kmx_lloyd_status_read after a relocation.  Iteration j reads the
+ * centroids and previous labels of its parity and writes those of the other one: centroids_even holds
+ * the initial centroids, and iteration 0 writes centroids_odd and labels_odd.  After KMX_NEED_RELOCATION the caller relocates, calls
  * kmx_lloyd_finalize and comes back with n_done = status.n_iter + 1 if the run goes on.  Waits for
  * the end of the run on the host (without synchronising the stream: launches that find the run over
  * may still be queued).  Safe to call from several threads on workspaces and streams of their own.

@@ -1246,11 +1246,9 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
     int enqueued = n_done;
     kmx_lloyd_status seen;
     std::memset(&seen, 0, sizeof(seen));
-    if (resident != nullptr && n_done > 0) {
-        // (what an earlier call found about the copy)
-        const int32_t rc = kmx_lloyd_status_read(workspace, &seen, stream_);
-        if (rc != KMX_OK) return rc;
-    }
+    // (what an earlier call found about the copy)
+    if (status_host->uncertified_iter > 0 && status_host->uncertified_iter <= n_done)
+        seen.uncertified_iter = status_host->uncertified_iter;
     seen.n_iter = n_done;
     seen.state = KMX_RUNNING;
     // Whether iteration `it` takes its labels from the copy.  What decides is known whenever an iteration is
