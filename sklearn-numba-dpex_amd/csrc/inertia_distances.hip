@@ -7,40 +7,6 @@
 
 namespace {
 
-// Four consecutive values of a row at i0 (128-bit accesses when `full`), zero past n.
-template <typename T>
-__device__ __forceinline__ void load4(const T* __restrict__ row, int64_t i0, int64_t n, bool full, T (&v)[4]) {
-    if (full) {
-        if constexpr (sizeof(T) == 4) {
-            const float4 q = *reinterpret_cast<const float4*>(row + i0);
-            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
-            const double2 a = *reinterpret_cast<const double2*>(row + i0);
-            const double2 b = *reinterpret_cast<const double2*>(row + i0 + 2);
-            v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (i0 + r < n) ? row[i0 + r] : T(0);
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void store4(T* __restrict__ row, int64_t i0, int64_t n, bool full, const T (&v)[4]) {
-    if (full) {
-        if constexpr (sizeof(T) == 4) {
-            *reinterpret_cast<float4*>(row + i0) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            *reinterpret_cast<double2*>(row + i0) = make_double2(v[0], v[1]);
-            *reinterpret_cast<double2*>(row + i0 + 2) = make_double2(v[2], v[3]);
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (i0 + r < n) row[i0 + r] = v[r];
-    }
-}
-
 // out[i] = w_i * sum_f (x_fi - c_f,label_i)^2, features accumulated in order.  A thread takes
 // four consecutive samples (128-bit loads of every feature row); the centroids are staged in
 // LDS when they fit (LDS_CENTROIDS), so that the per-sample gather of the label's centroid
@@ -54,7 +20,7 @@ template <typename T, bool LDS_CENTROIDS, bool SUM>
 __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight,
     const T* __restrict__ centroids_t, const uint32_t* __restrict__ labels, T* __restrict__ out,
-    double* __restrict__ partial, int64_t n, int d, int k, int vec_ok) {
+    double* __restrict__ partial, int64_t n, int d, int k) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* cs = reinterpret_cast<T*>(smem_raw);  // the workgroup's feature rows of centroids_t, same layout
     const int f_chunk = (d + (int)gridDim.y - 1) / (int)gridDim.y;
@@ -72,7 +38,7 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
     (void)total;
     for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n_groups; g += stride) {
         const int64_t i0 = g * 4;
-        const bool full = vec_ok && (i0 + 4 <= n);
+        const bool full = i0 + 4 <= n;
         uint32_t c[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) c[r] = (i0 + r < n) ? labels[i0 + r] : 0u;
@@ -80,7 +46,7 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
 #pragma unroll 4
         for (int f = f_begin; f < f_end; ++f) {
             T x[4];
-            load4<T>(X_t + (size_t)f * n, i0, n, full, x);
+            kmx_load4<T>(X_t + (size_t)f * n, i0, n, full, x);
             const T* __restrict__ crow = cent + (size_t)f * k;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -90,7 +56,7 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
         }
         if (sample_weight) {
             T w[4];
-            load4<T>(sample_weight, i0, n, full, w);
+            kmx_load4<T>(sample_weight, i0, n, full, w);
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[r] *= w[r];
         }
@@ -99,7 +65,7 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
 #pragma unroll
             for (int r = 0; r < 4; ++r) total += (i0 + r < n) ? (double)acc[r] : 0.0;
         } else {
-            store4<T>(out, i0, n, full, acc);
+            kmx_store4<T>(out, i0, n, full, acc);
         }
     }
     if constexpr (SUM) {
@@ -110,14 +76,16 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
 }
 
 // The same from the rows of a row-major copy of X and of the packed centroids: 16 lanes per sample and
-// 128-bit loads (VEC: rows of whole 16-byte groups), so that the gathered centroid is whole cache
-// lines too; lanes sum in T, the sample and the total in fp64.  Bound by reading X once.
+// 128-bit loads, so that the gathered centroid is whole cache lines too; lanes sum in T, the sample and
+// the total in fp64.  Bound by reading X once.  WHOLE: rows of whole 16-byte groups; else the last
+// values of a row are loaded one by one.
 // per-sample values to `out` (SUM false) or the workgroup's total to `partial`.
-template <typename T, bool VEC, bool SUM>
+template <typename T, bool WHOLE, bool SUM>
 __global__ __launch_bounds__(256) void rows_inertia_kernel(
     const T* __restrict__ X_rm, const T* __restrict__ sample_weight, const T* __restrict__ cpack,
     const uint32_t* __restrict__ labels, T* __restrict__ out, double* __restrict__ partial, int64_t n, int d, int dpad) {
-    constexpr int W = VEC ? 16 / (int)sizeof(T) : 1;
+    constexpr int W = 16 / (int)sizeof(T);
+    using V = typename KmxVec<T, W>::type;
     const int e = threadIdx.x & 15;
     const int64_t per_pass = (int64_t)gridDim.x * 32;  // two samples per group of lanes
     double total = 0.0;
@@ -137,14 +105,19 @@ __global__ __launch_bounds__(256) void rows_inertia_kernel(
             T x[2][W], c[2][W];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                if constexpr (VEC) {
-                    using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
+                if (WHOLE || f + W <= d) {
                     const V xv = *reinterpret_cast<const V*>(row[u] + f), cv = *reinterpret_cast<const V*>(cen[u] + f);
-                    __builtin_memcpy(x[u], &xv, 16);
-                    __builtin_memcpy(c[u], &cv, 16);
+#pragma unroll
+                    for (int j = 0; j < W; ++j) {
+                        x[u][j] = xv[j];
+                        c[u][j] = cv[j];
+                    }
                 } else {
-                    x[u][0] = row[u][f];
-                    c[u][0] = cen[u][f];
+#pragma unroll
+                    for (int j = 0; j < W; ++j) {
+                        x[u][j] = f + j < d ? row[u][f + j] : T(0);
+                        c[u][j] = f + j < d ? cen[u][f + j] : T(0);
+                    }
                 }
             }
 #pragma unroll
@@ -197,6 +170,15 @@ __device__ __forceinline__ float dist_sqrt(float a) {
 }
 __device__ __forceinline__ double dist_sqrt(double a) { return sqrt(a); }
 
+// Four consecutive values in LDS at a 16-byte boundary.
+template <typename T>
+__device__ __forceinline__ void lds_load4(const T* p, T (&v)[4]) {
+    struct alignas(16) Four { T e[4]; };
+    const Four q = *reinterpret_cast<const Four*>(p);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = q.e[r];
+}
+
 // distances_t[c, i] = sqrt(sum_f (c_fc - x_fi)^2).  Output bound (k values written per
 // sample).  A thread keeps the features of four consecutive samples in registers (d <= DREG);
 // the workgroup's share of the centroids (blockIdx.y: `c_chunk` of them, a multiple of 4) is
@@ -205,7 +187,7 @@ __device__ __forceinline__ double dist_sqrt(double a) { return sqrt(a); }
 template <typename T, int DREG>
 __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
     const T* __restrict__ X_t, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
-    int64_t n, int d, int k, int vec_ok, int c_chunk) {
+    int64_t n, int d, int k, int c_chunk) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* cs = reinterpret_cast<T*>(smem_raw);  // [d][c_chunk]
     const int c_begin = blockIdx.y * c_chunk;
@@ -218,12 +200,12 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
     const int64_t stride = (int64_t)gridDim.x * 256;
     for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n_groups; g += stride) {
         const int64_t i0 = g * 4;
-        const bool full = vec_ok && (i0 + 4 <= n);
+        const bool full = i0 + 4 <= n;
         T x[DREG][4];
 #pragma unroll
         for (int f = 0; f < DREG; ++f) {
             if (f < d) {
-                load4<T>(X_t + (size_t)f * n, i0, n, full, x[f]);
+                kmx_load4<T>(X_t + (size_t)f * n, i0, n, full, x[f]);
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) x[f][r] = T(0);
@@ -239,7 +221,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
             for (int f = 0; f < DREG; ++f) {
                 if (f < d) {
                     T cv[4];
-                    load4<T>(cs + f * c_chunk, c4, c_chunk, true, cv);  // same address in every lane
+                    lds_load4<T>(cs + f * c_chunk + c4, cv);  // same address in every lane
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -255,7 +237,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
                 if (c < k) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[j][r] = dist_sqrt(acc[j][r]);
-                    store4<T>(distances_t + (size_t)c * n, i0, n, full, acc[j]);
+                    kmx_store4<T>(distances_t + (size_t)c * n, i0, n, full, acc[j]);
                 }
             }
         }
@@ -264,7 +246,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
 
 // Any d: a workgroup owns a tile of DT_S samples x DC centroids, a thread a 4 x (DC / 8) block of
 // it; the features are staged DT_K at a time through LDS (both arrays are feature-major, as the
-// tiles: a stage is a copy of rows, 128-bit loads where alignment allows), the next stage's
+// tiles: a stage is a copy of rows, 128-bit loads), the next stage's
 // loads in flight during the arithmetic.  Per staged feature a thread reads its four samples
 // and its centroids from LDS (the centroid reads are broadcasts) and updates its sums with a
 // difference and a fused multiply-add each, features in order: vector-ALU bound.
@@ -281,33 +263,28 @@ constexpr int dt_vectors() {
 
 template <typename T, int COLS>
 __device__ __forceinline__ void dt_stage_load(T (*regs)[16 / sizeof(T)], const T* __restrict__ base, int64_t len,
-                                              int64_t c0, int d, int f0, bool vec_ok) {
+                                              int64_t c0, int d, int f0) {
     constexpr int V = 16 / sizeof(T);                 // elements per 128-bit vector
     constexpr int PER_ROW = COLS / V;                 // vectors per staged row
     constexpr int N = dt_vectors<T, COLS>();          // vectors per thread
+    // (the same for the whole workgroup: the loads of a stage that exists whole are straight-line code)
+    const bool whole = f0 + DT_K <= d && c0 + COLS <= len;
 #pragma unroll
     for (int l = 0; l < N; ++l) {
         const int g = threadIdx.x + 256 * l;
         const int f = f0 + g / PER_ROW;
         const int64_t c = c0 + (int64_t)V * (g % PER_ROW);
+        const T* __restrict__ src = base + (size_t)f * (size_t)len + c;
+        const bool used = g < DT_K * PER_ROW;  // (known at compile time but for a narrow tile)
+        if (whole) {
+            if (used) {
+                const auto v = *reinterpret_cast<const typename KmxVec<T, V>::type*>(src);
 #pragma unroll
-        for (int e = 0; e < V; ++e) regs[l][e] = T(0);
-        if (f < d && g < DT_K * PER_ROW) {
-            const T* __restrict__ src = base + (size_t)f * (size_t)len + c;
-            if (vec_ok && c + V <= len) {
-                using Vec = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-                union {
-                    Vec v;
-                    T s[V];
-                } u;
-                u.v = *reinterpret_cast<const Vec*>(src);
-#pragma unroll
-                for (int e = 0; e < V; ++e) regs[l][e] = u.s[e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < V; ++e)
-                    if (c + e < len) regs[l][e] = src[e];
+                for (int e = 0; e < V; ++e) regs[l][e] = v[e];
             }
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e) regs[l][e] = used && f < d && c + e < len ? src[e] : T(0);
         }
     }
 }
@@ -330,7 +307,7 @@ __device__ __forceinline__ void dt_stage_store(T (*tile)[COLS], const T (*regs)[
 template <typename T, int DC>
 __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
     const T* __restrict__ X_t, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
-    int64_t n, int d, int k, int x_vec, int c_vec, int out_vec) {
+    int64_t n, int d, int k) {
     constexpr int V = 16 / sizeof(T);
     constexpr int CT = DC / 8;  // centroids per thread
     __shared__ __align__(16) T xs[DT_K][DT_S];
@@ -345,8 +322,8 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[c][i] = T(0);
 
-    dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, 0, x_vec != 0);
-    dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, 0, c_vec != 0);
+    dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, 0);
+    dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, 0);
     const int n_stages = (d + DT_K - 1) / DT_K;
     for (int st = 0; st < n_stages; ++st) {
         __syncthreads();  // the previous stage's reads are over
@@ -354,8 +331,8 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
         dt_stage_store<T, DC>(cs, rc);
         __syncthreads();
         if (st + 1 < n_stages) {
-            dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, (st + 1) * DT_K, x_vec != 0);
-            dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, (st + 1) * DT_K, c_vec != 0);
+            dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, (st + 1) * DT_K);
+            dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, (st + 1) * DT_K);
         }
         // (rows past d hold zeros on both sides: their differences add nothing)
 #pragma unroll
@@ -380,14 +357,10 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
         const int cc = c0 + CT * ty + c;
         if (cc >= k) continue;
         T* __restrict__ dst = distances_t + (size_t)cc * (size_t)n + i;
-        if (sizeof(T) == 4 && out_vec && i + 4 <= n) {
-            *reinterpret_cast<float4*>(dst) = make_float4((float)dist_sqrt(acc[c][0]), (float)dist_sqrt(acc[c][1]),
-                                                          (float)dist_sqrt(acc[c][2]), (float)dist_sqrt(acc[c][3]));
-        } else {
+        T v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (i + e < n) dst[e] = dist_sqrt(acc[c][e]);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = dist_sqrt(acc[c][e]);
+        kmx_store4<T>(dst - i, i, n, i + 4 <= n, v);
     }
 }
 
@@ -450,9 +423,6 @@ static int32_t inertia_launch(const void* X_t, const void* sample_weight, const 
     const bool sum = partial != nullptr;
     const int grid = stream_grid(kmx_cdiv(n, 4));
     const size_t es = kmx_dtype_size(dtype);
-    auto al16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
-    const int vec_ok =
-        (n % 4 == 0) && al16(X_t) && (sum || al16(out)) && (sample_weight == nullptr || al16(sample_weight));
     // the sum over few samples of many features: the features split over the second grid dimension
     // until there are about four workgroups per compute unit (and at least 16 features each)
     int gy = 1;
@@ -468,7 +438,7 @@ static int32_t inertia_launch(const void* X_t, const void* sample_weight, const 
 #define KMX_INERTIA(T, L, S)                                                                       \
     hipLaunchKernelGGL((per_sample_inertia_kernel<T, L, S>), dim3(grid, gy), dim3(256), (L) ? lds : 0,  \
                        stream, (const T*)X_t, (const T*)sample_weight, (const T*)centroids_t,      \
-                       labels, (S) ? nullptr : (T*)out, partial, n, d, k, vec_ok)
+                       labels, (S) ? nullptr : (T*)out, partial, n, d, k)
 #define KMX_INERTIA_T(T)                                                        \
     do {                                                                        \
         if (in_lds && sum) KMX_INERTIA(T, true, true);                          \
@@ -541,15 +511,14 @@ int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, cons
     if (grid > 8 * (int64_t)kmx_num_cus()) grid = 8 * (int64_t)kmx_num_cus();
     if (grid > cap) grid = cap;
     const size_t es = kmx_dtype_size(dtype);
-    const bool vec = (size_t)d * es % 16 == 0 && (((uintptr_t)X_rowmajor) & 15) == 0 && (((uintptr_t)cpack) & 15) == 0 &&
-                     (size_t)dpad * es % 16 == 0;
+    const bool whole = (size_t)d * es % 16 == 0;
 #define KMX_ROWS_INERTIA(T, V, S)                                                                                     \
     hipLaunchKernelGGL((rows_inertia_kernel<T, V, S>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_rowmajor, \
                        (const T*)sample_weight, (const T*)cpack, labels, (S) ? nullptr : (T*)out, workspace, n, d, dpad)
 #define KMX_ROWS_INERTIA_T(T)                                                  \
     do {                                                                       \
-        if (vec && workspace) KMX_ROWS_INERTIA(T, true, true);                 \
-        else if (vec) KMX_ROWS_INERTIA(T, true, false);                        \
+        if (whole && workspace) KMX_ROWS_INERTIA(T, true, true);                 \
+        else if (whole) KMX_ROWS_INERTIA(T, true, false);                        \
         else if (workspace) KMX_ROWS_INERTIA(T, false, true);                  \
         else KMX_ROWS_INERTIA(T, false, false);                                \
     } while (0)
@@ -572,8 +541,6 @@ int32_t kmx_euclidean_distances(const void* X_t, const void* centroids_t, void* 
     if (n <= 0 || d <= 0 || k <= 0) return KMX_ERR_BAD_SHAPE;
     KMX_REQUIRE_DTYPE(dtype);
     hipStream_t stream = (hipStream_t)stream_;
-    auto al16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
-    const int vec_ok = (n % 4 == 0) && al16(X_t) && al16(distances_t);
     // register kernel: the centroid range is split over blockIdx.y until there are about six
     // workgroups per compute unit (a thread's walk over the centroids is one dependent chain)
     const int64_t wgx = stream_grid(kmx_cdiv(n, 4));
@@ -588,28 +555,23 @@ int32_t kmx_euclidean_distances(const void* X_t, const void* centroids_t, void* 
     if (dtype == KMX_F32 && d <= 32 && lds <= 64 * 1024) {
         if (d <= 16)
             hipLaunchKernelGGL((euclidean_distances_reg_kernel<float, 16>), rgrid, dim3(256), lds, stream,
-                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, vec_ok,
-                               c_chunk);
+                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, c_chunk);
         else
             hipLaunchKernelGGL((euclidean_distances_reg_kernel<float, 32>), rgrid, dim3(256), lds, stream,
-                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, vec_ok,
-                               c_chunk);
+                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, c_chunk);
     } else if (dtype == KMX_F64 && d <= 16 && lds <= 64 * 1024) {
         hipLaunchKernelGGL((euclidean_distances_reg_kernel<double, 16>), rgrid, dim3(256), lds, stream,
-                           (const double*)X_t, (const double*)centroids_t, (double*)distances_t, n, d, k, vec_ok,
-                           c_chunk);
+                           (const double*)X_t, (const double*)centroids_t, (double*)distances_t, n, d, k, c_chunk);
     } else {
         const int dc = k <= 2 * DT_C_FEW ? DT_C_FEW : DT_C;
         const dim3 tgrid((unsigned)kmx_cdiv(n, DT_S), (unsigned)kmx_cdiv(k, dc));
-        const int per_vec = (int)(16 / es);
-        const int x_vec = (n % per_vec == 0) && al16(X_t), c_vec = (k % per_vec == 0) && al16(centroids_t);
-#define KMX_DIST_TILED(T, DC, OUT_VEC)                                                                 \
+#define KMX_DIST_TILED(T, DC)                                                                          \
     hipLaunchKernelGGL((euclidean_distances_tiled_kernel<T, DC>), tgrid, dim3(256), 0, stream,         \
-                       (const T*)X_t, (const T*)centroids_t, (T*)distances_t, n, d, k, x_vec, c_vec, OUT_VEC)
+                       (const T*)X_t, (const T*)centroids_t, (T*)distances_t, n, d, k)
         if (dtype == KMX_F32) {
-            if (dc == DT_C_FEW) KMX_DIST_TILED(float, DT_C_FEW, vec_ok); else KMX_DIST_TILED(float, DT_C, vec_ok);
+            if (dc == DT_C_FEW) KMX_DIST_TILED(float, DT_C_FEW); else KMX_DIST_TILED(float, DT_C);
         } else {
-            if (dc == DT_C_FEW) KMX_DIST_TILED(double, DT_C_FEW, 0); else KMX_DIST_TILED(double, DT_C, 0);
+            if (dc == DT_C_FEW) KMX_DIST_TILED(double, DT_C_FEW); else KMX_DIST_TILED(double, DT_C);
         }
 #undef KMX_DIST_TILED
     }

@@ -28,7 +28,7 @@ constexpr int CHUNK = 1024;     // samples per workgroup (256 threads x 4)
 // Screened steps (kpp_screen_step_kernel): from these sizes on.  The copies they read cost about two
 // plain steps, and a step still writes all its rows: with few features there is little to save.
 // Measured, whole seedings, plain / screened steps: fp32 1e6 x 32, 128 centres 5.3 / 6.1 ms; 3e5 x 64,
-// 32 centres 1.35 / 1.22; 1e6 x 64, 256 centres 15.9 / 15.4; 1 000 003 x 64 (unaligned rows) 23.6 / 16.1;
+// 32 centres 1.35 / 1.22; 1e6 x 64, 256 centres 15.9 / 15.4;
 // 4e5 x 255, 100 centres 10.9 / 8.1; fp64 1e6 x 16, 128 centres 5.5 / 7.2; 5e5 x 50, 100 centres 5.0 / 5.0;
 // 5e5 x 64, 200 centres 11.5 / 9.4; 3e5 x 128, 64 centres 6.0 / 5.1.
 constexpr int64_t SCREEN_MIN_N = 1 << 17;
@@ -95,40 +95,6 @@ __device__ __forceinline__ T kpp_sq_acc(T diff, T acc) {
     }
 }
 
-// Four consecutive values of a row at i0 (one or two 128-bit accesses when `full`), zero past n.
-template <typename T>
-__device__ __forceinline__ void load4(const T* __restrict__ row, int64_t i0, int64_t n, bool full, T (&v)[4]) {
-    if (full) {
-        if constexpr (sizeof(T) == 4) {
-            const float4 q = *reinterpret_cast<const float4*>(row + i0);
-            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
-            const double2 a = *reinterpret_cast<const double2*>(row + i0);
-            const double2 b = *reinterpret_cast<const double2*>(row + i0 + 2);
-            v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (i0 + r < n) ? row[i0 + r] : T(0);
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void store4(T* __restrict__ row, int64_t i0, int64_t n, bool full, const T (&v)[4]) {
-    if (full) {
-        if constexpr (sizeof(T) == 4) {
-            *reinterpret_cast<float4*>(row + i0) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            *reinterpret_cast<double2*>(row + i0) = make_double2(v[0], v[1]);
-            *reinterpret_cast<double2*>(row + i0 + 2) = make_double2(v[2], v[3]);
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (i0 + r < n) row[i0 + r] = v[r];
-    }
-}
-
 // The value lane `src` (a constant) holds, as a wave-uniform scalar.
 template <typename T>
 __device__ __forceinline__ T kpp_readlane(T v, int src) {
@@ -182,7 +148,7 @@ __device__ __forceinline__ void kpp_finish_block(T* __restrict__ rows, double* _
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (i0 + r < n) pot[t] += (double)v[r];
-            store4<T>(rows + (size_t)t * n, i0, n, full, v);
+            kmx_store4<T>(rows + (size_t)t * n, i0, n, full, v);
         }
     }
     // all row sums of the workgroup with one barrier: waves first, then one thread per trial
@@ -210,15 +176,15 @@ template <typename T, int TN, bool FUSED, bool INIT>
 __global__ __launch_bounds__(256) void kpp_step_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight, const T* __restrict__ cand_rows,
     T* __restrict__ rows, double* __restrict__ block_pot, KppHeader* __restrict__ header,
-    int64_t n, int d, int k, int n_trials, int vec_ok, int32_t start, T* __restrict__ centers_t,
+    int64_t n, int d, int k, int n_trials, int32_t start, T* __restrict__ centers_t,
     int32_t* __restrict__ center_indices) {
     __shared__ double wave_pot[4][TN];
     const int best = INIT ? 0 : header->best_row;
     const int64_t i0 = (int64_t)blockIdx.x * CHUNK + threadIdx.x * 4;
     const int lane = threadIdx.x & 63;
-    // Whether the 128-bit accesses are legal is decided once per workgroup and known at compile
-    // time inside the body: with a test per access every load sat in a branch of its own and
-    // was waited for before the next one was issued.
+    // Whether every sample of the workgroup exists is decided once and known at compile time inside
+    // the body: with a test per access every load sat in a branch of its own and was waited for
+    // before the next one was issued.
     auto body = [&](auto full_tag) {
     constexpr bool full = decltype(full_tag)::value;
 
@@ -241,7 +207,7 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
         for (int j = 0; j < FB; ++j) {
             const int f = f0 + j < d ? f0 + j : d - 1;  // past the end: a valid row, ignored below
             const T* __restrict__ row = X_t + (size_t)f * n;
-            load4<T>(row, i0, n, full, xv[j]);
+            kmx_load4<T>(row, i0, n, full, xv[j]);
         }
         KppCandBatch<T, TN, FB> cand;
         if constexpr (INIT) {
@@ -251,8 +217,8 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
             cand.load(cand_rows, f0, d, n_trials, lane);
         }
         if (f0 + FB >= d) {
-            load4<T>(sample_weight, i0, n, full, w);
-            if constexpr (!INIT) load4<T>(rows + (size_t)best * n, i0, n, full, cl);
+            kmx_load4<T>(sample_weight, i0, n, full, w);
+            if constexpr (!INIT) kmx_load4<T>(rows + (size_t)best * n, i0, n, full, cl);
         }
         auto accumulate = [&](auto whole_tag) {
             constexpr bool whole = decltype(whole_tag)::value;  // all FB features exist
@@ -287,7 +253,7 @@ __global__ __launch_bounds__(256) void kpp_step_kernel(
         }
     });
     };
-    if (vec_ok && (int64_t)(blockIdx.x + 1) * CHUNK <= n)
+    if ((int64_t)(blockIdx.x + 1) * CHUNK <= n)
         body(std::true_type{});
     else
         body(std::false_type{});
@@ -339,8 +305,7 @@ template <typename T>
 __global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
     const T* __restrict__ X_t, const T* __restrict__ X_rm, KmxTiles tiles, const T* __restrict__ sample_weight,
     const int32_t* __restrict__ cand, const T* __restrict__ cand_rows, T* __restrict__ rows,
-    double* __restrict__ block_pot, const KppHeader* __restrict__ header, int64_t n, int d, int n_trials, int vec_ok,
-    int row_vec) {
+    double* __restrict__ block_pot, const KppHeader* __restrict__ header, int64_t n, int d, int n_trials) {
     extern __shared__ __align__(16) unsigned char screen_smem[];
     __shared__ double wave_pot[4][SCREEN_TN];
     __shared__ int queued_s;
@@ -457,7 +422,7 @@ __global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
     if (queued > SCREEN_QUEUE) {
         // (the same for the whole workgroup) every pair, two samples per thread from X itself
         const int sl = threadIdx.x * 2;
-        const bool pair = vec_ok && base + CHUNK <= n;
+        const bool pair = base + CHUNK <= n;
         T dist[SCREEN_TN][2];
 #pragma unroll
         for (int t = 0; t < SCREEN_TN; ++t) dist[t][0] = dist[t][1] = T(0);
@@ -468,9 +433,9 @@ __global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
             for (int q = 0; q < FB; ++q) {
                 const T* __restrict__ row = X_t + (size_t)(f0 + q < d ? f0 + q : d - 1) * n;
                 if (pair) {
-                    using V2 = std::conditional_t<sizeof(T) == 4, float2, double2>;
+                    using V2 = typename KmxVec<T, 2>::type;
                     const V2 v = *reinterpret_cast<const V2*>(row + base + sl);
-                    xv[q][0] = v.x; xv[q][1] = v.y;
+                    xv[q][0] = v[0]; xv[q][1] = v[1];
                 } else {
 #pragma unroll
                     for (int r = 0; r < 2; ++r) xv[q][r] = row[base + sl + r < n ? base + sl + r : n - 1];
@@ -507,18 +472,15 @@ __global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
             const T* __restrict__ row = X_rm + (size_t)(base + sl) * d;
             const T* __restrict__ c = cand_s + t * dp;
             T dist = T(0);
-            if (row_vec) {
+            const int whole = d & ~3;
 #pragma unroll 8
-                for (int f = 0; f < d; f += 4) {
-                    T v[4];
-                    load4<T>(row, f, d, true, v);
+            for (int f = 0; f < whole; f += 4) {
+                T v[4];
+                kmx_load4<T>(row, f, d, true, v);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) dist = kpp_sq_acc<true>(v[q] - c[f + q], dist);
-                }
-            } else {
-#pragma unroll 16
-                for (int f = 0; f < d; ++f) dist = kpp_sq_acc<true>(row[f] - c[f], dist);
+                for (int q = 0; q < 4; ++q) dist = kpp_sq_acc<true>(v[q] - c[f + q], dist);
             }
+            for (int f = whole; f < d; ++f) dist = kpp_sq_acc<true>(row[f] - c[f], dist);
             T* at = v_s + t * SCREEN_PITCH + sl;
             *at = fmin(dist * sample_weight[base + sl], *at);
         }
@@ -532,7 +494,7 @@ __global__ __launch_bounds__(512, 4) void kpp_screen_step_kernel(
                 for (int r = 0; r < 4; ++r) v[r] = v_s[t * SCREEN_PITCH + q4 + r];
             });
     };
-    if (vec_ok && base + CHUNK <= n)
+    if (base + CHUNK <= n)
         finish(std::true_type{});
     else
         finish(std::false_type{});
@@ -546,11 +508,11 @@ __device__ __forceinline__ void load_spt(const T* __restrict__ row, int64_t i0, 
         if constexpr (SPT == 1) {
             v[0] = row[i0];
         } else if constexpr (SPT == 2) {
-            using V2 = std::conditional_t<sizeof(T) == 4, float2, double2>;
+            using V2 = typename KmxVec<T, 2>::type;
             const V2 q = *reinterpret_cast<const V2*>(row + i0);
-            v[0] = q.x; v[1] = q.y;
+            v[0] = q[0]; v[1] = q[1];
         } else {
-            load4<T>(row, i0, n, true, v);
+            kmx_load4<T>(row, i0, n, true, v);
         }
     } else {
 #pragma unroll
@@ -571,7 +533,7 @@ template <typename T, int TN, int SPT, bool INIT, bool LITERAL>
 __global__ __launch_bounds__(256) void kpp_step_split_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight, const T* __restrict__ cand_rows,
     T* __restrict__ rows, double* __restrict__ block_pot, KppHeader* __restrict__ header, int64_t n,
-    int d, int k, int n_trials, int vec_ok, int32_t start, T* __restrict__ centers_t,
+    int d, int k, int n_trials, int32_t start, T* __restrict__ centers_t,
     int32_t* __restrict__ center_indices) {
     constexpr int S = 64 * SPT;
     __shared__ T part[4][TN][S];
@@ -645,7 +607,7 @@ __global__ __launch_bounds__(256) void kpp_step_split_kernel(
 #pragma unroll
                 for (int r = 0; r < SPT; ++r) part[wave][t][lane * SPT + r] = acc[t][r];
     };
-    if (vec_ok && base + S <= n)
+    if (base + S <= n)
         body(std::true_type{});
     else
         body(std::false_type{});
@@ -1066,11 +1028,10 @@ template <typename T>
 void launch_init(const void* X_t, const void* w, int32_t start, void* centers_t, int32_t* idx,
                  const KppPtrs& p, const KppLayout& L, int64_t n, int d, int k, hipStream_t s, bool literal) {
     if (L.split) {
-        const int vec_ok = (n % L.split == 0) && (((uintptr_t)X_t) % 16 == 0);
 #define KMX_KPP_INIT_SPLIT_(SPT, LIT)                                                                 \
     hipLaunchKernelGGL((kpp_step_split_kernel<T, 1, SPT, true, LIT>), dim3((unsigned)L.n_blocks),    \
                        dim3(256), 0, s, (const T*)X_t, (const T*)w, (const T*)nullptr, (T*)p.rows,    \
-                       p.block_pot, p.header, n, d, k, 1, vec_ok, start, (T*)centers_t, idx)
+                       p.block_pot, p.header, n, d, k, 1, start, (T*)centers_t, idx)
 #define KMX_KPP_INIT_SPLIT(SPT) \
     do { if (literal) KMX_KPP_INIT_SPLIT_(SPT, true); else KMX_KPP_INIT_SPLIT_(SPT, false); } while (0)
         if (L.split == 1) KMX_KPP_INIT_SPLIT(1);
@@ -1080,12 +1041,10 @@ void launch_init(const void* X_t, const void* w, int32_t start, void* centers_t,
 #undef KMX_KPP_INIT_SPLIT
         return;
     }
-    const int vec_ok = (n % 4 == 0) && (((uintptr_t)X_t) % 16 == 0) && (((uintptr_t)w) % 16 == 0) &&
-                       (((uintptr_t)p.rows) % 16 == 0);
 #define KMX_KPP_INIT(FUSED)                                                                          \
     hipLaunchKernelGGL((kpp_step_kernel<T, 1, FUSED, true>), dim3((unsigned)L.n_blocks), dim3(256), 0, s, \
                        (const T*)X_t, (const T*)w, (const T*)nullptr, (T*)p.rows, p.block_pot, p.header, \
-                       n, d, k, 1, vec_ok, start, (T*)centers_t, idx)
+                       n, d, k, 1, start, (T*)centers_t, idx)
     if (literal) KMX_KPP_INIT(false); else KMX_KPP_INIT(true);
 #undef KMX_KPP_INIT
 }
@@ -1095,11 +1054,10 @@ void launch_step(const void* X_t, const void* w, const int32_t* cand, const KppP
                  const KppLayout& L, int64_t n, int d, int n_trials, hipStream_t s, bool literal) {
     (void)cand;  // the candidates' rows were copied to p.cand_rows when they were sampled
     if (L.split) {
-        const int vec_split = (n % L.split == 0) && (((uintptr_t)X_t) % 16 == 0);
 #define KMX_KPP_STEP_SPLIT_(TN, SPT, LIT)                                                              \
     hipLaunchKernelGGL((kpp_step_split_kernel<T, TN, SPT, false, LIT>), dim3((unsigned)L.n_blocks),    \
                        dim3(256), 0, s, (const T*)X_t, (const T*)w, (const T*)p.cand_rows, (T*)p.rows, \
-                       p.block_pot, p.header, n, d, 0, n_trials, vec_split, 0, (T*)nullptr,            \
+                       p.block_pot, p.header, n, d, 0, n_trials, 0, (T*)nullptr,            \
                        (int32_t*)nullptr)
 #define KMX_KPP_STEP_SPLIT(TN, SPT) \
     do { if (literal) KMX_KPP_STEP_SPLIT_(TN, SPT, true); else KMX_KPP_STEP_SPLIT_(TN, SPT, false); } while (0)
@@ -1116,12 +1074,10 @@ void launch_step(const void* X_t, const void* w, const int32_t* cand, const KppP
 #undef KMX_KPP_STEP_SPLIT_
         return;
     }
-    const int vec_ok = (n % 4 == 0) && (((uintptr_t)X_t) % 16 == 0) && (((uintptr_t)w) % 16 == 0) &&
-                       (((uintptr_t)p.rows) % 16 == 0);
 #define KMX_KPP_STEP(TN, FUSED)                                                                      \
     hipLaunchKernelGGL((kpp_step_kernel<T, TN, FUSED, false>), dim3((unsigned)L.n_blocks), dim3(256), 0, s, \
                        (const T*)X_t, (const T*)w, (const T*)p.cand_rows, (T*)p.rows, p.block_pot,   \
-                       p.header, n, d, 0, n_trials, vec_ok, 0, (T*)nullptr, (int32_t*)nullptr)
+                       p.header, n, d, 0, n_trials, 0, (T*)nullptr, (int32_t*)nullptr)
     if (n_trials <= 8) {
         if (literal) KMX_KPP_STEP(8, false); else KMX_KPP_STEP(8, true);
     } else {
@@ -1145,8 +1101,6 @@ size_t screen_bytes(const KppLayout& L, int64_t n, int d, int k, int n_trials, i
 template <typename T>
 int32_t launch_screen_step(const void* X_t, const void* X_rm, const KmxTiles& tiles, const void* w, const int32_t* cand,
                            const KppPtrs& p, const KppLayout& L, int64_t n, int d, int n_trials, hipStream_t s) {
-    const int vec_ok = (n % 4 == 0) && (((uintptr_t)X_t) % 16 == 0) && (((uintptr_t)w) % 16 == 0) &&
-                       (((uintptr_t)p.rows) % 16 == 0);
     const size_t lds = screen_lds<T>(d, tiles.S);
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&kpp_screen_step_kernel<T>),
@@ -1155,7 +1109,7 @@ int32_t launch_screen_step(const void* X_t, const void* X_rm, const KmxTiles& ti
     }
     hipLaunchKernelGGL((kpp_screen_step_kernel<T>), dim3((unsigned)L.n_blocks), dim3(512), lds, s, (const T*)X_t,
                        (const T*)X_rm, tiles, (const T*)w, cand, (const T*)p.cand_rows, (T*)p.rows, p.block_pot,
-                       p.header, n, d, n_trials, vec_ok, d % 4 == 0 ? 1 : 0);
+                       p.header, n, d, n_trials);
     return KMX_OK;
 }
 

@@ -21,32 +21,17 @@
 
 namespace {
 
+// R consecutive samples of one feature row; one load where all of them exist.
 template <typename T, int R>
-struct VecOf;
-template <>
-struct VecOf<float, 1> { using type = float; };
-template <>
-struct VecOf<float, 2> { using type = float2; };
-template <>
-struct VecOf<float, 4> { using type = float4; };
-template <>
-struct VecOf<double, 1> { using type = double; };
-template <>
-struct VecOf<double, 2> { using type = double2; };
-
-// R consecutive samples of one feature row; vector load when the row is aligned.
-template <typename T, int R>
-__device__ __forceinline__ void load_row(const T* __restrict__ row, int64_t i0, int64_t n,
-                                         bool vec_ok, T (&out)[R]) {
-    if (vec_ok && i0 + R <= n) {
-        using V = typename VecOf<T, R>::type;
-        union {
-            V v;
-            T s[R];
-        } u;
-        u.v = *reinterpret_cast<const V*>(row + i0);
+__device__ __forceinline__ void load_row(const T* __restrict__ row, int64_t i0, int64_t n, T (&out)[R]) {
+    if (i0 + R <= n) {
+        if constexpr (R == 1) {
+            out[0] = row[i0];
+        } else {
+            const auto v = *reinterpret_cast<const typename KmxVec<T, R>::type*>(row + i0);
 #pragma unroll
-        for (int r = 0; r < R; ++r) out[r] = u.s[r];
+            for (int r = 0; r < R; ++r) out[r] = v[r];
+        }
     } else {
 #pragma unroll
         for (int r = 0; r < R; ++r) out[r] = (i0 + r < n) ? row[i0 + r] : T(0);
@@ -65,7 +50,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_reg_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight, const T* __restrict__ cpack,
     const T* __restrict__ half_norms, const uint32_t* __restrict__ labels_prev,
     uint32_t* __restrict__ labels, T* __restrict__ partial, kmx_lloyd_status* __restrict__ status,
-    int64_t n, int d, int k, int dpad, int n_copies, int vec_ok, int lds_copies) {
+    int64_t n, int d, int k, int dpad, int n_copies, int lds_copies) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
 
     // LDS accumulators are fp64 for both types: ds_add_f64 is fast on this hardware, ds_add_f32
@@ -93,7 +78,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_reg_kernel(
 #pragma unroll
         for (int f = 0; f < DREG; ++f) {
             if (f < d) {
-                load_row<T, R>(X_t + (size_t)f * n, i0, n, vec_ok != 0, x[f]);
+                load_row<T, R>(X_t + (size_t)f * n, i0, n, x[f]);
             } else {
 #pragma unroll
                 for (int r = 0; r < R; ++r) x[f][r] = T(0);
@@ -189,7 +174,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_stream_kernel(
     const T* __restrict__ centroids_t, const T* __restrict__ half_norms,
     const uint32_t* __restrict__ labels_prev, uint32_t* __restrict__ labels,
     T* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k,
-    int n_copies, int vec_ok, int lds_copies) {
+    int n_copies, int lds_copies) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
 
     // LDS accumulators are fp64 for both types: ds_add_f64 is fast on this hardware, ds_add_f32
@@ -231,7 +216,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_stream_kernel(
 #pragma unroll 4
             for (int f = 0; f < d; ++f) {
                 T xv[R];
-                load_row<T, R>(X_t + (size_t)f * n, i0, n, vec_ok != 0, xv);
+                load_row<T, R>(X_t + (size_t)f * n, i0, n, xv);
                 const T* __restrict__ crow = centroids_t + (size_t)f * k;  // wave-uniform
 #pragma unroll
                 for (int j = 0; j < KC; ++j) {
@@ -276,7 +261,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_stream_kernel(
 #pragma unroll 4
             for (int f = 0; f < d; ++f) {
                 T xv[R];
-                load_row<T, R>(X_t + (size_t)f * n, i0, n, vec_ok != 0, xv);
+                load_row<T, R>(X_t + (size_t)f * n, i0, n, xv);
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     if (i0 + r < n) {
@@ -659,10 +644,9 @@ void launch_reg(const LloydLayout& L, const void* X_t, const void* w, const T* c
                 kmx_lloyd_status* status, int64_t n, int d, int k, int grid, hipStream_t stream) {
     const int copies = lds_acc_copies(d, k);
     const size_t lds = (ACC == ACC_LDS) ? (size_t)(d + 1) * k * sizeof(double) * copies : 0;
-    const int vec_ok = (n % R == 0) && (((uintptr_t)X_t) % (R * sizeof(T)) == 0);
     hipLaunchKernelGGL((lloyd_fused_reg_kernel<T, DREG, R, ACC>), dim3(grid), dim3(256), lds, stream,
                        (const T*)X_t, (const T*)w, cpack, half_norms, labels_prev, labels, partial,
-                       status, n, d, k, L.dpad, L.n_partials, vec_ok, copies);
+                       status, n, d, k, L.dpad, L.n_partials, copies);
 }
 
 // Returns the status of the entry point it hands over to (a refusal there would leave `labels`
@@ -718,12 +702,11 @@ int32_t launch_fused(const LloydLayout& L, const void* X_t, const void* w, const
         if (lloyd_stream_samples_per_thread(n, sizeof(T) == 8 ? KMX_F64 : KMX_F32) == 1) {
             hipLaunchKernelGGL((lloyd_fused_stream_kernel<T, 1, KC, ACC>), dim3(grid), dim3(256), lds,
                                stream, (const T*)X_t, (const T*)w, (const T*)centroids_t, half_norms,
-                               labels_prev, labels, partial, status, n, d, k, L.n_partials, 0, copies);
+                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies);
         } else {
-            const int vec_ok = (n % RV == 0) && (((uintptr_t)X_t) % 16 == 0);
             hipLaunchKernelGGL((lloyd_fused_stream_kernel<T, RV, KC, ACC>), dim3(grid), dim3(256), lds,
                                stream, (const T*)X_t, (const T*)w, (const T*)centroids_t, half_norms,
-                               labels_prev, labels, partial, status, n, d, k, L.n_partials, vec_ok, copies);
+                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies);
         }
     }
     KMX_LAUNCH_CHECK();
@@ -1517,22 +1500,17 @@ size_t kmx_assign_workspace_bytes_for(int64_t n, int32_t d, int32_t k, int32_t d
 
 // fp64 labels of up to 64 features: the screen, or the fp64 product.  The screen saves matrix work; its
 // operands take longer to prepare, which few samples do not pay back, and features past a multiple of 16
-// are padding.  Rows that 128-bit loads cannot take (any n not divisible by 4) go through its loop of
-// scalar loads, where wide samples lose.  Measured, product -> screen, us (clusters as many as fit):
-//   128-bit loads: 1e6 x 14 311 -> 77, 50 333 -> 173, 64 307 -> 180; 128 000 x 50 57 -> 43, 64 49 -> 38;
-//     64 000 x 48 30 -> 28, 50 32 -> 36, 64 29 -> 32; 8 000 x 6 48 -> 37, 4 39 -> 41; 200 000 x 4 72 -> 51
-//   scalar loads: 300 001 x 17 96 -> 66, 36 100 -> 66, 56 102 -> 94, 64 89 -> 105; 128 001 x 16 39 -> 34,
-//     20 38 -> 41, 24 40 -> 43, 36 55 -> 38, 56 57 -> 49; 64 001 x 24 42 -> 39, 36 30 -> 34, 56 33 -> 46
+// are padding.  Measured, product -> screen, us (clusters as many as fit):
+//   1e6 x 14 311 -> 77, 50 333 -> 173, 64 307 -> 180; 128 000 x 50 57 -> 43, 64 49 -> 38;
+//   64 000 x 48 30 -> 28, 50 32 -> 36, 64 29 -> 32; 8 000 x 6 48 -> 37, 4 39 -> 41; 200 000 x 4 72 -> 51
+// Arrays of 4 GB or more go through its loop of scalar loads, where the widest samples lose
+// (300 001 x 56 102 -> 94, 64 89 -> 105).
 // Not below four features, where the margins of many clusters are too narrow for the certificate:
 // 1e6 x 1, 1 500 clusters 468 -> 1 202.
-static bool f64_labels_screened(const void* X_t, const void* labels, int64_t n, int d) {
+static bool f64_labels_screened(int64_t n, int d) {
     if (d < 6) return d >= 4 && n >= 200000;
-    const bool wide_loads = n % 4 == 0 && (uint64_t)n * (uint64_t)d < ((uint64_t)1 << 29) &&
-                            (((uintptr_t)X_t | (uintptr_t)labels) & 15) == 0;
-    if (wide_loads) return d <= 48 || n >= 100000;
-    if (d <= 16) return true;
-    if (d <= 32) return n >= 200000 || (d >= 24 && n <= 65536);
-    return d <= 56 && n >= 100000;
+    if ((uint64_t)n * (uint64_t)d >= ((uint64_t)1 << 29)) return d <= 56;
+    return d <= 48 || n >= 100000;
 }
 
 int32_t kmx_assign_labels(const void* X_t, const void* centroids_t, uint32_t* labels,
@@ -1589,7 +1567,7 @@ int32_t kmx_assign_labels(const void* X_t, const void* centroids_t, uint32_t* la
     } else {
         // fp64 inputs: the screened step's kernel without the update, also where its sums would
         // not fit the LDS beside the operands.
-        const bool labels_only = f64_labels_screened(X_t, labels, n, d) && (L.variant == KMX_VARIANT_MFMA_F64 || L.variant == KMX_VARIANT_GEMM) &&
+        const bool labels_only = f64_labels_screened(n, d) && (L.variant == KMX_VARIANT_MFMA_F64 || L.variant == KMX_VARIANT_GEMM) &&
                                  (flags & (KMX_FLAG_PATH_MASK | KMX_FLAG_LABELS_MASK)) == 0 &&
                                  kmx_mfma_screen_labels_fits(n, d, k, 8);
         if (L.screen64 || labels_only)

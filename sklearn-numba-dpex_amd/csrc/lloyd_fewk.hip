@@ -108,7 +108,7 @@ void lloyd_fewk_kernel(
     const float* __restrict__ X_t, const float* __restrict__ X_rm, const float* __restrict__ sample_weight,
     const float* __restrict__ centroids_t, const float* __restrict__ half_norms,
     const uint32_t* __restrict__ labels_prev, uint32_t* __restrict__ labels,
-    float* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int vec_ok) {
+    float* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k) {
     if (status->state != KMX_RUNNING) return;
     constexpr int FBW = KW / 4 + 1;  // blocks of 16 features per wave
     constexpr int PF = fewk_prefetch(KW, S_LOG, NW);
@@ -197,7 +197,7 @@ void lloyd_fewk_kernel(
     float w_next = 0.0f;
     uint32_t pl_next = 0u;
     auto fetch = [&](const int64_t s0) __attribute__((always_inline)) {
-        const bool whole = vec_ok && s0 + S <= n;  // workgroup-uniform
+        const bool whole = s0 + S <= n;  // workgroup-uniform
         if ((int)threadIdx.x < 4 * S && (threadIdx.x & 3) == 0 && s0 + (threadIdx.x >> 2) < n) {
             w_next = sample_weight[s0 + (threadIdx.x >> 2)];
             pl_next = labels_prev[s0 + (threadIdx.x >> 2)];
@@ -220,7 +220,8 @@ void lloyd_fewk_kernel(
                 if (f_t + u * RSTEP < d) {
                     const float* p = X_t + ((size_t)(u * RSTEP) * n + s0) + x_mine;
                     if (whole) {
-                        pf[u] = *reinterpret_cast<const float4*>(p);
+                        const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(p);
+                        pf[u] = make_float4(v[0], v[1], v[2], v[3]);
                     } else {
                         const int64_t i = s0 + 4 * q_t;
                         if (i < n) pf[u].x = p[0];
@@ -811,7 +812,7 @@ __global__ __launch_bounds__(512)
 __attribute__((amdgpu_waves_per_eu(fewk_labels_waves_per_simd(KW), fewk_labels_waves_per_simd(KW))))
 void fewk_labels_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t, const float* __restrict__ half_norms,
-    uint32_t* __restrict__ labels, int64_t n, int d, int k, int vec_ok) {
+    uint32_t* __restrict__ labels, int64_t n, int d, int k) {
     constexpr int NW = 8, TS = 16 * SV;  // waves, samples per tile
     constexpr int CH = SV == 4 ? 4 : 8;   // K steps whose loads are in flight together
     __shared__ __align__(16) float part[NW][SV][256];  // [wave][block][sample m][cluster]
@@ -836,7 +837,7 @@ void fewk_labels_kernel(
     const int64_t n_tiles = (n + TS - 1) / TS;
     for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
         const int64_t s0 = t * TS;
-        const bool whole = vec_ok && s0 + TS <= n;  // workgroup-uniform
+        const bool whole = s0 + TS <= n;  // workgroup-uniform
         v4f sc[SV];
 #pragma unroll
         for (int e = 0; e < SV; ++e) sc[e] = start;
@@ -852,13 +853,9 @@ void fewk_labels_kernel(
                     const float* p = X_t + (size_t)f * n + s0 + SV * m16;
                     if (s < KW) {
                         if (whole) {
-                            if constexpr (SV == 4) {
-                                const float4 v = *reinterpret_cast<const float4*>(p);
-                                b[j][0] = v.x; b[j][1] = v.y; b[j][2] = v.z; b[j][3] = v.w;
-                            } else {
-                                const float2 v = *reinterpret_cast<const float2*>(p);
-                                b[j][0] = v.x; b[j][1] = v.y;
-                            }
+                            const auto v = *reinterpret_cast<const typename KmxVec<float, SV>::type*>(p);
+#pragma unroll
+                            for (int e = 0; e < SV; ++e) b[j][e] = v[e];
                         } else {
 #pragma unroll
                             for (int e = 0; e < SV; ++e) b[j][e] = s0 + SV * m16 + e < n ? p[e] : 0.0f;
@@ -914,7 +911,7 @@ void fewk_labels_kernel(
 template <int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void fewk_labels_wave_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t, const float* __restrict__ half_norms,
-    uint32_t* __restrict__ labels, int64_t n, int d, int k, int vec_ok) {
+    uint32_t* __restrict__ labels, int64_t n, int d, int k) {
     constexpr int SV = 4, TS = 16 * SV, CH = 4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int g4 = lane >> 4, m16 = lane & 15;
@@ -936,7 +933,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const int64_t n_tiles = (n + TS - 1) / TS;
     for (int64_t t = (int64_t)blockIdx.x * 4 + wave; t < n_tiles; t += (int64_t)gridDim.x * 4) {
         const int64_t s0 = t * TS;
-        const bool whole = vec_ok && s0 + TS <= n;  // wave-uniform
+        const bool whole = s0 + TS <= n;  // wave-uniform
         v4f sc[SV];
 #pragma unroll
         for (int e = 0; e < SV; ++e) sc[e] = start;
@@ -949,8 +946,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                     const int f = 4 * (c0 + j) + g4 < d ? 4 * (c0 + j) + g4 : d - 1;
                     const float* p = X_t + (size_t)f * n + s0 + SV * m16;
                     if (whole) {
-                        const float4 v = *reinterpret_cast<const float4*>(p);
-                        b[j][0] = v.x; b[j][1] = v.y; b[j][2] = v.z; b[j][3] = v.w;
+                        const auto v = *reinterpret_cast<const typename KmxVec<float, SV>::type*>(p);
+#pragma unroll
+                        for (int e = 0; e < SV; ++e) b[j][e] = v[e];
                     } else {
 #pragma unroll
                         for (int e = 0; e < SV; ++e) b[j][e] = s0 + SV * m16 + e < n ? p[e] : 0.0f;
@@ -994,7 +992,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         if (g4 == 0) {
             const int64_t gi = s0 + SV * m16;
             if (whole) {
-                *reinterpret_cast<uint4*>(labels + gi) = make_uint4(lab[0], lab[1], lab[2], lab[3]);
+                *reinterpret_cast<KmxVec<uint32_t, 4>::type*>(labels + gi) =
+                    KmxVec<uint32_t, 4>::type{lab[0], lab[1], lab[2], lab[3]};
             } else {
 #pragma unroll
                 for (int e = 0; e < SV; ++e)
@@ -1102,7 +1101,6 @@ int32_t kmx_lloyd_iter_fewk(const LloydLayout& L, const void* X_t, const void* X
     const size_t slots = (size_t)sh.nw * (sh.kw / 4 + 1) * 256;  // partial sums of a workgroup of the instantiated kernel
     if ((size_t)grid * slots * sizeof(float) > L.partial_bytes) grid = (int)(L.partial_bytes / (slots * sizeof(float)));
     if (grid < 1) return KMX_ERR_WORKSPACE;
-    const int vec_ok = (n % 4 == 0) && ((((uintptr_t)X_t) & 15) == 0);
     // whole samples from the row-major copy when there is one whose rows are multiples of 16 bytes
     const bool rm = X_rowmajor != nullptr && d % 4 == 0 && ((((uintptr_t)X_rowmajor) & 15) == 0);
     if (events) (void)hipEventRecord(events[0], stream);
@@ -1157,7 +1155,7 @@ int32_t kmx_lloyd_iter_fewk(const LloydLayout& L, const void* X_t, const void* X
                            dim3(64 * NW_),                                                                \
                            sh.lds, stream, (const float*)X_t, (const float*)X_rowmajor, (const float*)w,  \
                            (const float*)centroids_t, half_norms, labels_prev, labels, partial, status,   \
-                           n, d, k, vec_ok);                                                              \
+                           n, d, k);                                                                      \
     } while (0)
 #define KMX_FEWK_LAUNCH(KW_, SL_, FBW_, NW_)                                \
     do {                                                                   \
@@ -1195,25 +1193,22 @@ int32_t kmx_assign_labels_fewk(const void* X_t, const void* centroids_t, const v
     // tiles of 64 samples; of 32 while those would not give every compute unit a few tiles
     const int64_t tiles64 = kmx_cdiv(n, 64);
     if (d <= 128 && tiles64 >= (int64_t)16 * kmx_num_cus()) {
-        // every wave on tiles of its own (labels are written 128 bits at a time: 16-byte aligned)
-        const int vec = (n % 4 == 0) && ((((uintptr_t)X_t) & 15) == 0) && ((((uintptr_t)labels) & 15) == 0);
+        // every wave on tiles of its own
         int64_t wg = (int64_t)3 * kmx_num_cus();
         if (wg > kmx_cdiv(tiles64, 4)) wg = kmx_cdiv(tiles64, 4);
         hipLaunchKernelGGL((fewk_labels_wave_kernel<32>), dim3((unsigned)wg), dim3(256), 0, stream, (const float*)X_t,
-                           (const float*)centroids_t, (const float*)half_norms, labels, n, d, k, vec);
+                           (const float*)centroids_t, (const float*)half_norms, labels, n, d, k);
         KMX_LAUNCH_CHECK();
         return KMX_OK;
     }
     const bool small = tiles64 < (int64_t)8 * kmx_num_cus();
     const int ts = small ? 32 : 64;
-    const int sv = ts / 16;
-    const int vec_ok = (n % sv == 0) && ((((uintptr_t)X_t) & (size_t)(4 * sv - 1)) == 0);
     int64_t grid = (int64_t)2 * kmx_num_cus();
     const int64_t tiles = kmx_cdiv(n, ts);
     if (grid > tiles) grid = tiles;
 #define KMX_FEWK_LABELS(KW_, SV_)                                                                                     \
     hipLaunchKernelGGL((fewk_labels_kernel<KW_, SV_>), dim3((unsigned)grid), dim3(512), 0, stream, (const float*)X_t, \
-                       (const float*)centroids_t, (const float*)half_norms, labels, n, d, k, vec_ok)
+                       (const float*)centroids_t, (const float*)half_norms, labels, n, d, k)
     const int kw = fewk_kw(d, 8);
     if (kw <= 16) {
         if (small) KMX_FEWK_LABELS(16, 2);

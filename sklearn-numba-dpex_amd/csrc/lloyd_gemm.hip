@@ -16,7 +16,7 @@
 //     tile of 32 or 64 for that few clusters); the
 //     features are staged 16 (fp32) or 8 (fp64) at a time through double-buffered LDS tiles.
 //     Both arrays are feature-major in memory, as the tiles are in LDS: a stage is a copy of
-//     rows (128-bit loads where alignment allows), rows padded so that the operand reads of a
+//     rows (128-bit loads), rows padded so that the operand reads of a
 //     wave fall on distinct banks.  The next stage's loads are in flight during the MFMAs.
 //   * A wave multiplies all 128 centroids of the tile with its own 32 samples: centroids are
 //     the rows of the MFMA result and samples its columns, so a lane holds scores of ONE
@@ -43,25 +43,28 @@ constexpr int GLD64 = GT + 16;  // in doubles: the K rows of a half-wave's read 
 // 64 centroids 32 or 16.
 template <int L, int GROUPS = 32>
 __device__ __forceinline__ void stage_load_f32(float4 (&r)[L], const float* __restrict__ base, int64_t len,
-                                               int64_t c0, int d, int f0, bool vec_ok) {
+                                               int64_t c0, int d, int f0) {
+    // (the same for the whole workgroup: the loads of a stage that exists whole are then straight-line
+    // code, none of them waited for in a branch of its own)
+    const bool whole = f0 + 256 * L / GROUPS <= d && c0 + 4 * GROUPS <= len;
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int g = threadIdx.x + 256 * l;
         const int f = f0 + g / GROUPS;
         const int64_t c = c0 + 4 * (g % GROUPS);
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (f < d) {
-            const float* __restrict__ src = base + (size_t)f * (size_t)len + c;
-            if (vec_ok && c + 4 <= len) {
-                v = *reinterpret_cast<const float4*>(src);
-            } else {
-                if (c + 0 < len) v.x = src[0];
-                if (c + 1 < len) v.y = src[1];
-                if (c + 2 < len) v.z = src[2];
-                if (c + 3 < len) v.w = src[3];
+        const float* __restrict__ src = base + (size_t)f * (size_t)len + c;
+        if (whole) {
+            const auto q = *reinterpret_cast<const KmxVec<float, 4>::type*>(src);
+            r[l] = make_float4(q[0], q[1], q[2], q[3]);
+        } else {
+            r[l] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (f < d) {
+                if (c + 0 < len) r[l].x = src[0];
+                if (c + 1 < len) r[l].y = src[1];
+                if (c + 2 < len) r[l].z = src[2];
+                if (c + 3 < len) r[l].w = src[3];
             }
         }
-        r[l] = v;
     }
 }
 
@@ -108,7 +111,7 @@ template <int NA, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
     const float* __restrict__ X_t, const float* __restrict__ centroids_t,
     const float* __restrict__ half_norms, uint32_t* __restrict__ labels,
-    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
+    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k,
     const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
     const unsigned int* __restrict__ all_count = nullptr, int64_t all_from = 0) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
@@ -143,10 +146,10 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
         }
         auto load_x = [&](float4(&r)[XL], const int f0) {
             if constexpr (LISTED) stage_load_listed_f32<XL>(r, X_t, n, cols, d, f0);
-            else stage_load_f32<XL>(r, X_t, n, i0, d, f0, x_vec != 0);
+            else stage_load_f32<XL>(r, X_t, n, i0, d, f0);
         };
         auto load_c = [&](float4(&r)[CL], const int c0, const int f0) {
-            stage_load_f32<CL, CG>(r, centroids_t, k, c0, d, f0, c_vec != 0);
+            stage_load_f32<CL, CG>(r, centroids_t, k, c0, d, f0);
         };
         for (int c0 = 0; c0 < k; c0 += 32 * NA) {
             __syncthreads();  // the previous tile's reads of hn and of the stage buffers are over
@@ -216,23 +219,24 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f32_kernel(
 // 2 (g % GROUPS)); GROUPS = 64 for 128 columns, 16 or 32 for a tile of 32 or 64 centroids.
 template <int L, int GROUPS = 64>
 __device__ __forceinline__ void stage_load_f64(double2 (&r)[L], const double* __restrict__ base, int64_t len,
-                                               int64_t c0, int d, int f0, bool vec_ok) {
+                                               int64_t c0, int d, int f0) {
+    const bool whole = f0 + 256 * L / GROUPS <= d && c0 + 2 * GROUPS <= len;  // (as above)
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int g = threadIdx.x + 256 * l;
         const int f = f0 + g / GROUPS;
         const int64_t c = c0 + 2 * (g % GROUPS);
-        double2 v = make_double2(0.0, 0.0);
-        if (f < d) {
-            const double* __restrict__ src = base + (size_t)f * (size_t)len + c;
-            if (vec_ok && c + 2 <= len) {
-                v = *reinterpret_cast<const double2*>(src);
-            } else {
-                if (c + 0 < len) v.x = src[0];
-                if (c + 1 < len) v.y = src[1];
+        const double* __restrict__ src = base + (size_t)f * (size_t)len + c;
+        if (whole) {
+            const auto q = *reinterpret_cast<const KmxVec<double, 2>::type*>(src);
+            r[l] = make_double2(q[0], q[1]);
+        } else {
+            r[l] = make_double2(0.0, 0.0);
+            if (f < d) {
+                if (c + 0 < len) r[l].x = src[0];
+                if (c + 1 < len) r[l].y = src[1];
             }
         }
-        r[l] = v;
     }
 }
 
@@ -273,7 +277,7 @@ template <int NA, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
     const double* __restrict__ X_t, const double* __restrict__ centroids_t,
     const double* __restrict__ half_norms, uint32_t* __restrict__ labels,
-    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k, int x_vec, int c_vec,
+    const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k,
     const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr,
     const unsigned int* __restrict__ all_count = nullptr, int64_t all_from = 0) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
@@ -308,7 +312,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
         }
         auto load_x = [&](double2(&r)[XL], const int f0) {
             if constexpr (LISTED) stage_load_listed_f64<XL>(r, X_t, n, cols, d, f0);
-            else stage_load_f64<XL>(r, X_t, n, i0, d, f0, x_vec != 0);
+            else stage_load_f64<XL>(r, X_t, n, i0, d, f0);
         };
         for (int c0 = 0; c0 < k; c0 += 16 * NA) {
             __syncthreads();
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
                 hn[threadIdx.x] = c0 + (int)threadIdx.x < k ? -half_norms[c0 + threadIdx.x] : -kmx_inf<double>();
             double2 rx[XL], rc[CL];
             load_x(rx, 0);
-            stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, 0, c_vec != 0);
+            stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, 0);
             stage_store_f64<XL, GLD64>(xs[0], rx);
             stage_store_f64<CL, CLD, CG>(cs[0], rc);
             __syncthreads();
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
                 const int cur = st & 1;
                 if (st + 1 < n_stages) {
                     load_x(rx, (st + 1) * GK);
-                    stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, (st + 1) * GK, c_vec != 0);
+                    stage_load_f64<CL, CG>(rc, centroids_t, k, c0, d, (st + 1) * GK);
                 }
 #pragma unroll
                 for (int s = 0; s < GK / 4; ++s) {
@@ -400,10 +404,6 @@ __global__ __launch_bounds__(256, 2) void lloyd_gemm_labels_f64_kernel(
 int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const void* half_norms,
                               uint32_t* labels, const kmx_lloyd_status* status, int64_t n, int d, int k,
                               int32_t dtype, hipStream_t stream) {
-    const size_t s = kmx_dtype_size(dtype);
-    const int per_vec = (int)(16 / s);
-    auto vec_ok = [&](const void* p, int64_t len) { return (len % per_vec == 0) && ((((uintptr_t)p) & 15) == 0); };
-    const int x_vec = vec_ok(X_t, n), c_vec = vec_ok(centroids_t, k);
     int64_t grid = kmx_cdiv(n, GT);
     // workgroups per compute unit: what registers and LDS allow (one workgroup per tile instead
     // measured 4 % slower)
@@ -412,7 +412,7 @@ int32_t kmx_lloyd_gemm_labels(const void* X_t, const void* centroids_t, const vo
     if (grid > cap) grid = cap;
 #define KMX_GEMM_LAUNCH(KERNEL, T)                                                                    \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t,             \
-                       (const T*)centroids_t, (const T*)half_norms, labels, status, n, d, k, x_vec, c_vec)
+                       (const T*)centroids_t, (const T*)half_norms, labels, status, n, d, k)
     // centroid tile: 32 / 64 for that few clusters, else 128
     if (dtype == KMX_F32) {
         if (k <= 32) KMX_GEMM_LAUNCH(lloyd_gemm_labels_f32_kernel<1>, float);
@@ -436,13 +436,12 @@ int32_t kmx_lloyd_gemm_labels_listed(const void* X_t, const void* centroids_t, c
                                      const unsigned int* list_count, int64_t n, int d, int k,
                                      int32_t dtype, hipStream_t stream, const unsigned int* all_count,
                                      int64_t all_from) {
-    const int c_vec = (k % (dtype == KMX_F32 ? 4 : 2) == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
     int64_t grid = kmx_cdiv(n, GT);
     const int64_t cap = (int64_t)(dtype == KMX_F32 ? 3 : 2) * kmx_num_cus();
     if (grid > cap) grid = cap;
 #define KMX_GEMM_LISTED(KERNEL, T)                                                                             \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t, (const T*)centroids_t, \
-                       (const T*)half_norms, labels, status, n, d, k, 0, c_vec, list, list_count, all_count, all_from)
+                       (const T*)half_norms, labels, status, n, d, k, list, list_count, all_count, all_from)
     if (dtype == KMX_F32) {
         if (k <= 32) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<1, true>), float);
         else if (k <= 64) KMX_GEMM_LISTED((lloyd_gemm_labels_f32_kernel<2, true>), float);

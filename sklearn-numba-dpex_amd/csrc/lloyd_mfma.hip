@@ -52,35 +52,34 @@ __global__ void absmax_zero_kernel(unsigned int* absmax, int count) {
 // Row r < d: max |X_t[r, :]|; row d: max |w|.  Non-negative floats order like their bits.
 // (fp64 inputs: the maximum of the values rounded to fp32, which is what the screened step works
 // with; its fixed-point exponents leave a factor of two of room above it)
-__device__ __forceinline__ float amax_vec(float a, const float4& v) {
-    return fmaxf(fmaxf(a, fabsf(v.x)), fmaxf(fabsf(v.y), fmaxf(fabsf(v.z), fabsf(v.w))));
+__device__ __forceinline__ float amax_vec(float a, KmxVec<float, 4>::type v) {
+    return fmaxf(fmaxf(a, fabsf(v[0])), fmaxf(fabsf(v[1]), fmaxf(fabsf(v[2]), fabsf(v[3]))));
 }
-__device__ __forceinline__ float amax_vec(float a, const double2& v) {
-    return fmaxf(a, fmaxf(fabsf((float)v.x), fabsf((float)v.y)));
+__device__ __forceinline__ float amax_vec(float a, KmxVec<double, 2>::type v) {
+    return fmaxf(a, fmaxf(fabsf((float)v[0]), fabsf((float)v[1])));
 }
 template <typename T>
 __global__ __launch_bounds__(256) void absmax_rows_kernel(const T* __restrict__ X_t,
                                                           const T* __restrict__ w,
                                                           unsigned int* __restrict__ absmax,
-                                                          int64_t n, int d, int vec_ok) {
+                                                          int64_t n, int d) {
     const int row = blockIdx.y;
     const T* __restrict__ p = row < d ? X_t + (size_t)row * n : w;
     float m = 0.0f;
     const int64_t stride = (int64_t)gridDim.x * 256;
-    if (vec_ok) {
-        // rows start 16-byte aligned and n is a multiple of 4: 128-bit loads
-        using V = std::conditional_t<sizeof(T) == 8, double2, float4>;
+    {
+        constexpr int W = 16 / (int)sizeof(T);
+        using V = typename KmxVec<T, W>::type;
         const V* __restrict__ p4 = reinterpret_cast<const V*>(p);
-        const int64_t n4 = n / (int64_t)(16 / sizeof(T));
+        const int64_t n4 = n / W;
         int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
         for (; g + 3 * stride < n4; g += 4 * stride) {  // four loads in flight per lane
             const V v0 = p4[g], v1 = p4[g + stride], v2 = p4[g + 2 * stride], v3 = p4[g + 3 * stride];
             m = amax_vec(amax_vec(amax_vec(amax_vec(m, v0), v1), v2), v3);
         }
         for (; g < n4; g += stride) m = amax_vec(m, p4[g]);
-    } else {
-        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride)
-            m = fmaxf(m, fabsf((float)p[i]));
+        // (the last values of a row)
+        if (blockIdx.x == 0 && n4 * W + threadIdx.x < n) m = fmaxf(m, fabsf((float)p[n4 * W + threadIdx.x]));
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
@@ -136,8 +135,7 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
     const float* __restrict__ X_t, const float* __restrict__ sample_weight,
     const float* __restrict__ centroids_t, const uint32_t* __restrict__ labels_prev,
     uint32_t* __restrict__ labels, kmx_lloyd_status* __restrict__ status,
-    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum, int64_t n, int d, int k,
-    int vec_ok) {
+    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum, int64_t n, int d, int k) {
     if (UPDATE && status->state != KMX_RUNNING) return;
 
     constexpr int WAVES = mfma_waves(NKS, MC), THREADS = 64 * WAVES;
@@ -200,7 +198,7 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
     // One tile of NC sample columns per lane: scores on the matrix cores, argmax, labels and
     // (UPDATE) the accumulation.  NC = 4: 128 samples, the lane's samples are i0 .. i0 + 3;
     // NC = 1: 32 samples (a quarter tile), the lane's sample is i0.  FULL: every sample of the
-    // tile exists and (NC = 4) 128-bit accesses are legal.  wv / pl: weights and previous
+    // tile exists.  wv / pl: weights and previous
     // labels of the lane's samples.
     // +inf the optimiser cannot see through (it would turn the median in the arg-max into a
     // maximum with two canonicalising instructions in front)
@@ -310,9 +308,10 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
 
         if (h == 0) {
             if constexpr (FULL && NC == 4) {
-                *reinterpret_cast<uint4*>(labels + i0) = make_uint4(lab[0], lab[1], lab[2], lab[3]);
+                *reinterpret_cast<KmxVec<uint32_t, 4>::type*>(labels + i0) =
+                    KmxVec<uint32_t, 4>::type{lab[0], lab[1], lab[2], lab[3]};
             } else if constexpr (FULL && NC == 2) {
-                *reinterpret_cast<uint2*>(labels + i0) = make_uint2(lab[0], lab[1]);
+                *reinterpret_cast<KmxVec<uint32_t, 2>::type*>(labels + i0) = KmxVec<uint32_t, 2>::type{lab[0], lab[1]};
             } else {
 #pragma unroll
                 for (int t = 0; t < NC; ++t)
@@ -359,10 +358,10 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
 
     const int64_t wt_step = (int64_t)gridDim.x * WAVES;
     const int64_t wt_first = (int64_t)blockIdx.x * WAVES + wave;
-    // Tiles that lie entirely inside the array, when vector accesses are legal: straight-line
+    // Tiles that lie entirely inside the array: straight-line
     // loads with the next tile's rows in flight during the current tile (the wave does not
     // stall on its own loads or on the completion of its label store).
-    const int64_t n_fast = vec_ok ? n / TILE : 0;
+    const int64_t n_fast = n / TILE;
     // The last round of full tiles would keep only n_fast % wt_step of the waves busy for a
     // whole tile time.  When it is at most three quarters full it is cut into single-column
     // tiles of 32 samples instead (one MFMA chain per wave), spread over all the waves.
@@ -378,13 +377,9 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
     const int last_row = 2 * (nks - 1) + h < d ? 2 * (nks - 1) + h : d - 1;
     const size_t last_row_off = (size_t)(last_row - h) * n;
     auto load_cols = [&](const float* __restrict__ p, float(&v)[MC]) {
-        if constexpr (MC == 4) {
-            const float4 q = *reinterpret_cast<const float4*>(p);
-            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-        } else {
-            const float2 q = *reinterpret_cast<const float2*>(p);
-            v[0] = q.x; v[1] = q.y;
-        }
+        const auto q = *reinterpret_cast<const typename KmxVec<float, MC>::type*>(p);
+#pragma unroll
+        for (int t = 0; t < MC; ++t) v[t] = q[t];
     };
     auto load_rows = [&](const int64_t wt, float(&dst)[NKS][MC]) {
         const float* __restrict__ p = xrow_base + wt * TILE;
@@ -425,13 +420,9 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
             }
             if (UPDATE) {
                 load_cols(sample_weight + i0, wv);
-                if constexpr (MC == 4) {
-                    const uint4 p4 = *reinterpret_cast<const uint4*>(labels_prev + i0);
-                    pl[0] = p4.x; pl[1] = p4.y; pl[2] = p4.z; pl[3] = p4.w;
-                } else {
-                    const uint2 p2 = *reinterpret_cast<const uint2*>(labels_prev + i0);
-                    pl[0] = p2.x; pl[1] = p2.y;
-                }
+                const auto p4 = *reinterpret_cast<const typename KmxVec<uint32_t, MC>::type*>(labels_prev + i0);
+#pragma unroll
+                for (int t = 0; t < MC; ++t) pl[t] = p4[t];
             }
             process(ColsM{}, std::true_type{}, x, wv, pl, i0);
         }
@@ -520,14 +511,11 @@ int32_t launch_mfma(const LloydLayout& L, const void* X_t, const void* w, const 
     const int cap = (L.wgs_per_cu > 0 ? L.wgs_per_cu : per_cu) * kmx_num_cus();
     if (grid > cap) grid = cap;
     if (grid < 1) grid = 1;
-    auto aligned16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
-    const int vec_ok = (n % 4 == 0) && aligned16(X_t) && aligned16(labels) &&
-                       (!UPDATE || (aligned16(w) && aligned16(labels_prev)));
 #define KMX_MFMA_LAUNCH(NKS, EXACT, MC)                                                           \
     hipLaunchKernelGGL((lloyd_mfma_kernel<NKS, EXACT, UPDATE, MC>), dim3((unsigned)grid),          \
                        dim3(64 * mfma_waves(NKS, MC)), lds, stream, (const float*)X_t,             \
                        (const float*)w, (const float*)centroids_t, labels_prev, labels, status,    \
-                       q_exp, gsum, n, d, k, vec_ok)
+                       q_exp, gsum, n, d, k)
 #define KMX_MFMA_CASE(NKS, EXACT)                    \
     do {                                             \
         if (mc == 2 && NKS <= 8)                     \
@@ -578,13 +566,12 @@ int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void
     int64_t gx = kmx_cdiv(n, 256 * 64);
     if (gx > 64) gx = 64;
     if (gx * (rows + 1) < 1024) gx = kmx_cdiv(1024, rows + 1) < kmx_cdiv(n, 1024) ? kmx_cdiv(1024, rows + 1) : kmx_cdiv(n, 1024);
-    const int vec_ok = (n % 4 == 0) && ((((uintptr_t)X_t) & 15) == 0) && ((((uintptr_t)w) & 15) == 0);
     if (dtype == KMX_F64)
         hipLaunchKernelGGL(absmax_rows_kernel<double>, dim3((unsigned)gx, (unsigned)(rows + 1)), dim3(256), 0,
-                           stream, (const double*)X_t, (const double*)w, first, n, rows, vec_ok);
+                           stream, (const double*)X_t, (const double*)w, first, n, rows);
     else
         hipLaunchKernelGGL(absmax_rows_kernel<float>, dim3((unsigned)gx, (unsigned)(rows + 1)), dim3(256), 0,
-                           stream, (const float*)X_t, (const float*)w, first, n, rows, vec_ok);
+                           stream, (const float*)X_t, (const float*)w, first, n, rows);
     hipLaunchKernelGGL(fixed_point_exponents_kernel, dim3((unsigned)kmx_cdiv(d + 1, 128)), dim3(128), 0,
                        stream, absmax, q_exp, n, d);
     const size_t words = (size_t)(d + 1) * L.k_for_gsum * 2;

@@ -38,9 +38,9 @@ template <int NC>
 __device__ __forceinline__ void load_cols(const double* __restrict__ p, double (&v)[NC]) {
 #pragma unroll
     for (int c = 0; c < NC; c += 2) {
-        const double2 a = *reinterpret_cast<const double2*>(p + c);
-        v[c] = a.x;
-        v[c + 1] = a.y;
+        const auto a = *reinterpret_cast<const KmxVec<double, 2>::type*>(p + c);
+        v[c] = a[0];
+        v[c + 1] = a[1];
     }
 }
 
@@ -52,8 +52,7 @@ __global__ __launch_bounds__(64 * f64_waves(NC)) void lloyd_mfma_f64_kernel(
     const double* __restrict__ X_t, const double* __restrict__ sample_weight,
     const double* __restrict__ centroids_t, const double* __restrict__ half_norms,
     const uint32_t* __restrict__ labels_prev, uint32_t* __restrict__ labels,
-    double* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k,
-    int vec_ok) {
+    double* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
     constexpr int F64_WAVES = f64_waves(NC);
     constexpr int THREADS = 64 * F64_WAVES;
@@ -91,7 +90,7 @@ __global__ __launch_bounds__(64 * f64_waves(NC)) void lloyd_mfma_f64_kernel(
     unsigned int changed = 0;
 
     // One tile: scores, arg-max, labels and (UPDATE) the accumulation.  FULL: every sample of
-    // the tile exists and 128-bit accesses are legal.
+    // the tile exists.
     auto process = [&](auto full_tag, const double(&x)[NKS][NC], const double(&wv)[NC],
                        const uint32_t(&pl)[NC], const int64_t i0) {
         constexpr bool FULL = decltype(full_tag)::value;
@@ -155,9 +154,10 @@ __global__ __launch_bounds__(64 * f64_waves(NC)) void lloyd_mfma_f64_kernel(
 
         if (g == 0) {
             if constexpr (FULL && NC == 4) {
-                *reinterpret_cast<uint4*>(labels + i0) = make_uint4(lab[0], lab[1], lab[2], lab[3]);
+                *reinterpret_cast<KmxVec<uint32_t, 4>::type*>(labels + i0) =
+                    KmxVec<uint32_t, 4>::type{lab[0], lab[1], lab[2], lab[3]};
             } else if constexpr (FULL && NC == 2) {
-                *reinterpret_cast<uint2*>(labels + i0) = make_uint2(lab[0], lab[1]);
+                *reinterpret_cast<KmxVec<uint32_t, 2>::type*>(labels + i0) = KmxVec<uint32_t, 2>::type{lab[0], lab[1]};
             } else {
 #pragma unroll
                 for (int t = 0; t < NC; ++t)
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(64 * f64_waves(NC)) void lloyd_mfma_f64_kernel(
 
     const int64_t wt_step = (int64_t)gridDim.x * F64_WAVES;
     const int64_t wt_first = (int64_t)blockIdx.x * F64_WAVES + wave;
-    const int64_t n_fast = vec_ok ? n / TILE : 0;  // tiles entirely inside the array
+    const int64_t n_fast = n / TILE;  // tiles entirely inside the array
     // rows 4 s + g of the lane's samples; a row past d - 1 reads row d - 1 (its A fragment is
     // zero and the update skips it), so that the loads are unconditional
     auto load_rows = [&](const int64_t wt, double(&dst)[NKS][NC]) {
@@ -224,18 +224,14 @@ __global__ __launch_bounds__(64 * f64_waves(NC)) void lloyd_mfma_f64_kernel(
             }
             if (UPDATE) {
                 load_cols<NC>(sample_weight + i0, wv);
-                if constexpr (NC == 4) {
-                    const uint4 p4 = *reinterpret_cast<const uint4*>(labels_prev + i0);
-                    pl[0] = p4.x; pl[1] = p4.y; pl[2] = p4.z; pl[3] = p4.w;
-                } else {
-                    const uint2 p2 = *reinterpret_cast<const uint2*>(labels_prev + i0);
-                    pl[0] = p2.x; pl[1] = p2.y;
-                }
+                const auto p4 = *reinterpret_cast<const typename KmxVec<uint32_t, NC>::type*>(labels_prev + i0);
+#pragma unroll
+                for (int t = 0; t < NC; ++t) pl[t] = p4[t];
             }
             process(std::true_type{}, x, wv, pl, i0);
         }
     }
-    // The rest: a partial last tile, or every tile when 128-bit accesses are not legal
+    // The rest: a partial last tile
     for (int64_t wt = n_fast + wt_first; wt < n_wtiles; wt += wt_step) {
         const int64_t i0 = wt * TILE + NC * j;
         double x[NKS][NC];
@@ -314,11 +310,6 @@ int32_t kmx_lloyd_step_mfma_f64(const void* X_t, const void* w, const void* cent
         return KMX_ERR_UNSUPPORTED;
     const size_t lds = mfma_f64_lds_bytes(d, k, update);
     const int grid = kmx_mfma_f64_grid(n, d, wgs_per_cu, cols_asked, max_slots);
-    auto aligned16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
-    // rows start 16-byte aligned when n is even; 4 samples per lane need n % 4 == 0 only for
-    // the 128-bit label accesses
-    const int vec_ok = (n % 4 == 0) && aligned16(X_t) && aligned16(labels) &&
-                       (!update || (aligned16(w) && aligned16(labels_prev)));
     const int cols = f64_cols(n, d, cols_asked);
 #define KMX_F64_LAUNCH(NKS, NC, UPD)                                                              \
     if (lds > 64 * 1024) {                                                                        \
@@ -330,7 +321,7 @@ int32_t kmx_lloyd_step_mfma_f64(const void* X_t, const void* w, const void* cent
     hipLaunchKernelGGL((lloyd_mfma_f64_kernel<NKS, NC, UPD>), dim3((unsigned)grid),                 \
                        dim3(64 * f64_waves(NC)), lds, stream, (const double*)X_t, (const double*)w, \
                        (const double*)centroids_t, (const double*)half_norms, labels_prev, labels,  \
-                       (double*)partial, status, n, d, k, vec_ok)
+                       (double*)partial, status, n, d, k)
 #define KMX_F64_CASE(NKS)                                    \
     do {                                                     \
         if (cols == 2) {                                     \

@@ -1833,11 +1833,9 @@ int32_t launch_screen(const void* X_t, const void* w, const void* centroids_t, c
     const int cap = (wgs_per_cu > 0 ? wgs_per_cu : per_cu) * kmx_num_cus();
     if (grid > cap) grid = cap;
     if (grid < 1) grid = 1;
-    auto aligned16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
-    // (the fast path addresses a lane's rows with 32-bit byte offsets from the tile's address in row 0)
-    const int vec_ok = ((uint64_t)d * (uint64_t)n * (uint64_t)ES < ((uint64_t)1 << 32)) && (n % 4 == 0) && aligned16(X_t) &&
-                       aligned16(labels) && aligned16(w) &&
-                       aligned16(labels_prev);
+    // (the fast path addresses a lane's rows with 32-bit byte offsets from the tile's address in row 0; its
+    // buffer loads take any row that is aligned to an element)
+    const int vec_ok = (uint64_t)d * (uint64_t)n * (uint64_t)ES < ((uint64_t)1 << 32);
     const size_t lds = screen_lds(d, k, nk, UPDATE, ES).total;
     // -0.5||c||^2 in a spare feature slot of the last K step whenever there is one
     const bool hk = d % 16 != 0;

@@ -41,7 +41,7 @@ __device__ __forceinline__ unsigned long long to_fixed(double scaled_plus_magic)
 // The chunk origin is wave-uniform (scalar base), the thread part a 32-bit offset, so no
 // per-chunk 64-bit addresses stay alive across the K loop.
 __device__ __forceinline__ void chunk_prefetch(float4 (&regs)[4], const float* __restrict__ centroids_t,
-                                               int f0, int c0, int d, int k, bool vec_ok) {
+                                               int f0, int c0, int d, int k) {
     const int col = (threadIdx.x & 31) * 4;
     const int row0 = threadIdx.x >> 5;
     const float* __restrict__ base = centroids_t + (size_t)f0 * k + c0;  // uniform
@@ -52,8 +52,9 @@ __device__ __forceinline__ void chunk_prefetch(float4 (&regs)[4], const float* _
         const int off = row * k + col;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (f0 + row < d) {
-            if (vec_ok && c + 4 <= k) {
-                v = *reinterpret_cast<const float4*>(base + off);
+            if (c + 4 <= k) {
+                const auto u = *reinterpret_cast<const KmxVec<float, 4>::type*>(base + off);
+                v = make_float4(u[0], u[1], u[2], u[3]);
             } else {
                 if (c + 0 < k) v.x = base[off + 0];
                 if (c + 1 < k) v.y = base[off + 1];
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_mfma_wide_kernel(
     const uint32_t* __restrict__ labels_prev, uint32_t* __restrict__ labels,
     kmx_lloyd_status* __restrict__ status, const int* __restrict__ q_exp,
     unsigned long long* __restrict__ gsum, int* __restrict__ counts, int* __restrict__ ranks,
-    int64_t n, int d, int k, int vec_ok, const float* __restrict__ X_rm = nullptr,
+    int64_t n, int d, int k, const float* __restrict__ X_rm = nullptr,
     const int* __restrict__ list = nullptr, const unsigned int* __restrict__ list_count = nullptr) {
     constexpr bool UPDATE = MODE != MODE_LABELS;
     if (UPDATE && status->state != KMX_RUNNING) return;
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_mfma_wide_kernel(
 
         float4 regs[4];
         __syncthreads();  // every wave is done with both LDS buffers (previous tile) and hneg_s is set
-        chunk_prefetch(regs, centroids_t, 0, 0, d, k, vec_ok != 0);
+        chunk_prefetch(regs, centroids_t, 0, 0, d, k);
         chunk_store(ctile[0], regs);
         __syncthreads();
 
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(256, 2) void lloyd_mfma_wide_kernel(
                 const bool has_next = (kc + 1 < NKC) || (cg + 1 < n_cg);
                 const int next_f0 = (kc + 1 < NKC) ? (kc + 1) * KC : 0;
                 const int next_c0 = (kc + 1 < NKC) ? cg * CG : (cg + 1) * CG;
-                if (has_next) chunk_prefetch(regs, centroids_t, next_f0, next_c0, d, k, vec_ok != 0);
+                if (has_next) chunk_prefetch(regs, centroids_t, next_f0, next_c0, d, k);
 
                 // A fragments of K step s + 1 are read from LDS while the MFMAs of step s run;
                 // the scheduling barriers keep the compiler from hoisting all 64 reads of the
@@ -279,11 +280,14 @@ __global__ __launch_bounds__(256) void bucket_accumulate_kernel(
     constexpr int U = 8;  // rows in flight per lane
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int f4 = lane * 4;
+    // VEC: the lane's load starts at feature fl, moved back for the lane whose four features do not all
+    // exist (what it reads twice, and what lanes past the row's end read, is dropped below)
+    const int fl = VEC && f4 + 4 > d ? d - 4 : f4;
     double sc[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = f4 + j < d ? (double)ldexpf(1.0f, q_exp[f4 + j]) : 0.0;
+    for (int j = 0; j < 4; ++j) sc[j] = fl + j < d ? (double)ldexpf(1.0f, q_exp[fl + j]) : 0.0;
     const double sc_w = (double)ldexpf(1.0f, q_exp[d]);
-    const float* __restrict__ col = X_rm + (f4 < d ? f4 : 0);
+    const float* __restrict__ col = X_rm + (fl < d ? fl : 0);
 
     int c = c_first;
     int pos = P0;
@@ -321,8 +325,9 @@ __global__ __launch_bounds__(256) void bucket_accumulate_kernel(
                     for (int u = 0; u < U; ++u) {
                         const float* __restrict__ row = col + (size_t)idx[u] * d;
                         if (VEC) {
-                            const float4 v = *reinterpret_cast<const float4*>(row);
-                            xv[u][0] = v.x; xv[u][1] = v.y; xv[u][2] = v.z; xv[u][3] = v.w;
+                            const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(row);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) xv[u][j] = v[j];
                         } else {
 #pragma unroll
                             for (int j = 0; j < 4; ++j) xv[u][j] = f4 + j < d ? row[j] : 0.0f;
@@ -343,7 +348,7 @@ __global__ __launch_bounds__(256) void bucket_accumulate_kernel(
             // the four waves' totals meet in LDS; one global atomic per feature and segment
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (f4 + j < WIDE_D_MAX) red[wave][f4 + j] = acc[j];
+                if (VEC ? fl + j >= f4 : f4 + j < WIDE_D_MAX) red[wave][fl + j] = acc[j];
             if (lane == 0) red[wave][WIDE_D_MAX] = wsum;
             __syncthreads();
             for (int f = threadIdx.x; f <= d; f += 256) {
@@ -371,11 +376,10 @@ int32_t launch_wide(const LloydLayout& L, const void* X_t, const void* w, const 
     if (grid > cap) grid = cap;
     if (grid < 1) grid = 1;
     (void)L;
-    const int vec_ok = (k % 4 == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
 #define KMX_WIDE_CASE(NKC)                                                                      \
     hipLaunchKernelGGL((lloyd_mfma_wide_kernel<NKC, MODE>), dim3((unsigned)grid), dim3(256), lds, \
                        stream, (const float*)X_t, (const float*)w, (const float*)centroids_t,     \
-                       half_norms, labels_prev, labels, status, q_exp, gsum, counts, ranks, n, d, k, vec_ok)
+                       half_norms, labels_prev, labels, status, q_exp, gsum, counts, ranks, n, d, k)
     switch ((d + KC - 1) / KC) {
         case 1: KMX_WIDE_CASE(1); break;
         case 2: KMX_WIDE_CASE(2); break;
@@ -407,12 +411,11 @@ int32_t launch_wide_listed(const void* X_t, const void* X_rm, const void* w, con
     const int64_t cap = 2 * (int64_t)kmx_num_cus();
     if (grid > cap) grid = cap;
     if (grid < 1) grid = 1;
-    const int vec_ok = (k % 4 == 0) && ((((uintptr_t)centroids_t) & 15) == 0);
 #define KMX_WIDE_CASE(NKC)                                                                             \
     hipLaunchKernelGGL((lloyd_mfma_wide_kernel<NKC, MODE, true>), dim3((unsigned)grid), dim3(256),       \
                        lds, stream, (const float*)X_t, (const float*)w, (const float*)centroids_t,       \
                        half_norms, labels_prev, labels, status, q_exp, gsum, counts, ranks, n, d, k,     \
-                       vec_ok, (const float*)X_rm, list, list_count)
+                       (const float*)X_rm, list, list_count)
     switch ((d + KC - 1) / KC) {
         case 1: KMX_WIDE_CASE(1); break;
         case 2: KMX_WIDE_CASE(2); break;
@@ -477,7 +480,7 @@ int32_t kmx_lloyd_step_mfma_wide_f32(const LloydLayout& L, const void* X_t, cons
     rc = kmx_bucket_order(labels, counts, offsets, ranks, order, status, n, k, stream);
     if (rc != KMX_OK) return rc;
     const unsigned ag = (unsigned)kmx_cdiv(n, ACC_CHUNK);
-    if (d % 4 == 0 && ((((uintptr_t)X_rowmajor) & 15) == 0))
+    if (d >= 4)
         hipLaunchKernelGGL((bucket_accumulate_kernel<true>), dim3(ag), dim3(256), 0, stream,
                            (const float*)X_rowmajor, (const float*)w, order, offsets, counts, q_exp,
                            gsum, status, (int)n, d, k);

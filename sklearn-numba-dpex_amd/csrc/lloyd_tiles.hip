@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
                                                             uint4* __restrict__ xt, float* __restrict__ norm,
                                                             float* __restrict__ err, const unsigned int* __restrict__ header,
                                                             unsigned int* __restrict__ absmax, int64_t n, int d, int S,
-                                                            int64_t n_pad, int x_vec) {
+                                                            int64_t n_pad) {
     constexpr int NS = 128, NF = 32;
     constexpr int W = 16 / (int)sizeof(T);      // samples per 128-bit load
     constexpr int TPR = NS / W;                 // threads per row of 128 samples
@@ -192,25 +192,22 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
         float sq = 0.0f, e2 = 0.0f;
         for (int f0 = 0; f0 < 16 * S; f0 += NF) {
             {
-                using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
                 const int col = (threadIdx.x % TPR) * W, row0 = threadIdx.x / TPR;
                 const int64_t i = i0 + col;
                 T v[NF / RPP][W];
+                // (the same for the whole workgroup: the loads of a stage that exists whole are straight-line code)
+                const bool whole = f0 + NF <= d && i0 + NS <= n;
 #pragma unroll
                 for (int p = 0; p < NF / RPP; ++p) {
                     const int f = f0 + row0 + p * RPP;
+                    const T* __restrict__ src = X_t + (size_t)f * n + i;
+                    if (whole) {
+                        const auto q = *reinterpret_cast<const typename KmxVec<T, W>::type*>(src);
 #pragma unroll
-                    for (int e = 0; e < W; ++e) v[p][e] = T(0);
-                    if (f < d) {
-                        const T* __restrict__ src = X_t + (size_t)f * n + i;
-                        if (x_vec && i + W <= n) {
-                            const V q = *reinterpret_cast<const V*>(src);
-                            __builtin_memcpy(v[p], &q, 16);
-                        } else {
+                        for (int e = 0; e < W; ++e) v[p][e] = q[e];
+                    } else {
 #pragma unroll
-                            for (int e = 0; e < W; ++e)
-                                if (i + e < n) v[p][e] = src[e];
-                        }
+                        for (int e = 0; e < W; ++e) v[p][e] = f < d && i + e < n ? src[e] : T(0);
                     }
                 }
                 __syncthreads();  // (the previous stage's reads are over)
@@ -889,10 +886,9 @@ static void tiles_copy(const void* X_t, void* X_rowmajor, char* area, unsigned i
     if (grid > cap) grid = cap;
 #define KMX_TILES_COPY(T)                                                                                                 \
     do {                                                                                                                  \
-        const int x_vec = n % (16 / (int)sizeof(T)) == 0 && (((uintptr_t)X_t) & 15) == 0;                                 \
         hipLaunchKernelGGL((tiles_prepare_kernel<T>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t,          \
                            (T*)X_rowmajor, (uint4*)(area + a.off_xt), (float*)(area + a.off_norm),                        \
-                           (float*)(area + a.off_err), header, absmax, n, d, a.S, n_pad, x_vec);                          \
+                           (float*)(area + a.off_err), header, absmax, n, d, a.S, n_pad);                          \
     } while (0)
     if (dtype == KMX_F32) KMX_TILES_COPY(float); else KMX_TILES_COPY(double);
 #undef KMX_TILES_COPY

@@ -13,44 +13,43 @@ namespace {
 constexpr int SUM_MAX_BLOCKS_PER_ROW = 256;
 constexpr int SUM_COL_CHUNKS = 64;
 
-// VEC: rows start 16-byte aligned and hold a whole number of 16-byte groups; a thread then
-// reads 16 bytes per load and keeps two loads in flight.
-template <typename T, bool VEC>
+// A thread's part of a row's sum: 16 bytes per load, two loads in flight; the values behind the last
+// whole load go to the first threads of the first workgroup.
+template <typename T>
+__device__ __forceinline__ double sum_row_part(const T* __restrict__ p, int64_t cols, int square) {
+    constexpr int W = 16 / (int)sizeof(T);
+    using V = typename KmxVec<T, W>::type;
+    const V* __restrict__ pv = reinterpret_cast<const V*>(p);
+    const int64_t groups = cols / W;
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    double acc = 0.0;
+    auto add_one = [&](const T e) {
+        const double x = (double)e;
+        acc += square ? x * x : x;
+    };
+    auto add = [&](const V v) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) add_one(v[j]);
+    };
+    for (; g + stride < groups; g += 2 * stride) {
+        const V a = pv[g];
+        const V b = pv[g + stride];
+        add(a);
+        add(b);
+    }
+    if (g < groups) add(pv[g]);
+    if (blockIdx.x == 0 && groups * W + threadIdx.x < cols) add_one(p[groups * W + threadIdx.x]);
+    return acc;
+}
+
+template <typename T>
 __global__ __launch_bounds__(256) void sum_rows_stage1(const T* __restrict__ in,
                                                        double* __restrict__ partial, int64_t cols,
                                                        int square) {
     const int64_t row = blockIdx.y;
     const T* __restrict__ p = in + (size_t)row * cols;
-    double acc = 0.0;
-    if constexpr (VEC) {
-        constexpr int W = 16 / sizeof(T);
-        using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-        const V* __restrict__ pv = reinterpret_cast<const V*>(p);
-        const int64_t groups = cols / W;
-        const int64_t stride = (int64_t)gridDim.x * 256;
-        int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-        auto add = [&](const V& v) {
-            const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const double x = (double)e[j];
-                acc += square ? x * x : x;
-            }
-        };
-        for (; g + stride < groups; g += 2 * stride) {
-            const V a = pv[g];
-            const V b = pv[g + stride];
-            add(a);
-            add(b);
-        }
-        if (g < groups) add(pv[g]);
-    } else {
-        const int64_t stride = (int64_t)gridDim.x * 256;
-        for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < cols; c += stride) {
-            const double v = (double)p[c];
-            acc += square ? v * v : v;
-        }
-    }
+    const double acc = sum_row_part<T>(p, cols, square);
     __shared__ double scratch[4];
     const double tot = kmx_block_sum<double>(acc, scratch);
     if (threadIdx.x == 0) partial[(size_t)row * gridDim.x + blockIdx.x] = tot;
@@ -78,41 +77,12 @@ constexpr int SUM_TICKET_SLOTS = 256;
 constexpr int SUM_TICKET_ROWS = 64;
 __device__ unsigned int sum_tickets[SUM_TICKET_SLOTS][SUM_TICKET_ROWS];
 
-template <typename T, bool VEC>
+template <typename T>
 __global__ __launch_bounds__(256) void sum_rows_fused(const T* __restrict__ in, double* __restrict__ partial,
                                                       T* __restrict__ out, int64_t cols, int square, int slot) {
     const int64_t row = blockIdx.y;
     const T* __restrict__ p = in + (size_t)row * cols;
-    double acc = 0.0;
-    if constexpr (VEC) {
-        constexpr int W = 16 / sizeof(T);
-        using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-        const V* __restrict__ pv = reinterpret_cast<const V*>(p);
-        const int64_t groups = cols / W;
-        const int64_t stride = (int64_t)gridDim.x * 256;
-        int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-        auto add = [&](const V& v) {
-            const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const double x = (double)e[j];
-                acc += square ? x * x : x;
-            }
-        };
-        for (; g + stride < groups; g += 2 * stride) {
-            const V a = pv[g];
-            const V b = pv[g + stride];
-            add(a);
-            add(b);
-        }
-        if (g < groups) add(pv[g]);
-    } else {
-        const int64_t stride = (int64_t)gridDim.x * 256;
-        for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < cols; c += stride) {
-            const double v = (double)p[c];
-            acc += square ? v * v : v;
-        }
-    }
+    const double acc = sum_row_part<T>(p, cols, square);
     __shared__ double scratch[4];
     __shared__ unsigned int is_last;
     const int n_partials = (int)gridDim.x;
@@ -205,7 +175,7 @@ __global__ __launch_bounds__(256) void half_sq_norms_kernel(const T* __restrict_
     out[c] = acc / T(2);
 }
 
-template <typename T, bool VEC>
+template <typename T>
 __global__ __launch_bounds__(256) void broadcast_rows_kernel(T* __restrict__ a,
                                                              const T* __restrict__ v, int64_t rows,
                                                              int64_t cols, int op) {
@@ -213,21 +183,18 @@ __global__ __launch_bounds__(256) void broadcast_rows_kernel(T* __restrict__ a,
     const T rv = op == 0 ? -v[row] : v[row];
     T* __restrict__ p = a + (size_t)row * cols;
     const int64_t stride = (int64_t)gridDim.x * 256;
-    if constexpr (VEC) {
-        constexpr int W = 16 / sizeof(T);
-        using V = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-        V* __restrict__ pv = reinterpret_cast<V*>(p);
-        const int64_t groups = cols / W;
-        for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += stride) {
-            V x = pv[g];
-            T* e = reinterpret_cast<T*>(&x);
+    constexpr int W = 16 / (int)sizeof(T);
+    using V = typename KmxVec<T, W>::type;
+    V* __restrict__ pv = reinterpret_cast<V*>(p);
+    const int64_t groups = cols / W;
+    for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += stride) {
+        V x = pv[g];
 #pragma unroll
-            for (int j = 0; j < W; ++j) e[j] = e[j] + rv;
-            pv[g] = x;
-        }
-    } else {
-        for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < cols; c += stride) p[c] = p[c] + rv;
+        for (int j = 0; j < W; ++j) x[j] = x[j] + rv;
+        pv[g] = x;
     }
+    const int64_t c = groups * W + threadIdx.x;  // the values behind the last whole vector
+    if (blockIdx.x == 0 && c < cols) p[c] = p[c] + rv;
 }
 
 template <typename T>
@@ -535,8 +502,6 @@ int32_t kmx_sum_rows(const void* in, void* out, int64_t rows, int64_t cols, int3
     if (workspace_bytes < (size_t)rows * b * sizeof(double)) return KMX_ERR_WORKSPACE;
     hipStream_t stream = (hipStream_t)stream_;
     double* partial = (double*)workspace;
-    const size_t es = kmx_dtype_size(dtype);
-    const bool vec = (((uintptr_t)in) % 16 == 0) && ((cols * es) % 16 == 0);
     // Few workgroups (one round of them on the chip): one launch, the last workgroup of a row
     // finishes it (same sums, same order).  The hand-over costs every workgroup two round trips
     // to memory at its end, which a launch of many short workgroups pays for more dearly than
@@ -544,23 +509,19 @@ int32_t kmx_sum_rows(const void* in, void* out, int64_t rows, int64_t cols, int3
     static std::atomic<unsigned int> next_slot{0};
     const bool fused = rows <= SUM_TICKET_ROWS && rows * (int64_t)b <= 2 * (int64_t)kmx_num_cus();
     const int slot = fused ? (int)(next_slot.fetch_add(1u) % (unsigned int)SUM_TICKET_SLOTS) : 0;
-#define KMX_SUM_ROWS(T, VEC)                                                                       \
+#define KMX_SUM_ROWS(T)                                                                            \
     do {                                                                                           \
         if (fused) {                                                                               \
-            hipLaunchKernelGGL((sum_rows_fused<T, VEC>), dim3(b, (unsigned)rows), dim3(256), 0, stream, \
+            hipLaunchKernelGGL((sum_rows_fused<T>), dim3(b, (unsigned)rows), dim3(256), 0, stream, \
                                (const T*)in, partial, (T*)out, cols, square, slot);                \
         } else {                                                                                   \
-            hipLaunchKernelGGL((sum_rows_stage1<T, VEC>), dim3(b, (unsigned)rows), dim3(256), 0, stream, \
+            hipLaunchKernelGGL((sum_rows_stage1<T>), dim3(b, (unsigned)rows), dim3(256), 0, stream, \
                                (const T*)in, partial, cols, square);                               \
             hipLaunchKernelGGL((sum_rows_stage2<T>), dim3((unsigned)rows), dim3(256), 0, stream,    \
                                partial, (T*)out, b);                                               \
         }                                                                                          \
     } while (0)
-    if (dtype == KMX_F32) {
-        if (vec) KMX_SUM_ROWS(float, true); else KMX_SUM_ROWS(float, false);
-    } else {
-        if (vec) KMX_SUM_ROWS(double, true); else KMX_SUM_ROWS(double, false);
-    }
+    if (dtype == KMX_F32) KMX_SUM_ROWS(float); else KMX_SUM_ROWS(double);
 #undef KMX_SUM_ROWS
     KMX_LAUNCH_CHECK();
     return KMX_OK;
@@ -732,16 +693,10 @@ int32_t kmx_broadcast_rows(void* a, const void* v, int64_t rows, int64_t cols, i
     hipStream_t stream = (hipStream_t)stream_;
     int64_t gx = kmx_cdiv(cols, 256 * 4);
     if (gx > 2048) gx = 2048;
-    const size_t es = kmx_dtype_size(dtype);
-    const bool vec = (((uintptr_t)a) % 16 == 0) && ((cols * es) % 16 == 0);
-#define KMX_BCAST(T, VEC)                                                                       \
-    hipLaunchKernelGGL((broadcast_rows_kernel<T, VEC>), dim3((unsigned)gx, (unsigned)rows),      \
+#define KMX_BCAST(T)                                                                            \
+    hipLaunchKernelGGL((broadcast_rows_kernel<T>), dim3((unsigned)gx, (unsigned)rows),           \
                        dim3(256), 0, stream, (T*)a, (const T*)v, rows, cols, op)
-    if (dtype == KMX_F32) {
-        if (vec) KMX_BCAST(float, true); else KMX_BCAST(float, false);
-    } else {
-        if (vec) KMX_BCAST(double, true); else KMX_BCAST(double, false);
-    }
+    if (dtype == KMX_F32) KMX_BCAST(float); else KMX_BCAST(double);
 #undef KMX_BCAST
     KMX_LAUNCH_CHECK();
     return KMX_OK;
