@@ -350,7 +350,13 @@ int32_t kmx_assign_labels_inertia(const void* X_t, const void* sample_weight,
 
 /* distances_t (k, n): sqrt(sum_f (c_f - x_f)^2).  Replaces
  * make_compute_euclidean_distances_fixed_window_kernel
- * (kmeans/kernels/compute_euclidean_distances.py:15-161). */
+ * (kmeans/kernels/compute_euclidean_distances.py:15-161).
+ * _rows: X is (n, d) row-major, as a caller of KMeans.transform has it, and *not_finite (device) = 1
+ * if it holds a NaN or an infinity, else 0 (kmx_transpose_finite's check, on the way); the distances
+ * of pairs with such values are then unspecified. */
+int32_t kmx_euclidean_distances_rows(const void* X, const void* centroids_t, void* distances_t,
+                                     int32_t* not_finite, int64_t n, int32_t d, int32_t k,
+                                     int32_t dtype, void* stream);
 int32_t kmx_euclidean_distances(const void* X_t, const void* centroids_t, void* distances_t,
                                 int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream);
 

@@ -1,6 +1,7 @@
 // Per-sample inertia, euclidean distances and empty-cluster relocation for gfx950.
-// All three are HBM-bound passes over X_t: one thread per sample, features read with
-// coalesced loads (consecutive lanes = consecutive samples of one feature row).
+// Inertia and relocation are HBM-bound passes over X_t: one thread per sample, features read with
+// coalesced loads (consecutive lanes = consecutive samples of one feature row).  Distances are taken
+// from either layout of X, in fp32 on the fp64 matrix cores.
 #include "kmx_common.h"
 
 #include <type_traits>
@@ -180,14 +181,21 @@ __device__ __forceinline__ void lds_load4(const T* p, T (&v)[4]) {
 }
 
 // distances_t[c, i] = sqrt(sum_f (c_fc - x_fi)^2).  Output bound (k values written per
-// sample).  A thread keeps the features of four consecutive samples in registers (d <= DREG);
-// the workgroup's share of the centroids (blockIdx.y: `c_chunk` of them, a multiple of 4) is
-// staged in LDS, and the thread walks it four centroids at a time: one 128-bit broadcast read
-// per feature, sixteen independent sums, one 128-bit store per centroid row.
-template <typename T, int DREG>
+// sample).  A thread keeps the features of four consecutive samples in registers (d <= DREG; up to
+// DREG_EXACT features the kernel is compiled for each d); the workgroup's share of the centroids
+// (blockIdx.y: `c_chunk` of them, a multiple of 4) is staged in LDS, and the thread walks it four
+// centroids at a time: one 128-bit broadcast read per feature, sixteen independent sums, one
+// 128-bit store per centroid row.
+// ROWS (exact d): X is (n, d); the thread's samples are 4 d consecutive values, and a NaN or an infinity in
+// them sets *not_finite; else (d, n).
+template <typename T>
+constexpr int DREG_EXACT = sizeof(T) == 4 ? 16 : 8;
+template <typename T, int DREG, bool ROWS>
 __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
-    const T* __restrict__ X_t, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
-    int64_t n, int d, int k, int c_chunk) {
+    const T* __restrict__ X, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
+    int32_t* __restrict__ not_finite, int64_t n, int d_, int k, int c_chunk) {
+    static_assert(!ROWS || DREG <= DREG_EXACT<T>, "rows are split at compile time");
+    const int d = DREG <= DREG_EXACT<T> ? DREG : d_;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* cs = reinterpret_cast<T*>(smem_raw);  // [d][c_chunk]
     const int c_begin = blockIdx.y * c_chunk;
@@ -198,17 +206,31 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
     __syncthreads();
     const int64_t n_groups = (n + 3) >> 2;
     const int64_t stride = (int64_t)gridDim.x * 256;
+    bool bad = false;
     for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n_groups; g += stride) {
         const int64_t i0 = g * 4;
         const bool full = i0 + 4 <= n;
         T x[DREG][4];
+        if constexpr (ROWS) {
+            T flat[DREG][4];  // 128 bits at a time (fp64: twice)
 #pragma unroll
-        for (int f = 0; f < DREG; ++f) {
-            if (f < d) {
-                kmx_load4<T>(X_t + (size_t)f * n, i0, n, full, x[f]);
-            } else {
+            for (int q = 0; q < DREG; ++q) kmx_load4<T>(X + (size_t)i0 * DREG, 4 * q, (n - i0) * DREG, full, flat[q]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) x[f][r] = T(0);
+            for (int f = 0; f < DREG; ++f)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    x[f][r] = flat[(r * DREG + f) / 4][(r * DREG + f) % 4];
+                    bad |= kmx_not_finite(x[f][r]);
+                }
+        } else {
+#pragma unroll
+            for (int f = 0; f < DREG; ++f) {
+                if (f < d) {
+                    kmx_load4<T>(X + (size_t)f * n, i0, n, full, x[f]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[f][r] = T(0);
+                }
             }
         }
         for (int c4 = 0; c4 < c_chunk; c4 += 4) {
@@ -242,6 +264,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
             }
         }
     }
+    if (ROWS && bad) *not_finite = 1;
 }
 
 // Any d: a workgroup owns a tile of DT_S samples x DC centroids, a thread a 4 x (DC / 8) block of
@@ -304,34 +327,79 @@ __device__ __forceinline__ void dt_stage_store(T (*tile)[COLS], const T (*regs)[
     }
 }
 
-template <typename T, int DC>
+// A stage of the samples from the (n, d) array: thread t takes 16 bytes of rows t / 8 + 32 l, and puts
+// them feature by feature into the tile (rows of DT_S + 2: the eight lanes of a sample and the four
+// samples beside them fall on all banks).
+template <typename T>
+__device__ __forceinline__ void dt_rows_load(T (*regs)[16 / sizeof(T)], const T* __restrict__ X, int64_t n, int64_t i0,
+                                             int d, int f0) {
+    constexpr int V = 16 / sizeof(T), PER_ROW = DT_K / V, N = DT_S * PER_ROW / 256;
+    const bool whole = f0 + DT_K <= d && i0 + DT_S <= n;  // (the same for the whole workgroup)
+#pragma unroll
+    for (int l = 0; l < N; ++l) {
+        const int64_t i = i0 + (threadIdx.x + 256 * l) / PER_ROW;
+        const int f = f0 + V * (threadIdx.x % PER_ROW);
+        const T* __restrict__ src = X + (size_t)i * d + f;
+        if (whole) {
+            const auto v = *reinterpret_cast<const typename KmxVec<T, V>::type*>(src);
+#pragma unroll
+            for (int e = 0; e < V; ++e) regs[l][e] = v[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e) regs[l][e] = i < n && f + e < d ? src[e] : T(0);
+        }
+    }
+}
+template <typename T>
+__device__ __forceinline__ bool dt_rows_store(T (*tile)[DT_S + 2], const T (*regs)[16 / sizeof(T)]) {
+    constexpr int V = 16 / sizeof(T), PER_ROW = DT_K / V, N = DT_S * PER_ROW / 256;
+    bool bad = false;
+#pragma unroll
+    for (int l = 0; l < N; ++l)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            tile[V * (threadIdx.x % PER_ROW) + e][(threadIdx.x + 256 * l) / PER_ROW] = regs[l][e];
+            bad |= kmx_not_finite(regs[l][e]);
+        }
+    return bad;
+}
+
+// ROWS: X is (n, d), and a NaN or an infinity in it sets *not_finite; else (d, n).
+template <typename T, int DC, bool ROWS>
 __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
-    const T* __restrict__ X_t, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
-    int64_t n, int d, int k) {
+    const T* __restrict__ X, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
+    int32_t* __restrict__ not_finite, int64_t n, int d, int k) {
     constexpr int V = 16 / sizeof(T);
     constexpr int CT = DC / 8;  // centroids per thread
-    __shared__ __align__(16) T xs[DT_K][DT_S];
+    constexpr int XP = ROWS ? DT_S + 2 : DT_S;
+    __shared__ __align__(16) T xs[DT_K][XP];
     __shared__ __align__(16) T cs[DT_K][DC];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const int64_t i0 = (int64_t)blockIdx.x * DT_S;
     const int c0 = blockIdx.y * DC;
     T rx[dt_vectors<T, DT_S>()][V], rc[dt_vectors<T, DC>()][V];
+    bool bad = false;
     T acc[CT][4];
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[c][i] = T(0);
 
-    dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, 0);
+    auto load_x = [&](const int f0) __attribute__((always_inline)) {
+        if constexpr (ROWS) dt_rows_load<T>(rx, X, n, i0, d, f0);
+        else dt_stage_load<T, DT_S>(rx, X, n, i0, d, f0);
+    };
+    load_x(0);
     dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, 0);
     const int n_stages = (d + DT_K - 1) / DT_K;
     for (int st = 0; st < n_stages; ++st) {
         __syncthreads();  // the previous stage's reads are over
-        dt_stage_store<T, DT_S>(xs, rx);
+        if constexpr (ROWS) bad |= dt_rows_store<T>(xs, rx);
+        else dt_stage_store<T, DT_S>(xs, rx);
         dt_stage_store<T, DC>(cs, rc);
         __syncthreads();
         if (st + 1 < n_stages) {
-            dt_stage_load<T, DT_S>(rx, X_t, n, i0, d, (st + 1) * DT_K);
+            load_x((st + 1) * DT_K);
             dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, (st + 1) * DT_K);
         }
         // (rows past d hold zeros on both sides: their differences add nothing)
@@ -351,6 +419,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
                 }
         }
     }
+    if (ROWS && bad) *not_finite = 1;
     const int64_t i = i0 + 4 * tx;
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
@@ -362,6 +431,319 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
         for (int e = 0; e < 4; ++e) v[e] = dist_sqrt(acc[c][e]);
         kmx_store4<T>(dst - i, i, n, i + 4 <= n, v);
     }
+}
+
+// ---------------------------------------------------------------------------- fp32 distances
+//
+// |x - c|^2 = |x - m|^2 + |c - m|^2 - 2 <x - m, c - m> with every term in fp64 (m: centroid 0, as far as DM_M
+// features; x and c are fp32, so the differences and products carry 53 bits), the inner products on the fp64 matrix cores.
+// Where the result is less than about d 2^-27 of what it is the difference of, rounding would show in
+// fp32: those few pairs are redone in the difference form, feature by feature in fp32, as are pairs that
+// involve values beyond 2^62, NaN or infinities.  What is left is one rounding to fp32 and the square root:
+// nearer the exact distance than d rounded additions.
+// Why: the difference form costs two vector instructions per pair and feature (98 us for 300 007 x 100 x 64
+// at the chip's rate without packed arithmetic), the fp64 matrix cores take 49 us for the same.  And the
+// rows of X are read where they are: a transposed copy of X for this one pass over it took 59 us there.
+// A workgroup keeps 16 NCT centroids and walks tiles of 128 samples, DM_K features at a time through LDS (the
+// operands of up to DM_K features stay there); the next stage's loads are in flight during the arithmetic.
+// A wave: two tiles of 16 samples (lane j: samples 2 j and 2 j + 1, so that results leave in pairs).
+// ROWS: X is (n, d), and a stage is kept sample by sample (DM_RP: sixteen lanes and four features on 64
+// banks); else (d, n) and feature by feature (DM_CP).
+// Nothing of the vector work hides behind these matrix instructions, so the end of a tile counts: square
+// root from one reciprocal root, one test of a lane's 32 results instead of one each, norms from LDS.
+// Bound by the matrix cores (42 TFLOP/s) and, with few features, by the end of a tile.  Kernel times, us, the
+// transposed copy and the differences it replaces / this: 300 007 x 100, 64 clusters 178 / 116; 1e5 x 784,
+// 300 clusters 1 340 / 1 065; 1e6 x 20, 16 clusters 90 / 60.  Reading the next step's operands ahead of the
+// matrix instructions: 292 -> 321 us at 1e6 x 96, 64 clusters (registers), not done.
+constexpr int DM_S = 128, DM_K = 32, DM_RP = DM_K + 2, DM_CP = DM_S + 32, DM_M = 1024;
+typedef double dm_v4d __attribute__((ext_vector_type(4)));
+
+template <int NCT, bool ROWS>
+__global__ __launch_bounds__(256, 3) void distances_f32_kernel(
+    const float* __restrict__ X, const float* __restrict__ centroids_t, float* __restrict__ distances_t,
+    int32_t* __restrict__ not_finite, int64_t n, int d, int k, int c_tiles, int slots) {
+    constexpr int PX = DM_S * DM_K / 256;            // values of X per thread and stage
+    constexpr int PC = NCT * 64 * (DM_K / 4) / 256;  // centroid values per thread and stage
+    __shared__ __align__(16) float xs[ROWS ? DM_S * DM_RP : DM_K * DM_CP];
+    __shared__ double cf[DM_K / 4][NCT][64];  // operand fragments
+    __shared__ double ms[DM_M + DM_K];        // m
+    __shared__ double cn[4][16 * NCT];        // |c - m|^2: the waves' parts, then the sums in row 0
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int g = lane >> 4, j = lane & 15;
+    // workgroup b: die b % 8, centroid tile (b / 8) % c_tiles, and of the die's sample tiles every slots-th:
+    // the workgroups that read the same samples run on one die, next to each other in time
+    const int c0 = (int)(blockIdx.x / 8 % c_tiles) * 16 * NCT;
+    const int64_t s_step = (int64_t)slots * 8, n_tiles = (n + DM_S - 1) / DM_S;
+    int64_t tile = (int64_t)(blockIdx.x / 8 / c_tiles) * 8 + blockIdx.x % 8;
+    if (tile >= n_tiles) return;
+
+    float rx[PX], rc[PC];
+    bool bad = false;
+    auto load = [&](const int64_t i0, const int f0, const bool centroids) __attribute__((always_inline)) {
+        const int here = n - i0 < DM_S ? (int)(n - i0) : DM_S;  // samples of the tile that exist
+        const int w = d - f0 < DM_K ? d - f0 : DM_K;            // features of the stage
+        const bool whole = w == DM_K && here == DM_S;
+        if constexpr (ROWS) {
+            if (whole) {
+#pragma unroll
+                for (int p = 0; p < PX / 4; ++p) {
+                    const int s = (threadIdx.x >> 3) + 32 * p, q = threadIdx.x & 7;
+                    const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(X + (size_t)(i0 + s) * d + f0 + 4 * q);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rx[4 * p + e] = v[e];
+                }
+            } else {
+                // the values one after the other (of up to DM_K features: whole cache lines); past the end
+                // the last sample's, dropped when they are stored
+                const int step_s = 256 / w, step_f = 256 - step_s * w;
+                int s = (int)threadIdx.x / w, f = (int)threadIdx.x - s * w;
+                asm volatile("" : "+v"(s), "+v"(f));  // (recomputed per stage instead of a register per value)
+                const float* __restrict__ from = X + (size_t)i0 * d + f0;
+#pragma unroll
+                for (int p = 0; p < PX; ++p) {
+                    if (256 * p < DM_S * w) rx[p] = from[(size_t)(s < here ? s : here - 1) * d + f];  // (uniform)
+                    s += step_s;
+                    f += step_f;
+                    if (f >= w) {
+                        f -= w;
+                        ++s;
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < PX / 4; ++p) {
+                const int f = (threadIdx.x >> 5) + 8 * p, s = 4 * (threadIdx.x & 31);
+                if (whole) {
+                    const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(X + (size_t)(f0 + f) * n + i0 + s);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rx[4 * p + e] = v[e];
+                } else {
+                    const float* __restrict__ row = X + (size_t)(f < w ? f0 + f : d - 1) * n + i0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rx[4 * p + e] = row[s + e < here ? s + e : here - 1];
+                }
+            }
+        }
+        // fragment value (step, tile, lane): feature f0 + 4 step + lane / 16 of centroid c0 + 16 tile + lane % 16
+        // (a thread's values are all of one centroid)
+        if (centroids) {
+            int c = c0 + 16 * (wave % NCT) + j;
+            asm volatile("" : "+v"(c));
+#pragma unroll
+            for (int p = 0; p < PC; ++p) {
+                const int f = f0 + 4 * ((wave + 4 * p) / NCT) + g;
+                rc[p] = centroids_t[(size_t)(f < d ? f : d - 1) * k + (c < k ? c : k - 1)];
+            }
+        }
+    };
+    double my_nc = 0.0;
+    auto store = [&](const int64_t i0, const int f0, const bool centroids, const bool first) __attribute__((always_inline)) {
+        const int here = n - i0 < DM_S ? (int)(n - i0) : DM_S;
+        const int w = d - f0 < DM_K ? d - f0 : DM_K;
+        if (ROWS && !(w == DM_K && here == DM_S)) {
+            const int step_s = 256 / w, step_f = 256 - step_s * w;
+            int s = (int)threadIdx.x / w, f = (int)threadIdx.x - s * w;
+            asm volatile("" : "+v"(s), "+v"(f));
+#pragma unroll
+            for (int p = 0; p < PX; ++p) {
+                if (256 * p < DM_S * w && s < DM_S) {
+                    xs[s * DM_RP + f] = rx[p];
+                    bad |= kmx_not_finite(rx[p]);
+                }
+                s += step_s;
+                f += step_f;
+                if (f >= w) {
+                    f -= w;
+                    ++s;
+                }
+            }
+            // (features up to the next step of four: zero, as the fragments are)
+            const int fill = -w & 3;
+            for (int u = threadIdx.x; u < DM_S * fill; u += 256) xs[u / fill * DM_RP + w + u % fill] = 0.0f;
+        } else if constexpr (ROWS) {
+#pragma unroll
+            for (int p = 0; p < PX / 4; ++p) {
+                const int s = (threadIdx.x >> 3) + 32 * p, q = threadIdx.x & 7;
+                float2* at = reinterpret_cast<float2*>(xs + s * DM_RP + 4 * q);
+                at[0] = make_float2(rx[4 * p], rx[4 * p + 1]);
+                at[1] = make_float2(rx[4 * p + 2], rx[4 * p + 3]);
+            }
+#pragma unroll
+            for (int p = 0; p < PX; ++p) bad |= kmx_not_finite(rx[p]);
+        } else {
+#pragma unroll
+            for (int p = 0; p < PX / 4; ++p) {
+                const int f = (threadIdx.x >> 5) + 8 * p;
+                float4 v = make_float4(rx[4 * p], rx[4 * p + 1], rx[4 * p + 2], rx[4 * p + 3]);
+                if (f >= w) v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                *reinterpret_cast<float4*>(xs + f * DM_CP + 4 * (threadIdx.x & 31)) = v;
+            }
+        }
+        if (centroids) {
+            int c = c0 + 16 * (wave % NCT) + j;
+            asm volatile("" : "+v"(c));
+            const double* m_at = ms + (f0 < DM_M ? f0 : DM_M) + g;
+#pragma unroll
+            for (int p = 0; p < PC; ++p) {
+                const int st = (wave + 4 * p) / NCT, f = 4 * st + g;
+                double v = (double)rc[p] - m_at[4 * st];
+                v = f < w && c < k ? v : 0.0;
+                cf[st][wave % NCT][lane] = v;
+                if (first) my_nc = fma(v, v, my_nc);
+            }
+        }
+    };
+
+    const bool resident = d <= DM_K;  // the operands of all features stay in LDS
+    bool first = true;
+    load(tile * DM_S, 0, true);
+    // (zero for the features past d, and for the stages past DM_M)
+    for (int f = threadIdx.x; f < DM_M + DM_K; f += 256)
+        if (f < (d + DM_K - 1) / DM_K * DM_K || f >= DM_M) ms[f] = f < d && f < DM_M ? (double)centroids_t[(size_t)f * k] : 0.0;
+    for (; tile < n_tiles; tile += s_step) {
+        const int64_t i0 = tile * DM_S, i_next = (tile + s_step) * DM_S;
+        dm_v4d acc[NCT][2];
+        double nx[2] = {0.0, 0.0};
+#pragma unroll
+        for (int a = 0; a < NCT; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = dm_v4d{0.0, 0.0, 0.0, 0.0};
+        for (int f0 = 0; f0 < d; f0 += DM_K) {
+            const bool last_stage = f0 + DM_K >= d;
+            __syncthreads();  // the previous stage's reads are over
+            store(i0, f0, first || !resident, first);
+            if (first && last_stage) {
+                // (the threads of a centroid: four lanes of the waves that hold its tile)
+                double v = my_nc;
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                if (g == 0) cn[wave / NCT][16 * (wave % NCT) + j] = v;
+            }
+            __syncthreads();
+            if (!last_stage || tile + s_step < n_tiles)
+                load(last_stage ? i_next : i0, last_stage ? 0 : f0 + DM_K, !resident);
+            const int steps = (d - f0 < DM_K ? d - f0 + 3 : DM_K) / 4;
+            const double* m_here = ms + (f0 < DM_M ? f0 : DM_M) + g;
+#pragma unroll 1
+            for (int st = 0; st < steps; ++st) {
+                const double m = m_here[4 * st];
+                double xb[2];
+                if constexpr (ROWS) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) xb[b] = (double)xs[(32 * wave + 2 * j + b) * DM_RP + 4 * st + g] - m;
+                } else {
+                    const float2 v = *reinterpret_cast<const float2*>(xs + (4 * st + g) * DM_CP + 32 * wave + 2 * j);
+                    xb[0] = (double)v.x - m;
+                    xb[1] = (double)v.y - m;
+                }
+#pragma unroll
+                for (int b = 0; b < 2; ++b) nx[b] = fma(xb[b], xb[b], nx[b]);
+#pragma unroll
+                for (int a = 0; a < NCT; ++a) {
+                    const double av = cf[st][a][lane];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, xb[b], acc[a][b], 0, 0, 0);
+                }
+            }
+        }
+        if (first && NCT < 4) {
+            if (threadIdx.x < 16 * NCT) {
+                double v = 0.0;
+#pragma unroll
+                for (int q = 0; q < 4 / NCT; ++q) v += cn[q][threadIdx.x];
+                cn[0][threadIdx.x] = v;
+            }
+            __syncthreads();
+        }
+        first = false;
+
+        // the four lanes that share a sample
+#pragma unroll
+        for (int off = 16; off <= 32; off <<= 1)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) nx[b] += __shfl_xor(nx[b], off, 64);
+        // accumulator r of lane (g, j): centroid 16 a + g + 4 r, samples 2 j + b of the wave
+        const int here = n - i0 < DM_S ? (int)(n - i0) : DM_S;
+        const int sl = 32 * wave + 2 * j;
+        // a result's high word less that of what it is the difference of: how many binades it lost (20 bits
+        // each); its least over the lane's results, the largest norm and the least result decide at once
+        int least = 0x7fffffff, most = max(__double2hiint(nx[0]), __double2hiint(nx[1]));
+        float low = kmx_inf<float>();
+        auto finish = [&](auto whole_tag) __attribute__((always_inline)) {
+            constexpr bool whole = decltype(whole_tag)::value;
+            float* __restrict__ dst = distances_t + (size_t)(c0 + g) * n + i0 + sl;
+            int c = c0 + g;
+#pragma unroll
+            for (int a = 0; a < NCT; ++a) {
+                __builtin_amdgcn_sched_barrier(0);  // (four norms at a time in registers)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const double c2 = cn[0][16 * a + g + 4 * r];
+                    most = max(most, __double2hiint(c2));
+                    float v[2];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const double of = nx[b] + c2, sq = fma(-2.0, acc[a][b][r], of);
+                        least = min(least, __double2hiint(sq) - __double2hiint(of));
+                        const float q = (float)sq;
+                        low = fminf(low, q);
+                        // root by one reciprocal root and a Newton step on the residual
+                        const float y = __builtin_amdgcn_rsqf(q), t = q * y;
+                        v[b] = fmaf(fmaf(-t, t, q), 0.5f * y, t);
+                    }
+                    // (the running extremes now, not as a tree over 32 results kept to the end)
+                    asm volatile("" : "+v"(least), "+v"(most), "+v"(low));
+                    if (c < k && (whole || sl + 1 < here))
+                        *reinterpret_cast<KmxVec<float, 2>::type*>(dst) = KmxVec<float, 2>::type{v[0], v[1]};
+                    else if (!whole && c < k && sl < here)
+                        dst[0] = v[0];
+                    dst += 4 * n;
+                    c += 4;
+                }
+            }
+        };
+        if (here == DM_S) finish(std::true_type{});  // (uniform)
+        else finish(std::false_type{});
+        // d 2^-27, in binades; 2^126: no square beyond it overflows; 1e-30: roots and their residuals are normal
+        const int lost = (26 - (31 - __builtin_clz(d))) << 20;
+        if (__any(least + lost <= 0 || most >= 0x47d00000 || !(low >= 1e-30f))) {
+            unsigned int redo = 0u;
+            asm volatile("" : "+v"(nx[0]), "+v"(nx[1]) : : "memory");  // (computed again, not kept in registers since above)
+#pragma unroll
+            for (int a = 0; a < NCT; ++a) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const double c2 = cn[0][16 * a + g + 4 * r];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const double of = nx[b] + c2, sq = fma(-2.0, acc[a][b][r], of);
+                        if (!(__double2hiint(sq) - __double2hiint(of) + lost > 0 && of < 0x1p126 && (float)sq >= 1e-30f))
+                            redo |= 1u << (8 * a + 2 * r + b);
+                    }
+                }
+            }
+            while (redo != 0u) {
+                const int u = __builtin_ctz(redo);
+                redo &= redo - 1u;
+                const int c = c0 + 16 * (u >> 3) + g + 4 * ((u >> 1) & 3), si = sl + (u & 1);
+                if (c >= k || si >= here) continue;
+                float* __restrict__ dst = distances_t + (size_t)c * n + i0 + si;
+                const float* __restrict__ x = ROWS ? X + (size_t)(i0 + si) * d : X + i0 + si;
+                const size_t step = ROWS ? 1 : (size_t)n;
+                float sum = 0.0f;
+#pragma unroll 4
+                for (int f = 0; f < d; ++f) {
+                    const float diff = centroids_t[(size_t)f * k + c] - x[f * step];
+                    sum = fmaf(diff, diff, sum);
+                }
+                *dst = dist_sqrt(sum);
+            }
+        }
+    }
+    if (ROWS && bad) *not_finite = 1;
 }
 
 // One workgroup per relocated cluster, threads over features.  Several relocations may take
@@ -414,6 +796,82 @@ int32_t kmx_inertia_total_launch(const double* partial, int count, void* out, in
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
+
+namespace {
+__global__ void clear_word_kernel(int32_t* word) {
+    if (threadIdx.x == 0) *word = 0;
+}
+
+// The register kernel for d features: DREG = 16 (any d up to it) or DREG = d.  Its centroid range is split over
+// blockIdx.y until there are about six workgroups per compute unit (a thread's walk over the centroids
+// is one dependent chain).
+template <typename T, int DREG, bool ROWS>
+int32_t launch_distances_reg(const void* X, const void* centroids_t, void* distances_t, int32_t* not_finite, int64_t n,
+                             int d, int k, hipStream_t stream) {
+    if constexpr (DREG <= DREG_EXACT<T> && DREG > 1) {
+        if (d < DREG)
+            return launch_distances_reg<T, DREG - 1, ROWS>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
+    }
+    const int64_t wgx = stream_grid(kmx_cdiv(n, 4));
+    int64_t gy = kmx_cdiv((int64_t)kmx_num_cus() * 6, wgx);
+    if (gy > kmx_cdiv(k, 16)) gy = kmx_cdiv(k, 16);
+    if (gy < 1) gy = 1;
+    int c_chunk = (int)(4 * kmx_cdiv(kmx_cdiv(k, gy), 4));
+    const int most = (int)(64 * 1024 / (d * sizeof(T))) & ~3;  // (the share within 64 KB of LDS)
+    if (c_chunk > most) c_chunk = most;
+    gy = kmx_cdiv(k, c_chunk);
+    if (gy > 65535) return KMX_ERR_BAD_SHAPE;
+    hipLaunchKernelGGL((euclidean_distances_reg_kernel<T, DREG, ROWS>), dim3((unsigned)wgx, (unsigned)gy), dim3(256),
+                       (size_t)d * c_chunk * sizeof(T), stream, (const T*)X, (const T*)centroids_t, (T*)distances_t,
+                       not_finite, n, d, k, c_chunk);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
+template <bool ROWS>
+int32_t launch_distances_f32(const void* X, const void* centroids_t, void* distances_t, int32_t* not_finite, int64_t n,
+                             int d, int k, hipStream_t stream) {
+    // few features: the differences are fewer instructions than what the end of a tile takes on the matrix cores
+    // (transform of 1e6 x d by k clusters, us, matrix cores / registers: d 3 k 5 87 / 57, d 8 k 64 127 / 112,
+    // d 9 k 64 133 / 113, d 9 k 5 94 / 64, and the copy and differences both took 79, 136, 142, 87 before)
+    if (d <= DREG_EXACT<float>)
+        return launch_distances_reg<float, DREG_EXACT<float>, ROWS>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
+    const int nct = k <= 16 ? 1 : k <= 32 ? 2 : 4;
+    const int64_t c_tiles = kmx_cdiv(k, 16 * nct), groups = kmx_cdiv(kmx_cdiv(n, DM_S), 8);
+    // as many workgroups as run at once, each on one centroid tile
+    int64_t slots = (int64_t)3 * kmx_num_cus() / (8 * c_tiles);
+    if (slots < 1) slots = 1;
+    if (slots > groups) slots = groups;
+    if (c_tiles * slots > INT32_MAX / 8) return KMX_ERR_BAD_SHAPE;
+#define KMX_DIST_F32(NCT)                                                                                         \
+    hipLaunchKernelGGL((distances_f32_kernel<NCT, ROWS>), dim3((unsigned)(8 * c_tiles * slots)), dim3(256), 0,    \
+                       stream, (const float*)X, (const float*)centroids_t, (float*)distances_t, not_finite, n, d, \
+                       k, (int)c_tiles, (int)slots)
+    if (nct == 1) KMX_DIST_F32(1); else if (nct == 2) KMX_DIST_F32(2); else KMX_DIST_F32(4);
+#undef KMX_DIST_F32
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
+template <bool ROWS>
+int32_t launch_distances_f64(const void* X, const void* centroids_t, void* distances_t, int32_t* not_finite, int64_t n,
+                             int d, int k, hipStream_t stream) {
+    if (d <= DREG_EXACT<double>)
+        return launch_distances_reg<double, DREG_EXACT<double>, ROWS>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
+    if constexpr (!ROWS) {
+        if (d <= 16) return launch_distances_reg<double, 16, ROWS>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
+    }
+    const int dc = k <= 2 * DT_C_FEW ? DT_C_FEW : DT_C;
+    const dim3 grid((unsigned)kmx_cdiv(n, DT_S), (unsigned)kmx_cdiv(k, dc));
+#define KMX_DIST_TILED(DC)                                                                                          \
+    hipLaunchKernelGGL((euclidean_distances_tiled_kernel<double, DC, ROWS>), grid, dim3(256), 0, stream,            \
+                       (const double*)X, (const double*)centroids_t, (double*)distances_t, not_finite, n, d, k)
+    if (dc == DT_C_FEW) KMX_DIST_TILED(DT_C_FEW); else KMX_DIST_TILED(DT_C);
+#undef KMX_DIST_TILED
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+}  // namespace
 
 extern "C" {
 
@@ -541,42 +999,23 @@ int32_t kmx_euclidean_distances(const void* X_t, const void* centroids_t, void* 
     if (n <= 0 || d <= 0 || k <= 0) return KMX_ERR_BAD_SHAPE;
     KMX_REQUIRE_DTYPE(dtype);
     hipStream_t stream = (hipStream_t)stream_;
-    // register kernel: the centroid range is split over blockIdx.y until there are about six
-    // workgroups per compute unit (a thread's walk over the centroids is one dependent chain)
-    const int64_t wgx = stream_grid(kmx_cdiv(n, 4));
-    int64_t gy = kmx_cdiv((int64_t)kmx_num_cus() * 6, wgx);
-    if (gy > kmx_cdiv(k, 16)) gy = kmx_cdiv(k, 16);
-    if (gy < 1) gy = 1;
-    const int c_chunk = (int)(4 * kmx_cdiv(kmx_cdiv(k, gy), 4));
-    gy = kmx_cdiv(k, c_chunk);
-    const size_t es = kmx_dtype_size(dtype);
-    const size_t lds = (size_t)d * c_chunk * es;
-    const dim3 rgrid((unsigned)wgx, (unsigned)gy);
-    if (dtype == KMX_F32 && d <= 32 && lds <= 64 * 1024) {
-        if (d <= 16)
-            hipLaunchKernelGGL((euclidean_distances_reg_kernel<float, 16>), rgrid, dim3(256), lds, stream,
-                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, c_chunk);
-        else
-            hipLaunchKernelGGL((euclidean_distances_reg_kernel<float, 32>), rgrid, dim3(256), lds, stream,
-                               (const float*)X_t, (const float*)centroids_t, (float*)distances_t, n, d, k, c_chunk);
-    } else if (dtype == KMX_F64 && d <= 16 && lds <= 64 * 1024) {
-        hipLaunchKernelGGL((euclidean_distances_reg_kernel<double, 16>), rgrid, dim3(256), lds, stream,
-                           (const double*)X_t, (const double*)centroids_t, (double*)distances_t, n, d, k, c_chunk);
-    } else {
-        const int dc = k <= 2 * DT_C_FEW ? DT_C_FEW : DT_C;
-        const dim3 tgrid((unsigned)kmx_cdiv(n, DT_S), (unsigned)kmx_cdiv(k, dc));
-#define KMX_DIST_TILED(T, DC)                                                                          \
-    hipLaunchKernelGGL((euclidean_distances_tiled_kernel<T, DC>), tgrid, dim3(256), 0, stream,         \
-                       (const T*)X_t, (const T*)centroids_t, (T*)distances_t, n, d, k)
-        if (dtype == KMX_F32) {
-            if (dc == DT_C_FEW) KMX_DIST_TILED(float, DT_C_FEW); else KMX_DIST_TILED(float, DT_C);
-        } else {
-            if (dc == DT_C_FEW) KMX_DIST_TILED(double, DT_C_FEW); else KMX_DIST_TILED(double, DT_C);
-        }
-#undef KMX_DIST_TILED
-    }
-    KMX_LAUNCH_CHECK();
-    return KMX_OK;
+    return dtype == KMX_F32 ? launch_distances_f32<false>(X_t, centroids_t, distances_t, nullptr, n, d, k, stream)
+                            : launch_distances_f64<false>(X_t, centroids_t, distances_t, nullptr, n, d, k, stream);
+}
+
+int32_t kmx_euclidean_distances_rows(const void* X, const void* centroids_t, void* distances_t, int32_t* not_finite,
+                                     int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream_) {
+    KMX_ENTRY();
+    KMX_REQUIRE_PTR(X);
+    KMX_REQUIRE_PTR(centroids_t);
+    KMX_REQUIRE_PTR(distances_t);
+    KMX_REQUIRE_PTR(not_finite);
+    if (n <= 0 || d <= 0 || k <= 0) return KMX_ERR_BAD_SHAPE;
+    KMX_REQUIRE_DTYPE(dtype);
+    hipStream_t stream = (hipStream_t)stream_;
+    hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(64), 0, stream, not_finite);
+    return dtype == KMX_F32 ? launch_distances_f32<true>(X, centroids_t, distances_t, not_finite, n, d, k, stream)
+                            : launch_distances_f64<true>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
 }
 
 int32_t kmx_relocate_empty_clusters(const void* X_t, const void* sample_weight,

@@ -104,6 +104,12 @@ __device__ __forceinline__ float kmx_inf<float>() { return __builtin_huge_valf()
 template <>
 __device__ __forceinline__ double kmx_inf<double>() { return __builtin_huge_val(); }
 
+// Whether a value is a NaN or an infinity: all bits of the exponent set.
+__device__ __forceinline__ bool kmx_not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+__device__ __forceinline__ bool kmx_not_finite(double v) {
+    return ((unsigned)(__double_as_longlong(v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
+}
+
 // Sum over the 64 lanes of a wave; every lane receives the total.
 template <typename T>
 __device__ __forceinline__ T kmx_wave_sum(T v) {

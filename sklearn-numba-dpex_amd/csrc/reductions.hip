@@ -335,13 +335,6 @@ int sum_blocks_per_row(int64_t cols) {
     return (int)(b < 1 ? 1 : b);
 }
 
-
-// Whether a value is a NaN or an infinity: all bits of the exponent set.
-__device__ __forceinline__ bool kmx_not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
-__device__ __forceinline__ bool kmx_not_finite(double v) {
-    return ((unsigned)(__double_as_longlong(v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
-}
-
 // The elements of a transposed tile that fit its LDS (33 KB: four workgroups' tiles and their
 // loads are in flight on a compute unit).
 template <typename T>

@@ -347,6 +347,20 @@ def get_euclidean_distances(X_t, Y_t):
     return distances_t.T
 
 
+def get_euclidean_distances_rows(X, Y_t, not_finite):
+    """`get_euclidean_distances` from the (n_samples, n_features) C-contiguous array that a caller of
+    `KMeans.transform` has.  `not_finite`, an int32 tensor of one element, is set to whether X holds a NaN
+    or an infinity."""
+    require_cuda()
+    Y_t = contiguous(Y_t)
+    n, d = X.shape
+    k = Y_t.shape[1]
+    distances_t = torch.empty((k, n), dtype=X.dtype, device=X.device)
+    check(lib.kmx_euclidean_distances_rows(ptr(X), ptr(Y_t), ptr(distances_t), ptr(not_finite), n, d, k, dcode(X),
+                                           _capi.current_stream()), "kmx_euclidean_distances_rows")
+    return distances_t.T
+
+
 def kpp_uniforms(n_clusters, n_local_trials, random_state, dtype):
     """Starting raw draw and the table U[c - 1, t] of the uniform that trial t draws when
     centre c is picked (state t serves trial t; state 0 first serves the raw draw that picks

@@ -40,6 +40,7 @@ from ..common._buffers import require_cuda, upload
 from ..common.kernels import all_finite, transposed_copy
 from .drivers import (
     get_euclidean_distances,
+    get_euclidean_distances_rows,
     get_labels_inertia,
     get_nb_distinct_clusters,
     is_same_clustering,
@@ -218,9 +219,24 @@ class KMeansEngine(_EngineBase):
         return X
 
     def get_euclidean_distances(self, X):
-        X = self._validate_data(X, reset=False)
-        cluster_centers = self._check_init(self.estimator.cluster_centers_, X, copy=False)
-        euclidean_distances = get_euclidean_distances(X.T, cluster_centers)
+        X_dev, X_host, owns_copy = self._to_device(X)
+        if X_dev.is_contiguous() and not X_dev.T.is_contiguous() and (
+            X_dev.shape[1] == getattr(self.estimator, "n_features_in_", X_dev.shape[1])
+        ):
+            # one pass over the rows where they are, which looks for non-finite values on the way
+            not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
+            try:
+                cluster_centers = self._check_init(self.estimator.cluster_centers_, X_dev, copy=False)
+            except Exception:
+                all_finite(X_dev, not_finite)  # (what is wrong with X is reported first)
+                self._assert_all_finite(not_finite, X_dev.T, X_host)
+                raise
+            euclidean_distances = get_euclidean_distances_rows(X_dev, cluster_centers, not_finite)
+            self._assert_all_finite(not_finite, X_dev.T, X_host)
+        else:
+            X = self._feature_major(X_dev, X_host, owns_copy, reset=False)
+            cluster_centers = self._check_init(self.estimator.cluster_centers_, X, copy=False)
+            euclidean_distances = get_euclidean_distances(X.T, cluster_centers)
         if self._is_in_testing_mode:
             euclidean_distances = _to_numpy(euclidean_distances).astype(
                 getattr(self.estimator, "_output_dtype", np.float64)
@@ -249,11 +265,11 @@ class KMeansEngine(_EngineBase):
         host = X_host if X_host is not None else X_t.T.cpu().numpy()
         _assert_all_finite(host, input_name="X", estimator_name=type(self.estimator).__name__)
 
-    def _validate_data(self, X, reset=True):
-        """Returns X on the device as the transposed view of a contiguous (d, n) buffer, dtype
-        float64 or float32 (other dtypes are converted to float64, as scikit-learn does)."""
+    def _to_device(self, X):
+        """(n_samples, n_features) device tensor of X as float64 or float32 (other dtypes are converted to
+        float64, as scikit-learn does), the host array it came from or None, and whether the tensor is this
+        engine's own.  Values are not looked at yet."""
         require_cuda()
-        estimator = self.estimator
         if sp.issparse(X):
             raise NotSupportedByEngineError("A sparse matrix was passed, but dense data is required.")
 
@@ -269,42 +285,42 @@ class KMeansEngine(_EngineBase):
                 raise ValueError(f"Found array with shape {tuple(X.shape)}: at least one sample and "
                                  "one feature are required.")
             out_dtype = X.dtype if X.dtype in _TORCH_FLOAT else torch.float64
-            n_features = X.shape[1]
             X_dev = X.to(device=self.device, dtype=out_dtype)
-            # (d, n) contiguous; already the case for an F-ordered tensor
-            X_t = X_dev.T
-            owns_copy = X_dev.data_ptr() != X.data_ptr()
-            not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
-            if X_dev.is_contiguous() and not X_t.is_contiguous():
-                X_t = transposed_copy(X_dev, not_finite)
-                owns_copy = True
-            else:
-                owns_copy = owns_copy or not X_t.is_contiguous()
-                X_t = X_t.contiguous()
-                all_finite(X_t, not_finite)
-            self._assert_all_finite(not_finite, X_t, None)
+            return X_dev, None, X_dev.data_ptr() != X.data_ptr()
+
+        X_np = check_array(
+            X,
+            accept_sparse=False,
+            dtype=list(_ACCEPTED_DTYPES),
+            order=None,
+            copy=False,
+            ensure_all_finite=False,  # checked on the device: the host pass costs more than the upload
+            estimator=self.estimator,
+            input_name="X",
+        )
+        # (through pinned staging buffers when the array is large; the upload is this engine's own copy)
+        if X_np.flags.f_contiguous:
+            return upload(np.ascontiguousarray(X_np.T), self.device).T, X_np, True
+        return upload(X_np, self.device), X_np, True
+
+    def _validate_data(self, X, reset=True):
+        """Returns X on the device as the transposed view of a contiguous (d, n) buffer."""
+        return self._feature_major(*self._to_device(X), reset)
+
+    def _feature_major(self, X_dev, X_host, owns_copy, reset):
+        estimator = self.estimator
+        n_features = X_dev.shape[1]
+        # (d, n) contiguous; already the case for an F-ordered array
+        X_t = X_dev.T
+        not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
+        if X_dev.is_contiguous() and not X_t.is_contiguous():
+            X_t = transposed_copy(X_dev, not_finite)
+            owns_copy = True
         else:
-            owns_copy = True  # the upload below is this engine's own device copy
-            X_np = check_array(
-                X,
-                accept_sparse=False,
-                dtype=list(_ACCEPTED_DTYPES),
-                order=None,
-                copy=False,
-                ensure_all_finite=False,  # checked on the device below: the host pass costs more than the upload
-                estimator=estimator,
-                input_name="X",
-            )
-            n_features = X_np.shape[1]
-            # upload, then transpose on the device: (d, n) contiguous
-            # (through pinned staging buffers when the array is large)
-            X_t = upload(np.ascontiguousarray(X_np.T) if X_np.flags.f_contiguous else X_np, self.device)
-            not_finite = torch.empty(1, dtype=torch.int32, device=X_t.device)
-            if X_np.flags.f_contiguous:
-                all_finite(X_t, not_finite)
-            else:
-                X_t = transposed_copy(X_t, not_finite)
-            self._assert_all_finite(not_finite, X_t, X_np)
+            owns_copy = owns_copy or not X_t.is_contiguous()
+            X_t = X_t.contiguous()
+            all_finite(X_t, not_finite)
+        self._assert_all_finite(not_finite, X_t, X_host)
 
         # prepare_fit centres the data in place when this buffer is not the caller's (or copy_x is off)
         self._owns_X = owns_copy

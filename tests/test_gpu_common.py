@@ -364,6 +364,66 @@ def test_distances_and_inertia_kernels(cuda, shape):
     np.testing.assert_allclose(total_unit[0], per_sample.sum(), rtol=rtol)
 
 
+# both layouts of X, at the edges of sample tiles (128), feature stages (32; 1 024 of the shift), centroid tiles
+# (16, 32, 64) and the kernels kept per number of features
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,k", [(1, 1, 1), (5, 1, 5), (130, 2, 17), (1023, 5, 600), (257, 7, 9), (127, 8, 64), (128, 9, 16),
+                                   (129, 15, 33), (1025, 16, 130), (4097, 16, 2100), (2049, 17, 1), (127, 31, 15),
+                                   (128, 32, 16), (1153, 33, 32), (640, 36, 65), (129, 64, 64), (300, 100, 129),
+                                   (200, 1023, 3), (131, 1056, 20), (70, 1500, 66)])
+def test_distances_from_either_layout(cuda, n, d, k, dtype):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + 7 * d + k)
+    C = rng.uniform(-4, 4, (k, d)).astype(dtype)
+    X = (C[rng.integers(0, k, n)] + rng.standard_normal((n, d))).astype(dtype)
+    X[n // 2] = C[k // 2]  # distance exactly 0
+    exact = np.sqrt(((X.astype(np.float64)[:, None, :] - C.astype(np.float64)[None, :, :]) ** 2).sum(axis=2))
+    # d additions of non-negative terms, each rounded, and the root
+    rtol = (d / 2 + 3) * np.finfo(dtype).eps if dtype == np.float64 or d <= 16 else 1.5 * np.finfo(dtype).eps
+    not_finite = torch.empty(1, dtype=torch.int32, device=cuda)
+    rows = drivers.get_euclidean_distances_rows(_dev(X, cuda), _dev(C.T, cuda), not_finite)
+    assert int(not_finite) == 0
+    for got in (rows, drivers.get_euclidean_distances(_dev(X.T, cuda), _dev(C.T, cuda))):
+        got = got.cpu().numpy()
+        assert got.shape == (n, k) and got.dtype == dtype
+        np.testing.assert_allclose(got, exact, rtol=rtol)
+        assert (got[exact == 0] == 0).all()
+    for i, f, value in ((0, 0, np.nan), (n - 1, d - 1, np.inf), (n // 2, d // 2, -np.inf)):
+        bad = X.copy()
+        bad[i, f] = value
+        drivers.get_euclidean_distances_rows(_dev(bad, cuda), _dev(C.T, cuda), not_finite)
+        assert int(not_finite) == 1
+
+
+# pairs that the inner products cannot settle: next to a centroid, far from the origin, tiny, and squares beyond
+# fp32 (infinite in the difference form too)
+@pytest.mark.parametrize("case", ["near", "offset", "tiny", "huge", "one far centroid"])
+def test_fp32_distances_of_close_and_extreme_pairs(cuda, case):
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(17)
+    n, d, k = 700, 40, 70
+    C = rng.uniform(-4, 4, (k, d))
+    X = C[rng.integers(0, k, n)] + rng.standard_normal((n, d))
+    if case == "near":
+        X = C[rng.integers(0, k, n)] * (1 + 1e-6 * rng.standard_normal((n, d)))
+    elif case == "offset":
+        C, X = C + 1e6, X + 1e6
+    elif case == "tiny":
+        C, X = C * 1e-17, X * 1e-17
+    elif case == "huge":
+        C, X = C * 1e17, X * 1e17
+    else:
+        C[5] = 1e8
+    C, X = C.astype(np.float32), X.astype(np.float32)
+    exact = np.sqrt(((X.astype(np.float64)[:, None, :] - C.astype(np.float64)[None, :, :]) ** 2).sum(axis=2))
+    got = drivers.get_euclidean_distances(_dev(X.T, cuda), _dev(C.T, cuda)).cpu().numpy()
+    np.testing.assert_allclose(got, exact, rtol=(d / 2 + 3) * 1.2e-7)  # (redone pairs: d rounded additions)
+
+
 def test_distances_with_few_samples_split_the_centroids(cuda):
     """With few samples the centroid range is split over the second grid dimension (ragged last
     share, k not a multiple of 4), and exact zeros / tiny distances go through the square root."""
