@@ -43,10 +43,11 @@ struct KppHeader {
 };
 
 struct KppLayout {
-    size_t off_header, off_cand, off_pot, off_cand_rows, off_block_pot, off_rows, total;
+    size_t off_header, off_cand, off_pot, off_cand_rows, off_block_pot, off_rows, off_rows2, total;
     int64_t n_blocks;
     int chunk;  // samples per block sum: CHUNK, or 64 * split
     int split;  // 0, or the samples per thread (1, 2, 4) of the feature-split step kernel
+    int joint;  // 0, or the samples per thread (1, 2, 4) of the kernel that selects, samples and steps at once
 };
 
 // Samples per thread of the feature-split step kernel, 0 when the shape keeps the plain one.
@@ -60,6 +61,23 @@ int kpp_split(int64_t n, int d, int n_trials, int dtype) {
     const int most = (dtype == KMX_F32 ? 4 : 2) / (n_trials > 8 ? 2 : 1);
     const int spt = n <= 65536 ? 1 : n <= 131072 ? 2 : n <= 262144 ? 4 : 8;
     return spt <= most ? spt : 0;
+}
+
+// Samples per thread of kpp_joint_kernel, 0 when a centre takes two launches: every workgroup repeats the
+// selection and the search for the candidates, which pays while there are at most JOINT_BLOCKS block sums
+// to look through and the candidates' rows are short.  Beyond one sample per thread a step is the time to
+// read X once it has more than JOINT_BYTES, and one workgroup per compute unit does not hide that.  Whole
+// seedings, us, two launches a centre / one: fp32 20 000 x 50, 200 centres 5 981 / 3 198; 80 223 x 9, 85 1 766 /
+// 1 162; 131 072 x 40 (21 MB), 50 1 068 / 892; 260 000 x 10, 100 2 008 / 1 640; 262 144 x 63 (66 MB), 30 946 / 1 137;
+// fp64 1 500 x 20, 8 252 / 212; 65 536 x 63, 100 3 065 / 1 958; 100 000 x 30 (24 MB), 20 516 / 503; 131 072 x 63
+// (66 MB), 30 1 010 / 1 061.
+constexpr int JOINT_BLOCKS = 256, JOINT_TN = 8, JOINT_D = 64;
+constexpr int64_t JOINT_BYTES = 24 << 20;
+int kpp_joint(int64_t n, int d, int n_trials, int dtype) {
+    if (d >= JOINT_D || n_trials > JOINT_TN || n > 4 * 256 * JOINT_BLOCKS) return 0;
+    if (n <= 256 * JOINT_BLOCKS) return 1;
+    if (n * d * (int64_t)kmx_dtype_size(dtype) > JOINT_BYTES) return 0;
+    return n <= 2 * 256 * JOINT_BLOCKS ? 2 : 4;
 }
 
 // The layout, the block sums included, depends on the shape only: calls with either sampler
@@ -76,6 +94,11 @@ KppLayout kpp_layout(int64_t n, int d, int n_trials, int dtype) {
     L.off_block_pot = L.off_cand_rows + kmx_align256((size_t)TN_MAX * d * kmx_dtype_size(dtype));
     L.off_rows = L.off_block_pot + kmx_align256((size_t)L.n_blocks * TN_MAX * sizeof(double));
     L.total = L.off_rows + kmx_align256((size_t)n_trials * n * kmx_dtype_size(dtype));
+    // (its steps read the rows of the one before while they write their own; two sets of block sums)
+    L.joint = kpp_joint(n, d, n_trials, dtype);
+    L.off_rows2 = L.total;
+    if (L.joint)
+        L.total += kmx_align256((size_t)n_trials * n * kmx_dtype_size(dtype)) + 2 * JOINT_TN * JOINT_BLOCKS * sizeof(double);
     return L;
 }
 
@@ -863,6 +886,268 @@ __global__ __launch_bounds__(256) void kpp_select_sample_kernel(
     for (int f = threadIdx.x; f < d; f += 256) cand_rows[(size_t)trial * d + f] = X_t[(size_t)f * n + cand];
 }
 
+// ---------------------------------------------------------------- one launch per centre
+//
+// Few samples: the two launches of a centre are chains of trips to memory on an idle chip, 8 us for the
+// selection and 12 for the step at 80 000 x 9.  Here every workgroup finds the winner of the last step and
+// this step's candidates by itself - the block sums (one per thread), the waves' share of the candidates'
+// blocks, their rows - while its own samples are on their way, and then steps.  What a workgroup looks up, all
+// others look up too, from L2.  The rows read are those of the step before, the rows written another set: no
+// workgroup waits for another.  Distances and roundings are those of the plain step; sums of sums are taken in
+// another order, in fp64.
+// INIT: the first distances, closest = w * ||x - x_start||^2, into row 0.
+
+// Sums over the wave of eight values at once: lane l returns the total of value l >> 3 (in its bits 5, 4, 3).
+__device__ __forceinline__ double wave_sum_of_eight(const double (&v)[8], int lane) {
+    double a[4], b[2], c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = (lane & 32 ? v[i + 4] : v[i]) + __shfl_xor(lane & 32 ? v[i] : v[i + 4], 32, 64);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) b[i] = (lane & 16 ? a[i + 2] : a[i]) + __shfl_xor(lane & 16 ? a[i] : a[i + 2], 16, 64);
+    c = (lane & 8 ? b[1] : b[0]) + __shfl_xor(lane & 8 ? b[0] : b[1], 8, 64);
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    return c;
+}
+
+__device__ __forceinline__ double wave_inclusive_scan(double v, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(v, off, 64);
+        if (lane >= off) v += o;
+    }
+    return v;
+}
+
+template <typename T, int SPT, bool INIT>
+__global__ __launch_bounds__(256) void kpp_joint_kernel(
+    const T* __restrict__ X_t, const T* __restrict__ sample_weight, const double* __restrict__ uniforms,
+    const int32_t* __restrict__ cand_prev, int32_t* __restrict__ cand_next, const T* __restrict__ rows_in,
+    T* __restrict__ rows_out, const double* __restrict__ pot_in, double* __restrict__ pot_out,
+    T* __restrict__ centers_t, int32_t* __restrict__ center_indices, double* __restrict__ potentials,
+    KppHeader* __restrict__ header, int64_t n, int d, int k, int n_trials, int center_slot, int32_t start) {
+    constexpr int TN = INIT ? 1 : JOINT_TN, CH = 256 * SPT;
+    constexpr int FB = 16 / SPT < 8 ? 8 : 16 / SPT;  // features of a batch
+    constexpr int V = 16 / (int)sizeof(T);
+    __shared__ double wave_pot[4][8], wave_tot[4], excl_s[256];
+    __shared__ int first_s[4][JOINT_TN], cand_s[JOINT_TN];
+    __shared__ __align__(16) T row_s[TN][JOINT_D];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int n_blocks = (int)gridDim.x;
+    const int64_t base = (int64_t)blockIdx.x * CH, i0 = base + threadIdx.x * SPT;
+    const bool full = base + CH <= n;  // (the same for the whole workgroup)
+
+    auto load_own = [&](const T* __restrict__ row, T(&v)[SPT]) __attribute__((always_inline)) {
+        if (SPT > 1 && full) {
+            if constexpr (SPT == 4) {
+                kmx_load4<T>(row, i0, n, true, v);
+            } else if constexpr (SPT == 2) {
+                const auto q = *reinterpret_cast<const typename KmxVec<T, 2>::type*>(row + i0);
+                v[0] = q[0]; v[1] = q[1];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < SPT; ++r) v[r] = row[i0 + r < n ? i0 + r : n - 1];
+        }
+    };
+    T xv[FB][SPT], w[SPT], cl[SPT];
+    auto load_batch = [&](const int f0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < FB; ++j) load_own(X_t + (size_t)(f0 + j < d ? f0 + j : d - 1) * n, xv[j]);
+    };
+    load_batch(0);
+    load_own(sample_weight, w);
+
+    if constexpr (INIT) {
+        if ((int)threadIdx.x < d) row_s[0][threadIdx.x] = X_t[(size_t)threadIdx.x * n + start];
+        __syncthreads();
+    } else {
+        // ---- the winner of the last step (slot 0: the starting sample is in row 0)
+        const int b = threadIdx.x, n_rows = center_slot > 0 ? n_trials : 1;
+        double own[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const double v = pot_in[(size_t)(t < n_rows ? t : 0) * n_blocks + (b < n_blocks ? b : 0)];
+            own[t] = b < n_blocks && t < n_rows ? v : 0.0;
+        }
+        const double part = wave_sum_of_eight(own, lane);
+        if ((lane & 7) == 0) wave_pot[wave][lane >> 3] = part;
+        __syncthreads();
+        int best = 0;
+        double best_pot = (wave_pot[0][0] + wave_pot[1][0]) + (wave_pot[2][0] + wave_pot[3][0]);
+        for (int t = 1; t < n_rows; ++t) {
+            const double pt = (wave_pot[0][t] + wave_pot[1][t]) + (wave_pot[2][t] + wave_pot[3][t]);
+            if (pt < best_pot) {
+                best_pot = pt;
+                best = t;
+            }
+        }
+        best = __builtin_amdgcn_readfirstlane(best);
+        const T* __restrict__ closest = rows_in + (size_t)best * n;
+        load_own(closest, cl);
+        if (blockIdx.x == 0 && center_slot > 0) {
+            const int32_t chosen = cand_prev[best];
+            if ((int)threadIdx.x < d) centers_t[(size_t)threadIdx.x * k + center_slot] = X_t[(size_t)threadIdx.x * n + chosen];
+            if ((int)threadIdx.x < n_trials)
+                potentials[threadIdx.x] = (wave_pot[0][threadIdx.x] + wave_pot[1][threadIdx.x]) +
+                                          (wave_pot[2][threadIdx.x] + wave_pot[3][threadIdx.x]);
+            if (threadIdx.x == 0) {
+                center_indices[center_slot] = chosen;
+                header->best_row = best;
+                header->total = best_pot;
+            }
+        }
+        // ---- the block of every candidate: the first whose inclusive sum reaches u * total
+        double mine = own[0];
+#pragma unroll
+        for (int t = 1; t < 8; ++t) mine = t == best ? own[t] : mine;
+        const double incl = wave_inclusive_scan(mine, lane);
+        if (lane == 63) wave_tot[wave] = incl;
+        __syncthreads();
+        double before = 0.0, total = 0.0;
+#pragma unroll
+        for (int w2 = 0; w2 < 4; ++w2) {
+            if (w2 == wave) before = total;
+            total += wave_tot[w2];
+        }
+        const double excl = before + incl - mine, cum = excl + mine;
+        excl_s[threadIdx.x] = excl;
+#pragma unroll
+        for (int t = 0; t < JOINT_TN; ++t) {
+            const double rv = uniforms[t < n_trials ? t : 0] * total;
+            const unsigned long long at = __ballot(b < n_blocks && cum >= rv);
+            if (lane == 0) first_s[wave][t] = at != 0ull ? 64 * wave + __builtin_ctzll(at) : n_blocks;
+        }
+        __syncthreads();
+        // ---- the sample in that block, trials wave and wave + 4
+        constexpr int PER = CH / 64;  // values per lane
+        T fv[2][PER];
+        int block[2];
+        double prefix[2], rv[2];
+        int64_t j0[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int t = wave + 4 * q < n_trials ? wave + 4 * q : 0;
+            const int at = min(min(first_s[0][t], first_s[1][t]), min(first_s[2][t], first_s[3][t]));
+            // (rounding: u * total above every inclusive sum)
+            block[q] = at < n_blocks ? at : n_blocks - 1;
+            prefix[q] = at < n_blocks ? excl_s[block[q]] : total;
+            rv[q] = uniforms[t] * total;
+            j0[q] = (int64_t)block[q] * CH + lane * PER;
+            if ((int64_t)(block[q] + 1) * CH <= n) {
+#pragma unroll
+                for (int r = 0; r < PER; r += 4) {
+                    T four[4];
+                    kmx_load4<T>(closest, j0[q] + r, n, true, four);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) fv[q][r + e] = four[e];
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < PER; ++r) fv[q][r] = j0[q] + r < n ? closest[j0[q] + r] : T(0);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            double s = 0.0;
+#pragma unroll
+            for (int r = 0; r < PER; ++r) s += (double)fv[q][r];
+            double c2 = prefix[q] + (wave_inclusive_scan(s, lane) - s);
+            int hit = -1;
+#pragma unroll
+            for (int r = 0; r < PER; ++r) {
+                c2 += (double)fv[q][r];
+                if (hit < 0 && j0[q] + r < n && c2 >= rv[q]) hit = (int)j0[q] + r;
+            }
+            const unsigned long long at = __ballot(hit >= 0);
+            // (rounding pushed the crossing just past the block)
+            int64_t cand = (int64_t)(block[q] + 1) * CH;
+            if (at != 0ull) cand = __builtin_amdgcn_readlane(hit, __builtin_ctzll(at));
+            if (cand > n - 1) cand = n - 1;
+            if (lane == 0) cand_s[wave + 4 * q] = (int)cand;
+        }
+        __syncthreads();
+        {
+            const int t = threadIdx.x >> 5, f = threadIdx.x & 31, c = cand_s[t];  // (past n_trials: trial 0's block, not used)
+            const T v0 = X_t[(size_t)(f < d ? f : d - 1) * n + c], v1 = X_t[(size_t)(f + 32 < d ? f + 32 : d - 1) * n + c];
+            row_s[t][f] = v0;
+            row_s[t][f + 32] = v1;
+            if (blockIdx.x == 0 && f == 0 && t < n_trials) cand_next[t] = c;
+        }
+        __syncthreads();
+    }
+
+    // ---- the step: features in order, as in kpp_step_kernel
+    T acc[TN][SPT];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int r = 0; r < SPT; ++r) acc[t][r] = T(0);
+    for (int f0 = 0; f0 < d; f0 += FB) {
+        auto accumulate = [&](auto whole_tag) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                if (t < n_trials) {
+#pragma unroll
+                    for (int j = 0; j < FB; j += V) {
+                        struct alignas(16) Piece { T e[V]; };
+                        const Piece cv = *reinterpret_cast<const Piece*>(&row_s[t][f0 + j]);  // (a broadcast)
+#pragma unroll
+                        for (int e = 0; e < V; ++e)
+                            if (decltype(whole_tag)::value || f0 + j + e < d) {
+#pragma unroll
+                                for (int r = 0; r < SPT; ++r) {
+                                    const T diff = xv[j + e][r] - cv.e[e];
+                                    acc[t][r] = kpp_sq_acc<true>(diff, acc[t][r]);
+                                }
+                            }
+                    }
+                }
+            }
+        };
+        if (f0 + FB <= d) accumulate(std::true_type{});
+        else accumulate(std::false_type{});
+        if (f0 + FB < d) load_batch(f0 + FB);
+    }
+    double pot[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        pot[t] = 0.0;
+        if (t < TN && t < n_trials) {
+            T v[SPT];
+#pragma unroll
+            for (int r = 0; r < SPT; ++r) {
+                v[r] = acc[t < TN ? t : 0][r] * w[r];
+                if constexpr (!INIT) v[r] = fmin(v[r], cl[r]);
+                if (full || i0 + r < n) pot[t] += (double)v[r];
+            }
+            T* __restrict__ to = rows_out + (size_t)t * n;
+            if constexpr (SPT == 4) {
+                kmx_store4<T>(to, i0, n, full, v);
+            } else {
+#pragma unroll
+                for (int r = 0; r < SPT; ++r)
+                    if (full || i0 + r < n) to[i0 + r] = v[r];
+            }
+        }
+    }
+    const double part = wave_sum_of_eight(pot, lane);
+    __syncthreads();  // (wave_pot has been read)
+    if ((lane & 7) == 0) wave_pot[wave][lane >> 3] = part;
+    __syncthreads();
+    if ((int)threadIdx.x < n_trials)
+        pot_out[(size_t)threadIdx.x * n_blocks + blockIdx.x] = (wave_pot[0][threadIdx.x] + wave_pot[1][threadIdx.x]) +
+                                                               (wave_pot[2][threadIdx.x] + wave_pot[3][threadIdx.x]);
+    if (INIT && blockIdx.x == 0) {
+        if ((int)threadIdx.x < d) centers_t[(size_t)threadIdx.x * k] = row_s[0][threadIdx.x];
+        if (threadIdx.x == 0) {
+            center_indices[0] = start;
+            header->best_row = 0;
+            header->total = 0.0;
+        }
+    }
+}
+
 // The reference's sampler taken literally (kmeans/kernels/kmeans_plusplus.py:79-100): a
 // running sum of `closest` in T, element by element from sample 0, and per trial the first j
 // whose running sum reaches rv_t = T(u_t) * T(total), clipped to n - 1.  A floating-point
@@ -1148,6 +1433,51 @@ void launch_select_sample(const void* X_t, const double* uniforms, const int32_t
 #undef KMX_KPP_SELECT
 }
 
+// A whole seeding with one launch per centre (L.joint).
+template <typename T>
+int32_t run_joint(const void* X_t, const void* w, const double* uniforms, int32_t start, void* centers_t, int32_t* idx,
+                  char* ws, const KppPtrs& p, const KppLayout& L, int64_t n, int d, int k, int n_trials, hipStream_t s) {
+    const int n_blocks = (int)kmx_cdiv(n, 256 * L.joint);
+    // step k - 1 writes the rows that kmx_kpp_closest_ptr names
+    T* rows[2];
+    rows[(k - 1) & 1] = (T*)p.rows;
+    rows[k & 1] = (T*)(ws + L.off_rows2);
+    double* pot = (double*)(ws + L.off_rows2 + kmx_align256((size_t)n_trials * n * sizeof(T)));
+    double* pots[2] = {pot, pot + JOINT_TN * JOINT_BLOCKS};
+#define KMX_KPP_JOINT(SPT, INIT, U, CP, CN, RI, RO, PI, PO, TRIALS, SLOT)                                                \
+    hipLaunchKernelGGL((kpp_joint_kernel<T, SPT, INIT>), dim3((unsigned)n_blocks), dim3(256), 0, s, (const T*)X_t,      \
+                       (const T*)w, U, CP, CN, RI, RO, PI, PO, (T*)centers_t, idx, p.potentials, p.header, n, d, k,     \
+                       TRIALS, SLOT, start)
+#define KMX_KPP_JOINT_SPT(...)                                              \
+    do {                                                                    \
+        if (L.joint == 1) KMX_KPP_JOINT(1, __VA_ARGS__);                    \
+        else if (L.joint == 2) KMX_KPP_JOINT(2, __VA_ARGS__);               \
+        else KMX_KPP_JOINT(4, __VA_ARGS__);                                 \
+    } while (0)
+    KMX_KPP_JOINT_SPT(true, (const double*)nullptr, (const int32_t*)nullptr, (int32_t*)nullptr, (const T*)nullptr, rows[0],
+                      (const double*)nullptr, pots[0], 1, 0);
+    KMX_LAUNCH_CHECK();
+    for (int c = 1; c < k; ++c) {
+        const double* u = uniforms + (size_t)(c - 1) * n_trials;
+        KMX_KPP_JOINT_SPT(false, u, p.cand + ((c - 1) & 1) * TN_MAX, p.cand + (c & 1) * TN_MAX, (const T*)rows[(c - 1) & 1],
+                          rows[c & 1], pots[(c - 1) & 1], pots[c & 1], n_trials, c - 1);
+        KMX_LAUNCH_CHECK();
+    }
+#undef KMX_KPP_JOINT_SPT
+#undef KMX_KPP_JOINT
+    if (k > 1) {
+        KppPtrs last = p;
+        last.block_pot = pots[(k - 1) & 1];
+        KppLayout geometry = L;
+        geometry.n_blocks = n_blocks;
+        geometry.chunk = 256 * L.joint;
+        launch_select_sample<T>(X_t, nullptr, p.cand + ((k - 1) & 1) * TN_MAX, nullptr, nullptr, centers_t, idx, last,
+                                geometry, n, d, k, n_trials, k - 1, 1, 0, s);
+        KMX_LAUNCH_CHECK();
+    }
+    return KMX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1246,14 +1576,27 @@ int32_t kmx_kpp_run(const void* X_t, const void* sample_weight, const double* un
     KMX_ENTRY();
     if (flags & ~(uint32_t)KMX_KPP_SAMPLER_LITERAL) return KMX_ERR_BAD_ARGUMENT;
     const bool literal = (flags & KMX_KPP_SAMPLER_LITERAL) != 0;
-    int32_t rc = kmx_kpp_init(X_t, sample_weight, start_index, centers_t, center_indices, workspace,
-                              workspace_bytes, n, d, k, n_trials, dtype, flags, stream_);
+    int32_t rc = kpp_check(X_t, sample_weight, workspace, workspace_bytes, n, d, k, n_trials, dtype);
     if (rc != KMX_OK) return rc;
-    if (k == 1) return KMX_OK;
-    KMX_REQUIRE_PTR(uniforms);
     const KppLayout L = kpp_layout(n, d, n_trials, dtype);
     const KppPtrs p = kpp_ptrs((char*)workspace, L);
     hipStream_t s = (hipStream_t)stream_;
+    if (L.joint && !literal && k > 1) {
+        KMX_REQUIRE_PTR(centers_t);
+        KMX_REQUIRE_PTR(center_indices);
+        KMX_REQUIRE_PTR(uniforms);
+        if (start_index < 0 || start_index >= n) return KMX_ERR_BAD_ARGUMENT;
+        return dtype == KMX_F32
+                   ? run_joint<float>(X_t, sample_weight, uniforms, start_index, centers_t, center_indices,
+                                      (char*)workspace, p, L, n, d, k, n_trials, s)
+                   : run_joint<double>(X_t, sample_weight, uniforms, start_index, centers_t, center_indices,
+                                       (char*)workspace, p, L, n, d, k, n_trials, s);
+    }
+    rc = kmx_kpp_init(X_t, sample_weight, start_index, centers_t, center_indices, workspace, workspace_bytes, n, d, k,
+                      n_trials, dtype, flags, stream_);
+    if (rc != KMX_OK) return rc;
+    if (k == 1) return KMX_OK;
+    KMX_REQUIRE_PTR(uniforms);
     const size_t extra = literal ? 0 : screen_bytes(L, n, d, k, n_trials, dtype);
     const bool screened = extra != 0 && workspace_bytes >= L.total + extra && ((uintptr_t)workspace & 15) == 0;
     void* X_rm = nullptr;

@@ -87,6 +87,38 @@ def test_seeding_at_the_limits_of_the_feature_split_step(cuda, n, d, dtype, samp
     np.testing.assert_array_equal(centers_t.cpu().numpy().T, X[ref_idx])
 
 
+# one launch per centre: samples per thread change at 65 536 and 131 072, it ends at 262 144, 63 features, 8 trials
+# (k 402) and 24 MB; fewer samples than a workgroup has threads, ragged last blocks
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,k", [(1, 3, 1), (2, 1, 2), (255, 33, 3), (256, 32, 8), (257, 63, 20), (513, 31, 402), (600, 5, 404),
+                                   (65_536, 2, 5), (65_537, 3, 5), (131_072, 24, 4), (131_073, 1, 6), (131_073, 23, 4),
+                                   (262_144, 4, 5), (262_145, 4, 5), (100_001, 31, 4)])
+def test_seeding_with_one_launch_per_centre(cuda, n, d, k, dtype):
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n + d + k)
+    X = rng.normal(size=(n, d)).astype(dtype)
+    w = rng.uniform(0.1, 3.0, n).astype(dtype)
+    centers_t, idx = drivers.kmeans_plusplus(_dev(X.T, cuda), _dev(w, cuda), k, 5)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ok.kmeans_plusplus(X, w, k, 5)[1])
+    np.testing.assert_array_equal(centers_t.cpu().numpy().T, X[idx.cpu().numpy()])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_seeding_of_equal_samples_and_zero_weights(cuda, dtype):
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    same = np.full((700, 3), 1.5, dtype=dtype)
+    w = np.ones(700, dtype=dtype)
+    _, idx = drivers.kmeans_plusplus(_dev(same.T, cuda), _dev(w, cuda), 4, 5)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ok.kmeans_plusplus(same, w, 4, 5)[1])
+    X = np.random.default_rng(3).normal(size=(700, 3)).astype(dtype)
+    w[50:] = 0  # only the first samples can be picked
+    _, idx = drivers.kmeans_plusplus(_dev(X.T, cuda), _dev(w, cuda), 4, 5)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ok.kmeans_plusplus(X, w, 4, 5)[1])
+    assert (idx.cpu().numpy()[1:] < 50).all()
+
+
 @pytest.mark.parametrize("shape", [(10_007, 6, 4), (66_001, 64, 12), (3_001, 70, 10), (140_000, 65, 3)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_step_kernels_through_c_abi(cuda, dtype, shape):
