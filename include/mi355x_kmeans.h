@@ -458,6 +458,15 @@ int32_t* kmx_kpp_candidates_ptr(void* workspace, int64_t n, int32_t d, int32_t k
 
 size_t kmx_sum_workspace_bytes(int64_t rows, int64_t cols);
 
+/* What a fit asks of its data, in one chain of launches and one array to read back
+ * (prepare_data_for_lloyd, kmeans/drivers.py:436-545): mean (rows) = the row means of X_t (rows, cols);
+ * dst = X_t - mean, which may be X_t itself; stats (4 values of the data type) = sum of mean^2, sum of
+ * the squares of dst, sum of sample_weight (cols), its first value.  All means zero: dst = X_t. */
+size_t kmx_center_workspace_bytes(int64_t rows, int64_t cols);
+int32_t kmx_center_rows(const void* X_t, void* dst, const void* sample_weight, void* mean, void* stats,
+                        void* workspace, size_t workspace_bytes, int64_t rows, int64_t cols,
+                        int32_t dtype, void* stream);
+
 /* out[r] = sum_c f(in[r, c]) with f = identity or square (first pass only).  Replaces
  * make_sum_reduction_2d_kernel with axis=1 and the 1-D form (common/reductions.py:214-460,
  * 643-890).  Accumulates in fp64, fixed order: results are reproducible run to run. */

@@ -9,7 +9,8 @@ from .. import _capi
 
 
 def require_cuda():
-    if not torch.cuda.is_available():
+    # (an initialised runtime has its GPU: is_available() reads the environment each time)
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError("sklearn_numba_dpex_amd needs a ROCm GPU (torch.cuda.is_available() is False)")
 
 

@@ -197,6 +197,77 @@ __global__ __launch_bounds__(256) void broadcast_rows_kernel(T* __restrict__ a,
     if (blockIdx.x == 0 && c < cols) p[c] = p[c] + rv;
 }
 
+// mean[r] = sums[r] / n in T (in place), stats[0] = sum of mean^2 (fp64, rounded to T).
+template <typename T>
+__global__ __launch_bounds__(256) void center_mean_kernel(T* __restrict__ mean, T* __restrict__ stats, int64_t rows, T n) {
+    __shared__ double scratch[4];
+    double acc = 0.0;
+    for (int64_t r = threadIdx.x; r < rows; r += 256) {
+        const T m = mean[r] / n;
+        mean[r] = m;
+        acc += (double)m * (double)m;
+    }
+    const double tot = kmx_block_sum<double>(acc, scratch);
+    if (threadIdx.x == 0) stats[0] = (T)tot;
+}
+
+// dst = src - mean per row (dst may be src; left as it is where stats[0] is zero and dst is src) and the
+// workgroups' sums of the new values' squares: a pass over X less than centring first and summing then.
+template <typename T>
+__global__ __launch_bounds__(256) void center_rows_kernel(const T* src, T* dst, const T* __restrict__ mean,
+                                                          const T* __restrict__ stats, double* __restrict__ partial,
+                                                          int64_t cols) {
+    const int64_t row = blockIdx.y;
+    const bool any = stats[0] != T(0);  // (NaN: yes)
+    const T rv = any ? -mean[row] : T(0);
+    const T* p = src + (size_t)row * cols;
+    T* q = dst + (size_t)row * cols;
+    const bool write = any || src != dst;
+    constexpr int W = 16 / (int)sizeof(T);
+    using V = typename KmxVec<T, W>::type;
+    const int64_t groups = cols / W, stride = (int64_t)gridDim.x * 256;
+    double acc = 0.0;
+    auto group = [&](const int64_t g, V x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            if (any) x[j] = x[j] + rv;
+            acc += (double)x[j] * (double)x[j];
+        }
+        if (write) *reinterpret_cast<V*>(q + g * W) = x;
+    };
+    int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (; g + stride < groups; g += 2 * stride) {  // two loads in flight
+        const V a = *reinterpret_cast<const V*>(p + g * W), b = *reinterpret_cast<const V*>(p + (g + stride) * W);
+        group(g, a);
+        group(g + stride, b);
+    }
+    if (g < groups) group(g, *reinterpret_cast<const V*>(p + g * W));
+    const int64_t c = groups * W + threadIdx.x;  // the values behind the last whole vector
+    if (blockIdx.x == 0 && c < cols) {
+        const T x = any ? p[c] + rv : p[c];
+        acc += (double)x * (double)x;
+        if (write) q[c] = x;
+    }
+    __shared__ double scratch[4];
+    const double tot = kmx_block_sum<double>(acc, scratch);
+    if (threadIdx.x == 0) partial[(size_t)row * gridDim.x + blockIdx.x] = tot;
+}
+
+// stats[1] = the total of the partial sums, stats[3] = the first weight.
+template <typename T>
+__global__ __launch_bounds__(1024) void center_total_kernel(const double* __restrict__ partial, int64_t count,
+                                                            const T* __restrict__ w, T* __restrict__ stats) {
+    __shared__ double scratch[16];
+    double acc = 0.0;
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < count; i += 1024) acc += partial[i];
+    const double tot = kmx_block_sum<double>(acc, scratch);
+    if (threadIdx.x == 0) {
+        stats[1] = (T)tot;
+        stats[3] = w[0];
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void broadcast_div_cols_kernel(T* __restrict__ a,
                                                                  const T* __restrict__ v,
@@ -327,6 +398,13 @@ int grid_for(int64_t n) {
     const int64_t cap = (int64_t)kmx_num_cus() * 8;
     if (blocks > cap) blocks = cap;
     return (int)(blocks < 1 ? 1 : blocks);
+}
+
+// Workgroups per row of the centring pass: 16 KB of a row each, 16 384 in all where that is more.
+int64_t center_blocks_per_row(int64_t rows, int64_t cols) {
+    int64_t b = kmx_cdiv(cols, 256 * 16);
+    if (b * rows > 16384) b = kmx_cdiv(16384, rows);
+    return b < 1 ? 1 : b;
 }
 
 int sum_blocks_per_row(int64_t cols) {
@@ -671,6 +749,48 @@ int32_t kmx_all_finite(const void* data, int64_t n_items, int32_t* not_finite, i
         if (vec) KMX_FINITE(double, true); else KMX_FINITE(double, false);
     }
 #undef KMX_FINITE
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
+size_t kmx_center_workspace_bytes(int64_t rows, int64_t cols) {
+    if (rows <= 0 || cols <= 0) return 0;
+    const size_t a = kmx_sum_workspace_bytes(rows, cols);
+    const size_t b = kmx_align256((size_t)rows * center_blocks_per_row(rows, cols) * sizeof(double));
+    return a > b ? a : b;
+}
+
+int32_t kmx_center_rows(const void* X_t, void* dst, const void* sample_weight, void* mean, void* stats, void* workspace,
+                        size_t workspace_bytes, int64_t rows, int64_t cols, int32_t dtype, void* stream_) {
+    KMX_ENTRY();
+    KMX_REQUIRE_PTR(X_t);
+    KMX_REQUIRE_PTR(dst);
+    KMX_REQUIRE_PTR(sample_weight);
+    KMX_REQUIRE_PTR(mean);
+    KMX_REQUIRE_PTR(stats);
+    KMX_REQUIRE_PTR(workspace);
+    if (rows <= 0 || cols <= 0 || rows > 65535) return KMX_ERR_BAD_SHAPE;
+    KMX_REQUIRE_DTYPE(dtype);
+    if (workspace_bytes < kmx_center_workspace_bytes(rows, cols)) return KMX_ERR_WORKSPACE;
+    hipStream_t stream = (hipStream_t)stream_;
+    // (one workspace: the launches follow one another on the stream)
+    int32_t rc = kmx_sum_rows(sample_weight, (char*)stats + 2 * kmx_dtype_size(dtype), 1, cols, 0, workspace,
+                              workspace_bytes, dtype, stream_);
+    if (rc != KMX_OK) return rc;
+    rc = kmx_sum_rows(X_t, mean, rows, cols, 0, workspace, workspace_bytes, dtype, stream_);
+    if (rc != KMX_OK) return rc;
+    const int64_t b = center_blocks_per_row(rows, cols);
+    double* partial = (double*)workspace;
+#define KMX_CENTER(T)                                                                                                  \
+    do {                                                                                                               \
+        hipLaunchKernelGGL((center_mean_kernel<T>), dim3(1), dim3(256), 0, stream, (T*)mean, (T*)stats, rows, (T)cols); \
+        hipLaunchKernelGGL((center_rows_kernel<T>), dim3((unsigned)b, (unsigned)rows), dim3(256), 0, stream,           \
+                           (const T*)X_t, (T*)dst, (const T*)mean, (const T*)stats, partial, cols);                    \
+        hipLaunchKernelGGL((center_total_kernel<T>), dim3(1), dim3(1024), 0, stream, partial, b * rows,                \
+                           (const T*)sample_weight, (T*)stats);                                                        \
+    } while (0)
+    if (dtype == KMX_F32) KMX_CENTER(float); else KMX_CENTER(double);
+#undef KMX_CENTER
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }

@@ -13,7 +13,7 @@ import torch
 from .. import _capi
 from .._capi import LloydStatus, check, lib, ptr
 from ..common._buffers import contiguous, dcode, require_cuda, room_for, workspace
-from ..common.kernels import broadcast_rows, divide_by, transposed_copy
+from ..common.kernels import broadcast_rows, transposed_copy
 from ..common.random import create_xoroshiro128pp_states, get_random_raw, raw_to_uniform
 from ..common.reductions import sum_reduction
 from ..common.topk import topk_idx
@@ -264,23 +264,27 @@ def prepare_data_for_lloyd(X_t, init, tol, sample_weight, copy_x):
     require_cuda()
     d, n = X_t.shape
     X_t = contiguous(X_t)
-    X_mean = sum_reduction(X_t, axis=1)
-    divide_by(X_mean, n)
-    X_sum_squared = sum_reduction(X_mean, square=True)
-    if float(X_sum_squared[0]) == 0.0:
+    fused = sample_weight.dtype == X_t.dtype and tuple(sample_weight.shape) == (n,)
+    weights = contiguous(sample_weight) if fused else X_t  # (any n values)
+    centred = torch.empty_like(X_t) if copy_x else X_t
+    X_mean = torch.empty(d, dtype=X_t.dtype, device=X_t.device)
+    stats = torch.empty(4, dtype=X_t.dtype, device=X_t.device)
+    ws_bytes = lib.kmx_center_workspace_bytes(d, n)
+    check(lib.kmx_center_rows(ptr(X_t), ptr(centred), ptr(weights), ptr(X_mean), ptr(stats),
+                              ptr(workspace(ws_bytes, X_t.device, tag="sum")), ws_bytes, d, n, dcode(X_t),
+                              _capi.current_stream()), "kmx_center_rows")
+    # everything the host needs to know about the data, read back once
+    mean_squares, variance, sample_weight_sum, first = stats.cpu().numpy()
+    if not fused:
+        sample_weight_sum = sum_reduction(sample_weight).cpu().numpy()[0]
+        first = sample_weight[:1].cpu().numpy()[0]
+    if mean_squares == 0.0:
         X_mean = None
     else:
-        if copy_x:
-            X_t = X_t.clone()
-        broadcast_rows(X_t, X_mean, "minus")
+        X_t = centred
         if isinstance(init, torch.Tensor):
             broadcast_rows(init, X_mean, "minus")
-
-    variance = sum_reduction(X_t.reshape(-1), square=True)
-    tol = (float(variance.cpu().numpy()[0]) / (d * n)) * tol
-
-    sample_weight_sum = sum_reduction(sample_weight).cpu().numpy()[0]
-    first = sample_weight[:1].cpu().numpy()[0]
+    tol = (float(variance) / (d * n)) * tol
     sample_weight_is_uniform = bool(sample_weight_sum == first * first.dtype.type(n))
     return X_t, X_mean, init, tol, sample_weight_is_uniform
 
