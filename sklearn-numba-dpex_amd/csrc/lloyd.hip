@@ -38,6 +38,60 @@ __device__ __forceinline__ void load_row(const T* __restrict__ row, int64_t i0, 
     }
 }
 
+// A workgroup's sums (lds_copies of them in LDS, fp64) to its slot of `partial`.  fuse_tail: there are few slots, and
+// the workgroup that gets done last adds them up (in fp64, in an order that does not depend on timing) and
+// finishes the iteration.
+template <typename T>
+__device__ __forceinline__ void hand_over_sums(double* all, int lds_copies, T* __restrict__ partial,
+                                               kmx_lloyd_status* status, int d, int k, const LloydTail<T>& tail,
+                                               const int fuse_tail) {
+    const int items = (d + 1) * k;
+    T* out = partial + (size_t)blockIdx.x * items;
+    for (int j = threadIdx.x; j < items; j += 256) {
+        double tot = all[j];
+        for (int c = 1; c < lds_copies; ++c) tot += all[(size_t)c * items + j];
+        if (fuse_tail) __hip_atomic_store(&out[j], (T)tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else out[j] = (T)tot;
+    }
+    if (!fuse_tail || !lloyd_last_workgroup(status)) return;
+    // thread (g, j): item j (and j + 256, ...) of every n_groups-th slot, eight loads in flight; the groups are
+    // then added in order
+    __shared__ double red[256];
+    const int n_groups = items < 256 ? 256 / items : 1, slots = (int)gridDim.x;
+    for (int base = 0; base < items; base += 256) {
+        const int g = items < 256 ? (int)threadIdx.x / items : 0;
+        const int j = items < 256 ? (int)threadIdx.x - g * items : base + (int)threadIdx.x;
+        double s = 0.0;
+        if (g < n_groups && j < items) {
+            const T* __restrict__ from = partial + j;
+            auto slot = [&](const int b) __attribute__((always_inline)) {
+                return __hip_atomic_load(from + (size_t)b * items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            };
+            int b = g;
+            for (; b + 7 * n_groups < slots; b += 8 * n_groups) {
+                T v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = slot(b + u * n_groups);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s += (double)v[u];
+            }
+            for (; b < slots; b += n_groups) s += (double)slot(b);
+        }
+        red[threadIdx.x] = s;
+        __syncthreads();
+        const int at = base + (int)threadIdx.x;
+        if (at < items && (items >= 256 || (int)threadIdx.x < items)) {
+            double tot = red[threadIdx.x];
+            for (int g2 = 1; g2 < n_groups; ++g2) tot += red[g2 * items + threadIdx.x];
+            if (at < d * k) tail.sums_t[at] = (T)tot;
+            else tail.sizes[at - d * k] = (T)tot;
+        }
+        __syncthreads();
+    }
+    lloyd_small_finalize_body<T, false, true>(nullptr, nullptr, tail, reinterpret_cast<T*>(all));
+    if (threadIdx.x == 0) status->ticket = 0u;
+}
+
 constexpr int ACC_NONE = 0;    // labels only
 constexpr int ACC_LDS = 1;     // workgroup-private LDS accumulators, flushed to partial[block]
 constexpr int ACC_GLOBAL = 2;  // hardware float atomics into partial[block % n_copies]
@@ -50,7 +104,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_reg_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight, const T* __restrict__ cpack,
     const T* __restrict__ half_norms, const uint32_t* __restrict__ labels_prev,
     uint32_t* __restrict__ labels, T* __restrict__ partial, kmx_lloyd_status* __restrict__ status,
-    int64_t n, int d, int k, int dpad, int n_copies, int lds_copies) {
+    int64_t n, int d, int k, int dpad, int n_copies, int lds_copies, const LloydTail<T> tail, const int fuse_tail) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
 
     // LDS accumulators are fp64 for both types: ds_add_f64 is fast on this hardware, ds_add_f32
@@ -151,15 +205,11 @@ __global__ __launch_bounds__(256) void lloyd_fused_reg_kernel(
         if (changed) atomicAdd(&changed_block, changed);
         __syncthreads();
         if (ACC == ACC_LDS) {
-            T* out = partial + (size_t)blockIdx.x * items;
-            const double* all = reinterpret_cast<const double*>(smem_raw);
-            for (int j = threadIdx.x; j < items; j += 256) {
-                double tot = all[j];
-                for (int c = 1; c < lds_copies; ++c) tot += all[(size_t)c * items + j];
-                out[j] = (T)tot;
-            }
+            if (threadIdx.x == 0 && changed_block) atomicAdd(&status->n_changed, changed_block);
+            hand_over_sums<T>(reinterpret_cast<double*>(smem_raw), lds_copies, partial, status, d, k, tail, fuse_tail);
+        } else if (threadIdx.x == 0 && changed_block) {
+            atomicAdd(&status->n_changed, changed_block);
         }
-        if (threadIdx.x == 0 && changed_block) atomicAdd(&status->n_changed, changed_block);
     }
 }
 
@@ -174,7 +224,7 @@ __global__ __launch_bounds__(256) void lloyd_fused_stream_kernel(
     const T* __restrict__ centroids_t, const T* __restrict__ half_norms,
     const uint32_t* __restrict__ labels_prev, uint32_t* __restrict__ labels,
     T* __restrict__ partial, kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k,
-    int n_copies, int lds_copies) {
+    int n_copies, int lds_copies, const LloydTail<T> tail, const int fuse_tail) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
 
     // LDS accumulators are fp64 for both types: ds_add_f64 is fast on this hardware, ds_add_f32
@@ -279,15 +329,11 @@ __global__ __launch_bounds__(256) void lloyd_fused_stream_kernel(
         if (changed) atomicAdd(&changed_block, changed);
         __syncthreads();
         if (ACC == ACC_LDS) {
-            T* out = partial + (size_t)blockIdx.x * items;
-            const double* all = reinterpret_cast<const double*>(smem_raw);
-            for (int j = threadIdx.x; j < items; j += 256) {
-                double tot = all[j];
-                for (int c = 1; c < lds_copies; ++c) tot += all[(size_t)c * items + j];
-                out[j] = (T)tot;
-            }
+            if (threadIdx.x == 0 && changed_block) atomicAdd(&status->n_changed, changed_block);
+            hand_over_sums<T>(reinterpret_cast<double*>(smem_raw), lds_copies, partial, status, d, k, tail, fuse_tail);
+        } else if (threadIdx.x == 0 && changed_block) {
+            atomicAdd(&status->n_changed, changed_block);
         }
-        if (threadIdx.x == 0 && changed_block) atomicAdd(&status->n_changed, changed_block);
     }
 }
 
@@ -641,12 +687,14 @@ static int lds_acc_copies(int d, int k) {
 template <typename T, int DREG, int R, int ACC>
 void launch_reg(const LloydLayout& L, const void* X_t, const void* w, const T* cpack,
                 const T* half_norms, const uint32_t* labels_prev, uint32_t* labels, T* partial,
-                kmx_lloyd_status* status, int64_t n, int d, int k, int grid, hipStream_t stream) {
+                kmx_lloyd_status* status, int64_t n, int d, int k, int grid, hipStream_t stream,
+                const LloydTail<T>* tail) {
     const int copies = lds_acc_copies(d, k);
     const size_t lds = (ACC == ACC_LDS) ? (size_t)(d + 1) * k * sizeof(double) * copies : 0;
     hipLaunchKernelGGL((lloyd_fused_reg_kernel<T, DREG, R, ACC>), dim3(grid), dim3(256), lds, stream,
                        (const T*)X_t, (const T*)w, cpack, half_norms, labels_prev, labels, partial,
-                       status, n, d, k, L.dpad, L.n_partials, copies);
+                       status, n, d, k, L.dpad, L.n_partials, copies, tail ? *tail : LloydTail<T>(),
+                       tail ? 1 : 0);
 }
 
 // Returns the status of the entry point it hands over to (a refusal there would leave `labels`
@@ -656,7 +704,7 @@ int32_t launch_fused(const LloydLayout& L, const void* X_t, const void* w, const
                   const T* cpack, const T* half_norms, const uint32_t* labels_prev,
                   uint32_t* labels, T* partial, kmx_lloyd_status* status, int64_t n, int d, int k,
                   hipStream_t stream, const unsigned int* screen_absmax = nullptr, char* screen_area = nullptr,
-                  const void* X_rowmajor = nullptr) {
+                  const void* X_rowmajor = nullptr, const LloydTail<T>* tail = nullptr) {
     const int grid = lloyd_fused_grid(L, n, d, sizeof(T) == 8 ? KMX_F64 : KMX_F32);
     if (L.variant == KMX_VARIANT_GEMM) {
         if (sizeof(T) == 4 && L.screen_labels)
@@ -674,7 +722,7 @@ int32_t launch_fused(const LloydLayout& L, const void* X_t, const void* w, const
     } else if (L.variant == KMX_VARIANT_REGISTER) {
 #define KMX_REG_CASE(DR, RR)                                                                    \
     launch_reg<T, DR, RR, ACC>(L, X_t, w, cpack, half_norms, labels_prev, labels, partial, status, \
-                               n, d, k, grid, stream)
+                               n, d, k, grid, stream, tail)
         if constexpr (sizeof(T) == 4) {
             if (d <= 8)
                 KMX_REG_CASE(8, 4);
@@ -702,16 +750,20 @@ int32_t launch_fused(const LloydLayout& L, const void* X_t, const void* w, const
         if (lloyd_stream_samples_per_thread(n, sizeof(T) == 8 ? KMX_F64 : KMX_F32) == 1) {
             hipLaunchKernelGGL((lloyd_fused_stream_kernel<T, 1, KC, ACC>), dim3(grid), dim3(256), lds,
                                stream, (const T*)X_t, (const T*)w, (const T*)centroids_t, half_norms,
-                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies);
+                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies,
+                               tail ? *tail : LloydTail<T>(), tail ? 1 : 0);
         } else {
             hipLaunchKernelGGL((lloyd_fused_stream_kernel<T, RV, KC, ACC>), dim3(grid), dim3(256), lds,
                                stream, (const T*)X_t, (const T*)w, (const T*)centroids_t, half_norms,
-                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies);
+                               labels_prev, labels, partial, status, n, d, k, L.n_partials, copies,
+                               tail ? *tail : LloydTail<T>(), tail ? 1 : 0);
         }
     }
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
+
+constexpr int64_t TAIL_PARTIALS = 16384;
 
 template <typename T>
 int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_rowmajor, const void* w,
@@ -724,6 +776,21 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
     T* half_norms = reinterpret_cast<T*>(ws + L.off_half);
     T* partial = reinterpret_cast<T*>(ws + L.off_partial);
     double* shift_partial = reinterpret_cast<double*>(ws + L.off_shift);
+    auto small_tail_args = [&] {
+        LloydTail<T> tail;
+        tail.sums_t = (T*)new_centroids_t;
+        tail.sizes = (T*)sizes;
+        tail.empty_clusters = empty_clusters;
+        tail.old_centroids_t = (const T*)centroids_t;
+        tail.cpack = cpack;
+        tail.half_norms = half_norms;
+        tail.status = status;
+        tail.d = d;
+        tail.k = k;
+        tail.dpad = L.dpad;
+        tail.progress = L.progress;
+        return tail;
+    };
 
     if (events) (void)hipEventRecord(events[0], stream);
     int n_partials_used = L.n_partials;
@@ -759,11 +826,23 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
             if (rc != KMX_OK) return rc;
         }
     } else if (L.acc_mode == ACC_LDS) {
+        n_partials_used = lloyd_fused_grid(L, n, d, sizeof(T) == 8 ? KMX_F64 : KMX_F32);
+        // Up to this many partial sums the step's last workgroup adds them up and ends the iteration, instead of
+        // two more launches; one workgroup reads them at 64 loads a thread.  Runs of 10 iterations, us, three
+        // launches / one: 800 000 x 4, 2 clusters fp64 485 / 431; 100 000 x 10, 8 fp32 335 / 306; 20 651 x 3, 6 fp64
+        // 259 / 239.
+        const bool fuse = (L.variant == KMX_VARIANT_REGISTER || L.variant == KMX_VARIANT_STREAM) &&
+                          (int64_t)n_partials_used * (d + 1) * k <= TAIL_PARTIALS && (d + 1) * k <= 6 * 1024;
+        const LloydTail<T> tail = small_tail_args();
         const int32_t rc_step =
             launch_fused<T, ACC_LDS>(L, X_t, w, centroids_t, cpack, half_norms, labels_prev, labels,
-                                     partial, status, n, d, k, stream, nullptr, nullptr, X_rowmajor);
+                                     partial, status, n, d, k, stream, nullptr, nullptr, X_rowmajor, fuse ? &tail : nullptr);
         if (rc_step != KMX_OK) return rc_step;
-        n_partials_used = lloyd_fused_grid(L, n, d, sizeof(T) == 8 ? KMX_F64 : KMX_F32);
+        if (fuse) {
+            if (events)
+                for (int i = 1; i < 4; ++i) (void)hipEventRecord(events[i], stream);
+            return KMX_OK;
+        }
     } else {
         const int32_t rc_step =
             launch_fused<T, ACC_GLOBAL>(L, X_t, w, centroids_t, cpack, half_norms, labels_prev, labels,
@@ -779,18 +858,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
             // 9 us for 1 900 sums, 27 us for 10 500; the conversion pass and the general
             // finalisation below take 18 us for 16 600)
             if (events) (void)hipEventRecord(events[2], stream);
-            LloydTail<float> tail;
-            tail.sums_t = (float*)new_centroids_t;
-            tail.sizes = (float*)sizes;
-            tail.empty_clusters = empty_clusters;
-            tail.old_centroids_t = (const float*)centroids_t;
-            tail.cpack = cpack;
-            tail.half_norms = half_norms;
-            tail.status = status;
-            tail.d = d;
-            tail.k = k;
-            tail.dpad = L.dpad;
-            tail.progress = L.progress;
+            const LloydTail<float> tail = small_tail_args();
             hipLaunchKernelGGL((lloyd_small_finalize_kernel<float, true>), dim3(1), dim3(256),
                                (size_t)items * sizeof(float), stream, gsum, q_exp, tail);
             KMX_LAUNCH_CHECK();
@@ -811,18 +879,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
     KMX_LAUNCH_CHECK();
     if (events) (void)hipEventRecord(events[2], stream);
     if (small_tail) {
-        LloydTail<T> tail;
-        tail.sums_t = (T*)new_centroids_t;
-        tail.sizes = (T*)sizes;
-        tail.empty_clusters = empty_clusters;
-        tail.old_centroids_t = (const T*)centroids_t;
-        tail.cpack = cpack;
-        tail.half_norms = half_norms;
-        tail.status = status;
-        tail.d = d;
-        tail.k = k;
-        tail.dpad = L.dpad;
-        tail.progress = L.progress;
+        const LloydTail<T> tail = small_tail_args();
         hipLaunchKernelGGL((lloyd_small_finalize_kernel<T, false>), dim3(1), dim3(256),
                            (size_t)items * sizeof(T), stream, nullptr, nullptr, tail);
     } else {

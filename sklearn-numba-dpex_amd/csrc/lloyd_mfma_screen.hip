@@ -1588,12 +1588,7 @@ __global__ __launch_bounds__(64 * scr_waves(NK), NK == 1 ? scr_waves(1) / 4 : 2)
         // side; each workgroup waits for its own before it draws its ticket, and the last one
         // reads them with device-scope loads.  No device-wide fence.
         if (fuse_tail) {
-            __shared__ unsigned int is_last;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            if (threadIdx.x == 0) is_last = (atomicAdd(&status->ticket, 1u) == gridDim.x - 1) ? 1u : 0u;
-            __syncthreads();
-            if (is_last != 0u) {
+            if (lloyd_last_workgroup(status)) {
                 // (the accumulators are flushed: their LDS holds the (d + 1) k sums as floats)
                 lloyd_small_finalize_body<TX, true, true>(gsum, q_exp, tail, reinterpret_cast<TX*>(smem_raw));
                 if (threadIdx.x == 0) status->ticket = 0u;

@@ -479,6 +479,18 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
     if (threadIdx.x == 0) lloyd_update_status(a.status, total, n_changed, a.progress);
 }
 
+// Every workgroup of a launch calls this behind what it hands over (device-scope atomics and stores) with all
+// its threads: true in the one that gets there last.  Each waits for its own accesses before it draws its
+// ticket, so that the last one finds everyone's with device-scope loads; no device-wide fence.
+__device__ __forceinline__ bool lloyd_last_workgroup(kmx_lloyd_status* status) {
+    __shared__ unsigned int last_s;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) last_s = atomicAdd(&status->ticket, 1u) == gridDim.x - 1 ? 1u : 0u;
+    __syncthreads();
+    return last_s != 0u;
+}
+
 // The same as a launch of its own: ordered after the producers of the sums by the kernel boundary.
 template <typename T, bool FROM_GSUM>
 __global__ __launch_bounds__(256) void lloyd_small_finalize_kernel(
