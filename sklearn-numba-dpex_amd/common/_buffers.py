@@ -70,6 +70,17 @@ def room_for(n_bytes, device):
     return 2 * n_bytes <= free
 
 
+def host_scalar(dtype):
+    """One value in pinned host memory for a kernel to write: `read_host_scalar` waits for the stream and
+    reads it, where a value in device memory takes a copy's launch and its wait as well (9 us a call)."""
+    return torch.empty(1, dtype=dtype, pin_memory=True)
+
+
+def read_host_scalar(out, device):
+    torch.cuda.current_stream(device).synchronize()
+    return out.numpy().copy()
+
+
 def dcode(t):
     return _capi.dtype_code(t.dtype)
 

@@ -12,7 +12,7 @@ import torch
 
 from .. import _capi
 from .._capi import LloydStatus, check, lib, ptr
-from ..common._buffers import contiguous, dcode, require_cuda, room_for, workspace
+from ..common._buffers import contiguous, dcode, host_scalar, read_host_scalar, require_cuda, room_for, workspace
 from ..common.kernels import broadcast_rows, transposed_copy
 from ..common.random import create_xoroshiro128pp_states, get_random_raw, raw_to_uniform
 from ..common.reductions import sum_reduction
@@ -154,13 +154,13 @@ def lloyd(
         inertia = _assign_with_inertia(X_t, sample_weight, best, assignments_idx, flags)[0]
     else:
         inertia_ws_bytes = lib.kmx_inertia_workspace_bytes(n)
-        out = torch.empty(1, dtype=dt, device=dev)
+        out = host_scalar(dt)
         check(lib.kmx_lloyd_labels_inertia(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(best),
                                            ptr(assignments_idx), ptr(out), ptr(ws), ws_bytes, ptr(resident),
                                            resident_bytes, n_iteration,
                                            ptr(workspace(inertia_ws_bytes, dev, tag="inertia")), inertia_ws_bytes,
                                            stream), "kmx_lloyd_labels_inertia")
-        inertia = out.cpu().numpy()[0]
+        inertia = read_host_scalar(out, dev)[0]
     return assignments_idx, inertia, best, n_iteration
 
 
@@ -184,11 +184,11 @@ def _assign_with_inertia(X_t, sample_weight, centroids_t, labels_out, flags=None
     flags = _capi.DEFAULT_FLAGS if flags is None else int(flags)
     ws_bytes = lib.kmx_assign_inertia_workspace_bytes(n, d, k, dc, flags)
     ws = workspace(ws_bytes, X_t.device, tag="assign_inertia")
-    out = torch.empty(1, dtype=X_t.dtype, device=X_t.device)
+    out = host_scalar(X_t.dtype)
     check(lib.kmx_assign_labels_inertia(ptr(X_t), ptr(sample_weight), ptr(centroids_t), ptr(labels_out), ptr(out),
                                         ptr(ws), ws_bytes, n, d, k, dc, flags, _capi.current_stream()),
           "kmx_assign_labels_inertia")
-    return out.cpu().numpy()
+    return read_host_scalar(out, X_t.device)
 
 
 def _per_sample_inertia(X_t, sample_weight, centroids_t, labels, out=None):
@@ -208,10 +208,10 @@ def _inertia_array(X_t, sample_weight, centroids_t, labels):
     k = centroids_t.shape[1]
     ws_bytes = lib.kmx_inertia_workspace_bytes(n)
     ws = workspace(ws_bytes, X_t.device, tag="inertia")
-    out = torch.empty(1, dtype=X_t.dtype, device=X_t.device)
+    out = host_scalar(X_t.dtype)
     check(lib.kmx_inertia(ptr(X_t), ptr(sample_weight), ptr(centroids_t), ptr(labels), ptr(out), ptr(ws), ws_bytes,
                           n, d, k, dcode(X_t), _capi.current_stream()), "kmx_inertia")
-    return out.cpu().numpy()
+    return read_host_scalar(out, X_t.device)
 
 
 def _inertia(X_t, sample_weight, centroids_t, labels):

@@ -36,7 +36,7 @@ except ImportError:  # stock scikit-learn
             self.estimator = estimator
 
 
-from ..common._buffers import require_cuda, upload
+from ..common._buffers import host_scalar, read_host_scalar, require_cuda, upload
 from ..common.kernels import all_finite, transposed_copy
 from .drivers import (
     get_euclidean_distances,
@@ -224,7 +224,7 @@ class KMeansEngine(_EngineBase):
             X_dev.shape[1] == getattr(self.estimator, "n_features_in_", X_dev.shape[1])
         ):
             # one pass over the rows where they are, which looks for non-finite values on the way
-            not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
+            not_finite = host_scalar(torch.int32)
             try:
                 cluster_centers = self._check_init(self.estimator.cluster_centers_, X_dev, copy=False)
             except Exception:
@@ -258,7 +258,7 @@ class KMeansEngine(_EngineBase):
         were looked at when they were transposed (or in one read of their own) instead of in a
         single-threaded host pass that costs more than the upload.  Non-finite data then get
         scikit-learn's own error from the host copy."""
-        if not int(not_finite):
+        if not read_host_scalar(not_finite, X_t.device)[0]:
             return
         from sklearn.utils.validation import _assert_all_finite
 
@@ -312,7 +312,7 @@ class KMeansEngine(_EngineBase):
         n_features = X_dev.shape[1]
         # (d, n) contiguous; already the case for an F-ordered array
         X_t = X_dev.T
-        not_finite = torch.empty(1, dtype=torch.int32, device=X_dev.device)
+        not_finite = host_scalar(torch.int32)
         if X_dev.is_contiguous() and not X_t.is_contiguous():
             X_t = transposed_copy(X_dev, not_finite)
             owns_copy = True

@@ -424,6 +424,45 @@ def test_fp32_distances_of_close_and_extreme_pairs(cuda, case):
     np.testing.assert_allclose(got, exact, rtol=(d / 2 + 3) * 1.2e-7)  # (redone pairs: d rounded additions)
 
 
+# a total that a kernel writes to the host: the same bits call after call, from several streams at once, and as a graph
+# that is replayed between other calls leaves it in device memory
+@pytest.mark.parametrize("n,d,k,dtype", [(1, 3, 2, np.float32), (20_001, 14, 40, np.float32), (30_003, 70, 9, np.float32),
+                                         (30_003, 20, 30, np.float64), (523_000, 3, 5, np.float64)])
+def test_inertia_totals_repeat_themselves(cuda, n, d, k, dtype):
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib, ptr
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(n)
+    X, C = rng.standard_normal((n, d)).astype(dtype), rng.standard_normal((k, d)).astype(dtype)
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    X_t, C_t, w_d = _dev(X.T, cuda), _dev(C.T, cuda), _dev(w, cuda)
+    labels, first = drivers.get_labels_inertia(X_t, C_t, w_d, True)
+    lab = labels.cpu().numpy()
+    exact = (w.astype(np.float64) * ((X.astype(np.float64) - C.astype(np.float64)[lab]) ** 2).sum(axis=1)).sum()
+    np.testing.assert_allclose(first[0], exact, rtol=2e-5 if dtype == np.float32 else 1e-12)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for s in streams:
+            with torch.cuda.stream(s):
+                assert drivers.get_labels_inertia(X_t, C_t, w_d, True)[1][0] == first[0]
+    dc = _capi.dtype_code(X_t.dtype)
+    ws_bytes = lib.kmx_assign_inertia_workspace_bytes(n, d, k, dc, 0)
+    ws, out = torch.empty(ws_bytes, dtype=torch.uint8, device=cuda), torch.empty(1, dtype=X_t.dtype, device=cuda)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _capi.check(lib.kmx_assign_labels_inertia(ptr(X_t), ptr(w_d), ptr(C_t), ptr(labels), ptr(out), ptr(ws), ws_bytes, n, d,
+                                                  k, dc, 0, _capi.current_stream()), "captured")
+    for _ in range(4):
+        out.fill_(-1)
+        graph.replay()
+        assert drivers.get_labels_inertia(X_t, C_t, w_d, True)[1][0] == first[0]
+        assert float(out[0]) == first[0]
+
+
 def test_distances_with_few_samples_split_the_centroids(cuda):
     """With few samples the centroid range is split over the second grid dimension (ragged last
     share, k not a multiple of 4), and exact zeros / tiny distances go through the square root."""
