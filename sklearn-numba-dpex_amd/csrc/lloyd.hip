@@ -587,7 +587,10 @@ __global__ __launch_bounds__(256) void lloyd_pack_kernel(const T* __restrict__ c
                                                          T* __restrict__ half_norms,
                                                          kmx_lloyd_status* __restrict__ status,
                                                          int d, int k, int dpad, int max_iter,
-                                                         double tol) {
+                                                         double tol, unsigned int* __restrict__ zero, int n_zero) {
+    // (words that the launches behind this one add to)
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < n_zero; i += 256) zero[i] = 0u;
     const int g = threadIdx.x & (LANES - 1);
     const int c = blockIdx.x * (256 / LANES) + (int)(threadIdx.x / LANES);
     T sq = T(0);
@@ -637,13 +640,16 @@ __global__ __launch_bounds__(256) void lloyd_pack_kernel(const T* __restrict__ c
 
 template <typename T>
 static void launch_pack(const void* centroids_t, void* cpack, void* half_norms, kmx_lloyd_status* status, int d, int k,
-                        int dpad, int max_iter, double tol, hipStream_t stream) {
+                        int dpad, int max_iter, double tol, hipStream_t stream, unsigned int* zero = nullptr,
+                        int n_zero = 0) {
     if (d >= 256)
         hipLaunchKernelGGL((lloyd_pack_kernel<T, 64>), dim3((unsigned)kmx_cdiv(k, 4)), dim3(256), 0, stream,
-                           (const T*)centroids_t, (T*)cpack, (T*)half_norms, status, d, k, dpad, max_iter, tol);
+                           (const T*)centroids_t, (T*)cpack, (T*)half_norms, status, d, k, dpad, max_iter, tol, zero,
+                           n_zero);
     else
         hipLaunchKernelGGL((lloyd_pack_kernel<T, 8>), dim3((unsigned)kmx_cdiv(k, 32)), dim3(256), 0, stream,
-                           (const T*)centroids_t, (T*)cpack, (T*)half_norms, status, d, k, dpad, max_iter, tol);
+                           (const T*)centroids_t, (T*)cpack, (T*)half_norms, status, d, k, dpad, max_iter, tol, zero,
+                           n_zero);
 }
 
 __global__ void fill_zero_bytes_kernel(uint32_t* __restrict__ p, size_t n_words) {
@@ -1088,19 +1094,22 @@ static int32_t lloyd_init_impl(const kmx_lloyd_plan* plan, void* workspace, size
     hipStream_t stream = (hipStream_t)stream_;
     char* ws = (char*)workspace;
     auto* status = reinterpret_cast<kmx_lloyd_status*>(ws + L.off_status);
+    const bool scales = L.variant == KMX_VARIANT_MFMA || L.variant == KMX_VARIANT_MFMA_WIDE || L.gemm_screen ||
+                        L.direct_sums || L.screen64 || L.variant == KMX_VARIANT_FEWK;
+    // (clears the words of the maxima for the pass that takes them)
+    unsigned int* absmax = scales ? reinterpret_cast<unsigned int*>(ws + L.off_scales) : nullptr;
     if (dtype == KMX_F32)
-        launch_pack<float>(centroids_t, ws + L.off_cpack, ws + L.off_half, status, d, k, L.dpad, max_iter, tol, stream);
+        launch_pack<float>(centroids_t, ws + L.off_cpack, ws + L.off_half, status, d, k, L.dpad, max_iter, tol, stream,
+                           absmax, scales ? d + 1 : 0);
     else
-        launch_pack<double>(centroids_t, ws + L.off_cpack, ws + L.off_half, status, d, k, L.dpad, max_iter, tol, stream);
+        launch_pack<double>(centroids_t, ws + L.off_cpack, ws + L.off_half, status, d, k, L.dpad, max_iter, tol, stream,
+                            absmax, scales ? d + 1 : 0);
     KMX_LAUNCH_CHECK();
-    if (L.variant == KMX_VARIANT_MFMA || L.variant == KMX_VARIANT_MFMA_WIDE || L.gemm_screen || L.direct_sums ||
-        L.screen64 || L.variant == KMX_VARIANT_FEWK) {
+    if (scales) {
         // (for the screened tiled product: max|x| per feature, from which its scale is taken)
         // (the pass over X that makes the resident copies takes the maxima along)
         if (resident != nullptr) {
-            kmx_lloyd_absmax_clear(L, ws, d, stream);
-            const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, centroids_t, resident,
-                                                 reinterpret_cast<unsigned int*>(ws + L.off_scales), n, d, k, dtype, stream);
+            const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, centroids_t, resident, absmax, n, d, k, dtype, stream);
             if (rc != KMX_OK) return rc;
         }
         const int32_t rc = kmx_lloyd_mfma_prepare(L, resident != nullptr ? nullptr : X_t, sample_weight, ws, n, d, dtype, stream);
@@ -1109,14 +1118,11 @@ static int32_t lloyd_init_impl(const kmx_lloyd_plan* plan, void* workspace, size
         const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, centroids_t, resident, nullptr, n, d, k, dtype, stream);
         if (rc != KMX_OK) return rc;
     }
-    if (L.variant == KMX_VARIANT_MFMA_WIDE || L.screen || L.screen64) {
-        // cluster counts of the wide path / the counter of uncertain samples of the screened one
-        hipLaunchKernelGGL(fill_zero_bytes_kernel, dim3(4), dim3(256), 0, stream,
-                           (uint32_t*)(ws + L.off_bucket),
-                           (L.screen || L.screen64) ? (size_t)64 : (size_t)k);
-        KMX_LAUNCH_CHECK();
-    }
+    // (the counter of uncertain samples of the screened steps was cleared with the sums)
     if (L.variant == KMX_VARIANT_MFMA_WIDE) {
+        // cluster counts
+        hipLaunchKernelGGL(fill_zero_bytes_kernel, dim3(4), dim3(256), 0, stream,
+                           (uint32_t*)(ws + L.off_bucket), (size_t)k);
         hipLaunchKernelGGL(fill_zero_bytes_kernel, dim3(1), dim3(64), 0, stream,
                            (uint32_t*)(ws + L.off_wscreen), (size_t)64);
         KMX_LAUNCH_CHECK();

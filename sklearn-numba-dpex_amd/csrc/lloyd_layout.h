@@ -322,8 +322,7 @@ static inline bool lloyd_tiles_wanted(const LloydLayout& L, int64_t n, int d, in
 
 // fp32 matrix-core implementations (lloyd_mfma.hip)
 // Fixed-point exponents from max|X_t row|, max|w| and n; clears the fixed-point sums.
-// X_t null: the words of max|X_t row| are there already (cleared by kmx_lloyd_absmax_clear, then filled)
-void kmx_lloyd_absmax_clear(const LloydLayout& L, char* ws, int d, hipStream_t stream);
+// The words of the maxima are zero on entry; X_t null: those of max|X_t row| have been taken already
 int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void* w, char* ws,
                                int64_t n, int d, int dtype, hipStream_t stream);
 int32_t kmx_lloyd_iter_mfma_f32(const LloydLayout& L, const void* X_t, const void* w,
@@ -376,7 +375,6 @@ int32_t kmx_assign_labels_inertia_mfma_screen(const void* X_t, const void* w, co
                                               int64_t n, int d, int k, int wgs_per_cu, hipStream_t stream);
 // out[0] = sum of `count` fp64 partial sums, in order (inertia_distances.hip)
 int32_t kmx_inertia_total_launch(const double* partial, int count, void* out, int32_t dtype, hipStream_t stream);
-int32_t kmx_sample_norms(const void* X_t, float* norms, int64_t n, int d, int dtype, hipStream_t stream);
 int32_t kmx_screen_scores_impl(const float* X_t, const float* centroids_t, float* scores,
                                float* bounds, float* half_norms, float* scale, unsigned int* scratch,
                                int64_t n, int d, int k, hipStream_t stream);

@@ -45,10 +45,6 @@ __device__ __forceinline__ unsigned long long to_fixed(double scaled_plus_magic)
 
 // ---------------------------------------------------------------------------- scales
 
-__global__ void absmax_zero_kernel(unsigned int* absmax, int count) {
-    for (int i = threadIdx.x; i < count; i += blockDim.x) absmax[i] = 0u;
-}
-
 // Row r < d: max |X_t[r, :]|; row d: max |w|.  Non-negative floats order like their bits.
 // (fp64 inputs: the maximum of the values rounded to fp32, which is what the screened step works
 // with; its fixed-point exponents leave a factor of two of room above it)
@@ -93,12 +89,98 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const T* __restrict__ 
     }
 }
 
+// The maxima above and ||x_i|| of every sample (fp32, features in order) in one pass over X_t, for
+// the steps that want both and d <= DM <= 64: a thread keeps the d maxima of its samples in
+// registers and meets the others once, at its end.  Bound by the read of X, which two kernels
+// read twice: 5 000 000 x 14 fp32 110 us -> 55 (5.8 TB/s with the norms written), 2 000 000 x 32 fp64
+// 182 -> 111 (4.9 TB/s), 1 000 000 x 60 fp32 79 -> 46, 100 000 x 14 17 -> 8.  Loads go out in batches of eight rows; a row behind the last one is read as the last
+// one again (a cache hit) and counts as zeros.
+constexpr int SCAN_D_MAX = 64;
+constexpr int SCAN_THREADS = 256;
+template <int W, typename V>
+__device__ __forceinline__ float scan_value(V v, int t) {
+    if constexpr (W == 1) return (float)v;
+    else return (float)v[t];
+}
+template <typename T, int W, int DM>
+__device__ __forceinline__ void scan_group(const T* __restrict__ X_t, const T* __restrict__ w,
+                                           float* __restrict__ norms, int64_t n, int d, int64_t i, float (&most)[DM],
+                                           float& w_most) {
+    using V = typename KmxVec<T, W>::type;
+    const V wv = *reinterpret_cast<const V*>(w + i);
+    float sq[W];
+#pragma unroll
+    for (int t = 0; t < W; ++t) {
+        sq[t] = 0.0f;
+        w_most = fmaxf(w_most, fabsf(scan_value<W>(wv, t)));
+    }
+#pragma unroll
+    for (int f0 = 0; f0 < DM; f0 += 8) {
+        if (f0 >= d) break;
+        // (opaque: else the offsets of all the rows are kept over the loop, beyond the registers)
+        int64_t row = n;
+        asm volatile("" : "+s"(row));
+        V v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int f = f0 + u < d ? f0 + u : d - 1;
+            v[u] = *reinterpret_cast<const V*>(X_t + (size_t)f * row + i);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int t = 0; t < W; ++t) {
+                const float x = f0 + u < d ? scan_value<W>(v[u], t) : 0.0f;
+                sq[t] = fmaf(x, x, sq[t]);
+                most[f0 + u] = fmaxf(most[f0 + u], fabsf(x));
+            }
+        // (opaque: else the values wait in registers for maxima taken together at the end)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(most[f0 + u]));
+    }
+#pragma unroll
+    for (int t = 0; t < W; ++t) norms[i + t] = sqrtf(sq[t]);
+}
+
+template <typename T, int DM>
+__global__ __launch_bounds__(SCAN_THREADS) void scan_samples_kernel(const T* __restrict__ X_t,
+                                                                    const T* __restrict__ w,
+                                                                    unsigned int* __restrict__ absmax,
+                                                                    float* __restrict__ norms, int64_t n, int d) {
+    constexpr int W = 16 / (int)sizeof(T);
+    __shared__ unsigned int wg_most[SCAN_D_MAX + 1];
+    for (int f = threadIdx.x; f <= d; f += SCAN_THREADS) wg_most[f] = 0u;
+    __syncthreads();
+    float most[DM], w_most = 0.0f;
+#pragma unroll
+    for (int f = 0; f < DM; ++f) most[f] = 0.0f;
+    const int64_t thread = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * SCAN_THREADS;
+    for (int64_t g = thread; g < n / W; g += stride) scan_group<T, W, DM>(X_t, w, norms, n, d, g * W, most, w_most);
+    if (thread < n % W) scan_group<T, 1, DM>(X_t, w, norms, n, d, n / W * W + thread, most, w_most);
+    // each exchange halves the features that a lane holds: lane l ends with feature l % DM
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int half = DM / 2; half > 0; half >>= 1)
+#pragma unroll
+        for (int f = 0; f < half; ++f) {
+            const bool high = (lane & half) != 0;
+            const float kept = high ? most[f + half] : most[f], sent = high ? most[f] : most[f + half];
+            most[f] = fmaxf(kept, __shfl_xor(sent, half, 64));
+        }
+#pragma unroll
+    for (int off = DM; off < 64; off <<= 1) most[0] = fmaxf(most[0], __shfl_xor(most[0], off, 64));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) w_most = fmaxf(w_most, __shfl_xor(w_most, off, 64));
+    if (lane < DM && lane < d) atomicMax(&wg_most[lane], __float_as_uint(most[0]));
+    if (lane == 0) atomicMax(&wg_most[d], __float_as_uint(w_most));
+    __syncthreads();
+    for (int f = threadIdx.x; f <= d; f += SCAN_THREADS) atomicMax(&absmax[f], wg_most[f]);
+}
+
 // q[f] for the sums of w * x_f, q[d] for the sums of w: the largest exponents such that
 // n * max|w| * max|x_f| * 2^q < 2^61 and one sample's contribution stays below 2^50.
-__global__ void fixed_point_exponents_kernel(const unsigned int* __restrict__ absmax,
-                                             int* __restrict__ q, int64_t n, int d) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f > d) return;
+__device__ __forceinline__ int fixed_point_exponent(const unsigned int* __restrict__ absmax, int64_t n, int d, int f) {
     const float wmax = __uint_as_float(absmax[d]);
     const float xmax = f < d ? __uint_as_float(absmax[f]) : 1.0f;
     int e = 0;  // log2 upper bound of one contribution
@@ -110,7 +192,19 @@ __global__ void fixed_point_exponents_kernel(const unsigned int* __restrict__ ab
     if (qv > 50 - e) qv = 50 - e;
     if (qv > 100) qv = 100;
     if (qv < -100) qv = -100;
-    q[f] = qv;
+    return qv;
+}
+
+// (the workgroups also clear the sums themselves and `n_words` words for the step)
+__global__ void fixed_point_exponents_kernel(const unsigned int* __restrict__ absmax,
+                                             int* __restrict__ q, int64_t n, int d,
+                                             unsigned long long* __restrict__ sums, int64_t n_sums,
+                                             uint32_t* __restrict__ words, int n_words) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_sums; i += (int64_t)gridDim.x * blockDim.x)
+        sums[i] = 0ull;
+    if (blockIdx.x != 0) return;
+    for (int i = threadIdx.x; i < n_words; i += blockDim.x) words[i] = 0u;
+    for (int f = threadIdx.x; f <= d; f += blockDim.x) q[f] = fixed_point_exponent(absmax, n, d, f);
 }
 
 // ---------------------------------------------------------------------------- fused step
@@ -554,20 +648,46 @@ int32_t launch_mfma(const LloydLayout& L, const void* X_t, const void* w, const 
 
 }  // namespace
 
-bool kmx_mfma_supported(int d, int k) {
-    return d <= 64 && k >= 16 && mfma_lds_bytes(d, k, true) <= 64 * 1024;
+// Exponents from the maxima; clears the sums and `n_words` words at `words` (one launch).
+static int32_t launch_scales(const LloydLayout& L, const unsigned int* absmax, int* q_exp, char* ws, uint32_t* words,
+                             int n_words, int64_t n, int d, hipStream_t stream) {
+    const int64_t sums = (int64_t)(d + 1) * L.k_for_gsum;
+    int64_t grid = kmx_cdiv(sums, 256 * 4);
+    if (grid > 64) grid = 64;
+    hipLaunchKernelGGL(fixed_point_exponents_kernel, dim3((unsigned)(grid < 1 ? 1 : grid)), dim3(256), 0, stream, absmax,
+                       q_exp, n, d, reinterpret_cast<unsigned long long*>(ws + L.off_gsum), sums, words, n_words);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
 }
 
-void kmx_lloyd_absmax_clear(const LloydLayout& L, char* ws, int d, hipStream_t stream) {
-    hipLaunchKernelGGL(absmax_zero_kernel, dim3(1), dim3(256), 0, stream,
-                       reinterpret_cast<unsigned int*>(ws + L.off_scales), d + 1);
+bool kmx_mfma_supported(int d, int k) {
+    return d <= 64 && k >= 16 && mfma_lds_bytes(d, k, true) <= 64 * 1024;
 }
 
 int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void* w, char* ws,
                                int64_t n, int d, int dtype, hipStream_t stream) {
     unsigned int* absmax = reinterpret_cast<unsigned int*>(ws + L.off_scales);
     int* q_exp = reinterpret_cast<int*>(absmax + (d + 1));
-    if (X_t != nullptr) kmx_lloyd_absmax_clear(L, ws, d, stream);
+    // the screened steps compare score gaps with a bound proportional to ||x_i||, taken in one pass with
+    // the maxima (all of them: d <= 64).  Two workgroups per compute unit keep 64 KB of loads in flight there.
+    const bool screened = (L.screen || L.screen64) && X_t != nullptr;
+    uint32_t* bucket = reinterpret_cast<uint32_t*>(ws + L.off_bucket);
+    if (screened) {
+        float* norms = reinterpret_cast<float*>(bucket + 64);
+        const int64_t groups = kmx_cdiv(n, dtype == KMX_F64 ? 2 : 4);
+        int64_t grid = kmx_cdiv(groups, SCAN_THREADS);
+        if (grid > 2 * kmx_num_cus()) grid = 2 * kmx_num_cus();
+#define KMX_SCAN(T, DM)                                                                                       \
+    hipLaunchKernelGGL((scan_samples_kernel<T, DM>), dim3((unsigned)grid), dim3(SCAN_THREADS), 0, stream,     \
+                       (const T*)X_t, (const T*)w, absmax, norms, n, d)
+        if (dtype == KMX_F64) {
+            if (d <= 16) KMX_SCAN(double, 16); else if (d <= 32) KMX_SCAN(double, 32); else KMX_SCAN(double, 64);
+        } else {
+            if (d <= 16) KMX_SCAN(float, 16); else if (d <= 32) KMX_SCAN(float, 32); else KMX_SCAN(float, 64);
+        }
+#undef KMX_SCAN
+        return launch_scales(L, absmax, q_exp, ws, bucket, 64, n, d, stream);
+    }
     // (without X_t: one row, the weights)
     const int rows = X_t != nullptr ? d : 0;
     unsigned int* first = absmax + (d - rows);
@@ -580,16 +700,7 @@ int32_t kmx_lloyd_mfma_prepare(const LloydLayout& L, const void* X_t, const void
     else
         hipLaunchKernelGGL(absmax_rows_kernel<float>, dim3((unsigned)gx, (unsigned)(rows + 1)), dim3(256), 0,
                            stream, (const float*)X_t, (const float*)w, first, n, rows);
-    hipLaunchKernelGGL(fixed_point_exponents_kernel, dim3((unsigned)kmx_cdiv(d + 1, 128)), dim3(128), 0,
-                       stream, absmax, q_exp, n, d);
-    const size_t words = (size_t)(d + 1) * L.k_for_gsum * 2;
-    hipLaunchKernelGGL(absmax_zero_kernel, dim3(1), dim3(1024), 0, stream,
-                       reinterpret_cast<unsigned int*>(ws + L.off_gsum), (int)words);
-    KMX_LAUNCH_CHECK();
-    // the screened step compares score gaps with a bound proportional to ||x_i||
-    if (L.screen || L.screen64)
-        return kmx_sample_norms(X_t, reinterpret_cast<float*>(ws + L.off_bucket + 256), n, d, dtype, stream);
-    return KMX_OK;
+    return launch_scales(L, absmax, q_exp, ws, bucket, 0, n, d, stream);
 }
 
 int32_t kmx_lloyd_iter_mfma_f32(const LloydLayout& L, const void* X_t, const void* w,

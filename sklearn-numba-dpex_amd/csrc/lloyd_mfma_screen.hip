@@ -1867,7 +1867,7 @@ int32_t launch_screen(const void* X_t, const void* w, const void* centroids_t, c
 // Screened fused step.  `uncertain_count`: one word the kernel adds the number of samples it
 // evaluated in fp32 to (zero on entry; the finalisation that follows moves it to the next word
 // and clears it).  `absmax`: bits of max|X_t row| per feature, as kmx_lloyd_mfma_prepare leaves
-// them; `norms`: ||x_i|| per sample (kmx_sample_norms).
+// them; `norms`: ||x_i|| per sample (likewise).
 // `tail` (may be null): what the finalisation of the iteration needs; the workgroup of the step
 // that gets done last then runs it, and no finalisation launch must follow.
 int32_t kmx_lloyd_step_mfma_screen(const void* X_t, const void* w, const void* centroids_t,
@@ -1948,35 +1948,6 @@ int32_t kmx_screen_scores_impl(const float* X_t, const float* centroids_t, float
         default: KMX_DIAG_CASE(16); break;
     }
 #undef KMX_DIAG_CASE
-    KMX_LAUNCH_CHECK();
-    return KMX_OK;
-}
-
-namespace {
-// ||x_i|| in fp32, features in order; one thread per sample (consecutive threads, consecutive
-// addresses in every feature row).
-// (fp64 inputs: rounded to fp32 first, as the screen sees them)
-template <typename TX>
-__global__ __launch_bounds__(256) void sample_norms_kernel(const TX* __restrict__ X_t,
-                                                           float* __restrict__ norms, int64_t n, int d) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float sq = 0.0f;
-#pragma unroll 8
-    for (int f = 0; f < d; ++f) {
-        const float v = (float)X_t[(size_t)f * n + i];
-        sq = fmaf(v, v, sq);
-    }
-    norms[i] = sqrtf(sq);
-}
-}  // namespace
-
-int32_t kmx_sample_norms(const void* X_t, float* norms, int64_t n, int d, int dtype, hipStream_t stream) {
-    const dim3 grid((unsigned)kmx_cdiv(n, 256));
-    if (dtype == KMX_F64)
-        hipLaunchKernelGGL(sample_norms_kernel<double>, grid, dim3(256), 0, stream, (const double*)X_t, norms, n, d);
-    else
-        hipLaunchKernelGGL(sample_norms_kernel<float>, grid, dim3(256), 0, stream, (const float*)X_t, norms, n, d);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import kmeans as ok
-from tests._parity import assert_centers_close, assert_labels_match
+from tests._parity import RTOL, assert_centers_close, assert_labels_match
 
 pytestmark = pytest.mark.gpu
 
@@ -904,3 +904,35 @@ def test_fp64_certificate_passes_no_label_that_fp64_would_not_give(cuda, d, k, s
     bad = np.flatnonzero(got != ref)
     gap = (dist[bad, got[bad]] - dist[bad, ref[bad]]) / dist[bad].max(axis=1)
     assert np.all(gap <= 1e-14), f"assign: {bad.size} labels differ, worst relative gap {gap.max():.3e}"
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("d", [1, 8, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n", [40, 1_025, 4_099, 530_000])
+def test_scales_see_every_sample_feature_and_weight(cuda, n, d, dtype):
+    """One value, then one weight, 2^14 times the others, at the first and last places of the vectors, of their
+    remainder and of the features: contributions are scaled to stay below 2^50 (and n of them below 2^61), and a
+    maximum that missed it would let it pass 2^51, where rounding to fixed point breaks."""
+    rng = np.random.default_rng(n + d)
+    k = 20
+    base = rng.uniform(1.0, 2.0, (n, d)).astype(dtype)
+    weights = rng.uniform(1.0, 2.0, n).astype(dtype)
+    rows = rng.choice(n, k, replace=False)
+    places = {(0, 0), (n - 1, d - 1), (n - 1 - n % 4, d // 2), (n // 2, min(d - 1, 16))}
+    for i, f in sorted(places) if n < 10_000 else [(n - 1, d - 1)]:
+        for heavy in (False, True):
+            X, w = base.copy(), weights.copy()
+            (w if heavy else X)[i if heavy else (i, f)] = 2.0 ** 14
+            init = X[rows].copy()  # (samples: no cluster is empty)
+            labels, c_out, sizes, status, variant, _ = _one_iteration(X, w, init, cuda)
+            assert variant in (61, 71) and status.n_empty == 0
+            # (the sums of the labels the step gave: with one feature within [1, 2) and a centre so close to the next
+            # the fp32 scores, up to 4 with 2^-24 of it rounded off per operation, decide no tie closer than 1e-6)
+            assert labels.min() >= 0 and labels.max() < k
+            sums, ref_sizes = ok.weighted_sums(X.astype(np.float64), w.astype(np.float64), labels, k)
+            # weights are at least 1, so half a unit of the fixed point per sample is at most half a unit of the mean
+            bits = np.ceil(np.log2(np.abs(X).max(axis=0)) + 1e-9) + np.ceil(np.log2(w.max()) + 1e-9)
+            unit = 2.0 ** -np.minimum(50 - bits, 61 - bits - np.ceil(np.log2(n)))
+            exact = sums / ref_sizes[:, None]
+            bound = RTOL[X.dtype] * np.abs(exact).max(axis=1, keepdims=True) + unit * (1 + np.abs(exact))
+            assert (np.abs(c_out - exact) <= bound).all()
