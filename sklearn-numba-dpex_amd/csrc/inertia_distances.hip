@@ -37,10 +37,10 @@ __global__ __launch_bounds__(256) void per_sample_inertia_kernel(
     const int64_t stride = (int64_t)gridDim.x * 256;
     double total = 0.0;
     (void)total;
-    // Rows in flight: eight where few workgroups wait for memory (30 002 x 500 fp64, the values of a relocation:
-    // 161 us with four, 139 with eight; 206 with a branch per row, 144 as single loads), four for the sum over
-    // large arrays (1 000 003 x 100 fp64: 145 us, 150 with eight).
-    constexpr int WALK = SUM ? 4 : 8;
+    // Rows in flight: eight where few workgroups wait for memory, the values of a relocation among many features
+    // (30 002 x 500 fp64: 161 us with four, 139 with eight; 206 with a branch per row, 144 as single loads); else
+    // four (1 000 003 x 100 fp64, sum: 145 us, 150 with eight; 2e6 x 32 fp64, values: 93 and 99).
+    constexpr int WALK = SUM || LDS_CENTROIDS ? 4 : 8;
     for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < n_groups; g += stride) {
         const int64_t i0 = g * 4;
         const bool full = i0 + 4 <= n;
