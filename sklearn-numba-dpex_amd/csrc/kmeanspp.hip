@@ -703,6 +703,8 @@ __device__ __forceinline__ int64_t block_min_i64(int64_t v, int64_t* scratch) {
 //              centre slot and does not sample.
 //   do_sample: candidate t = first j with scan(closest)_j >= uniforms[t] * total, and the
 //              candidate's feature row for the step kernel.
+//   merge:     0, or how many of these block sums make one of `merged`, which the last workgroup then writes
+//              row by row (the end of a run with one launch per centre: the sums that calls step by step read).
 // Thread i owns the block sums [i * P, (i + 1) * P); with P <= KPP_OWN they are read once and
 // stay in registers for the row totals, the coarse scan and the search.
 // Bound by the latency of its chain of loads.  The block sums lie row by row, so that neighbouring
@@ -717,7 +719,7 @@ __global__ __launch_bounds__(256) void kpp_select_sample_kernel(
     int32_t* __restrict__ center_indices, const T* __restrict__ rows,
     const double* __restrict__ block_pot, double* __restrict__ potentials,
     KppHeader* __restrict__ header, T* __restrict__ cand_rows, int64_t n, int64_t n_blocks, int chunk,
-    int d, int k, int n_trials, int center_slot, int do_select, int do_sample) {
+    int d, int k, int n_trials, int center_slot, int do_select, int do_sample, double* __restrict__ merged, int merge) {
     __shared__ double wave_tot[4];
     __shared__ double wave_pot[4][TN];
     __shared__ int64_t iscratch[4];
@@ -800,6 +802,15 @@ __global__ __launch_bounds__(256) void kpp_select_sample_kernel(
                 center_indices[center_slot] = chosen;
                 header->best_row = best;
                 header->total = best_pot;
+            }
+            if (merge > 0) {
+                const int n_merged = (int)((n_blocks + merge - 1) / merge);
+                for (int i = threadIdx.x; i < n_trials * n_merged; i += 256) {
+                    const int t = i / n_merged, first = (i - t * n_merged) * merge;
+                    double sum = 0.0;
+                    for (int b = first; b < first + merge && b < n_blocks; ++b) sum += block_pot[(size_t)t * n_blocks + b];
+                    merged[i] = sum;
+                }
             }
             return;
         }
@@ -1403,7 +1414,7 @@ void launch_select_sample(const void* X_t, const double* uniforms, const int32_t
                           int32_t* cand_next, int32_t* cand_out, void* centers_t, int32_t* idx,
                           const KppPtrs& p, const KppLayout& L, int64_t n, int d, int k,
                           int n_trials, int slot, int do_select, int do_sample, hipStream_t s,
-                          bool literal = false) {
+                          bool literal = false, double* merged = nullptr, int merge = 0) {
     if (literal) {
         // the selection alone (potentials compared in T), then the serial walk of one workgroup
         if (do_select)
@@ -1422,7 +1433,7 @@ void launch_select_sample(const void* X_t, const double* uniforms, const int32_t
     hipLaunchKernelGGL((kpp_select_sample_kernel<T, __VA_ARGS__>), dim3(grid), dim3(256), 0, s,    \
                        (const T*)X_t, uniforms, cand_prev, cand_next, cand_out, (T*)centers_t, idx, \
                        (const T*)p.rows, p.block_pot, p.potentials, p.header, (T*)p.cand_rows, n,   \
-                       L.n_blocks, L.chunk, d, k, n_trials, slot, do_select, do_sample)
+                       L.n_blocks, L.chunk, d, k, n_trials, slot, do_select, do_sample, merged, merge)
     if (n_trials <= 8) {
         // (more than four block sums per thread: eight in registers rather than re-read)
         if (L.n_blocks > 4 * 256 && L.n_blocks <= 8 * 256) KMX_KPP_SELECT(8, 8);
@@ -1471,8 +1482,9 @@ int32_t run_joint(const void* X_t, const void* w, const double* uniforms, int32_
         KppLayout geometry = L;
         geometry.n_blocks = n_blocks;
         geometry.chunk = 256 * L.joint;
+        static_assert(JOINT_D <= SPLIT_MIN_D, "the block sums of the layout are those of CHUNK samples");
         launch_select_sample<T>(X_t, nullptr, p.cand + ((k - 1) & 1) * TN_MAX, nullptr, nullptr, centers_t, idx, last,
-                                geometry, n, d, k, n_trials, k - 1, 1, 0, s);
+                                geometry, n, d, k, n_trials, k - 1, 1, 0, s, false, p.block_pot, CHUNK / geometry.chunk);
         KMX_LAUNCH_CHECK();
     }
     return KMX_OK;

@@ -193,6 +193,40 @@ def test_step_kernels_through_c_abi(cuda, dtype, shape):
         closest = got_rows[best_row].copy()
 
 
+# 1, 2 and 4 samples per thread with one launch per centre, ragged last blocks; two launches per centre
+@pytest.mark.parametrize("n", [700, 10_007, 70_001, 140_003, 262_145])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_calls_step_by_step_go_on_from_a_whole_run(cuda, dtype, n):
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib, ptr
+
+    rng = np.random.default_rng(n)
+    d, k, tn, dc = 3, 4, 5, _capi.dtype_code(dtype)
+    X = rng.normal(size=(n, d)).astype(dtype)
+    X_t = _dev(X.T, cuda)
+    w_d = torch.ones(n, dtype=X_t.dtype, device=cuda)
+    centers_t, indices = torch.zeros((d, k), dtype=X_t.dtype, device=cuda), torch.zeros(k, dtype=torch.int32, device=cuda)
+    cand = torch.zeros(tn, dtype=torch.int32, device=cuda)
+    ws_bytes = lib.kmx_kpp_workspace_bytes(n, d, k, tn, dc)
+    ws = torch.full((ws_bytes,), 0x55, dtype=torch.uint8, device=cuda)
+    shape, u = (n, d, k, tn, dc, 0, _capi.current_stream()), rng.random((k, tn))
+    _capi.check(lib.kmx_kpp_run(ptr(X_t), ptr(w_d), ptr(_dev(u[:-1], cuda)), n // 3, ptr(centers_t), ptr(indices), ptr(ws),
+                                ws_bytes, *shape), "kpp_run")
+
+    def view(at, count, of):
+        off = at - ws.data_ptr()
+        return ws[off: off + count * np.dtype(of).itemsize].cpu().numpy().view(of)
+
+    pots = view(lib.kmx_kpp_potentials_ptr(ptr(ws), n, d, k, tn, dc), tn, np.float64)
+    rows = view(lib.kmx_kpp_closest_ptr(ptr(ws), n, d, k, tn, dc), tn * n, dtype).reshape(tn, n)
+    np.testing.assert_allclose(pots, rows.sum(axis=1, dtype=np.float64), rtol=1e-12)
+    _capi.check(lib.kmx_kpp_sample_candidates(ptr(X_t), ptr(_dev(u[-1], cuda)), ptr(cand), ptr(ws), ws_bytes, *shape), "sample")
+    closest = rows[int(np.argmin(pots))]
+    np.testing.assert_array_equal(cand.cpu().numpy(), [ok._sample_exact(closest, uu) for uu in u[-1]])
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_known_answer_through_the_engine(cuda, dtype):
     """reference kmeans/tests/test_kmeans.py:251-325: mean score over seeds 0..9 of the
