@@ -73,7 +73,7 @@ def room_for(n_bytes, device):
 def host_scalar(dtype):
     """One value in pinned host memory for a kernel to write: `read_host_scalar` waits for the stream and
     reads it, where a value in device memory takes a copy's launch and its wait as well (9 us a call)."""
-    return torch.empty(1, dtype=dtype, pin_memory=True)
+    return torch.empty(1, dtype=dtype, device="cpu", pin_memory=True)  # (whatever torch's default device is)
 
 
 def read_host_scalar(out, device):
@@ -105,7 +105,7 @@ _stage_lock = threading.Lock()   # one upload at a time: the two buffers and the
 def _staging():
     global _stage
     if _stage is None:
-        _stage = [(torch.empty(_STAGE_BYTES, dtype=torch.uint8, pin_memory=True), torch.cuda.Event())
+        _stage = [(torch.empty(_STAGE_BYTES, dtype=torch.uint8, device="cpu", pin_memory=True), torch.cuda.Event())
                   for _ in range(2)]
     return _stage
 

@@ -374,6 +374,29 @@ def test_dlpack_inputs_give_the_same_fit(cuda, dtype):
     assert a.n_iter_ == b.n_iter_
 
 
+# a program whose default device is the GPU: small and staged (over 4 MiB) host arrays, device arrays
+@pytest.mark.parametrize("n", [200, 200_000])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_calls_under_a_default_device(cuda, dtype, n, monkeypatch):
+    import torch
+
+    from sklearn_numba_dpex_amd.common import _buffers
+    from sklearn_numba_dpex_amd.kmeans.estimator import KMeans
+
+    X = np.random.default_rng(7).standard_normal((n, 6)).astype(dtype)
+    expected = KMeans(n_clusters=4, n_init=1, random_state=0, max_iter=3).fit(X)
+    monkeypatch.setattr(_buffers, "_stage", None)
+    for data in (X, _as_cuda(X, dtype)):
+        with torch.device(cuda):
+            model = KMeans(n_clusters=4, n_init=1, random_state=0, max_iter=3).fit(data)
+            labels, distances, score = model.predict(data), model.transform(data), model.score(data)
+        # (sums within a workgroup are added in no fixed order)
+        assert_allclose(_np(model.cluster_centers_), _np(expected.cluster_centers_), rtol=1e-5, atol=1e-6)
+        assert_array_equal(_np(labels), _np(expected.predict(X)))
+        assert_allclose(_np(distances), _np(expected.transform(X)), rtol=1e-5)
+        assert_allclose(score, expected.score(X), rtol=1e-5)
+
+
 def test_numpy_inputs_are_uploaded_through_pinned_staging(cuda):
     """Large numpy inputs travel through two pinned staging buffers (several chunks, a ragged
     last one); the device copy is bit-identical to the host array, for every dtype and for
