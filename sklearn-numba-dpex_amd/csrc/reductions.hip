@@ -753,11 +753,12 @@ int32_t kmx_all_finite(const void* data, int64_t n_items, int32_t* not_finite, i
     return KMX_OK;
 }
 
+// The partial sums of the rows (those of the weights are one row's) or of the centring pass, one after the other:
+// not the column sums' scratch of kmx_sum_workspace_bytes, 512 bytes a column.
 size_t kmx_center_workspace_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0) return 0;
-    const size_t a = kmx_sum_workspace_bytes(rows, cols);
-    const size_t b = kmx_align256((size_t)rows * center_blocks_per_row(rows, cols) * sizeof(double));
-    return a > b ? a : b;
+    const int64_t a = sum_blocks_per_row(cols), b = center_blocks_per_row(rows, cols);
+    return kmx_align256((size_t)rows * (size_t)(a > b ? a : b) * sizeof(double));
 }
 
 int32_t kmx_center_rows(const void* X_t, void* dst, const void* sample_weight, void* mean, void* stats, void* workspace,

@@ -101,6 +101,10 @@ def test_workspace_queries():
     assert lib.kmx_topk_rows_workspace_bytes(7, 1000, 10, 0) == 7 * one_row
     assert lib.kmx_topk_rows_workspace_bytes(7, 1000, 10, 5) == 0
     assert lib.kmx_sum_workspace_bytes(7, 1_000_000) >= 7 * 256 * 8
+    # the data pass of a fit: partial sums only, of at most 256 workgroups a row and about 16 384 in all
+    assert lib.kmx_center_workspace_bytes(0, 5) == 0 and lib.kmx_center_workspace_bytes(1, 1) == 256
+    for rows, cols in [(14, 5_000_000), (1, 200_000_000), (65_535, 3), (800, 1_000_000), (64, 300_002)]:
+        assert lib.kmx_center_workspace_bytes(rows, cols) <= 8 * max(256 * rows, 16_384 + rows) + 256, (rows, cols)
 
 
 def test_kernel_variant_selection():

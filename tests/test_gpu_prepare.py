@@ -36,6 +36,27 @@ def test_centring_variance_and_weights(cuda, n, d, dtype, copy_x):
     assert uniform == (n == 1)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (2, 70_001), (14, 1_000_003), (900, 20_000), (1_500, 40)])
+def test_centring_stays_within_its_workspace(cuda, rows, cols):
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib, ptr
+
+    X_t = torch.randn((rows, cols), device=cuda, dtype=torch.float64) + 3
+    w, mean, stats = torch.ones(cols, device=cuda, dtype=X_t.dtype), X_t.new_empty(rows), X_t.new_empty(4)
+    out, size = torch.empty_like(X_t), lib.kmx_center_workspace_bytes(rows, cols)
+    ws = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device=cuda)
+    args = (rows, cols, _capi.KMX_F64, _capi.current_stream())
+    assert lib.kmx_center_rows(ptr(X_t), ptr(out), ptr(w), ptr(mean), ptr(stats), ptr(ws), size - 1, *args) != 0
+    _capi.check(lib.kmx_center_rows(ptr(X_t), ptr(out), ptr(w), ptr(mean), ptr(stats), ptr(ws), size, *args), "kmx_center_rows")
+    assert bool((ws[size:] == 0x5A).all())
+    torch.testing.assert_close(mean, X_t.mean(1), rtol=1e-12, atol=1e-13)
+    torch.testing.assert_close(out, X_t - mean[:, None], rtol=0, atol=0)
+    assert float(stats[2]) == cols and float(stats[3]) == 1
+    torch.testing.assert_close(stats[1], (out * out).sum(), rtol=1e-11, atol=1e-300)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_means_of_zero_leave_the_data_alone(cuda, dtype):
     import torch
