@@ -13,7 +13,7 @@ import torch
 from .. import _capi
 from .._capi import LloydStatus, check, lib, ptr
 from ..common._buffers import contiguous, dcode, host_scalar, read_host_scalar, require_cuda, room_for, workspace
-from ..common.kernels import broadcast_rows, transposed_copy
+from ..common.kernels import broadcast_rows, divide_by, transposed_copy
 from ..common.random import create_xoroshiro128pp_states, get_random_raw, raw_to_uniform
 from ..common.reductions import sum_reduction
 from ..common.topk import topk_idx
@@ -253,6 +253,19 @@ def _relocate_empty_clusters(
                                           _capi.current_stream()), "kmx_relocate_empty_clusters")
 
 
+def _room_for_centred(X_t):
+    """Memory for a centred copy of X_t.  Where there is none, and none is wanted because every mean is zero,
+    X_t itself: nothing is written then."""
+    try:
+        return torch.empty_like(X_t)
+    except torch.OutOfMemoryError:
+        X_mean = sum_reduction(X_t, axis=1)
+        divide_by(X_mean, X_t.shape[1])
+        if float(sum_reduction(X_mean, square=True)[0]) != 0.0:
+            raise
+        return X_t
+
+
 def prepare_data_for_lloyd(X_t, init, tol, sample_weight, copy_x):
     """Centres X (and an array `init`) on the feature means, scales `tol` by the mean feature
     variance and tests whether the weights are uniform (reference: kmeans/drivers.py:436-545).
@@ -266,7 +279,7 @@ def prepare_data_for_lloyd(X_t, init, tol, sample_weight, copy_x):
     X_t = contiguous(X_t)
     fused = sample_weight.dtype == X_t.dtype and tuple(sample_weight.shape) == (n,)
     weights = contiguous(sample_weight) if fused else X_t  # (any n values)
-    centred = torch.empty_like(X_t) if copy_x else X_t
+    centred = _room_for_centred(X_t) if copy_x else X_t
     X_mean = torch.empty(d, dtype=X_t.dtype, device=X_t.device)
     stats = torch.empty(4, dtype=X_t.dtype, device=X_t.device)
     ws_bytes = lib.kmx_center_workspace_bytes(d, n)

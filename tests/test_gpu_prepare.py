@@ -57,6 +57,26 @@ def test_centring_stays_within_its_workspace(cuda, rows, cols):
     torch.testing.assert_close(stats[1], (out * out).sum(), rtol=1e-11, atol=1e-300)
 
 
+# memory for the centred copy is asked for ahead of the means; means of zero do without it
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_means_of_zero_need_no_memory_for_a_copy(cuda, dtype, monkeypatch):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    X_t = torch.as_tensor(np.tile(np.array([[3, -3], [1, -1]], dtype=dtype), (1, 100)), device=cuda)
+    before, ones = X_t.clone(), torch.ones(200, dtype=X_t.dtype, device=cuda)
+
+    def none_left(*args, **kwargs):
+        raise torch.OutOfMemoryError("no memory for a copy")
+
+    monkeypatch.setattr(torch, "empty_like", none_left)
+    out, mean, _, tol, uniform = drivers.prepare_data_for_lloyd(X_t, "random", 1.0, ones, True)
+    assert mean is None and out.data_ptr() == X_t.data_ptr() and torch.equal(X_t, before) and tol == 5.0 and uniform
+    with pytest.raises(torch.OutOfMemoryError):
+        drivers.prepare_data_for_lloyd(X_t + 1, "random", 1.0, ones, True)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_means_of_zero_leave_the_data_alone(cuda, dtype):
     import torch
