@@ -36,7 +36,11 @@ HIPCC_FLAGS = [
 # Per source file.  lloyd_mfma_screen.hip: atomics stay as written - the rewrite of an atomic on a
 # uniform address into a wave-wide reduction reads the returned value at once, and the kernel
 # wants the answer of its chunk counter a tile later, not on the spot.
+# inertia_distances.hip: loops begin on a cache line.  With one workgroup per compute unit the fp32
+# distances took up to 4 % longer or not as their inner loop happened to fall (20 000 x 1 500 by 64,
+# rows: 259 us aligned, 269 after an unrelated change before the loop).
 EXTRA_FLAGS = {
+    "inertia_distances.hip": ["-falign-loops=64"],
     "lloyd_mfma_screen.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
 }
 

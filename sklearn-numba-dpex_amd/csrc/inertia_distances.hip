@@ -444,12 +444,15 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
 
 // ---------------------------------------------------------------------------- fp32 distances
 //
-// |x - c|^2 = |x - m|^2 + |c - m|^2 - 2 <x - m, c - m> with every term in fp64 (m: centroid 0, as far as DM_M
-// features; x and c are fp32, so the differences and products carry 53 bits), the inner products on the fp64 matrix cores.
+// |x - c|^2 = |x - m|^2 + |c - m|^2 - 2 <x - m, c - m> with every term in fp64 (x and c are fp32, so the differences
+// and products carry 53 bits), the inner products on the fp64 matrix cores.  m lies among the centroids, as far as
+// DM_M features: coordinate by coordinate the median of five of them, which an outlier among them does not move.
 // Where the result is less than about d 2^-27 of what it is the difference of, rounding would show in
-// fp32: those few pairs are redone in the difference form, feature by feature in fp32, as are pairs that
-// involve values beyond 2^62, NaN or infinities.  What is left is one rounding to fp32 and the square root:
-// nearer the exact distance than d rounded additions.
+// fp32: those pairs are redone in the difference form, feature by feature in fp32, as are pairs that
+// involve values beyond 2^62 or infinities.  They are few, and their lanes redo them; where many of a wave's are
+// (two groups a thousand times as far apart as they are wide, an offset beyond DM_M features) the wave does
+// (dm_redo_wave), and a call takes two to four times as long.  What is left is one rounding to fp32 and the
+// square root: nearer the exact distance than d rounded additions.
 // Why: the difference form costs two vector instructions per pair and feature (98 us for 300 007 x 100 x 64
 // at the chip's rate without packed arithmetic), the fp64 matrix cores take 49 us for the same.  And the
 // rows of X are read where they are: a transposed copy of X for this one pass over it took 59 us there.
@@ -464,8 +467,133 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
 // transposed copy and the differences it replaces / this: 300 007 x 100, 64 clusters 178 / 116; 1e5 x 784,
 // 300 clusters 1 340 / 1 065; 1e6 x 20, 16 clusters 90 / 60.  Reading the next step's operands ahead of the
 // matrix instructions: 292 -> 321 us at 1e6 x 96, 64 clusters (registers), not done.
-constexpr int DM_S = 128, DM_K = 32, DM_RP = DM_K + 2, DM_CP = DM_S + 32, DM_M = 1024;
+constexpr int DM_S = 128, DM_K = 32, DM_RP = DM_K + 2, DM_CP = DM_S + 32, DM_M = 1792;
+// pairs of a wave, per centroid tile, beyond which it redoes them all at once, and features at a time then (one after the
+// other: about 2.5 us a pair of 100 features; at once: 18 us for one tile of centroids, 65 for four)
+constexpr int DM_REDO = 5, DM_R = 8;
 typedef double dm_v4d __attribute__((ext_vector_type(4)));
+
+// The median of five values, 0 where it is not finite.
+__device__ __forceinline__ double dm_middle(const float (&v)[5]) {
+    const float low = fmaxf(fminf(v[0], v[1]), fminf(v[2], v[3]));
+    const float high = fminf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+    // (of the four, low and high are the middle ones, in either order)
+    const float middle = __builtin_amdgcn_fmed3f(v[4], low, high);
+    return kmx_not_finite(middle) ? 0.0 : (double)middle;
+}
+
+// The pairs of a wave that `redo` names (bit 8 tile + 2 r + b of lane (g, j): centroid c0 + 16 tile + g + 4 r, sample
+// 2 j + b of the wave) in the difference form, features in order.  A few of them: one after the other, a feature per lane,
+// 256 features' loads in flight; the lanes' differences are then added up in their order.
+template <bool ROWS>
+__device__ __forceinline__ void dm_redo_pairs(const float* __restrict__ X, const float* __restrict__ centroids_t,
+                                              float* __restrict__ distances_t, unsigned int redo, int64_t i0, int here,
+                                              int c0, int64_t n, int d, int k, int lane, int wave) {
+    asm volatile("" : "+v"(lane));  // (what follows from it is made here, not kept over the tiles)
+    for (unsigned long long lanes = __ballot(redo != 0u); lanes != 0ull; lanes = __ballot(redo != 0u)) {
+        const int from = __builtin_ctzll(lanes), u = __builtin_ctz((unsigned int)__builtin_amdgcn_readlane((int)redo, from));
+        if (lane == from) redo &= redo - 1u;
+        const int c = c0 + 16 * (u >> 3) + (from >> 4) + 4 * ((u >> 1) & 3), si = 32 * wave + 2 * (from & 15) + (u & 1);
+        if (c >= k || si >= here) continue;
+        float sum = 0.0f;
+        for (int f0 = 0; f0 < d; f0 += 256) {
+            float diff[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int fi = f0 + 64 * q + lane, f = fi < d ? fi : d - 1;
+                diff[q] = 0.0f;
+                if (f0 + 64 * q < d) {
+                    const float v = centroids_t[(size_t)f * k + c] - (ROWS ? X[(size_t)(i0 + si) * d + f] : X[(size_t)f * n + i0 + si]);
+                    diff[q] = fi < d ? v : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                for (int l = 0; l < 64 && f0 + 64 * q + l < d; l += 16)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(diff[q]), l + e));
+                        sum = fmaf(v, v, sum);
+                    }
+        }
+        if (lane == 0) distances_t[(size_t)c * n + i0 + si] = dist_sqrt(sum);
+    }
+}
+
+// Many of them: all the wave's pairs, DM_R features at a time through `own`, the part of xs that only this wave reads (its
+// samples'; rows of 32 floats): [feature][sample], then [feature][g][tile][r] of the centroids.  Bound by its loads'
+// latency.  300 007 x 100, 64 clusters in two groups (half of all pairs): 315 us, 1 630 with each lane on its own pairs;
+// 121 with none to redo.
+template <int NCT, bool ROWS>
+__device__ __forceinline__ void dm_redo_wave(const float* __restrict__ X, const float* __restrict__ centroids_t,
+                                             float* __restrict__ distances_t, float* own, unsigned int redo, int64_t i0,
+                                             int here, int c0, int64_t n, int d, int k, int lane, int wave) {
+    asm volatile("" : "+v"(lane));  // (what follows from it is made here, not kept over the tiles)
+    constexpr int PITCH = ROWS ? 36 : DM_CP;
+    constexpr int NA = NCT > 2 ? 2 : NCT, CW = 16 * NA;  // NA tiles of centroids at a time (registers)
+    static_assert(ROWS ? PITCH * (DM_R + DM_R * CW / 32) <= 32 * DM_RP : DM_R + DM_R * CW / 32 <= DM_K, "fits xs");
+    const int s0 = 32 * wave, g = lane >> 4, j = lane & 15;
+    for (int a0 = 0; a0 < NCT; a0 += NA) {
+        const int c00 = c0 + 16 * a0;
+        float sum[NA][4][2];
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[a][r][0] = sum[a][r][1] = 0.0f;
+        for (int f0 = 0; f0 < d; f0 += DM_R) {
+            float xv[DM_R / 2], cv[DM_R * CW / 64];
+#pragma unroll
+            for (int p = 0; p < DM_R / 2; ++p) {
+                const int u = lane + 64 * p, fi = f0 + (ROWS ? u % DM_R : u / 32), si = s0 + (ROWS ? u / DM_R : u % 32);
+                const int s = si < here ? si : here - 1, f = fi < d ? fi : d - 1;
+                xv[p] = ROWS ? X[(size_t)(i0 + s) * d + f] : X[(size_t)f * n + i0 + s];
+            }
+#pragma unroll
+            for (int p = 0; p < DM_R * CW / 64; ++p) {
+                const int u = lane + 64 * p, fi = f0 + u / CW, c = c00 + u % CW;
+                cv[p] = centroids_t[(size_t)(fi < d ? fi : d - 1) * k + (c < k ? c : k - 1)];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of the previous stage are over
+#pragma unroll
+            for (int p = 0; p < DM_R / 2; ++p) {
+                const int u = lane + 64 * p;
+                own[(ROWS ? u % DM_R : u / 32) * PITCH + (ROWS ? u / DM_R : u % 32)] = xv[p];
+            }
+#pragma unroll
+            for (int p = 0; p < DM_R * CW / 64; ++p) {
+                const int u = lane + 64 * p, c = u % CW, at = u / CW * CW + (c & 3) * 4 * NA + (c >> 4) * 4 + (c >> 2 & 3);
+                own[(DM_R + at / 32) * PITCH + at % 32] = cv[p];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const int w = d - f0 < DM_R ? d - f0 : DM_R;
+            for (int f = 0; f < w; ++f) {
+                const float2 x = *reinterpret_cast<const float2*>(own + f * PITCH + 2 * j);
+#pragma unroll
+                for (int a = 0; a < NA; ++a) {
+                    float c[4];
+                    const int at = f * CW + g * 4 * NA + 4 * a;
+                    lds_load4<float>(own + (DM_R + at / 32) * PITCH + at % 32, c);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float d0 = c[r] - x.x, d1 = c[r] - x.y;
+                        sum[a][r][0] = fmaf(d0, d0, sum[a][r][0]);
+                        sum[a][r][1] = fmaf(d1, d1, sum[a][r][1]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const int c = c00 + 16 * a + g + 4 * r, si = s0 + 2 * j + b;
+                    if ((redo >> (8 * (a0 + a) + 2 * r + b) & 1u) && c < k && si < here)
+                        distances_t[(size_t)c * n + i0 + si] = dist_sqrt(sum[a][r][b]);
+                }
+    }
+}
 
 template <int NCT, bool ROWS>
 __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
@@ -519,19 +647,21 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
                     }
                 }
             }
+        } else if (whole) {
+#pragma unroll
+            for (int p = 0; p < PX / 4; ++p) {
+                const int f = (threadIdx.x >> 5) + 8 * p, s = 4 * (threadIdx.x & 31);
+                const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(X + (size_t)(f0 + f) * n + i0 + s);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rx[4 * p + e] = v[e];
+            }
         } else {
 #pragma unroll
             for (int p = 0; p < PX / 4; ++p) {
                 const int f = (threadIdx.x >> 5) + 8 * p, s = 4 * (threadIdx.x & 31);
-                if (whole) {
-                    const auto v = *reinterpret_cast<const KmxVec<float, 4>::type*>(X + (size_t)(f0 + f) * n + i0 + s);
+                const float* __restrict__ row = X + (size_t)(f < w ? f0 + f : d - 1) * n + i0;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) rx[4 * p + e] = v[e];
-                } else {
-                    const float* __restrict__ row = X + (size_t)(f < w ? f0 + f : d - 1) * n + i0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) rx[4 * p + e] = row[s + e < here ? s + e : here - 1];
-                }
+                for (int e = 0; e < 4; ++e) rx[4 * p + e] = row[s + e < here ? s + e : here - 1];
             }
         }
         // fragment value (step, tile, lane): feature f0 + 4 step + lane / 16 of centroid c0 + 16 tile + lane % 16
@@ -608,8 +738,37 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
     bool first = true;
     load(tile * DM_S, 0, true);
     // (zero for the features past d, and for the stages past DM_M)
-    for (int f = threadIdx.x; f < DM_M + DM_K; f += 256)
-        if (f < (d + DM_K - 1) / DM_K * DM_K || f >= DM_M) ms[f] = f < d && f < DM_M ? (double)centroids_t[(size_t)f * k] : 0.0;
+    {
+        // m: the median of the last five centroids (kmeans++ takes outliers early; in a row they are two loads)
+        constexpr int P = DM_M / 256;
+        const int most = d < DM_M ? d : DM_M;
+        float v[P][5];
+        if (k >= 5) {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                if (256 * p >= most) break;  // (uniform)
+                const int f = threadIdx.x + 256 * p;
+                const float* __restrict__ row = centroids_t + (size_t)(f < most ? f : most - 1) * k + k - 5;
+                const auto q = *reinterpret_cast<const KmxVec<float, 4>::type*>(row);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[p][i] = q[i];
+                v[p][4] = row[4];
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int f = threadIdx.x + 256 * p;
+#pragma unroll
+                for (int i = 0; i < 5; ++i) v[p][i] = centroids_t[(size_t)(f < most ? f : most - 1) * k + (i < k ? i : k - 1)];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const int f = threadIdx.x + 256 * p;
+            if (256 * p < most + DM_K) ms[f] = f < most ? dm_middle(v[p]) : 0.0;
+        }
+        if (threadIdx.x < DM_K) ms[DM_M + threadIdx.x] = 0.0;
+    }
     for (; tile < n_tiles; tile += s_step) {
         const int64_t i0 = tile * DM_S, i_next = (tile + s_step) * DM_S;
         dm_v4d acc[NCT][2];
@@ -734,22 +893,11 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
                     }
                 }
             }
-            while (redo != 0u) {
-                const int u = __builtin_ctz(redo);
-                redo &= redo - 1u;
-                const int c = c0 + 16 * (u >> 3) + g + 4 * ((u >> 1) & 3), si = sl + (u & 1);
-                if (c >= k || si >= here) continue;
-                float* __restrict__ dst = distances_t + (size_t)c * n + i0 + si;
-                const float* __restrict__ x = ROWS ? X + (size_t)(i0 + si) * d : X + i0 + si;
-                const size_t step = ROWS ? 1 : (size_t)n;
-                float sum = 0.0f;
-#pragma unroll 4
-                for (int f = 0; f < d; ++f) {
-                    const float diff = centroids_t[(size_t)f * k + c] - x[f * step];
-                    sum = fmaf(diff, diff, sum);
-                }
-                *dst = dist_sqrt(sum);
-            }
+            if (kmx_wave_sum<int>(__popc(redo)) > DM_REDO * NCT)
+                dm_redo_wave<NCT, ROWS>(X, centroids_t, distances_t, xs + 32 * wave * (ROWS ? DM_RP : 1), redo, i0, here, c0,
+                                        n, d, k, lane, wave);
+            else
+                dm_redo_pairs<ROWS>(X, centroids_t, distances_t, redo, i0, here, c0, n, d, k, lane, wave);
         }
     }
     if (ROWS && bad) *not_finite = 1;

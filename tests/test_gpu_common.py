@@ -370,7 +370,7 @@ def test_distances_and_inertia_kernels(cuda, shape):
 @pytest.mark.parametrize("n,d,k", [(1, 1, 1), (5, 1, 5), (130, 2, 17), (1023, 5, 600), (257, 7, 9), (127, 8, 64), (128, 9, 16),
                                    (129, 15, 33), (1025, 16, 130), (4097, 16, 2100), (2049, 17, 1), (127, 31, 15),
                                    (128, 32, 16), (1153, 33, 32), (640, 36, 65), (129, 64, 64), (300, 100, 129),
-                                   (200, 1023, 3), (131, 1056, 20), (70, 1500, 66)])
+                                   (200, 1023, 3), (131, 1056, 20), (70, 1500, 66), (70, 1793, 9)])
 def test_distances_from_either_layout(cuda, n, d, k, dtype):
     import torch
 
@@ -422,6 +422,73 @@ def test_fp32_distances_of_close_and_extreme_pairs(cuda, case):
     exact = np.sqrt(((X.astype(np.float64)[:, None, :] - C.astype(np.float64)[None, :, :]) ** 2).sum(axis=2))
     got = drivers.get_euclidean_distances(_dev(X.T, cuda), _dev(C.T, cuda)).cpu().numpy()
     np.testing.assert_allclose(got, exact, rtol=(d / 2 + 3) * 1.2e-7)  # (redone pairs: d rounded additions)
+
+
+# pairs lost against the kernel's shift, many or all of a tile's: centroids far from everything (the first of them one),
+# two groups far apart (mixed, and in turn by 128 samples), an offset (the shift ends at 1 792 features), huge samples.
+# 16, 32 and 64 centroids a workgroup, its operands resident (d <= 32) or not, partial tiles, several tiles a workgroup.
+@pytest.mark.parametrize("case", ["far first", "far at both ends", "two groups", "groups by turns", "offset", "huge samples"])
+@pytest.mark.parametrize("n,d,k", [(1, 17, 1), (129, 20, 16), (300, 32, 31), (257, 100, 64), (700, 40, 70), (131, 1900, 5),
+                                   (200_003, 24, 20), (130_001, 33, 40)])
+def test_fp32_distances_far_from_the_shift(cuda, n, d, k, case):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    gen = torch.Generator(device=cuda).manual_seed(n + k)
+    C = torch.rand(k, d, generator=gen, device=cuda) * 8 - 4
+    lab = torch.randint(0, k, (n,), generator=gen, device=cuda)
+    if case == "far first":
+        C[0] = 1e6
+    elif case == "far at both ends":
+        C[0], C[-1] = 1e6, -2e6
+    elif case in ("two groups", "groups by turns"):
+        C[: (k + 1) // 2] += 1e6
+        if case == "groups by turns":
+            lab = torch.where(torch.arange(n, device=cuda) // 128 % 3 == 1, 0, k - 1)
+    elif case == "offset":
+        C += 1e5
+    X = C[lab] + torch.randn(n, d, generator=gen, device=cuda)
+    if case == "huge samples":
+        X[::3] *= (1.1e38 / (6.3 * d)) ** 0.5  # squares about 2^126, below the largest fp32
+    exact = torch.stack([(X.double() - c.double()).square().sum(1).sqrt() for c in C], dim=1)
+    not_finite = torch.empty(1, dtype=torch.int32, device=cuda)
+    for got in (drivers.get_euclidean_distances_rows(X, C.T.contiguous(), not_finite),
+                drivers.get_euclidean_distances(X.T.contiguous(), C.T.contiguous())):
+        # (redone pairs: d rounded additions)
+        torch.testing.assert_close(got.double(), exact, rtol=(d / 2 + 3) * 1.2e-7, atol=0)
+    assert int(not_finite) == 0
+
+
+def test_fp32_distances_take_as_long_with_a_far_centroid(cuda):
+    """The time does not hang on which centroid is an outlier, and not by more than a factor on how many pairs are redone
+    (before: 25 times as long with a far centroid 0, 13 with two groups)."""
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    n, d, k = 200_000, 100, 64
+    gen = torch.Generator(device=cuda).manual_seed(1)
+    C = torch.rand(k, d, generator=gen, device=cuda) * 8 - 4
+    lab = torch.randint(0, k, (n,), generator=gen, device=cuda)
+
+    def least(C):
+        X_t, C_t, times = (C[lab] + torch.randn(n, d, generator=gen, device=cuda)).T.contiguous(), C.T.contiguous(), []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            drivers.get_euclidean_distances(X_t, C_t)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    usual = least(C)
+    far, groups = C.clone(), C.clone()
+    far[0] = 1e6
+    groups[: k // 2] += 1e6
+    assert least(far) < 1.5 * usual
+    assert least(groups) < 6 * usual
 
 
 # a total that a kernel writes to the host: the same bits call after call, from several streams at once, and as a graph
