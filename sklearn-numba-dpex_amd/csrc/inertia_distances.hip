@@ -837,7 +837,13 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
         const int sl = 32 * wave + 2 * j;
         // a result's high word less that of what it is the difference of: how many binades it lost (20 bits
         // each); its least over the lane's results, the largest norm and the least result decide at once
-        int least = 0x7fffffff, most = max(__double2hiint(nx[0]), __double2hiint(nx[1]));
+        // (norms as unsigned words: infinities and NaN of either sign are the largest)
+        auto binades_lost = [](const double sq, const double of) __attribute__((always_inline)) {
+            return (int)((unsigned int)__double2hiint(sq) - (unsigned int)__double2hiint(of));
+        };
+        auto norm_word = [](const double v) __attribute__((always_inline)) { return (unsigned int)__double2hiint(v); };
+        int least = 0x7fffffff;
+        unsigned int most = max(norm_word(nx[0]), norm_word(nx[1]));
         float low = kmx_inf<float>();
         auto finish = [&](auto whole_tag) __attribute__((always_inline)) {
             constexpr bool whole = decltype(whole_tag)::value;
@@ -849,12 +855,12 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const double c2 = cn[0][16 * a + g + 4 * r];
-                    most = max(most, __double2hiint(c2));
+                    most = max(most, norm_word(c2));
                     float v[2];
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
                         const double of = nx[b] + c2, sq = fma(-2.0, acc[a][b][r], of);
-                        least = min(least, __double2hiint(sq) - __double2hiint(of));
+                        least = min(least, binades_lost(sq, of));
                         const float q = (float)sq;
                         low = fminf(low, q);
                         // root by one reciprocal root and a Newton step on the residual
@@ -876,7 +882,7 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
         else finish(std::false_type{});
         // d 2^-27, in binades; 2^126: no square beyond it overflows; 1e-30: roots and their residuals are normal
         const int lost = (26 - (31 - __builtin_clz(d))) << 20;
-        if (__any(least + lost <= 0 || most >= 0x47d00000 || !(low >= 1e-30f))) {
+        if (__any(least + lost <= 0 || most >= 0x47d00000u || !(low >= 1e-30f))) {
             unsigned int redo = 0u;
             asm volatile("" : "+v"(nx[0]), "+v"(nx[1]) : : "memory");  // (computed again, not kept in registers since above)
 #pragma unroll
@@ -888,7 +894,7 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
                         const double of = nx[b] + c2, sq = fma(-2.0, acc[a][b][r], of);
-                        if (!(__double2hiint(sq) - __double2hiint(of) + lost > 0 && of < 0x1p126 && (float)sq >= 1e-30f))
+                        if (!(binades_lost(sq, of) + lost > 0 && of < 0x1p126 && (float)sq >= 1e-30f))
                             redo |= 1u << (8 * a + 2 * r + b);
                     }
                 }

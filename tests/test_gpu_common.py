@@ -491,6 +491,24 @@ def test_fp32_distances_take_as_long_with_a_far_centroid(cuda):
     assert least(groups) < 6 * usual
 
 
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("d,k,at", [(20, 5, 0), (40, 70, 0), (40, 70, 69), (17, 2, 1), (1100, 20, 0)])
+def test_fp32_distances_to_a_centroid_with_nan(cuda, d, k, at, sign):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    rng = np.random.default_rng(d)
+    X, C = rng.standard_normal((300, d)).astype(np.float32), rng.standard_normal((k, d)).astype(np.float32)
+    for f in (0, d // 2, d - 1):
+        C[at, f] = np.copysign(np.float32(np.nan), np.float32(sign))
+    exact = np.sqrt(((X.astype(np.float64)[:, None, :] - C.astype(np.float64)[None, :, :]) ** 2).sum(axis=2))
+    not_finite = torch.empty(1, dtype=torch.int32, device=cuda)
+    for got in (drivers.get_euclidean_distances_rows(_dev(X, cuda), _dev(C.T, cuda), not_finite),
+                drivers.get_euclidean_distances(_dev(X.T, cuda), _dev(C.T, cuda))):
+        np.testing.assert_allclose(got.cpu().numpy(), exact, rtol=1.5 * 1.2e-7)  # (NaN in the column of `at` alone)
+
+
 # a total that a kernel writes to the host: the same bits call after call, from several streams at once, and as a graph
 # that is replayed between other calls leaves it in device memory
 @pytest.mark.parametrize("n,d,k,dtype", [(1, 3, 2, np.float32), (20_001, 14, 40, np.float32), (30_003, 70, 9, np.float32),
