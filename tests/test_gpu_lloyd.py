@@ -559,6 +559,40 @@ def test_iterations_behind_a_stop_leave_everything_alone(cuda, n, d, k, dtype):
     np.testing.assert_array_equal(sizes.cpu().numpy(), np.bincount(got, minlength=k))
 
 
+# iterations that the step's last workgroup ends: either side of 16 384 partial sums (workgroups x (d + 1) k), of 256
+# sums (several groups of threads per sum, several sums per thread), one and two clusters, a single workgroup; the kernels
+# with the samples in registers (11), streaming them (1) and on the fp32 matrix cores (31), also at most of 64 KB of LDS
+@pytest.mark.parametrize("n,d,k,dtype,flags,variant", [
+    (418_816, 4, 8, np.float32, 0, 11), (418_817, 4, 8, np.float32, 0, 11), (65_536, 16, 15, np.float32, 0, 11),
+    (65_537, 16, 15, np.float32, 0, 11), (32_768, 31, 8, np.float32, 0, 11), (32_769, 31, 8, np.float32, 0, 11),
+    (5_000, 60, 12, np.float32, 0, 11), (6_000, 60, 12, np.float32, 0, 11), (700, 2, 1, np.float32, 0, 11),
+    (32_768, 16, 15, np.float64, 0, 11), (32_769, 16, 15, np.float64, 0, 11), (9_001, 40, 8, np.float64, 0, 11),
+    (700, 2, 2, np.float64, 0, 11), (100, 3, 4, np.float64, 0, 11), (20_001, 20, 8, np.float32, 1, 1),
+    (7_000, 70, 8, np.float64, 1, 1), (7_700, 70, 8, np.float64, 1, 1), (20_001, 9, 45, np.float32, 0x10, 31),
+    (129, 14, 16, np.float32, 0x10, 31), (9_001, 42, 126, np.float32, 0x10, 31)])
+def test_iterations_ended_by_the_last_workgroup(cuda, n, d, k, dtype, flags, variant):
+    """Runs of one to three iterations, the first with a relocation out of the step, against the oracle."""
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    assert _capi.lloyd_plan(n, d, k, _capi.dtype_code(dtype), flags).variant == variant
+    rng = np.random.default_rng(n + d)
+    y = np.arange(n) % k
+    X = (rng.uniform(-50, 50, (k, d))[y] + rng.standard_normal((n, d))).astype(dtype)
+    X[n // 2] *= 4  # the farthest sample
+    init, w = X[:k].copy(), rng.uniform(0.5, 1.5, n).astype(dtype)
+    if k > 2:
+        init[k // 2] = 1e4
+    X_t, w_d = _dev(X.T, cuda), _dev(w, cuda)
+    for it in ok.lloyd_iterations(X, w, init, max_iter=3):
+        assert it["n_empty"] == (1 if k > 2 and it["n_iter"] == 1 else 0)
+        labels, _, centers_t, n_iter = drivers.lloyd(X_t, w_d, _dev(init.T, cuda), False, it["n_iter"], False, 0.0, flags=flags)
+        assert n_iter == it["n_iter"]
+        centers = centers_t.cpu().numpy().T
+        assert_centers_close(centers, it["centers"], dtype)
+        assert_labels_match(labels.cpu().numpy().astype(np.int64), ok.assign_labels(X, centers), X, centers)
+
+
 def _small_configs():
     return {
         "C1": lambda: datasets.config1(n=100_000),
