@@ -276,62 +276,60 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
     if (ROWS && bad) *not_finite = 1;
 }
 
-// Any d: a workgroup owns a tile of DT_S samples x DC centroids, a thread a 4 x (DC / 8) block of
-// it; the features are staged DT_K at a time through LDS (both arrays are feature-major, as the
-// tiles: a stage is a copy of rows, 128-bit loads), the next stage's
-// loads in flight during the arithmetic.  Per staged feature a thread reads its four samples
+// fp64, any d: a workgroup owns a tile of DT_S samples x DC centroids, a thread a 4 x (DC / 8) block of
+// it; the features are staged DT_K at a time through LDS (feature-major arrays: a stage is a copy of
+// rows, 128-bit loads), the next stage's loads in flight during the arithmetic.  Per staged feature a thread reads its four samples
 // and its centroids from LDS (the centroid reads are broadcasts) and updates its sums with a
 // difference and a fused multiply-add each, features in order: vector-ALU bound.
 // DC = 64, or 16 for up to 32 clusters: with 10 clusters a tile of 64 is five sixths padding,
 // and the kernel took ten times what reading X takes.
 constexpr int DT_S = 128, DT_C = 64, DT_C_FEW = 16, DT_K = 16;
+constexpr int DT_V = 2;  // elements per 128-bit vector
 
 // 128-bit vectors per thread of a staged tile of COLS columns (fewer vectors than threads: the
 // first threads take one)
-template <typename T, int COLS>
+template <int COLS>
 constexpr int dt_vectors() {
-    return (DT_K * (COLS / (16 / (int)sizeof(T))) + 255) / 256;
+    return (DT_K * (COLS / DT_V) + 255) / 256;
 }
 
-template <typename T, int COLS>
-__device__ __forceinline__ void dt_stage_load(T (*regs)[16 / sizeof(T)], const T* __restrict__ base, int64_t len,
+template <int COLS>
+__device__ __forceinline__ void dt_stage_load(double (*regs)[DT_V], const double* __restrict__ base, int64_t len,
                                               int64_t c0, int d, int f0) {
-    constexpr int V = 16 / sizeof(T);                 // elements per 128-bit vector
-    constexpr int PER_ROW = COLS / V;                 // vectors per staged row
-    constexpr int N = dt_vectors<T, COLS>();          // vectors per thread
+    constexpr int PER_ROW = COLS / DT_V;     // vectors per staged row
+    constexpr int N = dt_vectors<COLS>();    // vectors per thread
     // (the same for the whole workgroup: the loads of a stage that exists whole are straight-line code)
     const bool whole = f0 + DT_K <= d && c0 + COLS <= len;
 #pragma unroll
     for (int l = 0; l < N; ++l) {
         const int g = threadIdx.x + 256 * l;
         const int f = f0 + g / PER_ROW;
-        const int64_t c = c0 + (int64_t)V * (g % PER_ROW);
-        const T* __restrict__ src = base + (size_t)f * (size_t)len + c;
+        const int64_t c = c0 + (int64_t)DT_V * (g % PER_ROW);
+        const double* __restrict__ src = base + (size_t)f * (size_t)len + c;
         const bool used = g < DT_K * PER_ROW;  // (known at compile time but for a narrow tile)
         if (whole) {
             if (used) {
-                const auto v = *reinterpret_cast<const typename KmxVec<T, V>::type*>(src);
+                const auto v = *reinterpret_cast<const KmxVec<double, DT_V>::type*>(src);
 #pragma unroll
-                for (int e = 0; e < V; ++e) regs[l][e] = v[e];
+                for (int e = 0; e < DT_V; ++e) regs[l][e] = v[e];
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < V; ++e) regs[l][e] = used && f < d && c + e < len ? src[e] : T(0);
+            for (int e = 0; e < DT_V; ++e) regs[l][e] = used && f < d && c + e < len ? src[e] : 0.0;
         }
     }
 }
 
-template <typename T, int COLS>
-__device__ __forceinline__ void dt_stage_store(T (*tile)[COLS], const T (*regs)[16 / sizeof(T)]) {
-    constexpr int V = 16 / sizeof(T);
-    constexpr int PER_ROW = COLS / V;
-    constexpr int N = dt_vectors<T, COLS>();
+template <int COLS>
+__device__ __forceinline__ void dt_stage_store(double (*tile)[COLS], const double (*regs)[DT_V]) {
+    constexpr int PER_ROW = COLS / DT_V;
+    constexpr int N = dt_vectors<COLS>();
 #pragma unroll
     for (int l = 0; l < N; ++l) {
         const int g = threadIdx.x + 256 * l;
         if (g < DT_K * PER_ROW) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) tile[g / PER_ROW][V * (g % PER_ROW) + e] = regs[l][e];
+            for (int e = 0; e < DT_V; ++e) tile[g / PER_ROW][DT_V * (g % PER_ROW) + e] = regs[l][e];
         }
     }
 }
@@ -339,82 +337,79 @@ __device__ __forceinline__ void dt_stage_store(T (*tile)[COLS], const T (*regs)[
 // A stage of the samples from the (n, d) array: thread t takes 16 bytes of rows t / 8 + 32 l, and puts
 // them feature by feature into the tile (rows of DT_S + 2: the eight lanes of a sample and the four
 // samples beside them fall on all banks).
-template <typename T>
-__device__ __forceinline__ void dt_rows_load(T (*regs)[16 / sizeof(T)], const T* __restrict__ X, int64_t n, int64_t i0,
+__device__ __forceinline__ void dt_rows_load(double (*regs)[DT_V], const double* __restrict__ X, int64_t n, int64_t i0,
                                              int d, int f0) {
-    constexpr int V = 16 / sizeof(T), PER_ROW = DT_K / V, N = DT_S * PER_ROW / 256;
+    constexpr int PER_ROW = DT_K / DT_V, N = DT_S * PER_ROW / 256;
     const bool whole = f0 + DT_K <= d && i0 + DT_S <= n;  // (the same for the whole workgroup)
 #pragma unroll
     for (int l = 0; l < N; ++l) {
         const int64_t i = i0 + (threadIdx.x + 256 * l) / PER_ROW;
-        const int f = f0 + V * (threadIdx.x % PER_ROW);
-        const T* __restrict__ src = X + (size_t)i * d + f;
+        const int f = f0 + DT_V * (threadIdx.x % PER_ROW);
+        const double* __restrict__ src = X + (size_t)i * d + f;
         if (whole) {
-            const auto v = *reinterpret_cast<const typename KmxVec<T, V>::type*>(src);
+            const auto v = *reinterpret_cast<const KmxVec<double, DT_V>::type*>(src);
 #pragma unroll
-            for (int e = 0; e < V; ++e) regs[l][e] = v[e];
+            for (int e = 0; e < DT_V; ++e) regs[l][e] = v[e];
         } else {
 #pragma unroll
-            for (int e = 0; e < V; ++e) regs[l][e] = i < n && f + e < d ? src[e] : T(0);
+            for (int e = 0; e < DT_V; ++e) regs[l][e] = i < n && f + e < d ? src[e] : 0.0;
         }
     }
 }
-template <typename T>
-__device__ __forceinline__ bool dt_rows_store(T (*tile)[DT_S + 2], const T (*regs)[16 / sizeof(T)]) {
-    constexpr int V = 16 / sizeof(T), PER_ROW = DT_K / V, N = DT_S * PER_ROW / 256;
+__device__ __forceinline__ bool dt_rows_store(double (*tile)[DT_S + 2], const double (*regs)[DT_V]) {
+    constexpr int PER_ROW = DT_K / DT_V, N = DT_S * PER_ROW / 256;
     bool bad = false;
 #pragma unroll
     for (int l = 0; l < N; ++l)
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            tile[V * (threadIdx.x % PER_ROW) + e][(threadIdx.x + 256 * l) / PER_ROW] = regs[l][e];
+        for (int e = 0; e < DT_V; ++e) {
+            tile[DT_V * (threadIdx.x % PER_ROW) + e][(threadIdx.x + 256 * l) / PER_ROW] = regs[l][e];
             bad |= kmx_not_finite(regs[l][e]);
         }
     return bad;
 }
 
 // ROWS: X is (n, d), and a NaN or an infinity in it sets *not_finite; else (d, n).
-template <typename T, int DC, bool ROWS>
+template <int DC, bool ROWS>
 __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
-    const T* __restrict__ X, const T* __restrict__ centroids_t, T* __restrict__ distances_t,
+    const double* __restrict__ X, const double* __restrict__ centroids_t, double* __restrict__ distances_t,
     int32_t* __restrict__ not_finite, int64_t n, int d, int k) {
-    constexpr int V = 16 / sizeof(T);
     constexpr int CT = DC / 8;  // centroids per thread
     constexpr int XP = ROWS ? DT_S + 2 : DT_S;
-    __shared__ __align__(16) T xs[DT_K][XP];
-    __shared__ __align__(16) T cs[DT_K][DC];
+    __shared__ __align__(16) double xs[DT_K][XP];
+    __shared__ __align__(16) double cs[DT_K][DC];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const int64_t i0 = (int64_t)blockIdx.x * DT_S;
     const int c0 = blockIdx.y * DC;
-    T rx[dt_vectors<T, DT_S>()][V], rc[dt_vectors<T, DC>()][V];
+    double rx[dt_vectors<DT_S>()][DT_V], rc[dt_vectors<DC>()][DT_V];
     bool bad = false;
-    T acc[CT][4];
+    double acc[CT][4];
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[c][i] = T(0);
+        for (int i = 0; i < 4; ++i) acc[c][i] = 0.0;
 
     auto load_x = [&](const int f0) __attribute__((always_inline)) {
-        if constexpr (ROWS) dt_rows_load<T>(rx, X, n, i0, d, f0);
-        else dt_stage_load<T, DT_S>(rx, X, n, i0, d, f0);
+        if constexpr (ROWS) dt_rows_load(rx, X, n, i0, d, f0);
+        else dt_stage_load<DT_S>(rx, X, n, i0, d, f0);
     };
     load_x(0);
-    dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, 0);
+    dt_stage_load<DC>(rc, centroids_t, k, c0, d, 0);
     const int n_stages = (d + DT_K - 1) / DT_K;
     for (int st = 0; st < n_stages; ++st) {
         __syncthreads();  // the previous stage's reads are over
-        if constexpr (ROWS) bad |= dt_rows_store<T>(xs, rx);
-        else dt_stage_store<T, DT_S>(xs, rx);
-        dt_stage_store<T, DC>(cs, rc);
+        if constexpr (ROWS) bad |= dt_rows_store(xs, rx);
+        else dt_stage_store<DT_S>(xs, rx);
+        dt_stage_store<DC>(cs, rc);
         __syncthreads();
         if (st + 1 < n_stages) {
             load_x((st + 1) * DT_K);
-            dt_stage_load<T, DC>(rc, centroids_t, k, c0, d, (st + 1) * DT_K);
+            dt_stage_load<DC>(rc, centroids_t, k, c0, d, (st + 1) * DT_K);
         }
         // (rows past d hold zeros on both sides: their differences add nothing)
 #pragma unroll
         for (int kk = 0; kk < DT_K; ++kk) {
-            T xv[4], cv[CT];
+            double xv[4], cv[CT];
 #pragma unroll
             for (int i = 0; i < 4; ++i) xv[i] = xs[kk][4 * tx + i];
 #pragma unroll
@@ -423,7 +418,7 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
             for (int c = 0; c < CT; ++c)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const T diff = cv[c] - xv[i];
+                    const double diff = cv[c] - xv[i];
                     acc[c][i] = fma(diff, diff, acc[c][i]);
                 }
         }
@@ -434,11 +429,11 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
     for (int c = 0; c < CT; ++c) {
         const int cc = c0 + CT * ty + c;
         if (cc >= k) continue;
-        T* __restrict__ dst = distances_t + (size_t)cc * (size_t)n + i;
-        T v[4];
+        double* __restrict__ dst = distances_t + (size_t)cc * (size_t)n + i;
+        double v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = dist_sqrt(acc[c][e]);
-        kmx_store4<T>(dst - i, i, n, i + 4 <= n, v);
+        kmx_store4<double>(dst - i, i, n, i + 4 <= n, v);
     }
 }
 
@@ -503,8 +498,8 @@ __device__ __forceinline__ void dm_redo_pairs(const float* __restrict__ X, const
                 const int fi = f0 + 64 * q + lane, f = fi < d ? fi : d - 1;
                 diff[q] = 0.0f;
                 if (f0 + 64 * q < d) {
-                    const float v = centroids_t[(size_t)f * k + c] - (ROWS ? X[(size_t)(i0 + si) * d + f] : X[(size_t)f * n + i0 + si]);
-                    diff[q] = fi < d ? v : 0.0f;
+                    const float x = ROWS ? X[(size_t)(i0 + si) * d + f] : X[(size_t)f * n + i0 + si];
+                    diff[q] = fi < d ? centroids_t[(size_t)f * k + c] - x : 0.0f;
                 }
             }
 #pragma unroll
@@ -1027,7 +1022,7 @@ int32_t launch_distances_f64(const void* X, const void* centroids_t, void* dista
     const int dc = k <= 2 * DT_C_FEW ? DT_C_FEW : DT_C;
     const dim3 grid((unsigned)kmx_cdiv(n, DT_S), (unsigned)kmx_cdiv(k, dc));
 #define KMX_DIST_TILED(DC)                                                                                          \
-    hipLaunchKernelGGL((euclidean_distances_tiled_kernel<double, DC, ROWS>), grid, dim3(256), 0, stream,            \
+    hipLaunchKernelGGL((euclidean_distances_tiled_kernel<DC, ROWS>), grid, dim3(256), 0, stream,            \
                        (const double*)X, (const double*)centroids_t, (double*)distances_t, not_finite, n, d, k)
     if (dc == DT_C_FEW) KMX_DIST_TILED(DT_C_FEW); else KMX_DIST_TILED(DT_C);
 #undef KMX_DIST_TILED

@@ -838,7 +838,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         // launches / one: 800 000 x 4, 2 clusters fp64 485 / 431; 100 000 x 10, 8 fp32 335 / 306; 20 651 x 3, 6 fp64
         // 259 / 239.
         const bool fuse = (L.variant == KMX_VARIANT_REGISTER || L.variant == KMX_VARIANT_STREAM) &&
-                          (int64_t)n_partials_used * (d + 1) * k <= TAIL_PARTIALS && (d + 1) * k <= 6 * 1024;
+                          (int64_t)n_partials_used * (d + 1) * k <= TAIL_PARTIALS;  // (the sums fit: KMX_LDS_ACC_LIMIT)
         const LloydTail<T> tail = small_tail_args();
         const int32_t rc_step =
             launch_fused<T, ACC_LDS>(L, X_t, w, centroids_t, cpack, half_norms, labels_prev, labels,

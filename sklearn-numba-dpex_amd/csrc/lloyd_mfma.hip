@@ -93,8 +93,8 @@ __global__ __launch_bounds__(256) void absmax_rows_kernel(const T* __restrict__ 
 // the steps that want both and d <= DM <= 64: a thread keeps the d maxima of its samples in
 // registers and meets the others once, at its end.  Bound by the read of X, which two kernels
 // read twice: 5 000 000 x 14 fp32 110 us -> 55 (5.8 TB/s with the norms written), 2 000 000 x 32 fp64
-// 182 -> 111 (4.9 TB/s), 1 000 000 x 60 fp32 79 -> 46, 100 000 x 14 17 -> 8.  Loads go out in batches of eight rows; a row behind the last one is read as the last
-// one again (a cache hit) and counts as zeros.
+// 182 -> 111 (4.9 TB/s), 1 000 000 x 60 fp32 79 -> 46, 100 000 x 14 17 -> 8.  Loads go out in batches of
+// eight rows; a row behind the last one is read as the last one again (a cache hit) and counts as zeros.
 constexpr int SCAN_D_MAX = 64;
 constexpr int SCAN_THREADS = 256;
 template <int W, typename V>
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(64 * mfma_waves(NKS, MC)) void lloyd_mfma_kernel(
             process(Cols1{}, std::true_type{}, x, wv, pl, i0);
         }
     }
-    // The rest: a partial last tile, or every tile when vector accesses are not legal
+    // The rest: a partial last tile
     for (int64_t wt = n_fast + wt_first; wt < n_wtiles; wt += wt_step) {
         const int64_t i0 = wt * TILE + MC * j;
         float x[NKS][MC];

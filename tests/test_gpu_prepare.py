@@ -77,23 +77,34 @@ def test_means_of_zero_need_no_memory_for_a_copy(cuda, dtype, monkeypatch):
         drivers.prepare_data_for_lloyd(X_t + 1, "random", 1.0, ones, True)
 
 
+@pytest.mark.parametrize("copy_x", [True, False])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_means_of_zero_leave_the_data_alone(cuda, dtype):
+def test_means_of_zero_leave_the_data_alone(cuda, dtype, copy_x):
     import torch
 
     from sklearn_numba_dpex_amd.kmeans import drivers
 
-    half = np.random.default_rng(2).standard_normal((5, 301)).astype(dtype)
+    # small whole numbers: the sums are exact in any order
+    half = np.random.default_rng(2).integers(-9, 10, (5, 301)).astype(dtype)
     X_t = torch.as_tensor(np.concatenate([half, -half], axis=1), device=cuda)
     before = X_t.cpu().numpy().copy()
     ones = torch.full((602,), 0.25, dtype=X_t.dtype, device=cuda)
-    for copy_x in (True, False):
-        out, mean, init, tol, uniform = drivers.prepare_data_for_lloyd(X_t, "random", 1.0, ones, copy_x)
-        if mean is None:  # (the order of the additions decides whether opposite values cancel)
-            assert out.data_ptr() == X_t.data_ptr() and uniform and init == "random"
-            np.testing.assert_array_equal(out.cpu().numpy(), before)
-            assert tol == pytest.approx((before.astype(np.float64) ** 2).mean(), rel=1e-6)
-    zeros = torch.zeros((3, 77), dtype=X_t.dtype, device=cuda)
-    assert drivers.prepare_data_for_lloyd(zeros, "random", 1.0, ones[:77].contiguous(), False)[1] is None
-    # weights of another type or length than the data's are looked at by themselves
-    assert drivers.prepare_data_for_lloyd(zeros, "random", 1.0, torch.ones(77, dtype=torch.float64, device=cuda).float(), True)[4]
+    out, mean, init, tol, uniform = drivers.prepare_data_for_lloyd(X_t, "random", 1.0, ones, copy_x)
+    assert mean is None and out.data_ptr() == X_t.data_ptr() and uniform and init == "random"
+    np.testing.assert_array_equal(X_t.cpu().numpy(), before)
+    assert tol == pytest.approx((before.astype(np.float64) ** 2).mean(), rel=1e-6)
+
+
+@pytest.mark.parametrize("dtype,other", [(np.float32, np.float64), (np.float64, np.float32)])
+def test_weights_of_another_type_or_length_are_looked_at_by_themselves(cuda, dtype, other):
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    X_t = torch.as_tensor(np.random.default_rng(3).standard_normal((3, 77)).astype(dtype), device=cuda)
+    same = drivers.prepare_data_for_lloyd(X_t, "random", 1.0, torch.ones(77, dtype=X_t.dtype, device=cuda), True)
+    for weights, uniform in ((np.full(77, 0.5), True), (np.arange(1.0, 78.0), False), (np.arange(1.0, 6.0), False)):
+        for w in (weights.astype(other), weights.astype(dtype)):
+            got = drivers.prepare_data_for_lloyd(X_t, "random", 1.0, torch.as_tensor(w, device=cuda), True)
+            assert got[4] == uniform and got[3] == same[3]
+            assert torch.equal(got[0], same[0]) and torch.equal(got[1], same[1])
