@@ -278,9 +278,9 @@ __global__ __launch_bounds__(256) void euclidean_distances_reg_kernel(
 
 // fp64, any d: a workgroup owns a tile of DT_S samples x DC centroids, a thread a 4 x (DC / 8) block of
 // it; the features are staged DT_K at a time through LDS (feature-major arrays: a stage is a copy of
-// rows, 128-bit loads), the next stage's loads in flight during the arithmetic.  Per staged feature a thread reads its four samples
-// and its centroids from LDS (the centroid reads are broadcasts) and updates its sums with a
-// difference and a fused multiply-add each, features in order: vector-ALU bound.
+// rows, 128-bit loads), the next stage's loads in flight during the arithmetic.  Per staged feature a
+// thread reads its four samples and its centroids from LDS (the centroid reads are broadcasts) and updates
+// its sums with a difference and a fused multiply-add each, features in order: vector-ALU bound.
 // DC = 64, or 16 for up to 32 clusters: with 10 clusters a tile of 64 is five sixths padding,
 // and the kernel took ten times what reading X takes.
 constexpr int DT_S = 128, DT_C = 64, DT_C_FEW = 16, DT_K = 16;
@@ -444,10 +444,11 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
 // DM_M features: coordinate by coordinate the median of five of them, which an outlier among them does not move.
 // Where the result is less than about d 2^-27 of what it is the difference of, rounding would show in
 // fp32: those pairs are redone in the difference form, feature by feature in fp32, as are pairs that
-// involve values beyond 2^62 or infinities.  They are few, and their lanes redo them; where many of a wave's are
-// (two groups a thousand times as far apart as they are wide, an offset beyond DM_M features) the wave does
-// (dm_redo_wave), and a call takes two to four times as long.  What is left is one rounding to fp32 and the
-// square root: nearer the exact distance than d rounded additions.
+// involve values beyond 2^62 or infinities: a few one after the other (dm_redo_pairs), many of a wave's (two groups
+// a thousand times as far apart as they are wide, an offset beyond DM_M features) all at once (dm_redo_wave), and
+// a call takes two to four times as long.  What is left is one rounding of the square to fp32 and one of its root:
+// relative error at 300 007 x 100, 64 clusters 3.3e-8 root mean square and 8.9e-8 at most, of d rounded additions
+// 8.1e-8 and 4.6e-7.
 // Why: the difference form costs two vector instructions per pair and feature (98 us for 300 007 x 100 x 64
 // at the chip's rate without packed arithmetic), the fp64 matrix cores take 49 us for the same.  And the
 // rows of X are read where they are: a transposed copy of X for this one pass over it took 59 us there.
@@ -458,9 +459,10 @@ __global__ __launch_bounds__(256) void euclidean_distances_tiled_kernel(
 // banks); else (d, n) and feature by feature (DM_CP).
 // Nothing of the vector work hides behind these matrix instructions, so the end of a tile counts: square
 // root from one reciprocal root, one test of a lane's 32 results instead of one each, norms from LDS.
-// Bound by the matrix cores (42 TFLOP/s) and, with few features, by the end of a tile.  Kernel times, us, the
-// transposed copy and the differences it replaces / this: 300 007 x 100, 64 clusters 178 / 116; 1e5 x 784,
-// 300 clusters 1 340 / 1 065; 1e6 x 20, 16 clusters 90 / 60.  Reading the next step's operands ahead of the
+// Bound by the matrix work and the vector work one after the other (34 TFLOP/s at 300 007 x 100, 64 clusters,
+// 44 at 1e5 x 784, 300) and, with few features, by the end of a tile.  Kernel times, us, the transposed copy and
+// the differences it replaces / this: 300 007 x 100, 64 clusters 178 / 114; 1e5 x 784, 300 clusters 1 340 / 1 065;
+// 1e6 x 20, 16 clusters 90 / 60.  Reading the next step's operands ahead of the
 // matrix instructions: 292 -> 321 us at 1e6 x 96, 64 clusters (registers), not done.
 constexpr int DM_S = 128, DM_K = 32, DM_RP = DM_K + 2, DM_CP = DM_S + 32, DM_M = 1792;
 // pairs of a wave, per centroid tile, beyond which it redoes them all at once, and features at a time then (one after the
