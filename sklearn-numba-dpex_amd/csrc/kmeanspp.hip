@@ -72,9 +72,9 @@ int kpp_split(int64_t n, int d, int n_trials, int dtype) {
 // fp64 1 500 x 20, 8 252 / 212; 65 536 x 63, 100 3 065 / 1 958; 100 000 x 30 (24 MB), 20 516 / 503; 131 072 x 63
 // (66 MB), 30 1 010 / 1 061.
 // The line is where the first kind of shape loses; some of the others would gain a little beyond it.  50 centres,
-// two launches / one: fp32, two samples per thread, 131 072 x 48 (25 MB) 954 / 953, 56 (29 MB) 1 203 / 1 013, 63 (33 MB)
-// 1 266 / 1 143; four, 262 144 x 32 (34 MB) 1 053 / 1 177, 40 1 281 / 1 333, 48 (50 MB) 1 311 / 1 470; fp64 131 072 x 32
-// (34 MB) 1 164 / 1 076, 48 (50 MB) 1 393 / 1 363; 200 000 x 20 (32 MB) 1 119 / 1 171; 262 144 x 24 (50 MB) 1 309 / 1 245.
+// two launches / one: fp32, two samples per thread, 131 072 x 56 (29 MB) 1 203 / 1 013, 63 (33 MB) 1 266 / 1 143; four,
+// 262 144 x 32 (34 MB) 1 053 / 1 177, 40 1 281 / 1 333, 48 (50 MB) 1 311 / 1 470; fp64 131 072 x 32 (34 MB) 1 164 / 1 076,
+// 48 (50 MB) 1 393 / 1 363; 200 000 x 20 (32 MB) 1 119 / 1 171; 262 144 x 24 (50 MB) 1 309 / 1 245.
 constexpr int JOINT_BLOCKS = 256, JOINT_TN = 8, JOINT_D = 64;
 constexpr int64_t JOINT_BYTES = 24 << 20;
 int kpp_joint(int64_t n, int d, int n_trials, int dtype) {
