@@ -231,6 +231,11 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
  * They have no counterpart in the reference, which computes from one layout of X in its own type
  * (kmeans/drivers.py:146-391). */
 size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan);
+/* Bytes that kmx_lloyd_run takes as `resident` for plans without a half-precision copy whose iterations can look
+ * only at the samples whose label may have changed (0: the plan has no such iterations).  Uninitialised; used
+ * within the call only.  Same labels, centroids and counts with it and without; without it (`resident` NULL
+ * or smaller) every iteration reads all of X_t.  No counterpart in the reference. */
+size_t kmx_lloyd_bounds_bytes(const kmx_lloyd_plan* plan);
 /* Squared distance of every sample to the centroid of its label among those an iteration started
  * from (their packed copy in the workspace), for the relocation: out (n).  X_rowmajor: (n, d).
  * Replaces the distance pass of kmeans/drivers.py:239-259. */

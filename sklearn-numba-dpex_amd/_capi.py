@@ -114,6 +114,7 @@ SIGNATURES = {
     "kmx_lloyd_run": (_I32, [_PLAN, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _SZ, _I32, _I32,
                              POINTER(LloydStatus), _P]),
     "kmx_lloyd_resident_bytes": (_SZ, [_PLAN]),
+    "kmx_lloyd_bounds_bytes": (_SZ, [_PLAN]),
     "kmx_lloyd_sample_distances": (_I32, [_PLAN, _P, _P, _P, _P, _P]),
     "kmx_lloyd_init_resident": (_I32, [_PLAN, _P, _SZ, _P, _P, _P, _I32, c_double, _P, _P, _SZ, _P]),
     "kmx_lloyd_labels_inertia": (_I32, [_PLAN, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _SZ, _I32, _P, _SZ, _P]),

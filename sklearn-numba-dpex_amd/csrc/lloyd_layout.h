@@ -52,6 +52,7 @@ static inline bool kmx_flags_valid(uint32_t flags) {
 // Shapes the fp32 matrix-core fused step covers (operands and accumulators fit in LDS), and
 // those its wide-sample variant covers (samples in registers, centroids streamed).
 bool kmx_mfma_supported(int d, int k);
+bool kmx_bounds_fit(int64_t n, int d, int k, int dtype);  // (lloyd_bounds.hip)
 bool kmx_mfma_wide_supported(int d, int k);
 bool kmx_mfma_f64_supported(int d, int k);
 bool kmx_mfma_f64_labels_supported(int d, int k);  // without the accumulators in LDS
@@ -320,6 +321,20 @@ static inline bool lloyd_tiles_wanted(const LloydLayout& L, int64_t n, int d, in
     return products >= least && kmx_tiles_fit(n, d, k);
 }
 
+// Whether a run of the plan's kernels goes over to bounded iterations (lloyd_bounds.hip) where the caller has
+// memory for their rows and words.  A bounded iteration takes 40 us or more however few samples it looks at (a chain
+// of trips to memory), so the line is drawn at the time of a screened step without its own 15 us: the read of
+// X and the work per sample and centroid.  Measured, runs of 20 / 10 iterations on blobs, bounded over not:
+//   14 features, 127 clusters, fp32: 400 000 samples (the estimate says 10 us) 1.07 / 1.02, 800 000 (20) 1.00 /
+//     1.02, 1 600 000 (40) 0.91 / 1.01; 20, 200: 200 000 (12) 0.93 / 1.01, 400 000 (23) 0.83 / 1.01; 8, 127:
+//     800 000 (16) 1.03 / 1.03, 1 600 000 (31) 1.00 / 1.00; 48, 64: 400 000 (25) 0.93 / 1.00
+//   fp64, 32, 64: 200 000 (14) 0.91 / 1.01, 400 000 (28) 0.90 / 0.97; 60, 30: 200 000 (24) 0.73 / 0.87
+static inline bool lloyd_bounds_wanted(const LloydLayout& L, int64_t n, int d, int k, int dtype) {
+    if ((L.flags & (KMX_FLAG_PATH_MASK | KMX_FLAG_LABELS_MASK)) != 0 || !(L.screen || L.screen64)) return false;
+    const double us = (double)n * d * kmx_dtype_size(dtype) / 4.5e6 + (double)n * k * ((d + 15) / 16) * 1e-7;
+    return us >= 20.0 && kmx_bounds_fit(n, d, k, dtype);
+}
+
 // fp32 matrix-core implementations (lloyd_mfma.hip)
 // Fixed-point exponents from max|X_t row|, max|w| and n; clears the fixed-point sums.
 // The words of the maxima are zero on entry; X_t null: those of max|X_t row| have been taken already
@@ -367,6 +382,14 @@ int32_t kmx_lloyd_iter_fewk(const LloydLayout& L, const void* X_t, const void* X
                             const void* centroids_t, void* new_centroids_t, const uint32_t* labels_prev,
                             uint32_t* labels, void* sizes, uint32_t* empty_clusters, char* ws, int64_t n, int d,
                             int k, hipStream_t stream, hipEvent_t* events);
+// iterations of the screened steps that look only at samples whose label can have changed (lloyd_bounds.hip)
+size_t kmx_bounds_bytes(int64_t n, int d, int k);
+int32_t kmx_bounds_spread(const void* X_t, const void* centroids_t, const uint32_t* labels, const kmx_lloyd_status* status,
+                          unsigned long long* out, int64_t n, int d, int k, int dtype, hipStream_t stream);
+int32_t kmx_lloyd_iter_bounds(const LloydLayout& L, bool enter, char* area, int parity, const void* X_t, const void* w,
+                              const void* centroids_t, void* new_centroids_t, uint32_t* labels_a, uint32_t* labels_b,
+                              void* sizes, uint32_t* empty_clusters, char* ws, int64_t n, int d, int k, int dtype,
+                              hipStream_t stream);
 // labels only, screened the same way (scale from the centroids, norms taken per tile)
 int32_t kmx_assign_labels_mfma_screen(const void* X_t, const void* centroids_t, uint32_t* labels,
                                       int64_t n, int d, int k, int wgs_per_cu, hipStream_t stream);

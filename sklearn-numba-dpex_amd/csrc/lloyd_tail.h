@@ -12,6 +12,9 @@
 // GPU, more than many an iteration).  The words reach the host in any order; the last one is the
 // exclusive or of the others, and the host takes no notice of words that do not fit together.
 constexpr int KMX_PROGRESS_WORDS = 4;
+// Beside them hints, in no order with the others, that choose between steps with the same results: labels
+// changed (low half) and samples without a certificate, or looked at, by the last iteration; a distance (fp64).
+constexpr int KMX_PROGRESS_HINT = 4, KMX_PROGRESS_SPREAD = 5;
 constexpr unsigned long long KMX_PROGRESS_MARK = 0x6b6d78206c6c6f79ull;
 __host__ __device__ inline unsigned long long lloyd_progress_check(unsigned long long a, unsigned long long b,
                                                                    unsigned long long c) {
@@ -476,7 +479,12 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         }
     }
     const double total = kmx_block_sum<double>(shift, scratch);
-    if (threadIdx.x == 0) lloyd_update_status(a.status, total, n_changed, a.progress);
+    if (threadIdx.x == 0) {
+        if (a.progress != nullptr && a.clear_word != nullptr)
+            __hip_atomic_store(&a.progress[KMX_PROGRESS_HINT], (unsigned long long)n_changed | (unsigned long long)counter_word << 32,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        lloyd_update_status(a.status, total, n_changed, a.progress);
+    }
 }
 
 // Every workgroup of a launch calls this behind what it hands over (device-scope atomics and stores) with all

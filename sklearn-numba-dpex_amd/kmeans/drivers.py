@@ -26,6 +26,10 @@ def _iterations_per_call(n, d, k, itemsize):
     return max(16, int(0.1 / seconds))
 
 
+# a run shorter than this ends before its bounded iterations have paid for the one that prepares them
+_BOUNDS_LEAST_ITERATIONS = 8
+
+
 def lloyd(
     X_t,
     sample_weight,
@@ -100,6 +104,16 @@ def lloyd(
                                  float(tol), stream),
               "kmx_lloyd_init")
 
+    # room for iterations that look only at the samples whose label can have changed
+    extra, extra_bytes = resident, resident_bytes
+    if resident is None and not verbose and int(max_iter) >= _BOUNDS_LEAST_ITERATIONS:
+        extra_bytes = lib.kmx_lloyd_bounds_bytes(plan)
+        try:
+            if extra_bytes and room_for(extra_bytes, dev):
+                extra = torch.empty(extra_bytes, dtype=torch.uint8, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            extra = None
+
     status = LloydStatus()
     n_done, max_iter = 0, int(max_iter)
     per_call = _iterations_per_call(n, d, k, X_t.element_size())
@@ -108,7 +122,7 @@ def lloyd(
         until = min(n_done + (1 if verbose else per_call), max_iter)
         check(lib.kmx_lloyd_run(plan, ptr(X_t), ptr(X_rm), ptr(sample_weight), ptr(cent[0]), ptr(cent[1]),
                                 ptr(labels[0]), ptr(labels[1]), ptr(sizes), ptr(empty_list), ptr(ws), ws_bytes,
-                                ptr(resident), resident_bytes, n_done, until, status, stream), "kmx_lloyd_run")
+                                ptr(extra), extra_bytes, n_done, until, status, stream), "kmx_lloyd_run")
 
         if status.state == _capi.KMX_NEED_RELOCATION:
             j = status.n_iter  # the iteration that stopped: reads cent[j % 2], wrote sums to the other

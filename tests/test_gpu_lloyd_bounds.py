@@ -1,0 +1,135 @@
+"""GPU tests of the Lloyd iterations that look only at samples whose label can have changed
+(csrc/lloyd_bounds.hip): whole runs with the memory they need and without it, which has every
+iteration read all of X.  Labels, centroids, cluster sizes and the number of iterations are the same bit
+for bit: sums are integers, and what is passed over is proven unchanged.  The screened steps
+themselves are compared with the oracle in test_gpu_lloyd_screen.py."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+MARK = 0xFF
+
+
+def _run(X_t, w, init_t, max_iter, with_bounds):
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import check, lib, ptr
+
+    (d, n), k, dev = X_t.shape, init_t.shape[1], X_t.device
+    plan = _capi.lloyd_plan(n, d, k, _capi.dtype_code(X_t.dtype), 0)
+    need = lib.kmx_lloyd_bounds_bytes(plan)
+    assert need > 0
+    area = torch.full((need,), MARK, dtype=torch.uint8, device=dev) if with_bounds else None
+    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=dev)
+    cent = [init_t.clone(), torch.empty_like(init_t)]
+    labels = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(2)]
+    sizes, empty = torch.empty(k, dtype=X_t.dtype, device=dev), torch.empty(k, dtype=torch.int32, device=dev)
+    status, stream = _capi.LloydStatus(), _capi.current_stream()
+    check(lib.kmx_lloyd_init(plan, ptr(ws), ws.numel(), ptr(X_t), ptr(w), ptr(cent[0]), max_iter, 0.0, stream), "init")
+    check(lib.kmx_lloyd_run(plan, ptr(X_t), None, ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]), ptr(labels[1]),
+                            ptr(sizes), ptr(empty), ptr(ws), ws.numel(), ptr(area), need, 0, max_iter, status, stream), "run")
+    torch.cuda.synchronize()
+    if with_bounds:
+        # drift of the labels (two copies), then a word per sample: every one has been written, and some
+        # samples were passed over at least once (what they have seen of the drift is behind it by then)
+        words = area[(2 * k * 4 + 255) // 256 * 256:][: 4 * n].view(torch.int32)
+        assert bool((words != -1).all()), "no bounded iteration has run"
+        assert bool(((words & 0x7FF) < k).all())
+    at = status.n_iter % 2
+    return dict(n_iter=status.n_iter, state=status.state, labels=labels[at], cent=cent[at], sizes=sizes)
+
+
+def _same(a, b):
+    assert (a["n_iter"], a["state"]) == (b["n_iter"], b["state"])
+    for name in ("labels", "sizes", "cent"):
+        assert bool((a[name] == b[name]).all()), name
+
+
+def _blobs(n, d, k, dtype, seed, cuda, spread=5.0):
+    import torch
+
+    gen = torch.Generator(device=cuda).manual_seed(seed)
+    blobs = k * 3 // 4  # (every third blob has two centroids: labels keep moving, and no cluster empties)
+    centres = (torch.rand(blobs, d, generator=gen, device=cuda) * 2 - 1) * spread
+    std = 0.5 + 1.5 * torch.rand(blobs, generator=gen, device=cuda)
+    which = torch.arange(n, device=cuda) % blobs
+    X = centres[which] + std[which, None] * torch.randn(n, d, generator=gen, device=cuda)
+    X_t = X.to(dtype).T.contiguous()
+    w = 0.5 + torch.rand(n, generator=gen, device=cuda, dtype=dtype)
+    init = X_t[:, :k].contiguous()
+    return X_t, w, init
+
+
+# feature counts on both sides of the steps of 16 and of rows of 8; clusters on both sides of 32 and 64; sample
+# counts off every unit (128 words, 32 samples); each number of K steps in both types
+@pytest.mark.parametrize("n, d, k, dtype", [
+    (900_001, 14, 127, "float32"), (1_300_033, 16, 33, "float32"), (800_127, 17, 64, "float32"),
+    (500_031, 33, 65, "float32"), (400_001, 48, 100, "float32"), (400_129, 49, 31, "float32"), (300_001, 64, 100, "float32"),
+    (800_001, 13, 64, "float64"), (400_003, 32, 64, "float64"), (330_000, 33, 17, "float64"), (250_127, 49, 40, "float64"),
+    (200_001, 64, 48, "float64"),
+])
+def test_same_as_iterations_over_all_samples(n, d, k, dtype, cuda):
+    import torch
+
+    X_t, w, init = _blobs(n, d, k, getattr(torch, dtype), 7, cuda)
+    a = _run(X_t, w, init, 40, False)
+    b = _run(X_t, w, init, 40, True)
+    assert a["n_iter"] > 10
+    _same(a, b)
+
+
+def test_samples_on_the_bisector_and_more_of_them_than_the_list_holds(cuda):
+    """Two clusters that mirror each other exactly, and samples of weight zero on the plane between them: ties in
+    every iteration, which go to the lower index; with 5e6 samples and 2.9 % on the plane a workgroup meets
+    about 570 of them, beside some 200 that are close by themselves, and its list holds 640."""
+    import torch
+
+    n, d, k = 5_000_000, 10, 20
+    X_t, w, init = _blobs(n, d, k, torch.float32, 3, cuda)
+    half, on_plane = 200_000, int(0.029 * n)
+    gen = torch.Generator(device=cuda).manual_seed(1)
+    side = 40.0 + torch.randn(d, half, generator=gen, device=cuda)
+    X_t[:, :half] = side
+    X_t[:, half:2 * half] = side
+    X_t[0, half:2 * half] *= -1.0
+    w[half:2 * half] = w[:half]
+    plane = slice(2 * half, 2 * half + on_plane)
+    X_t[:, plane] = 40.0 + torch.randn(d, on_plane, generator=gen, device=cuda)
+    X_t[0, plane] = 0.0
+    w[plane] = 0.0
+    order = torch.randperm(n, generator=gen, device=cuda)
+    init[:, 3], init[:, 11] = X_t[:, 0], X_t[:, half]
+    X_t, w = X_t[:, order].contiguous(), w[order].contiguous()
+    a = _run(X_t, w, init, 24, False)
+    b = _run(X_t, w, init, 24, True)
+    _same(a, b)
+    tied = (X_t[0] == 0.0) & (w == 0.0)
+    assert int(tied.sum()) == on_plane
+    assert float(a["cent"][0, 3]) == -float(a["cent"][0, 11])  # the ties are exact
+    assert bool((b["labels"][tied] == 3).all())
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_run_with_relocated_clusters(dtype, cuda, monkeypatch):
+    """Through the driver: relocations end a call to the library, and the run goes on with another."""
+    import torch
+
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    X_t, w, init = _blobs(420_001, 32, 64, getattr(torch, dtype), 5, cuda)
+    for j in range(8):
+        init[:, 63 - j] = 1e3 * (1 + j * 1e-3)
+    with_bounds = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
+
+    class NoBounds:
+        def __getattr__(self, name):
+            return (lambda plan: 0) if name == "kmx_lloyd_bounds_bytes" else getattr(lib, name)
+
+    lib = drivers.lib
+    monkeypatch.setattr(drivers, "lib", NoBounds())
+    without = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
+    assert with_bounds[3] == without[3] and with_bounds[1] == without[1]
+    assert bool((with_bounds[0] == without[0]).all()) and bool((with_bounds[2] == without[2]).all())
