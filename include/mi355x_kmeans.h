@@ -234,7 +234,8 @@ size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan);
 /* Bytes that kmx_lloyd_run takes as `resident` for plans without a half-precision copy whose iterations can look
  * only at the samples whose label may have changed (0: the plan has no such iterations).  Uninitialised; used
  * within the call only.  Same labels, centroids and counts with it and without; without it (`resident` NULL
- * or smaller) every iteration reads all of X_t.  No counterpart in the reference. */
+ * or smaller) every iteration reads all of X_t, as in the reference (kmeans/drivers.py:188-343), which has no
+ * counterpart. */
 size_t kmx_lloyd_bounds_bytes(const kmx_lloyd_plan* plan);
 /* Squared distance of every sample to the centroid of its label among those an iteration started
  * from (their packed copy in the workspace), for the relocation: out (n).  X_rowmajor: (n, d).
