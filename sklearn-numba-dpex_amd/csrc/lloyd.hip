@@ -574,7 +574,7 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
             total += __builtin_nontemporal_load(shift_partial + b);
         status->ticket = 0;
         if (force) status->uncertified_iter = 0;  // (other centroids: the half-precision copy is tried again)
-        lloyd_update_status(status, total, status->n_changed, progress);
+        lloyd_update_status(status, lloyd_before(status), total, status->n_changed, progress);
     }
 }
 

@@ -121,109 +121,32 @@ __device__ inline int lloyd_list_empty(const T* sizes, uint32_t* empty_clusters,
     return base;
 }
 
-// The same for at most 64 clusters, by the first wave alone and with one barrier (the general
-// routine above passes five, each a wait for all the waves of the workgroup).
-template <typename T>
-__device__ inline int lloyd_list_empty_one_wave(const T* sizes, uint32_t* empty_clusters, int k,
-                                                int* heaviest_out) {
-    __shared__ int one_wave_result[2];
-    if (threadIdx.x < 64) {
-        const int c = (int)threadIdx.x;
-        const bool in = c < k;
-        const T sz = in ? sizes[c] : T(1);
-        const bool flag = in && sz == T(0);
-        const unsigned long long mask = __ballot(flag);
-        if (flag) empty_clusters[__popcll(mask & ((1ull << c) - 1ull))] = (uint32_t)c;
-        T my_max = in ? sz : -kmx_inf<T>();
-        int my_arg = in ? c : 0x7fffffff;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const T ov = __shfl_xor(my_max, off, 64);
-            const int oi = __shfl_xor(my_arg, off, 64);
-            if (ov > my_max || (ov == my_max && oi < my_arg)) {
-                my_max = ov;
-                my_arg = oi;
-            }
-        }
-        if (c == 0) {
-            one_wave_result[0] = my_arg;
-            one_wave_result[1] = __popcll(mask);
-        }
-    }
-    __syncthreads();
-    *heaviest_out = one_wave_result[0];
-    return one_wave_result[1];
-}
-
 // End of an iteration, by one thread: iteration count, shift, and the next state (strict
 // convergence from the second iteration on, then the tolerance, then the iteration limit).
-__device__ inline void lloyd_update_status(kmx_lloyd_status* st, double total_shift, unsigned int changed,
-                                           unsigned long long* progress) {
-    const int n_iter = st->n_iter + 1;
+// `was`: n_iter, max_iter and tol as they stood when the iteration began (asked for early by callers that wait for
+// other loads anyway).
+struct LloydBefore {
+    int n_iter, max_iter;
+    double tol;
+};
+__device__ inline LloydBefore lloyd_before(const kmx_lloyd_status* st) { return {st->n_iter, st->max_iter, st->tol}; }
+__device__ inline void lloyd_update_status(kmx_lloyd_status* st, const LloydBefore& was, double total_shift,
+                                           unsigned int changed, unsigned long long* progress) {
+    const int n_iter = was.n_iter + 1;
     st->n_iter = n_iter;
     st->shift_sum = total_shift;
     st->n_changed = 0;
     int next = KMX_RUNNING;
     if (n_iter > 1 && changed == 0)
         next = KMX_CONVERGED_STRICT;
-    else if (!(total_shift > st->tol))
+    else if (!(total_shift > was.tol))
         next = KMX_CONVERGED_TOL;
-    else if (n_iter >= st->max_iter)
+    else if (n_iter >= was.max_iter)
         next = KMX_MAX_ITER;
     st->state = next;
     st->reserved[1] = (int64_t)changed;
     lloyd_publish(progress, st, n_iter, next, 0, total_shift);
 }
-
-// Division, packed copy, half norms, shift and convergence test by ONE workgroup of 256
-// threads (thread per cluster, features in order).  `sums_t` becomes the new centroids.
-template <typename T>
-__device__ inline void lloyd_finalize_block(const LloydTail<T>& a, int n_empty, int heaviest) {
-    __shared__ double scratch[4];
-    const int d = a.d, k = a.k, dpad = a.dpad;
-    double shift = 0.0;
-    for (int c = threadIdx.x; c < k; c += 256) {
-        const T sz = a.sizes[c];
-        if (sz != T(0)) {
-            T sq = T(0), sh = T(0);
-#pragma unroll 2
-            for (int f = 0; f < d; ++f) {
-                const T nv = a.sums_t[(size_t)f * k + c] / sz;
-                const T df = a.old_centroids_t[(size_t)f * k + c] - nv;
-                sh += df * df;
-                sq += nv * nv;
-                a.cpack[(size_t)c * dpad + f] = nv;
-                a.sums_t[(size_t)f * k + c] = nv;
-            }
-            for (int f = d; f < dpad; ++f) a.cpack[(size_t)c * dpad + f] = T(0);
-            a.half_norms[c] = sq / T(2);
-            shift += (double)sh;
-        }
-    }
-    __syncthreads();
-    if (n_empty > 0) {
-        // still-empty clusters (nothing could be relocated) are parked on the heaviest one
-        for (int c = threadIdx.x; c < k; c += 256) {
-            if (a.sizes[c] == T(0)) {
-                T sq = T(0), sh = T(0);
-                for (int f = 0; f < d; ++f) {
-                    const T nv = a.cpack[(size_t)heaviest * dpad + f];
-                    const T df = a.old_centroids_t[(size_t)f * k + c] - nv;
-                    sh += df * df;
-                    sq += nv * nv;
-                    a.cpack[(size_t)c * dpad + f] = nv;
-                    a.sums_t[(size_t)f * k + c] = nv;
-                }
-                for (int f = d; f < dpad; ++f) a.cpack[(size_t)c * dpad + f] = T(0);
-                a.half_norms[c] = sq / T(2);
-                shift += (double)sh;
-            }
-        }
-    }
-    const double total = kmx_block_sum<double>(shift, scratch);
-    if (threadIdx.x == 0) lloyd_update_status(a.status, total, a.status->n_changed, a.progress);
-}
-
 
 // One workgroup (every thread of it, up to 1024) finishes an iteration whose (d + 1) * k sums fit
 // in LDS: empty-cluster list and, if no cluster is empty, division by the sizes, packed copy and
@@ -294,6 +217,8 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
             q_v[i] = mine ? q_exp[feature_of(jx, i)] : 0;
         }
     }
+    LloydBefore was = {};
+    if constexpr (!WIDE) was = lloyd_before(a.status);  // (WIDE has no registers left for it)
     unsigned int counter_word = 0u;
     if (a.clear_word != nullptr && threadIdx.x == 0)
         counter_word = COHERENT ? __hip_atomic_load(&a.clear_word[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
@@ -325,10 +250,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
             // (times 2^-q, built from its exponent field: exact, like ldexp)
             const T val = (T)((double)iv * __hiloint2double((1023 - q) << 20, 0));
             vals[jx] = val;
-            if (f < d)
-                out_t[jx] = val;
-            else
-                a.sizes[jx - dk] = val;
+            if (f == d) a.sizes[jx - dk] = val;
         };
         if (sums_ahead) {
 #pragma unroll
@@ -368,24 +290,30 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         for (int jx = threadIdx.x; jx < items; jx += n_threads) vals[jx] = jx < dk ? out_t[jx] : a.sizes[jx - dk];
     }
     __syncthreads();
-    int heaviest = 0;
-    const int n_empty = (WIDE && k <= 64) ? lloyd_list_empty_one_wave<T>(sizes_s, a.empty_clusters, k, &heaviest)
-                                          : lloyd_list_empty<T>(sizes_s, a.empty_clusters, k, &heaviest);
-    if (threadIdx.x == 0) {
-        a.status->n_empty = n_empty;
-        a.status->reserved[0] = heaviest;
-    }
-    if (n_empty > 0) {
-        // the host relocates and finishes the iteration; the next step rebuilds the sums
+    // Whether any cluster is empty, by every wave for itself; the list of them and the heaviest one, which take
+    // five barriers (3.4 us of an end of 14), only if there is one.
+    bool any_empty = false;
+    for (int c = (int)threadIdx.x & 63; c < k; c += 64) any_empty |= sizes_s[c] == T(0);
+    if (threadIdx.x == 0) a.status->n_empty = 0;
+    if (__any(any_empty)) {  // (the same in all waves)
+        int heaviest = 0;
+        const int n_empty = lloyd_list_empty<T>(sizes_s, a.empty_clusters, k, &heaviest);
+        if (threadIdx.x == 0) {
+            a.status->n_empty = n_empty;
+            a.status->reserved[0] = heaviest;
+        }
+        // the host relocates and finishes the iteration (from the raw sums); the next step rebuilds the sums
         if constexpr (FROM_GSUM) {
             if (keep_sums)
                 for (int jx = threadIdx.x; jx < items; jx += n_threads) gsum[jx] = 0ull;
-            if (fused) {  // (the raw sums, as the relocation reads them)
+            if (fused) {
 #pragma unroll
                 for (int i = 0; i < SUMS_AHEAD; ++i) {
                     const int jx = (int)threadIdx.x + stride * i;
                     if (lane_on && jx < dk) out_t[jx] = raw_v[i];
                 }
+            } else {
+                for (int jx = threadIdx.x; jx < dk; jx += n_threads) out_t[jx] = vals[jx];
             }
         }
         if (threadIdx.x == 0) {
@@ -483,7 +411,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         if (a.progress != nullptr && a.clear_word != nullptr)
             __hip_atomic_store(&a.progress[KMX_PROGRESS_HINT], (unsigned long long)n_changed | (unsigned long long)counter_word << 32,
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        lloyd_update_status(a.status, total, n_changed, a.progress);
+        lloyd_update_status(a.status, WIDE ? lloyd_before(a.status) : was, total, n_changed, a.progress);
     }
 }
 
