@@ -350,10 +350,30 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
     T* __restrict__ sizes, uint32_t* __restrict__ empty_clusters,
     kmx_lloyd_status* __restrict__ status, int d, int k,
     unsigned long long* __restrict__ gsum, const int* __restrict__ q_exp, int with_tail,
-    unsigned long long* __restrict__ progress) {
+    unsigned long long* __restrict__ progress, KmxKept kept, int rest) {
     if (status->state != KMX_RUNNING) return;
     const int items = (d + 1) * k;
-    if (gsum != nullptr) {
+    if (kept.hi != nullptr) {
+        // the sums that a run keeps (lloyd_moves.hip): converted with one rounding, and left as they are
+#pragma unroll 4
+        for (int item = blockIdx.x * 256 + threadIdx.x; item < items; item += gridDim.x * 256) {
+            const int q = q_exp[item / k];
+            const double unit = __hiloint2double((1023 - q) << 20, 0);  // 2^-q
+            const long long hi = (long long)kept.hi[item];
+            const double a = (double)hi;
+            double v = a * unit;
+            if (sizeof(T) == 8) {
+                const double small = (double)(long long)kept.lo[item] * __hiloint2double((1023 - q - rest) << 20, 0);
+                v += (double)(hi - (long long)a) * unit + small;
+            }
+            const T out = (T)(v + kept.odd[item]);
+            if (item < d * k)
+                sums_t[item] = out;
+            else
+                sizes[item - d * k] = out;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) kept.header[KMX_TH_SUMS] = (unsigned int)(status->n_iter + 1);
+    } else if (gsum != nullptr) {
         // 64-bit fixed-point sums of the matrix-core step: converted and cleared by a grid-stride
         // loop of few blocks (every block ends with one atomic on the same ticket)
         for (int item = blockIdx.x * 256 + threadIdx.x; item < items; item += gridDim.x * 256) {
@@ -483,12 +503,12 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
 // ------------------------------------------------------------------------------------------
 // Finalisation: LANES threads per cluster (256 / LANES clusters per workgroup), lane g on the
 // features g, g + LANES, ... (division, packed copy, half squared norm, squared shift); the lanes
-// meet in LDS in lane order.  8 lanes, or 64 for a few clusters of wide samples, where a
-// workgroup or two of eight-lane clusters would each walk a hundred features, a trip to memory
-// per value.  The last block sums the per-block shifts in block order and runs the convergence
-// test.
+// meet in LDS in lane order.  8 lanes, 32 where they would walk eight features or more, a trip to
+// memory per value, or 64 for a few clusters of wide samples, which leave the chip empty.  The last
+// block sums the per-block shifts in block order and runs the convergence test.
 // ------------------------------------------------------------------------------------------
-constexpr int fin_lanes(int d, int k) { return (d >= 256 && k <= 128) ? 64 : 8; }
+// (from 64 features on 32: 1 024 clusters of 256 features 24 -> 12 us, 100 of 100 12 -> 8)
+constexpr int fin_lanes(int d, int k) { return (d >= 256 && k <= 128) ? 64 : d >= 64 ? 32 : 8; }
 constexpr int fin_grid(int d, int k) { return (k + 256 / fin_lanes(d, k) - 1) / (256 / fin_lanes(d, k)); }
 
 template <typename T, int LANES>
@@ -567,11 +587,10 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
             }
         }
     }
+    for (unsigned int b = threadIdx.x; b < gridDim.x; b += 256) parked_shift += __builtin_nontemporal_load(shift_partial + b);
     parked_shift = kmx_block_sum<double>(parked_shift, scratch);
     if (threadIdx.x == 0) {
-        double total = parked_shift;
-        for (unsigned int b = 0; b < gridDim.x; ++b)
-            total += __builtin_nontemporal_load(shift_partial + b);
+        const double total = parked_shift;
         status->ticket = 0;
         if (force) status->uncertified_iter = 0;  // (other centroids: the half-precision copy is tried again)
         lloyd_update_status(status, lloyd_before(status), total, status->n_changed, progress);
@@ -803,7 +822,24 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
     int n_partials_used = L.n_partials;
     unsigned long long* gsum = nullptr;
     const int* q_exp = nullptr;
-    if (L.variant == KMX_VARIANT_MFMA_WIDE) {
+    KmxKept kept;
+    if (L.tiles != nullptr && d >= 4) {
+        // labels from the half-precision copy, and sums that are corrected for the samples that move (their rows
+        // are read four features at a time: narrower ones are summed as without the copy, below)
+        const unsigned int* absmax = reinterpret_cast<const unsigned int*>(ws + L.off_scales);
+        kept = kmx_tiles_kept(L.tiles, n, d, k);
+        q_exp = reinterpret_cast<const int*>(absmax + (d + 1));
+        constexpr int32_t dtype = sizeof(T) == 8 ? KMX_F64 : KMX_F32;
+        unsigned int* const listed = L.variant == KMX_VARIANT_MFMA_WIDE
+                                         ? const_cast<unsigned int*>(kmx_wide_screen_counter(ws + L.off_wscreen))
+                                         : nullptr;
+        int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, cpack, half_norms, L.tiles, status, labels, n, d, L.dpad,
+                                      k, dtype, stream, listed, labels_prev, absmax);
+        if (rc != KMX_OK) return rc;
+        rc = kmx_lloyd_kept_sums(X_rowmajor, w, labels_prev, labels, q_exp, kept, status, ws + L.off_bucket, n, d, k, dtype,
+                                 stream);
+        if (rc != KMX_OK) return rc;
+    } else if (L.variant == KMX_VARIANT_MFMA_WIDE) {
         if constexpr (sizeof(T) == 4) {
             const int32_t rc = kmx_lloyd_step_mfma_wide_f32(L, X_t, X_rowmajor, w, centroids_t,
                                                             labels_prev, labels, ws, n, d, k, stream);
@@ -873,7 +909,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
             return KMX_OK;
         }
     }
-    const int64_t reduce_grid = (gsum != nullptr || n_partials_used == 1)
+    const int64_t reduce_grid = (kept.hi != nullptr || gsum != nullptr || n_partials_used == 1)
                                     ? (kmx_cdiv(items, 256) < 128 ? kmx_cdiv(items, 256) : 128)
                                     : kmx_cdiv(items, RED_ITEMS);
     // sums that fit in LDS are finished by one workgroup (no device-wide fences or tickets)
@@ -882,7 +918,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
                        stream, partial, n_partials_used,
                        ((L.acc_mode == ACC_GLOBAL || L.acc_mode == KMX_ACC_BUCKET) && gsum == nullptr) ? 1 : 0,
                        (T*)new_centroids_t, (T*)sizes, empty_clusters, status, d, k, gsum, q_exp,
-                       small_tail ? 0 : 1, L.progress);
+                       small_tail ? 0 : 1, L.progress, kept, kmx_kept_rest(n));
     KMX_LAUNCH_CHECK();
     if (events) (void)hipEventRecord(events[2], stream);
     if (small_tail) {
@@ -890,7 +926,11 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         hipLaunchKernelGGL((lloyd_small_finalize_kernel<T, false>), dim3(1), dim3(256),
                            (size_t)items * sizeof(T), stream, nullptr, nullptr, tail);
     } else {
-        if (fin_lanes(d, k) == 64)
+        if (fin_lanes(d, k) == 32)
+            hipLaunchKernelGGL((lloyd_finalize_kernel<T, 32>), dim3((unsigned)fin_grid(d, k)), dim3(256), 0,
+                               stream, (const T*)centroids_t, (T*)new_centroids_t, (const T*)sizes, cpack,
+                               half_norms, shift_partial, status, d, k, L.dpad, 0, L.progress);
+        else if (fin_lanes(d, k) == 64)
             hipLaunchKernelGGL((lloyd_finalize_kernel<T, 64>), dim3((unsigned)fin_grid(d, k)), dim3(256), 0,
                                stream, (const T*)centroids_t, (T*)new_centroids_t, (const T*)sizes, cpack,
                                half_norms, shift_partial, status, d, k, L.dpad, 0, L.progress);
@@ -1103,7 +1143,7 @@ static int32_t lloyd_init_impl(const kmx_lloyd_plan* plan, void* workspace, size
     hipStream_t stream = (hipStream_t)stream_;
     char* ws = (char*)workspace;
     auto* status = reinterpret_cast<kmx_lloyd_status*>(ws + L.off_status);
-    const bool scales = L.variant == KMX_VARIANT_MFMA || L.variant == KMX_VARIANT_MFMA_WIDE || L.gemm_screen ||
+    const bool scales = resident != nullptr || L.variant == KMX_VARIANT_MFMA || L.variant == KMX_VARIANT_MFMA_WIDE || L.gemm_screen ||
                         L.direct_sums || L.screen64 || L.variant == KMX_VARIANT_FEWK;
     // (clears the words of the maxima for the pass that takes them)
     unsigned int* absmax = scales ? reinterpret_cast<unsigned int*>(ws + L.off_scales) : nullptr;
@@ -1122,9 +1162,6 @@ static int32_t lloyd_init_impl(const kmx_lloyd_plan* plan, void* workspace, size
             if (rc != KMX_OK) return rc;
         }
         const int32_t rc = kmx_lloyd_mfma_prepare(L, resident != nullptr ? nullptr : X_t, sample_weight, ws, n, d, dtype, stream);
-        if (rc != KMX_OK) return rc;
-    } else if (resident != nullptr) {
-        const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, centroids_t, resident, nullptr, n, d, k, dtype, stream);
         if (rc != KMX_OK) return rc;
     }
     // (the counter of uncertain samples of the screened steps was cleared with the sums)
@@ -1540,9 +1577,9 @@ int32_t kmx_lloyd_finalize(const kmx_lloyd_plan* plan, const void* centroids_t,
                        (T*)(ws + L.off_cpack), (T*)(ws + L.off_half), shift_partial, status, d, k,    \
                        L.dpad, 1, (unsigned long long*)nullptr)
     if (dtype == KMX_F32) {
-        if (fin_lanes(d, k) == 64) KMX_FINALIZE(float, 64); else KMX_FINALIZE(float, 8);
+        if (fin_lanes(d, k) == 64) KMX_FINALIZE(float, 64); else if (fin_lanes(d, k) == 32) KMX_FINALIZE(float, 32); else KMX_FINALIZE(float, 8);
     } else {
-        if (fin_lanes(d, k) == 64) KMX_FINALIZE(double, 64); else KMX_FINALIZE(double, 8);
+        if (fin_lanes(d, k) == 64) KMX_FINALIZE(double, 64); else if (fin_lanes(d, k) == 32) KMX_FINALIZE(double, 32); else KMX_FINALIZE(double, 8);
     }
 #undef KMX_FINALIZE
     KMX_LAUNCH_CHECK();

@@ -307,10 +307,17 @@ __global__ __launch_bounds__(DS_THREADS) void direct_sums_kernel(
 
 size_t kmx_bucket_bytes(int64_t n, int k) { return ((size_t)2 * k + 1 + 2 * (size_t)n) * sizeof(int); }
 
+int32_t kmx_bucket_offsets(const int* counts, int* offsets, const kmx_lloyd_status* status, int k, hipStream_t stream) {
+    hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, k, status);
+    KMX_LAUNCH_CHECK();
+    return KMX_OK;
+}
+
 // offsets and order from counts and ranks (also used by the wide fp32 path)
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,
                          int* order, const kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream) {
-    hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, k, status);
+    const int32_t rc = kmx_bucket_offsets(counts, offsets, status, k, stream);
+    if (rc != KMX_OK) return rc;
     int64_t sg = kmx_cdiv(n, 256 * 4);
     if (sg > 2048) sg = 2048;
     hipLaunchKernelGGL(bucket_scatter_kernel, dim3((unsigned)sg), dim3(256), 0, stream, labels, offsets, ranks,

@@ -73,7 +73,37 @@ int32_t kmx_lloyd_gemm_screen_labels(const void* X_t, const void* centroids_t, c
                                      const unsigned int* absmax, char* area, uint32_t* labels,
                                      const kmx_lloyd_status* status, int64_t n, int d, int k,
                                      hipStream_t stream);
-// labels from a half-precision copy of X kept for the run (lloyd_tiles.hip)
+// labels from a half-precision copy of X kept for the run (lloyd_tiles.hip), with the sums of its labels (lloyd_moves.hip)
+// Words of the copy's header.  The counts belong to one labelling and are cleared by its first kernel: whatever
+// was labelled before (a run that goes on, a call repeated, another run on the same copy) leaves
+// nothing behind that could run the lists past their n entries.
+constexpr int KMX_TH_SCALE = 0;    // bits of the scale
+constexpr int KMX_TH_LISTED = 1;   // samples without a certificate
+constexpr int KMX_TH_REST = 2;     // samples left to the tiled product
+constexpr int KMX_TH_MOVED = 3;    // samples with a certificate whose label is another one than before
+constexpr int KMX_TH_ENTRIES = 4;  // two for every sample that moved
+constexpr int KMX_TH_KEEP = 5;     // whether the kept sums are those of the labels before
+constexpr int KMX_TH_FINITE = 6;   // no NaN or infinity among samples and weights
+constexpr int KMX_TH_SUMS = 7;     // iterations behind the kept sums (0: none)
+constexpr int KMX_TH_WORDS = 64;
+struct KmxKept {
+    unsigned int* header = nullptr;
+    unsigned long long* hi = nullptr;   // (d + 1, k) sums, 64-bit fixed point with the run's scales
+    unsigned long long* lo = nullptr;   // fp64: what the terms of `hi` leave out, kmx_kept_rest more binary places
+    double* odd = nullptr;              // values that are not finite
+    uint32_t* entry = nullptr;          // samples that moved, twice, and their clusters
+    uint32_t* entry_cluster = nullptr;
+};
+// the rests of n terms, each at most half a unit of `hi`, stay within 2^59
+__host__ __device__ inline int kmx_kept_rest(int64_t n) {
+    int en = 9;
+    while (((int64_t)1 << en) < n && en < 31) ++en;  // n <= 2^en
+    return 59 - en;
+}
+KmxKept kmx_tiles_kept(char* area, int64_t n, int d, int k);
+int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_t* labels_prev, const uint32_t* labels,
+                            const int* q_exp, const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d,
+                            int k, int32_t dtype, hipStream_t stream);
 bool kmx_tiles_fit(int64_t n, int d, int k);
 size_t kmx_tiles_bytes(int64_t n, int d, int k);
 int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
@@ -98,9 +128,11 @@ int32_t kmx_inertia_rows(const void* X_rowmajor, const void* sample_weight, cons
 char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k);  // room for k half norms
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out = nullptr);
+                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out = nullptr,
+                         const uint32_t* labels_prev = nullptr, const unsigned int* absmax = nullptr);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
+int32_t kmx_bucket_offsets(const int* counts, int* offsets, const kmx_lloyd_status* status, int k, hipStream_t stream);
 int32_t kmx_bucket_order(const uint32_t* labels, const int* counts, int* offsets, const int* ranks,
                          int* order, const kmx_lloyd_status* status, int64_t n, int k, hipStream_t stream);
 int32_t kmx_bucket_count(const uint32_t* labels_prev, const uint32_t* labels, int* counts, int* ranks,

@@ -51,19 +51,11 @@ constexpr int GRP = 8;               // accumulator registers per arg-max group
 constexpr float ULP = 1.1920929e-7f; // 2^-23
 constexpr float HALF_MIN = 6.1035156e-5f;  // 2^-14: smaller magnitudes are rounded to zero (no fp16 subnormals)
 
-// Header words.  The two counts belong to one labelling and are cleared by its first kernel: whatever
-// was labelled before (a run that goes on, a call repeated, another run on the same copy) leaves
-// nothing behind that could run the lists past their n entries.
-constexpr int TH_SCALE = 0;      // bits of the scale
-constexpr int TH_LISTED = 1;     // samples without a certificate
-constexpr int TH_REST = 2;       // samples left to the tiled product
-constexpr int TH_WORDS = 64;
-
 struct TileArea {
     int S;              // steps of 16 features
     int n_blocks;       // blocks of 32 centroids
     int64_t n_tiles;    // tiles of 32 samples (even)
-    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_half, off_list, off_thr, off_rest, total;
+    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_half, off_list, off_thr, off_rest, off_hi, off_lo, off_odd, total;
 };
 
 inline TileArea tile_area(int64_t n, int d, int k) {
@@ -71,7 +63,7 @@ inline TileArea tile_area(int64_t n, int d, int k) {
     a.S = (d + 15) / 16;
     a.n_blocks = (k + 31) / 32;
     a.n_tiles = 2 * kmx_cdiv(n, 64);
-    a.off_xt = kmx_align256(TH_WORDS * sizeof(unsigned int));
+    a.off_xt = kmx_align256(KMX_TH_WORDS * sizeof(unsigned int));
     a.off_norm = a.off_xt + (size_t)a.n_tiles * a.S * 1024;
     a.off_err = a.off_norm + kmx_align256((size_t)a.n_tiles * 32 * sizeof(float));
     a.off_ct = a.off_err + kmx_align256((size_t)a.n_tiles * 32 * sizeof(float));
@@ -81,7 +73,10 @@ inline TileArea tile_area(int64_t n, int d, int k) {
     a.off_list = a.off_half + kmx_align256((size_t)k * sizeof(double));
     a.off_thr = a.off_list + kmx_align256((size_t)n * sizeof(int));
     a.off_rest = a.off_thr + kmx_align256((size_t)n * sizeof(float));
-    a.total = a.off_rest + kmx_align256((size_t)n * sizeof(int));
+    a.off_hi = a.off_rest + kmx_align256((size_t)n * sizeof(int));
+    a.off_lo = a.off_hi + kmx_align256((size_t)(d + 1) * k * 8);
+    a.off_odd = a.off_lo + kmx_align256((size_t)(d + 1) * k * 8);
+    a.total = a.off_odd + kmx_align256((size_t)(d + 1) * k * 8);
     return a;
 }
 
@@ -116,7 +111,7 @@ __device__ __forceinline__ void tiles_write_scale(float high, float low, float (
         m_s[1][threadIdx.x >> 6] = low;
     }
     __syncthreads();
-    if (threadIdx.x < TH_WORDS) header[threadIdx.x] = 0u;
+    if (threadIdx.x < KMX_TH_WORDS) header[threadIdx.x] = 0u;
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int i = 1; i < 16; ++i) {
@@ -124,7 +119,7 @@ __device__ __forceinline__ void tiles_write_scale(float high, float low, float (
             low = fmaxf(low, m_s[1][i]);
         }
         const int eh = scale_exponent(high, 10), el = scale_exponent(low, 0), e = eh > el ? eh : el;
-        header[TH_SCALE] = __float_as_uint(e == NO_EXPONENT ? 1.0f : ldexpf(1.0f, e));
+        header[KMX_TH_SCALE] = __float_as_uint(e == NO_EXPONENT ? 1.0f : ldexpf(1.0f, e));
     }
 }
 
@@ -186,7 +181,7 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
     __shared__ float part[2][2][NS];
     __shared__ unsigned int amax[TILE_D_MAX];
     for (int f = threadIdx.x; f < TILE_D_MAX; f += 256) amax[f] = 0u;
-    const float xs = __uint_as_float(header[TH_SCALE]);
+    const float xs = __uint_as_float(header[KMX_TH_SCALE]);
     const int s = threadIdx.x & (NS - 1), g2 = threadIdx.x >> 7;   // sample, pair of groups of 8 features
     for (int64_t i0 = (int64_t)blockIdx.x * NS; i0 < n_pad; i0 += (int64_t)gridDim.x * NS) {
         float sq = 0.0f, e2 = 0.0f;
@@ -277,19 +272,22 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
 
 // The centroids of a labelling: their tiles (32 centroids x 16 features, laid out like those of
 // the samples), -0.5 |c'|^2 (-inf past the last one), and per block of 32 the maxima of 0.5 |c'|^2 and
-// |e_c|.  A workgroup per block; four waves share the steps.  The first one clears the counts.
+// |e_c|.  A workgroup per block; its sixteen waves
+// take a step each (four took four trips to memory: 11 us, now 6).  The first one clears the counts.
+constexpr int CENT_WAVES = 16;
 template <typename T>
-__global__ __launch_bounds__(256) void tiles_centroids_kernel(const T* __restrict__ centroids_t, uint4* __restrict__ ct,
+__global__ __launch_bounds__(64 * CENT_WAVES) void tiles_centroids_kernel(const T* __restrict__ centroids_t, uint4* __restrict__ ct,
                                                               float* __restrict__ hneg, float2* __restrict__ cmax,
                                                               unsigned int* __restrict__ header,
-                                                              const kmx_lloyd_status* __restrict__ status, int d, int k, int S) {
+                                                              const kmx_lloyd_status* __restrict__ status,
+                                                              const unsigned int* __restrict__ absmax, int d, int k, int S) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
-    __shared__ double part[2][4][64];
-    const float xs = __uint_as_float(header[TH_SCALE]);
+    __shared__ double part[2][CENT_WAVES][64];
+    const float xs = __uint_as_float(header[KMX_TH_SCALE]);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = blockIdx.x * 32 + (lane & 31), h = lane >> 5;
     double sq = 0.0, e2 = 0.0;
-    for (int st = wave; st < S; st += 4) {
+    for (int st = wave; st < S; st += CENT_WAVES) {
         v8h hv;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -310,7 +308,7 @@ __global__ __launch_bounds__(256) void tiles_centroids_kernel(const T* __restric
         float hm = 0.0f, em = 0.0f;
         if (threadIdx.x < 32) {
             double s = 0.0, q = 0.0;
-            for (int w = 0; w < 4; ++w) {
+            for (int w = 0; w < (S < CENT_WAVES ? S : CENT_WAVES); ++w) {
                 s += part[0][w][lane] + part[0][w][lane + 32];
                 q += part[1][w][lane] + part[1][w][lane + 32];
             }
@@ -331,9 +329,21 @@ __global__ __launch_bounds__(256) void tiles_centroids_kernel(const T* __restric
         if (threadIdx.x == 0) {
             cmax[blockIdx.x] = make_float2(hm, em);
             if (blockIdx.x == 0) {
-                header[TH_LISTED] = 0u;
-                header[TH_REST] = 0u;
+                header[KMX_TH_LISTED] = 0u;
+                header[KMX_TH_REST] = 0u;
+                header[KMX_TH_MOVED] = 0u;
+                header[KMX_TH_ENTRIES] = 0u;
             }
+        }
+    }
+    // (an iteration: whether the sums kept from the one before can be corrected)
+    if (blockIdx.x == 0 && absmax != nullptr) {
+        bool finite = true;
+        for (int f = threadIdx.x; f <= d; f += 64 * CENT_WAVES) finite &= !kmx_not_finite(__uint_as_float(absmax[f]));
+        const bool all = __syncthreads_and(finite ? 1 : 0) != 0;
+        if (threadIdx.x == 0) {
+            header[KMX_TH_FINITE] = all ? 1u : 0u;
+            header[KMX_TH_KEEP] = all && status->n_iter > 0 && header[KMX_TH_SUMS] == (unsigned int)status->n_iter ? 1u : 0u;
         }
     }
 }
@@ -383,7 +393,8 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     const uint4* __restrict__ xt, const float* __restrict__ norm, const float* __restrict__ err,
     const uint4* __restrict__ ct, const float* __restrict__ hneg, const float2* __restrict__ block_max,
     unsigned int* __restrict__ header, const kmx_lloyd_status* __restrict__ status, uint32_t* __restrict__ labels,
-    int* __restrict__ list, float* __restrict__ list_thr, int64_t n, int n_blocks, float prod_rho) {
+    const uint32_t* __restrict__ labels_prev, int* __restrict__ list, float* __restrict__ list_thr, int64_t n, int n_blocks,
+    float prod_rho) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
     extern __shared__ __align__(16) unsigned char tiles_lds[];
     constexpr int CB = STREAM ? stream_blocks(S) : 1;
@@ -399,9 +410,12 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
     __shared__ int pend_i[8][PEND];
     __shared__ float pend_thr[8][PEND];
     int pending = 0;  // (the same in all lanes)
+    __shared__ unsigned int moved_block;
+    if (threadIdx.x == 0) moved_block = 0u;
+    unsigned int moved = 0u;
     auto flush = [&]() __attribute__((always_inline)) {
         unsigned int base = 0;
-        if (lane == 0) base = atomicAdd(header + TH_LISTED, (unsigned int)pending);
+        if (lane == 0) base = atomicAdd(header + KMX_TH_LISTED, (unsigned int)pending);
         base = (unsigned int)__builtin_amdgcn_readfirstlane((int)base);
         for (int e = lane; e < pending; e += 64) {
             list[base + e] = pend_i[wave][e];
@@ -594,6 +608,7 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
             const int64_t i = (grp_r * NCOL + cl) * 32 + j;
             const bool mine = live_group && h == 0 && i < n;
             const float nx2 = mine ? norm[i] : 0.0f, ex = mine ? err[i] : 0.0f;
+            const uint32_t was = mine && labels_prev != nullptr ? labels_prev[i] : 0u;
             const float delta = rho * fmaf(sqrtf(nx2) * 1.0001f, cmax, hmax);
             const float eps = (ex + emax) * 1.0001f;
             const float d2 = fmaxf(nx2 * 1.00005f - 2.0f * bb + 2.0f * delta, 0.0f);
@@ -617,12 +632,20 @@ __global__ __launch_bounds__(512, 2) void tiles_label_kernel(
                 pending += __popcll(um);
                 if (pending > PEND - 32) flush();
             }
-            if (mine && !unsure) labels[i] = (uint32_t)c;
+            if (mine && !unsure) {
+                labels[i] = (uint32_t)c;
+                moved += was != (uint32_t)c ? 1u : 0u;
+            }
         };
         finish(best0, second0, code0, w00, w01, w02, w03, 0);
         if constexpr (NCOL > 1) finish(best1, second1, code1, w10, w11, w12, w13, 1);
     }
     if (pending > 0) flush();
+    if (labels_prev != nullptr) {
+        if (moved != 0u) atomicAdd(&moved_block, moved);
+        __syncthreads();
+        if (threadIdx.x == 0 && moved_block != 0u) atomicAdd(header + KMX_TH_MOVED, moved_block);
+    }
 }
 
 // The listed samples: the centroids whose score reaches the sample's threshold are looked up again
@@ -652,11 +675,11 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
     double c_most = 0.0;  // max |c|, unscaled
     if constexpr (MATCH) {
         const float2 most = reduce_block_max(block_max, n_blocks);
-        c_most = (sqrt(2.0 * (double)most.x) * 1.0001 + (double)most.y) / (double)__uint_as_float(header[TH_SCALE]);
+        c_most = (sqrt(2.0 * (double)most.x) * 1.0001 + (double)most.y) / (double)__uint_as_float(header[KMX_TH_SCALE]);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = lane >> 5, j = lane & 31;
-    const int64_t n_listed = (int64_t)header[TH_LISTED];
+    const int64_t n_listed = (int64_t)header[KMX_TH_LISTED];
     if (listed_out != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *listed_out = (unsigned int)n_listed;
     if (n_listed > (n >> 3)) {  // the tiled product takes all samples
         if (status != nullptr && blockIdx.x == 0 && threadIdx.x == 0 && status->uncertified_iter == 0)
@@ -777,7 +800,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
             if (fine && arg < k)
                 labels[is] = (uint32_t)arg;
             else
-                rest[atomicAdd(header + TH_REST, 1u)] = is;
+                rest[atomicAdd(header + KMX_TH_REST, 1u)] = is;
         }
         __syncthreads();
         if constexpr (MATCH) {
@@ -822,7 +845,7 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
                 }
                 const int ic = list[t0 + j];
                 if (finite) labels[ic] = (uint32_t)lab;
-                else rest[atomicAdd(header + TH_REST, 1u)] = ic;
+                else rest[atomicAdd(header + KMX_TH_REST, 1u)] = ic;
             }
             __syncthreads();
         }
@@ -830,8 +853,8 @@ __global__ __launch_bounds__(256) void tiles_resolve_kernel(
 }
 
 template <int S, int NCOL, bool STREAM>
-int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                      float prod_rho, hipStream_t stream) {
+int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels,
+                      const uint32_t* labels_prev, int64_t n, float prod_rho, hipStream_t stream) {
     const size_t hneg_bytes = ((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023;
     const size_t lds = hneg_bytes + (STREAM ? (size_t)3 * stream_blocks(S) * S * 1024 : (size_t)a.n_blocks * S * 1024);
     if (lds > 64 * 1024) {
@@ -844,7 +867,7 @@ int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* sta
     hipLaunchKernelGGL((tiles_label_kernel<S, NCOL, STREAM>), dim3((unsigned)grid), dim3(512), lds, stream,
                        (const uint4*)(area + a.off_xt), (const float*)(area + a.off_norm), (const float*)(area + a.off_err),
                        (const uint4*)(area + a.off_ct), (const float*)(area + a.off_hneg),
-                       (const float2*)(area + a.off_cmax), (unsigned int*)area, status, labels,
+                       (const float2*)(area + a.off_cmax), (unsigned int*)area, status, labels, labels_prev,
                        (int*)(area + a.off_list), (float*)(area + a.off_thr), n, a.n_blocks, prod_rho);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
@@ -853,18 +876,18 @@ int32_t launch_labels(const TileArea& a, char* area, const kmx_lloyd_status* sta
 constexpr size_t TILES_LDS_MAX = 148 * 1024;  // (beside the 8 KB of the waves' list entries)
 
 template <int S>
-int32_t launch_labels_s(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                        float prod_rho, hipStream_t stream) {
+int32_t launch_labels_s(const TileArea& a, char* area, const kmx_lloyd_status* status, uint32_t* labels,
+                        const uint32_t* labels_prev, int64_t n, float prod_rho, hipStream_t stream) {
     const size_t resident = (((size_t)a.n_blocks * 128 + 1023) & ~(size_t)1023) + (size_t)a.n_blocks * S * 1024;
     const bool in_lds = resident <= TILES_LDS_MAX;
     // two columns per wave (a centroid fragment read from LDS serves two products) unless that leaves
     // compute units without a wave
     const bool two = n >= (int64_t)64 * 8 * kmx_num_cus() / 2;
     if (in_lds)
-        return two ? launch_labels<S, 2, false>(a, area, status, labels, n, prod_rho, stream)
-                   : launch_labels<S, 1, false>(a, area, status, labels, n, prod_rho, stream);
-    return two ? launch_labels<S, 2, true>(a, area, status, labels, n, prod_rho, stream)
-               : launch_labels<S, 1, true>(a, area, status, labels, n, prod_rho, stream);
+        return two ? launch_labels<S, 2, false>(a, area, status, labels, labels_prev, n, prod_rho, stream)
+                   : launch_labels<S, 1, false>(a, area, status, labels, labels_prev, n, prod_rho, stream);
+    return two ? launch_labels<S, 2, true>(a, area, status, labels, labels_prev, n, prod_rho, stream)
+               : launch_labels<S, 1, true>(a, area, status, labels, labels_prev, n, prod_rho, stream);
 }
 
 }  // namespace
@@ -927,34 +950,49 @@ int32_t kmx_tiles_prepare_samples(const void* X_t, void* X_rowmajor, char* area,
 KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
     const TileArea a = tile_area(n, d, 0);
     return {(const uint4*)(area + a.off_xt), (const float*)(area + a.off_norm), (const float*)(area + a.off_err),
-            (const float*)area + TH_SCALE, a.S};
+            (const float*)area + KMX_TH_SCALE, a.S};
+}
+
+KmxKept kmx_tiles_kept(char* area, int64_t n, int d, int k) {
+    const TileArea a = tile_area(n, d, k);
+    KmxKept kept;
+    kept.header = (unsigned int*)area;
+    kept.hi = (unsigned long long*)(area + a.off_hi);
+    kept.lo = (unsigned long long*)(area + a.off_lo);
+    kept.odd = (double*)(area + a.off_odd);
+    // (the lists of a labelling, which is over when the sums begin)
+    kept.entry = (uint32_t*)(area + a.off_list);
+    kept.entry_cluster = (uint32_t*)(area + a.off_thr);
+    return kept;
 }
 
 char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k) { return area + tile_area(n, d, k).off_half; }
 
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace
 // holds them).  `status` null: labels whatever the state, those of kmx_assign_labels, whose half norms
-// `half_norms` are then.  listed_out (or null): the number of samples without a certificate.
+// `half_norms` are then.  listed_out (or null): the number of samples without a certificate.  An iteration whose
+// sums are kept hands over the labels before and the bits of max |x| per feature and max |w| (else null).
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
-                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out) {
+                         int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out,
+                         const uint32_t* labels_prev, const unsigned int* absmax) {
     const TileArea a = tile_area(n, d, k);
     unsigned int* header = (unsigned int*)area;
     uint4* ct = (uint4*)(area + a.off_ct);
     float* hneg = (float*)(area + a.off_hneg);
     float2* cmax = (float2*)(area + a.off_cmax);
     if (dtype == KMX_F32)
-        hipLaunchKernelGGL((tiles_centroids_kernel<float>), dim3((unsigned)a.n_blocks), dim3(256), 0, stream,
-                           (const float*)centroids_t, ct, hneg, cmax, header, status, d, k, a.S);
+        hipLaunchKernelGGL((tiles_centroids_kernel<float>), dim3((unsigned)a.n_blocks), dim3(64 * CENT_WAVES), 0, stream,
+                           (const float*)centroids_t, ct, hneg, cmax, header, status, absmax, d, k, a.S);
     else
-        hipLaunchKernelGGL((tiles_centroids_kernel<double>), dim3((unsigned)a.n_blocks), dim3(256), 0, stream,
-                           (const double*)centroids_t, ct, hneg, cmax, header, status, d, k, a.S);
+        hipLaunchKernelGGL((tiles_centroids_kernel<double>), dim3((unsigned)a.n_blocks), dim3(64 * CENT_WAVES), 0, stream,
+                           (const double*)centroids_t, ct, hneg, cmax, header, status, absmax, d, k, a.S);
     // (an fp32 score: d + 1 roundings of partial sums, as many of the half norm)
     const bool match = status == nullptr && dtype == KMX_F32;
     const float prod_rho = match ? ULP * (float)(d + 8) : 0.0f;
     int32_t rc = KMX_ERR_UNSUPPORTED;
     switch (a.S) {
-#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, n, prod_rho, stream); break
+#define KMX_TILES_CASE(S_) case S_: rc = launch_labels_s<S_>(a, area, status, labels, labels_prev, n, prod_rho, stream); break
         KMX_TILES_CASE(1); KMX_TILES_CASE(2); KMX_TILES_CASE(3); KMX_TILES_CASE(4);
         KMX_TILES_CASE(5); KMX_TILES_CASE(6); KMX_TILES_CASE(7); KMX_TILES_CASE(8);
         KMX_TILES_CASE(9); KMX_TILES_CASE(10); KMX_TILES_CASE(11); KMX_TILES_CASE(12);
@@ -986,6 +1024,6 @@ int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* ce
     }
 #undef KMX_TILES_RESOLVE
     KMX_LAUNCH_CHECK();
-    return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + TH_REST, n, d, k, dtype,
-                                        stream, header + TH_LISTED, (n >> 3) + 1);
+    return kmx_lloyd_gemm_labels_listed(X_t, centroids_t, half_norms, labels, status, rest, header + KMX_TH_REST, n, d, k, dtype,
+                                        stream, header + KMX_TH_LISTED, (n >> 3) + 1);
 }

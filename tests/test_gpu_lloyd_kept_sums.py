@@ -1,0 +1,81 @@
+"""GPU tests of the sums that a run with the half-precision copy keeps and corrects for the samples that move
+(csrc/lloyd_moves.hip): the centroids of corrected sums are those of rebuilt ones bit for bit (integers),
+and both are the weighted means of the samples of a label."""
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_lloyd import _ResidentRun
+
+pytestmark = pytest.mark.gpu
+
+HEADER_SUMS = 7  # word of the copy's header: iterations behind the kept sums
+HEADER_KEEP = 5  # whether the last iteration had sums to correct
+HEADER_ENTRIES = 4
+
+
+def _words(run):
+    import torch
+
+    return run.resident[:32].view(torch.int32)
+
+
+def _blobs(n, d, k, dtype, seed=0, spread=2.0):
+    rng = np.random.default_rng(seed)
+    blobs = k * 3 // 4  # (every third blob has two centroids: labels keep moving, and no cluster empties)
+    centres = rng.uniform(-spread, spread, (blobs, d))
+    X = (centres[np.arange(n) % blobs] + rng.standard_normal((n, d))).astype(dtype)
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    w[::17] = 0.0
+    return X, w, X[:k].copy()
+
+
+# rows of 16, 32 and 64 lanes in both types, features beyond one pass of the lanes, widths that are no multiple of
+# a lane's values, stretches of the order that begin and end inside clusters, more clusters than stretches
+@pytest.mark.parametrize("n,d,k,dtype", [
+    (20_001, 16, 1300, np.float64), (20_011, 33, 620, np.float64), (65_603, 100, 100, np.float64), (20_001, 255, 130, np.float64),
+    (20_063, 129, 288, np.float32), (30_001, 70, 300, np.float32), (66_001, 191, 1025, np.float32), (66_001, 66, 400, np.float32),
+])
+def test_corrected_sums_are_rebuilt_sums(cuda, n, d, k, dtype):
+    X, w, init = _blobs(n, d, k, dtype, n + d)
+    steps = 8
+    corrected, rebuilt = _ResidentRun(cuda, X, w, init, steps), _ResidentRun(cuda, X, w, init, steps)
+    n_corrected = 0
+    for step in range(1, steps + 1):
+        a = corrected.run(step)
+        _words(rebuilt)[HEADER_SUMS] = 0
+        b = rebuilt.run(step)
+        if corrected.status.state not in (0, 3) or corrected.n_done < step:  # (KMX_RUNNING, KMX_MAX_ITER)
+            break
+        assert bool((a == b).all()) and bool((corrected.sizes == rebuilt.sizes).all())
+        assert bool((corrected.labels[step % 2] == rebuilt.labels[step % 2]).all())
+        keep, entries = int(_words(corrected)[HEADER_KEEP]), int(_words(corrected)[HEADER_ENTRIES])
+        assert int(_words(rebuilt)[HEADER_KEEP]) == 0 and keep == (1 if step > 1 else 0)
+        n_corrected += 1 if entries > 0 else 0
+        lab = corrected.labels[step % 2].cpu().numpy()
+        sizes = np.bincount(lab, weights=w.astype(np.float64), minlength=k)
+        full = sizes > 0
+        for f in (0, d // 2, d - 1):
+            want = np.bincount(lab, weights=X[:, f].astype(np.float64) * w, minlength=k)[full] / sizes[full]
+            got = a[f].cpu().numpy().astype(np.float64)[full]
+            # (the rounding of the result, and of the comparison's own sums; weights down to one sample's)
+            tol = 4 * np.finfo(dtype).eps if dtype == np.float32 else 1e-13
+            np.testing.assert_allclose(got, want, rtol=tol, atol=tol * np.abs(X[:, f]).max())
+    assert n_corrected >= 3
+
+
+@pytest.mark.parametrize("n,d,k,dtype", [(30_001, 100, 200, np.float64), (20_063, 129, 288, np.float32)])
+def test_values_that_are_not_finite_stay_in_their_clusters(cuda, n, d, k, dtype):
+    """One infinite coordinate: the cluster that holds the sample has an infinite or undefined mean there, every other
+    mean is finite, and no iteration corrects sums with such values in them."""
+    X, w, init = _blobs(n, d, k, dtype, 3)
+    X[n - 5, 7] = np.inf
+    w[n - 5] = 1.0
+    run = _ResidentRun(cuda, X, w, init, 3)
+    for step in (1, 2):
+        run.run(step, resident=True)
+        assert int(_words(run)[HEADER_KEEP]) == 0
+    lab = run.labels[run.n_done % 2].cpu().numpy()
+    c = run.cent[run.n_done % 2].cpu().numpy()
+    bad = ~np.isfinite(c)
+    assert bad[7, lab[n - 5]] and set(np.nonzero(bad)[1]) <= {int(lab[n - 5])} and set(np.nonzero(bad)[0]) == {7}
