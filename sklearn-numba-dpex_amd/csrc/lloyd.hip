@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
         // the sums that a run keeps (lloyd_moves.hip): converted with one rounding, and left as they are
 #pragma unroll 4
         for (int item = blockIdx.x * 256 + threadIdx.x; item < items; item += gridDim.x * 256) {
-            const int q = q_exp[item / k];
+            const int q = kmx_kept_exponent(kept.absmax, kept.n, d, item / k);
             const double unit = __hiloint2double((1023 - q) << 20, 0);  // 2^-q
             const long long hi = (long long)kept.hi[item];
             const double a = (double)hi;
@@ -827,8 +827,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         // labels from the half-precision copy, and sums that are corrected for the samples that move (their rows
         // are read four features at a time: narrower ones are summed as without the copy, below)
         const unsigned int* absmax = reinterpret_cast<const unsigned int*>(ws + L.off_scales);
-        kept = kmx_tiles_kept(L.tiles, n, d, k);
-        q_exp = reinterpret_cast<const int*>(absmax + (d + 1));
+        kept = kmx_tiles_kept(L.tiles, absmax, n, d, k);
         constexpr int32_t dtype = sizeof(T) == 8 ? KMX_F64 : KMX_F32;
         unsigned int* const listed = L.variant == KMX_VARIANT_MFMA_WIDE
                                          ? const_cast<unsigned int*>(kmx_wide_screen_counter(ws + L.off_wscreen))
@@ -836,8 +835,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, cpack, half_norms, L.tiles, status, labels, n, d, L.dpad,
                                       k, dtype, stream, listed, labels_prev, absmax);
         if (rc != KMX_OK) return rc;
-        rc = kmx_lloyd_kept_sums(X_rowmajor, w, labels_prev, labels, q_exp, kept, status, ws + L.off_bucket, n, d, k, dtype,
-                                 stream);
+        rc = kmx_lloyd_kept_sums(X_rowmajor, w, labels_prev, labels, kept, status, ws + L.off_bucket, n, d, k, dtype, stream);
         if (rc != KMX_OK) return rc;
     } else if (L.variant == KMX_VARIANT_MFMA_WIDE) {
         if constexpr (sizeof(T) == 4) {

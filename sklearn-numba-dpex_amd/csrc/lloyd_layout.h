@@ -83,12 +83,15 @@ constexpr int KMX_TH_REST = 2;     // samples left to the tiled product
 constexpr int KMX_TH_MOVED = 3;    // samples with a certificate whose label is another one than before
 constexpr int KMX_TH_ENTRIES = 4;  // two for every sample that moved
 constexpr int KMX_TH_KEEP = 5;     // whether the kept sums are those of the labels before
-constexpr int KMX_TH_FINITE = 6;   // no NaN or infinity among samples and weights
+constexpr int KMX_TH_FINITE = 6;   // no NaN or infinity, no maximum past fp32's largest, not all of them below its smallest
 constexpr int KMX_TH_SUMS = 7;     // iterations behind the kept sums (0: none)
+constexpr int KMX_TH_ODD = 8;      // NaN or infinity seen: among the samples (preparation), among the weights (sums)
 constexpr int KMX_TH_WORDS = 64;
 struct KmxKept {
     unsigned int* header = nullptr;
-    unsigned long long* hi = nullptr;   // (d + 1, k) sums, 64-bit fixed point with the run's scales
+    const unsigned int* absmax = nullptr;  // bits of max |x| per feature and of max |w|, in fp32
+    int64_t n = 0;
+    unsigned long long* hi = nullptr;   // (d + 1, k) sums, 64-bit fixed point (kmx_kept_exponent)
     unsigned long long* lo = nullptr;   // fp64: what the terms of `hi` leave out, kmx_kept_rest more binary places
     double* odd = nullptr;              // values that are not finite
     uint32_t* entry = nullptr;          // samples that moved, twice, and their clusters
@@ -100,10 +103,20 @@ __host__ __device__ inline int kmx_kept_rest(int64_t n) {
     while (((int64_t)1 << en) < n && en < 31) ++en;  // n <= 2^en
     return 59 - en;
 }
-KmxKept kmx_tiles_kept(char* area, int64_t n, int d, int k);
+// Exponent of the sums of feature f (f = d: of the weights): n terms stay within 2^61, one within 2^50.  No clamp,
+// unlike the fused steps' (they scale in fp32): -226 to 346 are exponents that fp64 has, so data of any
+// magnitude keep their digits.  A maximum of zero may be fp64 values below fp32's smallest.
+__device__ inline int kmx_kept_exponent(const unsigned int* __restrict__ absmax, int64_t n, int d, int f) {
+    const float w = __uint_as_float(absmax[d]), x = f < d ? __uint_as_float(absmax[f]) : 1.0f;
+    int e = kmx_not_finite(w) ? 0 : w > 0.0f ? ilogbf(w) + 1 : -149;
+    if (f < d) e += kmx_not_finite(x) ? 0 : x > 0.0f ? ilogbf(x) + 1 : -149;
+    const int en = n > 2 ? 64 - __clzll(n - 1) : 1;  // n <= 2^en
+    return (61 - en < 50 ? 61 - en : 50) - e;
+}
+KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k);
 int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_t* labels_prev, const uint32_t* labels,
-                            const int* q_exp, const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d,
-                            int k, int32_t dtype, hipStream_t stream);
+                            const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d, int k,
+                            int32_t dtype, hipStream_t stream);
 bool kmx_tiles_fit(int64_t n, int d, int k);
 size_t kmx_tiles_bytes(int64_t n, int d, int k);
 int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,

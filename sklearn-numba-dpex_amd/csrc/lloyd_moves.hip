@@ -10,8 +10,9 @@
 // and corrections of the same labels are then the same bits in any order, and the
 // sum that an iteration divides has one rounding (fp64 additions in an order of their own before).
 //
-// Values that are not finite have no such terms.  They are added up as they are, in sums of their own that join in
-// the end, and a run with any among its data rebuilds every iteration.
+// Values that are not finite, and those of a feature whose largest fp32 does not hold, have no such terms.  They are
+// added up as they are, in sums of their own that join in the end, and a run with any among its data rebuilds every
+// iteration (of fp64 features below fp32's smallest only where there are no others: beside those they are good to 2^-240).
 //
 // Bound by the read of rows (a rebuild: 4.8 TB/s) or by a chain of trips to memory (corrections).  moves_sum_kernel, every
 // iteration a rebuild before: 1e6 x 256 fp32, 1 024 clusters 216 us, now 215 / 112 / 45 / 27 / 22 in the first five
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(256) void moves_scatter_kernel(const uint32_t* __re
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_rm, const T* __restrict__ sample_weight,
                                                         const uint32_t* __restrict__ order, const int* __restrict__ offsets,
-                                                        int* __restrict__ counts, const int* __restrict__ q_exp, KmxKept kept,
+                                                        int* __restrict__ counts, KmxKept kept,
                                                         const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k) {
     if (status->state != KMX_RUNNING) return;
     constexpr bool TWO = sizeof(T) == 8;
@@ -185,13 +186,20 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
     const bool lane_on = f0 < d;
     const int rest = kmx_kept_rest(n);
     double m_hi[V], m_lo[V];
+    auto out_of_range = [&](const int f) __attribute__((always_inline)) {
+        const unsigned int bits = kept.absmax[f];
+        return kmx_not_finite(__uint_as_float(bits)) || (TWO && bits == 0u);
+    };
+    const bool w_as_is = out_of_range(d);
+    unsigned int as_is = 0u;  // bit j: the values of the lane's feature j are added up as they are
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-        const int q = q_exp[fl + j];
+        const int q = kmx_kept_exponent(kept.absmax, n, d, fl + j);
+        if (w_as_is || out_of_range(fl + j)) as_is |= 1u << j;
         m_hi[j] = fix_magic(q);
         m_lo[j] = fix_magic(q + rest);
     }
-    const int q_w = q_exp[d];
+    const int q_w = kmx_kept_exponent(kept.absmax, n, d, d);
     const double mw_hi = fix_magic(q_w), mw_lo = fix_magic(q_w + rest);
     const T* __restrict__ col = X_rm + fl;
 
@@ -229,9 +237,11 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (!FINITE && !(fabs(wv[u]) < kmx_inf<double>())) {
-                        // (a weight that is not finite: its terms as they are)
+                    const bool there = r0 + 4 * RPW * u + sub < n_here;
+                    if (!(fabs(wv[u]) < kmx_inf<double>())) {
+                        // (a weight that is not finite: its terms as they are; from the next iteration on FINITE is false)
                         if (lane_on) {
+                            kept.header[KMX_TH_ODD] = 1u;
 #pragma unroll
                             for (int j = 0; j < V; ++j)
                                 if (fl + j >= f0) kmx_atomic_add(kept.odd + (size_t)(fl + j) * k + c, (double)xv[u][j] * wv[u]);
@@ -242,13 +252,17 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
                         const double x = (double)xv[u][j];
-                        if (!FINITE && !(fabs(x) < kmx_inf<double>() && fabs(x * wv[u]) < 1e300)) {
-                            if (lane_on && fl + j >= f0 && wv[u] != 0.0) kmx_atomic_add(kept.odd + (size_t)(fl + j) * k + c, x * wv[u]);
+                        if (!FINITE && (((as_is >> j) & 1u) != 0u || !(fabs(x) < kmx_inf<double>()))) {
+                            if (lane_on && fl + j >= f0 && there && x != 0.0) kmx_atomic_add(kept.odd + (size_t)(fl + j) * k + c, x * wv[u]);
                             continue;
                         }
                         const double t = fma(x, wv[u], m_hi[j]);
                         hi[j] += to_fixed_q(t, m_hi[j]);
                         if constexpr (TWO) lo[j] += to_fixed_q(fma(x, wv[u], m_hi[j] - t) + m_lo[j], m_lo[j]);
+                    }
+                    if (!FINITE && w_as_is) {
+                        if (lane_on && f0 == 0 && there) kmx_atomic_add(kept.odd + (size_t)d * k + c, wv[u]);
+                        continue;
                     }
                     const double t = wv[u] + mw_hi;
                     w_hi += to_fixed_q(t, mw_hi);
@@ -312,14 +326,14 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
 }
 
 template <typename T>
-int32_t launch_sums(const void* X_rm, const void* w, const uint32_t* order, const int* offsets, int* counts, const int* q_exp,
-                    const KmxKept& kept, const kmx_lloyd_status* status, int64_t n, int d, int k, hipStream_t stream) {
+int32_t launch_sums(const void* X_rm, const void* w, const uint32_t* order, const int* offsets, int* counts, const KmxKept& kept,
+                    const kmx_lloyd_status* status, int64_t n, int d, int k, hipStream_t stream) {
     constexpr int V = 16 / (int)sizeof(T);
     // workgroups: a chunk each, or about four per compute unit where there are fewer chunks
     const unsigned gx = (unsigned)kmx_cdiv(n, CHUNK);
 #define KMX_MOVES_SUM(LPR_)                                                                                                  \
     hipLaunchKernelGGL((moves_sum_kernel<T, LPR_>), dim3(gx, (unsigned)kmx_cdiv(d, LPR_ * V)), dim3(256), 0, stream, (const T*)X_rm, \
-                       (const T*)w, order, offsets, counts, q_exp, kept, status, n, d, k)
+                       (const T*)w, order, offsets, counts, kept, status, n, d, k)
     if (d <= 16 * V) KMX_MOVES_SUM(16);
     else if (d <= 32 * V) KMX_MOVES_SUM(32);
     else KMX_MOVES_SUM(64);
@@ -333,8 +347,8 @@ int32_t launch_sums(const void* X_rm, const void* w, const uint32_t* order, cons
 // After kmx_tiles_labels: the kept sums are those of `labels`, and status->n_changed.  `bucket`: kmx_bucket_bytes, whose
 // first k words (the counts) are zero on entry and on return.
 int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_t* labels_prev, const uint32_t* labels,
-                            const int* q_exp, const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d,
-                            int k, int32_t dtype, hipStream_t stream) {
+                            const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d, int k,
+                            int32_t dtype, hipStream_t stream) {
     int* counts = reinterpret_cast<int*>(bucket);
     int* offsets = counts + k;
     uint32_t* order = reinterpret_cast<uint32_t*>(offsets + (k + 1));
@@ -351,6 +365,6 @@ int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_
     hipLaunchKernelGGL(moves_scatter_kernel, dim3((unsigned)sg), dim3(256), 0, stream, labels, kept, offsets, ranks, order, n,
                        (d + 1) * k, dtype == KMX_F64, status);
     KMX_LAUNCH_CHECK();
-    return dtype == KMX_F32 ? launch_sums<float>(X_rowmajor, w, order, offsets, counts, q_exp, kept, status, n, d, k, stream)
-                            : launch_sums<double>(X_rowmajor, w, order, offsets, counts, q_exp, kept, status, n, d, k, stream);
+    return dtype == KMX_F32 ? launch_sums<float>(X_rowmajor, w, order, offsets, counts, kept, status, n, d, k, stream)
+                            : launch_sums<double>(X_rowmajor, w, order, offsets, counts, kept, status, n, d, k, stream);
 }

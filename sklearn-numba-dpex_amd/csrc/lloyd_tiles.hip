@@ -170,7 +170,7 @@ __global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __res
 template <typename T>
 __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict__ X_t, T* __restrict__ X_rm,
                                                             uint4* __restrict__ xt, float* __restrict__ norm,
-                                                            float* __restrict__ err, const unsigned int* __restrict__ header,
+                                                            float* __restrict__ err, unsigned int* __restrict__ header,
                                                             unsigned int* __restrict__ absmax, int64_t n, int d, int S,
                                                             int64_t n_pad) {
     constexpr int NS = 128, NF = 32;
@@ -183,6 +183,7 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
     for (int f = threadIdx.x; f < TILE_D_MAX; f += 256) amax[f] = 0u;
     const float xs = __uint_as_float(header[KMX_TH_SCALE]);
     const int s = threadIdx.x & (NS - 1), g2 = threadIdx.x >> 7;   // sample, pair of groups of 8 features
+    float odd = 0.0f;  // (NaN once a value is NaN or infinite; the maxima leave NaN out)
     for (int64_t i0 = (int64_t)blockIdx.x * NS; i0 < n_pad; i0 += (int64_t)gridDim.x * NS) {
         float sq = 0.0f, e2 = 0.0f;
         for (int f0 = 0; f0 < 16 * S; f0 += NF) {
@@ -239,6 +240,7 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
                         sq = fmaf(hf, hf, sq);
                         const float r = v - hf;
                         e2 = fmaf(r, r, e2);
+                        odd = fmaf(v, 0.0f, odd);
                     }
                     // step (f0 + 8 g) / 16, half h = g & 1
                     const int st = f0 / 16 + (g >> 1);
@@ -267,6 +269,7 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
     if (absmax != nullptr) {
         __syncthreads();
         for (int f = threadIdx.x; f < d; f += 256) atomicMax(absmax + f, amax[f]);
+        if (odd != 0.0f) header[KMX_TH_ODD] = 1u;  // (true for NaN)
     }
 }
 
@@ -338,9 +341,13 @@ __global__ __launch_bounds__(64 * CENT_WAVES) void tiles_centroids_kernel(const 
     }
     // (an iteration: whether the sums kept from the one before can be corrected)
     if (blockIdx.x == 0 && absmax != nullptr) {
-        bool finite = true;
-        for (int f = threadIdx.x; f <= d; f += 64 * CENT_WAVES) finite &= !kmx_not_finite(__uint_as_float(absmax[f]));
-        const bool all = __syncthreads_and(finite ? 1 : 0) != 0;
+        bool finite = header[KMX_TH_ODD] == 0u && absmax[d] != 0u, some = false;
+        for (int f = threadIdx.x; f <= d; f += 64 * CENT_WAVES) {
+            finite &= !kmx_not_finite(__uint_as_float(absmax[f]));
+            some |= f < d && absmax[f] != 0u;
+        }
+        const bool any = __syncthreads_or(some ? 1 : 0) != 0;
+        const bool all = __syncthreads_and(finite && any ? 1 : 0) != 0;
         if (threadIdx.x == 0) {
             header[KMX_TH_FINITE] = all ? 1u : 0u;
             header[KMX_TH_KEEP] = all && status->n_iter > 0 && header[KMX_TH_SUMS] == (unsigned int)status->n_iter ? 1u : 0u;
@@ -902,7 +909,7 @@ size_t kmx_tiles_bytes(int64_t n, int d, int k) { return tile_area(n, d, k).tota
 static void tiles_copy(const void* X_t, void* X_rowmajor, char* area, unsigned int* absmax, int64_t n, int d, int dtype,
                        hipStream_t stream) {
     const TileArea a = tile_area(n, d, 0);  // (the samples' part depends on n and d alone)
-    const unsigned int* header = (const unsigned int*)area;
+    unsigned int* header = (unsigned int*)area;
     const int64_t n_pad = a.n_tiles * 32;
     int64_t grid = kmx_cdiv(n_pad, 128);
     const int64_t cap = (int64_t)(dtype == KMX_F32 ? 8 : 4) * kmx_num_cus();
@@ -953,10 +960,12 @@ KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
             (const float*)area + KMX_TH_SCALE, a.S};
 }
 
-KmxKept kmx_tiles_kept(char* area, int64_t n, int d, int k) {
+KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k) {
     const TileArea a = tile_area(n, d, k);
     KmxKept kept;
     kept.header = (unsigned int*)area;
+    kept.absmax = absmax;
+    kept.n = n;
     kept.hi = (unsigned long long*)(area + a.off_hi);
     kept.lo = (unsigned long long*)(area + a.off_lo);
     kept.odd = (double*)(area + a.off_odd);

@@ -64,18 +64,58 @@ def test_corrected_sums_are_rebuilt_sums(cuda, n, d, k, dtype):
     assert n_corrected >= 3
 
 
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("weight", [1.0, 0.0])
 @pytest.mark.parametrize("n,d,k,dtype", [(30_001, 100, 200, np.float64), (20_063, 129, 288, np.float32)])
-def test_values_that_are_not_finite_stay_in_their_clusters(cuda, n, d, k, dtype):
-    """One infinite coordinate: the cluster that holds the sample has an infinite or undefined mean there, every other
-    mean is finite, and no iteration corrects sums with such values in them."""
+def test_values_that_are_not_finite_stay_in_their_clusters(cuda, n, d, k, dtype, weight, value):
+    """One infinite or undefined coordinate: the cluster that holds the sample has an infinite or undefined mean there
+    (also with a weight of zero), every other mean is finite, and no iteration corrects sums with such values
+    in them."""
     X, w, init = _blobs(n, d, k, dtype, 3)
-    X[n - 5, 7] = np.inf
-    w[n - 5] = 1.0
+    X[n - 5, 7] = value
+    w[n - 5] = weight
     run = _ResidentRun(cuda, X, w, init, 3)
     for step in (1, 2):
         run.run(step, resident=True)
         assert int(_words(run)[HEADER_KEEP]) == 0
-    lab = run.labels[run.n_done % 2].cpu().numpy()
-    c = run.cent[run.n_done % 2].cpu().numpy()
-    bad = ~np.isfinite(c)
-    assert bad[7, lab[n - 5]] and set(np.nonzero(bad)[1]) <= {int(lab[n - 5])} and set(np.nonzero(bad)[0]) == {7}
+        if step == 1 or run.n_done == 2:
+            lab = run.labels[run.n_done % 2].cpu().numpy()
+            c = run.cent[run.n_done % 2].cpu().numpy()
+            bad = ~np.isfinite(c)
+            assert bad[7, lab[n - 5]] and set(np.nonzero(bad)[1]) <= {int(lab[n - 5])} and set(np.nonzero(bad)[0]) == {7}
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("n,d,k,dtype", [(30_001, 100, 200, np.float64), (20_063, 129, 288, np.float32)])
+def test_weights_that_are_not_finite_stay_in_their_clusters(cuda, n, d, k, dtype, value):
+    X, w, init = _blobs(n, d, k, dtype, 4)
+    w[n - 5] = value
+    run = _ResidentRun(cuda, X, w, init, 3)
+    run.run(1)
+    lab, c = run.labels[1].cpu().numpy(), run.cent[1].cpu().numpy()
+    held = np.arange(k) == lab[n - 5]
+    assert not np.isfinite(c[:, held]).any() and np.isfinite(c[:, ~held]).all()
+    run.run(2)
+    assert int(_words(run)[HEADER_KEEP]) == 0
+
+
+# magnitudes that the fused steps' fixed point and the fp32 maxima do not hold; one feature far below the others
+@pytest.mark.parametrize("scale,weight_scale,dtype", [
+    (1e10, 1e20, np.float32), (1e-17, 1e-12, np.float32), (1e-35, 1.0, np.float64),
+    (1e-80, 1.0, np.float64), (1e45, 1.0, np.float64), (1.0, 1e45, np.float64), (1.0, 1e-60, np.float64),
+])
+def test_sums_of_data_of_any_magnitude(cuda, scale, weight_scale, dtype):
+    n, d, k = (30_001, 100, 200) if dtype == np.float64 else (20_063, 129, 288)
+    X, w, init = _blobs(n, d, k, np.float64, 5)
+    X[:, 3] *= 1e-20 if dtype == np.float64 else 1e-5
+    X, w = (X * scale).astype(dtype), (w * weight_scale).astype(dtype)
+    run = _ResidentRun(cuda, X, w, X[:k].copy(), 2)
+    c = run.run(1).cpu().numpy().astype(np.float64)
+    assert run.n_done == 1 and run.status.state in (0, 3)  # (no cluster is empty)
+    lab = run.labels[1].cpu().numpy()
+    sizes = np.bincount(lab, weights=w.astype(np.float64), minlength=k)
+    full = sizes > 0
+    for f in (0, 3, d - 1):
+        want = np.bincount(lab, weights=X[:, f].astype(np.float64) * w, minlength=k)[full] / sizes[full]
+        tol = 4 * np.finfo(dtype).eps if dtype == np.float32 else 1e-13  # (as above)
+        np.testing.assert_allclose(c[f][full], want, rtol=tol, atol=tol * float(np.abs(X[:, f]).max()))
