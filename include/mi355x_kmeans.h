@@ -201,7 +201,8 @@ int32_t kmx_lloyd_trace_collect(float* kernel_ms_mean, float* kernel_ms_min, int
  * given to kmx_lloyd_init) is reached: enqueues kmx_lloyd_iter a few ahead of the last one that has
  * announced itself to the host and returns with what it learned in status_host (n_iter, state,
  * n_empty, shift_sum, uncertified_iter).  For a run that goes on (n_done > 0) status_host holds, on entry,
- * what the call before returned, or kmx_lloyd_status_read after a relocation.  Iteration j reads the
+ * what the call before returned, or kmx_lloyd_status_read after a relocation (without it the state is
+ * still KMX_NEED_RELOCATION: a run that the finalisation has ended then says so, without iterations).  Iteration j reads the
  * centroids and previous labels of its parity and writes those of the other one: centroids_even holds
  * the initial centroids, and iteration 0 writes centroids_odd and labels_odd.  After KMX_NEED_RELOCATION the caller relocates, calls
  * kmx_lloyd_finalize and comes back with n_done = status.n_iter + 1 if the run goes on.  Waits for
@@ -375,6 +376,13 @@ int32_t kmx_relocate_empty_clusters(const void* X_t, const void* sample_weight,
                                     const uint32_t* empty_clusters, int32_t n_relocated,
                                     void* per_sample_inertia, void* sums_t, void* cluster_sizes,
                                     int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream);
+/* The same if sq_dist (n) of the first far sample is above zero, else nothing (kmeans/drivers.py:239-259
+ * relocates either way): what the host would wait for before it relocates. */
+int32_t kmx_relocate_empty_clusters_if(const void* X_t, const void* sample_weight, const uint32_t* labels,
+                                       const int64_t* far_samples, const uint32_t* empty_clusters,
+                                       int32_t n_relocated, const void* sq_dist, void* sums_t,
+                                       void* cluster_sizes, int64_t n, int32_t d, int32_t k, int32_t dtype,
+                                       void* stream);
 
 /* ------------------------------------------------------------------------------------ *
  * kmeans++ seeding                                                                      *

@@ -139,6 +139,7 @@ SIGNATURES = {
     "kmx_euclidean_distances": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _P]),
     "kmx_euclidean_distances_rows": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P]),
     "kmx_relocate_empty_clusters": (_I32, [_P, _P, _P, _P, _P, _I32, _P, _P, _P, _I64, _I32, _I32, _I32, _P]),
+    "kmx_relocate_empty_clusters_if": (_I32, [_P, _P, _P, _P, _P, _I32, _P, _P, _P, _I64, _I32, _I32, _I32, _P]),
     "kmx_rng_init_states": (_I32, [ctypes.c_uint64, _I32, _I32, _P]),
     "kmx_rng_next_raw": (_I32, [_P, _I32, _I32, _P]),
     "kmx_kpp_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32]),

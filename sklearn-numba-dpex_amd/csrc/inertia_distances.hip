@@ -907,14 +907,16 @@ __global__ __launch_bounds__(256, 3) void distances_f32_kernel(
 }
 
 // One workgroup per relocated cluster, threads over features.  Several relocations may take
-// samples from the same old cluster, hence the atomic subtraction.
+// samples from the same old cluster, hence the atomic subtraction.  sq_dist (or null): nothing is
+// moved if the first sample, the farthest, has no distance above zero.
 template <typename T>
 __global__ __launch_bounds__(256) void relocate_kernel(
     const T* __restrict__ X_t, const T* __restrict__ sample_weight,
     const uint32_t* __restrict__ labels, const int64_t* __restrict__ far_samples,
     const uint32_t* __restrict__ empty_clusters, T* __restrict__ per_sample_inertia,
-    T* __restrict__ sums_t, T* __restrict__ sizes, int64_t n, int d, int k) {
+    T* __restrict__ sums_t, T* __restrict__ sizes, const T* __restrict__ sq_dist, int64_t n, int d, int k) {
     const int r = blockIdx.x;
+    if (sq_dist != nullptr && !(sq_dist[far_samples[0]] > T(0))) return;
     const uint32_t cluster = empty_clusters[r];
     const int64_t sample = far_samples[r];
     const uint32_t old = labels[sample];
@@ -1178,11 +1180,10 @@ int32_t kmx_euclidean_distances_rows(const void* X, const void* centroids_t, voi
                             : launch_distances_f64<true>(X, centroids_t, distances_t, not_finite, n, d, k, stream);
 }
 
-int32_t kmx_relocate_empty_clusters(const void* X_t, const void* sample_weight,
-                                    const uint32_t* labels, const int64_t* far_samples,
-                                    const uint32_t* empty_clusters, int32_t n_relocated,
-                                    void* per_sample_inertia, void* sums_t, void* cluster_sizes,
-                                    int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream_) {
+static int32_t relocate(const void* X_t, const void* sample_weight, const uint32_t* labels, const int64_t* far_samples,
+                        const uint32_t* empty_clusters, int32_t n_relocated, void* per_sample_inertia, void* sums_t,
+                        void* cluster_sizes, const void* sq_dist, int64_t n, int32_t d, int32_t k, int32_t dtype,
+                        void* stream_) {
     KMX_ENTRY();
     KMX_REQUIRE_PTR(X_t);
     KMX_REQUIRE_PTR(sample_weight);
@@ -1199,14 +1200,32 @@ int32_t kmx_relocate_empty_clusters(const void* X_t, const void* sample_weight,
         hipLaunchKernelGGL((relocate_kernel<float>), dim3(n_relocated), dim3(256), 0, stream,
                            (const float*)X_t, (const float*)sample_weight, labels, far_samples,
                            empty_clusters, (float*)per_sample_inertia, (float*)sums_t,
-                           (float*)cluster_sizes, n, d, k);
+                           (float*)cluster_sizes, (const float*)sq_dist, n, d, k);
     else
         hipLaunchKernelGGL((relocate_kernel<double>), dim3(n_relocated), dim3(256), 0, stream,
                            (const double*)X_t, (const double*)sample_weight, labels, far_samples,
                            empty_clusters, (double*)per_sample_inertia, (double*)sums_t,
-                           (double*)cluster_sizes, n, d, k);
+                           (double*)cluster_sizes, (const double*)sq_dist, n, d, k);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
+}
+
+int32_t kmx_relocate_empty_clusters(const void* X_t, const void* sample_weight,
+                                    const uint32_t* labels, const int64_t* far_samples,
+                                    const uint32_t* empty_clusters, int32_t n_relocated,
+                                    void* per_sample_inertia, void* sums_t, void* cluster_sizes,
+                                    int64_t n, int32_t d, int32_t k, int32_t dtype, void* stream) {
+    return relocate(X_t, sample_weight, labels, far_samples, empty_clusters, n_relocated, per_sample_inertia, sums_t,
+                    cluster_sizes, nullptr, n, d, k, dtype, stream);
+}
+
+int32_t kmx_relocate_empty_clusters_if(const void* X_t, const void* sample_weight, const uint32_t* labels,
+                                       const int64_t* far_samples, const uint32_t* empty_clusters, int32_t n_relocated,
+                                       const void* sq_dist, void* sums_t, void* cluster_sizes, int64_t n, int32_t d,
+                                       int32_t k, int32_t dtype, void* stream) {
+    KMX_REQUIRE_PTR(sq_dist);
+    return relocate(X_t, sample_weight, labels, far_samples, empty_clusters, n_relocated, nullptr, sums_t, cluster_sizes,
+                    sq_dist, n, d, k, dtype, stream);
 }
 
 }  // extern "C"

@@ -1300,6 +1300,10 @@ static void progress_give_back(unsigned long long* slot) {
     std::lock_guard<std::mutex> guard(progress_mutex);
     progress_free |= 1ull << ((slot - progress_page) / KMX_PROGRESS_STRIDE);
 }
+static __global__ void announce_end_kernel(const kmx_lloyd_status* __restrict__ status, unsigned long long* __restrict__ progress) {
+    if (threadIdx.x == 0 && status->state != KMX_RUNNING)
+        lloyd_publish(progress, status, status->n_iter, status->state, status->n_empty, status->shift_sum);
+}
 static bool progress_look(const unsigned long long* slot, kmx_lloyd_status* out) {
     const unsigned long long a = __atomic_load_n(&slot[0], __ATOMIC_RELAXED), b = __atomic_load_n(&slot[1], __ATOMIC_RELAXED),
                              c = __atomic_load_n(&slot[2], __ATOMIC_RELAXED);
@@ -1345,8 +1349,9 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
     int enqueued = n_done;
     kmx_lloyd_status seen;
     std::memset(&seen, 0, sizeof(seen));
-    // (what an earlier call found about the copy)
-    if (status_host->uncertified_iter > 0 && status_host->uncertified_iter <= n_done)
+    // (what an earlier call found about the copy; a relocation starts it anew)
+    const bool relocated = n_done > 0 && status_host->state == KMX_NEED_RELOCATION;
+    if (!relocated && status_host->uncertified_iter > 0 && status_host->uncertified_iter <= n_done)
         seen.uncertified_iter = status_host->uncertified_iter;
     seen.n_iter = n_done;
     seen.state = KMX_RUNNING;
@@ -1430,6 +1435,16 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
         else (void)hipGetLastError();
         return rc;
     };
+    // The caller has finalised a relocation and not asked how that ended (a copy and a wait of 50 us): if it ended the
+    // run, the iterations below do nothing, and this says so.
+    if (relocated) {
+        LloydLayout L = lloyd_layout(plan->n, plan->d, plan->k, plan->dtype, plan->flags);
+        if (workspace == nullptr || workspace_bytes < L.total) return give_up(workspace == nullptr ? KMX_ERR_NULL_POINTER : KMX_ERR_WORKSPACE);
+        hipLaunchKernelGGL(announce_end_kernel, dim3(1), dim3(64), 0, stream,
+                           (const kmx_lloyd_status*)((const char*)workspace + L.off_status), slot);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return give_up((int32_t)e);
+    }
     unsigned int spins = 0;
     while (true) {
         const int ahead = resident != nullptr && seen.n_iter == 0 ? 1 : bounds != nullptr && entered < 0 ? 2 : AHEAD;

@@ -139,6 +139,9 @@ def lloyd(
             )
             check(lib.kmx_lloyd_finalize(plan, ptr(cent[a]), ptr(cent[b]), ptr(sizes), ptr(ws), ws_bytes,
                                          stream), "kmx_lloyd_finalize")
+            if not verbose:  # (the next call says whether that has ended the run)
+                n_done = j + 1
+                continue
             check(lib.kmx_lloyd_status_read(ptr(ws), status, stream), "kmx_lloyd_status_read")
 
         if verbose:
@@ -257,14 +260,12 @@ def _relocate_empty_clusters(
     if sq_dist is None:
         sq_dist = _per_sample_inertia(X_t, None, distance_centroids_t, assignments_idx)
     far = topk_idx(sq_dist, int(n_empty_clusters))
-    if not float(sq_dist[far[0]]) > 0.0:
-        # more clusters than distinct samples: nothing to relocate; the finalisation parks
-        # the empty clusters on the heaviest one
-        return
-    check(lib.kmx_relocate_empty_clusters(ptr(X_t), ptr(sample_weight), ptr(assignments_idx), ptr(far),
-                                          ptr(empty_clusters_list), int(n_empty_clusters), None,
-                                          ptr(centroids_t), ptr(cluster_sizes), n, d, k, dcode(X_t),
-                                          _capi.current_stream()), "kmx_relocate_empty_clusters")
+    # (with more clusters than distinct samples there is nothing to relocate, which the kernel sees for
+    # itself; the finalisation parks the empty clusters on the heaviest one)
+    check(lib.kmx_relocate_empty_clusters_if(ptr(X_t), ptr(sample_weight), ptr(assignments_idx), ptr(far),
+                                             ptr(empty_clusters_list), int(n_empty_clusters), ptr(sq_dist),
+                                             ptr(centroids_t), ptr(cluster_sizes), n, d, k, dcode(X_t),
+                                             _capi.current_stream()), "kmx_relocate_empty_clusters_if")
 
 
 def _room_for_centred(X_t):

@@ -506,3 +506,32 @@ def test_finite_input_whose_sum_overflows_is_accepted(cuda):
     keep[[5, 9]] = False
     for arg in (X_big, _as_cuda(X_big, np.float32)):
         assert_array_equal(_np(km.predict(arg))[keep], _np(km.predict(X))[keep])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+# (not to convergence: in fp32 the iteration at which the last near tie is settled is not the oracle's)
+@pytest.mark.parametrize("max_iter,tol", [(1, 0.0), (5, 1e30), (2, 0.0), (4, 0.0)])
+@pytest.mark.parametrize("n,d,k", [(500, 3, 9), (30_000, 80, 70)])
+def test_a_run_that_ends_with_its_relocation(cuda, dtype, max_iter, tol, n, d, k):
+    """The finalisation of a relocation reaches the last iteration or the tolerance, or the run goes on: iterations and
+    centroids of the oracle."""
+    import torch
+
+    from oracle import kmeans as ok
+    from sklearn_numba_dpex_amd.kmeans import drivers
+    from tests._parity import assert_centers_close
+
+    rng = np.random.default_rng(n)
+    centres = rng.uniform(-30, 30, (k - 3, d))
+    X = (centres[np.arange(n) % (k - 3)] + rng.standard_normal((n, d))).astype(dtype)
+    X[[5, 50, 499]] *= np.array([[4], [5], [6]], dtype=dtype)  # (far apart in rank)
+    X -= X.mean(axis=0)
+    w = np.ones(n, dtype=dtype)
+    init = np.concatenate([X[:k - 3], np.full((3, d), 1e4)]).astype(dtype)
+    init[:, 0] += 0.1  # (no sample lies on its centroid)
+    labels, inertia, centroids_t, n_iter = drivers.lloyd(
+        torch.as_tensor(np.ascontiguousarray(X.T), device=cuda), torch.as_tensor(w, device=cuda),
+        torch.as_tensor(np.ascontiguousarray(init.T), device=cuda), True, max_iter, False, tol)
+    _, _, ref_centres, ref_n_iter = ok.lloyd(X, w, init, max_iter=max_iter, tol=tol)
+    assert n_iter == ref_n_iter == (1 if tol else max_iter)
+    assert_centers_close(centroids_t.cpu().numpy().T, ref_centres, dtype, scale_rtol=5e-5 if dtype == np.float32 else 1e-11)
