@@ -327,7 +327,7 @@ def gpu_lloyd_step_time(cfg, reps, consecutive=False, flags=0):
             torch.cuda.synchronize()
             return time.perf_counter() - t0, int(n_iter)
 
-        run(2)
+        run(5 + reps)  # (the first launch of a kernel loads its code, 2.6 ms: also of those that only later iterations use)
         t_short, it_short = run(5)
         t_long, it_long = run(5 + reps)
         if it_long <= it_short:
