@@ -355,10 +355,10 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
     const int items = (d + 1) * k;
     if (kept.hi != nullptr) {
         // The sums that a run keeps (lloyd_moves.hip): converted with one rounding, and left as they are.  The first
-        // workgroup takes the sizes and, if one is zero, the end below, a thread what it has written itself; the others
-        // take the sums.  None waits for another, and the list is made only if there is one: with a ticket and
-        // fences at the end of each of 128 workgroups, and the list always, 1 024 clusters of 256 features took 22 us,
-        // 100 of 100 (fp64) 9, now 5 both.
+        // workgroup takes the sizes and, if one is zero, the list below, a thread what it has written itself; the others
+        // take the sums.  None waits for another, so none may write the state that all of them ask for on entry:
+        // the finalisation behind this launch stops the run.  With a ticket and fences at the end of each of
+        // 128 workgroups, and the list always, 1 024 clusters of 256 features took 22 us, 100 of 100 (fp64) 9, now 5 both.
         const bool odd = kept.header[KMX_TH_FINITE] == 0u || kept.header[KMX_TH_ODD] != 0u;
         auto converted = [&](const int item, const int q) __attribute__((always_inline)) {
             const double unit = __hiloint2double((1023 - q) << 20, 0);  // 2^-q
@@ -512,7 +512,7 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
         status->reserved[0] = bidx;
         status->n_empty = base;
         status->ticket = 0;
-        if (base > 0) {
+        if (base > 0 && kept.hi == nullptr) {  // (the last workgroup: all have asked for the state)
             status->state = KMX_NEED_RELOCATION;
             lloyd_publish(progress, status, status->n_iter, KMX_NEED_RELOCATION, base, status->shift_sum);
         }
@@ -539,6 +539,15 @@ __global__ __launch_bounds__(256) void lloyd_finalize_kernel(
     const int state = status->state;
     if (force ? (state != KMX_NEED_RELOCATION && state != KMX_RUNNING) : (state != KMX_RUNNING))
         return;
+    if (!force && status->n_empty > 0) {
+        // (sums kept by the run: the launch before has left this to be said here.  Workgroups that see it said
+        // already return all the same)
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            status->state = KMX_NEED_RELOCATION;
+            lloyd_publish(progress, status, status->n_iter, KMX_NEED_RELOCATION, status->n_empty, status->shift_sum);
+        }
+        return;
+    }
     constexpr int CPW = 256 / LANES;  // clusters per workgroup
     const int cl = threadIdx.x & (CPW - 1), grp = threadIdx.x / CPW;
     const int c = blockIdx.x * CPW + cl;

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 HEADER_SUMS = 7  # word of the copy's header: iterations behind the kept sums
 HEADER_KEEP = 5  # whether the last iteration had sums to correct
 HEADER_ENTRIES = 4
+KMX_NEED_RELOCATION = 4
 
 
 def _words(run):
@@ -119,3 +120,38 @@ def test_sums_of_data_of_any_magnitude(cuda, scale, weight_scale, dtype):
         want = np.bincount(lab, weights=X[:, f].astype(np.float64) * w, minlength=k)[full] / sizes[full]
         tol = 4 * np.finfo(dtype).eps if dtype == np.float32 else 1e-13  # (as above)
         np.testing.assert_allclose(c[f][full], want, rtol=tol, atol=tol * float(np.abs(X[:, f]).max()))
+
+
+def test_all_sums_are_converted_when_the_gpu_is_busy(cuda):
+    """An iteration that ends with empty clusters: the workgroup that finds them is the launch's first and does not wait
+    for the 1 024 that convert the sums.  Another stream keeps the GPU busy with workgroups of a thousand threads, each
+    on a long row, so that many of them start behind its end."""
+    import torch
+
+    n, d, k = 20_003, 256, 1024
+    X, w, init = _blobs(n, d, k, np.float32, 6)
+    init[-16:] = 1e4
+    load = torch.rand(1024, 1 << 19, device=cuda)
+    out = torch.empty_like(load)
+    side = torch.cuda.Stream()
+    expected = None
+    for busy in [False] + [True] * 8:
+        run = _ResidentRun(cuda, X, w, init, 2)
+        run.cent[1].fill_(float("nan"))
+        torch.cuda.synchronize()
+        if busy:
+            with torch.cuda.stream(side):
+                for _ in range(20):
+                    torch.softmax(load, 1, out=out)
+        run.run(1)
+        torch.cuda.synchronize()
+        assert (run.status.state, run.status.n_empty, run.status.n_iter) == (KMX_NEED_RELOCATION, 16, 0)
+        assert sorted(run.empty[:16].tolist()) == list(range(k - 16, k))
+        sums = run.cent[1].cpu().numpy()
+        assert np.isfinite(sums).all()
+        if expected is None:
+            lab, expected = run.labels[1].cpu().numpy(), sums
+            for f in (0, d - 1):
+                want = np.bincount(lab, weights=X[:, f].astype(np.float64) * w, minlength=k)
+                np.testing.assert_allclose(sums[f], want, rtol=1e-6, atol=1e-6 * np.abs(X[:, f]).max())
+        np.testing.assert_array_equal(sums, expected)
