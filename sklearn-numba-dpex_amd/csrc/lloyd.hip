@@ -1407,8 +1407,9 @@ int32_t kmx_lloyd_run(const kmx_lloyd_plan* plan, const void* X_t, const void* X
             if (max_iter - enqueued < 4 || changed * 16 > plan->n || looked * 24 > plan->n) return false;
             if (!spread_asked) {
                 spread_asked = true;
+                const LloydLayout L = lloyd_layout(plan->n, plan->d, plan->k, plan->dtype, plan->flags);
                 bounds_rc = kmx_bounds_spread(X_t, cent[a], labels[a], (const kmx_lloyd_status*)workspace,
-                                              slot + KMX_PROGRESS_SPREAD, plan->n, plan->d, plan->k, plan->dtype, stream);
+                                              (const unsigned int*)((const char*)workspace + L.off_scales), slot + KMX_PROGRESS_SPREAD, plan->n, plan->d, plan->k, plan->dtype, stream);
                 return false;
             }
             // The share of the samples that it will look at is about two and a half times the root of the squared

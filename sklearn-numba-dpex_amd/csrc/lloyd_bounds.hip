@@ -18,7 +18,8 @@
 // other are further apart than two errors E of the chain: with r of the margin left and D the distance to the
 // own centroid those scores are at least r D + r^2 / 2 apart, and D is still at least D0 - (margin - r); the word
 // leaves out as much of the margin as makes that exceed 2 E, with E for the largest centroid that means of the
-// data can be.  The sums are fixed point: a sample that moves is taken off its old cluster and added to the new
+// data can be.  Scores, margins and drift are those of scaled values (the largest coordinate in
+// [2^12, 2^13)): squares of the data themselves leave fp32 from 1e-19 and 1e19 on, with the bounds made of them.  The sums are fixed point: a sample that moves is taken off its old cluster and added to the new
 // one, exactly.
 //
 // bounds_kernel<ENTER> is an iteration over all samples that also writes the words and, in fp32, the rows of X side
@@ -95,16 +96,18 @@ inline BoundsArea bounds_area(int64_t n, int d, int k) {
 }
 
 // What a chain of d fused multiply-adds from the half norm (d more) can be off by is chain_ulp (d + 8)
-// (|x| R + R^2), R the largest centroid norm, and chain_tiny (d + 8) where products underflow.
+// (|x| R + R^2), R the largest centroid norm, and chain_tiny (d + 8) where products underflow: in fp32 those of the
+// values themselves, not of scaled ones.
 template <typename T>
 constexpr float chain_ulp() { return sizeof(T) == 8 ? 2.3e-16f : 1.2e-7f; }
-constexpr float chain_tiny = 2e-36f;  // (fp64 too: margins are fp32)
+template <typename T>
+__device__ __forceinline__ float chain_tiny(const float xs) { return sizeof(T) == 8 ? 2e-36f : fmaxf(2e-36f * xs * xs, 2e-36f); }
 
 __device__ __forceinline__ float chain_fma(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double chain_fma(double a, double b, double c) { return fma(a, b, c); }
 
 // The margin of a sample, rounded down (zero: look at it next time, whatever the drift).  x_sq = |x|^2 to within
-// rel, best and second scores to within e_score, e_chain: E above.
+// rel, best and second scores to within e_score, e_chain: E above, all of scaled values.
 __device__ __forceinline__ float margin_of(const float x_sq, const float best, const float second, const float rel,
                                            const float e_score, const float e_chain) {
     const float spread = rel * x_sq + 2.01f * e_score;
@@ -140,8 +143,8 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     TX* frag = reinterpret_cast<TX*>(bounds_raw + lay.off_frag);                   // the chain's centroids
     TX* half_s = reinterpret_cast<TX*>(bounds_raw + lay.off_half);                 // -0.5 |c|^2, -inf past k
     float* drift_s = reinterpret_cast<float*>(bounds_raw + lay.off_drift);         // drift by now
-    float* step_s = drift_s + lay.kp;                                              // |c_new - c_old|
-    float* norm_s = step_s + lay.kp;                                               // |c|, rounded up
+    float* step_s = drift_s + lay.kp;                                              // |c_new - c_old|, scaled
+    float* norm_s = step_s + lay.kp;                                               // |c|, scaled, rounded up
     float* part_s = reinterpret_cast<float*>(bounds_raw + lay.off_part);           // its square, by eight features
     uint32_t* moved = reinterpret_cast<uint32_t*>(bounds_raw + lay.off_moved);     // [MOVED_MAX][2]: sample; old and new label
     uint32_t* u_index = reinterpret_cast<uint32_t*>(bounds_raw + lay.off_unsure);  // samples without a certificate
@@ -195,16 +198,17 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     if ((int)threadIdx.x <= d) q_s[threadIdx.x] = my_q;
     if (threadIdx.x == 0) queued = unsure_count = moved_count = changed_s = 0u;
     for (int i = threadIdx.x; i < (d + 1) * k; i += THREADS) acc[i] = 0ull;
-    // The largest coordinate sets the screen's scale (a centroid beyond it overflows, and costs certificates
-    // only); the box they span bounds the norm of any mean of the data.
-    float x_most = __uint_as_float(my_absmax), box = x_most * x_most;
+    // The largest coordinate sets the scale (a centroid beyond it overflows, and costs certificates only); the box
+    // they span bounds the norm of any mean of the data.
+    float x_most = __uint_as_float(my_absmax);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        box += __shfl_xor(box, off, 64);
-        x_most = fmaxf(x_most, __shfl_xor(x_most, off, 64));
-    }
-    box = sqrtf(box) * 1.0002f;
+    for (int off = 32; off > 0; off >>= 1) x_most = fmaxf(x_most, __shfl_xor(x_most, off, 64));
     const float xs = __uint_as_float((unsigned int)__builtin_amdgcn_readfirstlane((int)__float_as_uint(screen_scale(x_most))));
+    float box = __uint_as_float(my_absmax) * xs;
+    box *= box;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) box += __shfl_xor(box, off, 64);
+    box = sqrtf(box) * 1.0002f;
     // Centroid (f, c) of the chain: fp32 v_mfma_f32_32x32x2, lane (c % 32, f % 2), pair f / 2, four pairs side by
     // side; fp64 v_mfma_f64_16x16x4, lane (c % 16, f % 4), step f / 4, two steps side by side.
     auto place = [&](const int f, const int c) __attribute__((always_inline)) {
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
         v8h hi, lo;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const TX diff = now[e] - was[e];
+            const TX diff = (now[e] - was[e]) * (TX)xs;
             df = chain_fma(diff, diff, df);
             frag[place(8 * g + e, c)] = now[e];
             const float v = (float)now[e] * xs;
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     }
     __syncthreads();
     for (int c = threadIdx.x; c < kp; c += THREADS) {
-        TX sq = TX(0);
+        TX sq = TX(0), sq_scaled = TX(0);
         float df = 0.0f;
 #pragma unroll 1
         for (int g = 0; g < 2 * NK; ++g) {
@@ -242,13 +246,17 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = frag[place(8 * g + e, c)];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) sq = chain_fma(v[e], v[e], sq);  // (fused as in the other steps: near ties hang on it)
+            for (int e = 0; e < 8; ++e) {
+                sq = chain_fma(v[e], v[e], sq);  // (fused as in the other steps: near ties hang on it)
+                const TX vs = v[e] * (TX)xs;
+                sq_scaled = chain_fma(vs, vs, sq_scaled);
+            }
             if (!ENTER) df += part_s[g * kp + c];
         }
         half_s[c] = c < k ? -(sq / TX(2)) : -kmx_inf<TX>();
-        hneg_s[c] = c < k ? -((float)sq / 2.0f) * xs * xs : -kmx_inf<float>();
-        norm_s[c] = sqrtf((float)sq * 1.000001f) * 1.000001f;
-        step_s[c] = !ENTER && c < k ? sqrtf(df) * 1.00001f + 1e-17f : 0.0f;
+        hneg_s[c] = c < k ? -((float)sq_scaled / 2.0f) : -kmx_inf<float>();
+        norm_s[c] = sqrtf((float)sq_scaled * 1.000001f) * 1.000001f;
+        step_s[c] = !ENTER && c < k ? sqrtf(df) * 1.00001f + 1e-17f : 0.0f;  // (squares that underflow: 1e-21 of the data)
     }
     __syncthreads();
     // The largest norm and the two largest steps, by every wave for itself (as bits: a NaN is the largest).
@@ -283,13 +291,13 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     }
     __syncthreads();
 
-    // bounds of a score's error: of the chain now and later, of the screen (scaled; E of lloyd_mfma_screen.hip)
+    // bounds of a score's error: of the chain now and later, of the screen (E of lloyd_mfma_screen.hip)
     const float n_round = (float)(d + 8), rel = n_round * 1.2e-7f;
-    const float cmax = norm_most * xs, hmax = 0.5f * cmax * cmax;
+    const float chain_0 = n_round * chain_tiny<TX>(xs);
+    const float cmax = norm_most, hmax = 0.5f * cmax * cmax;
     const float round_term = SCR_ERR_ROUND * 51.0f * (float)NK, abs_term = SCR_ERR_ABS * sqrtf((float)d);
     const float scr_x = 1.001f * ((F64 ? SCR_ERR_SPLIT_F64 : SCR_ERR_SPLIT) + round_term) * cmax + abs_term;
     const float scr_0 = 1.001f * (round_term + (F64 ? SCR_ERR_HNEG_F64 : 0.0f)) * hmax + abs_term * cmax;
-    const float unscale = 1.0f / xs;
     const float neg_inf = -kmx_inf<float>();
     float pos_inf = kmx_inf<float>();
     asm volatile("" : "+s"(pos_inf));  // (keeps the first maximum of a group an instruction the compiler sees as such)
@@ -453,7 +461,10 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
                 xh[s] = __builtin_bit_cast(v8h, make_uint4(hw[0], hw[1], hw[2], hw[3]));
                 xl[s] = __builtin_bit_cast(v8h, make_uint4(lw[0], lw[1], lw[2], lw[3]));
 #pragma unroll
-                for (int e = 0; e < 8; ++e) sq = fmaf(x[s][e], x[s][e], sq);
+                for (int e = 0; e < 8; ++e) {
+                    const float v = x[s][e] * xs_sc;
+                    sq = fmaf(v, v, sq);
+                }
             }
         }
         sq += __shfl_xor(sq, 32, 64);
@@ -527,14 +538,12 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
         }
         // certain when the lead exceeds two errors (a NaN anywhere makes it uncertain)
         const float norm = sqrtf(sq) * 1.001f;
-        const float e_scr = fmaf(scr_x, norm * xs, scr_0);
+        const float e_scr = fmaf(scr_x, norm, scr_0);
         const bool owner = valid && h == 0;
         const bool unsure = owner && !(best - second > 2.01f * e_scr);
         if (owner && !unsure) {
-            const float e_chain = n_round * chain_ulp<TX>() * (norm + r_max) * r_max + n_round * chain_tiny;
-            settle(idx, old_label, (uint32_t)label,
-                   margin_of(sq, best * unscale * unscale, second * unscale * unscale, rel,
-                                    e_scr * unscale * unscale, e_chain));
+            const float e_chain = n_round * chain_ulp<TX>() * (norm + r_max) * r_max + chain_0;
+            settle(idx, old_label, (uint32_t)label, margin_of(sq, best, second, rel, e_scr, e_chain));
         }
         const unsigned long long um = __ballot(unsure);
         if (um != 0ull) {
@@ -764,13 +773,23 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
 
 // Root mean square distance of a thousand samples to their centroids, for the host (system scope): how far
 // centroids may move before bounds are of no use.  One workgroup; 64 samples in a row at sixteen places (a thousand
-// places take 30 to 110 us, a page of memory and its translation per value).
+// places take 30 to 110 us, a page of memory and its translation per value).  Zero, no use at all, for data beyond
+// these magnitudes: an fp32 chain whose products leave its range does not find what the screen certifies, and which
+// sample goes which way then decides its label.  Rounding to a multiple of fp32's smallest normal number is 4e-3 of
+// scaled squares at the lower end, a hundredth of the least lead that the screen certifies where the largest centroid is
+// a tenth of the largest coordinate; at the upper end 64 squares stay within fp32.
+constexpr float BOUNDS_LEAST = 5.7e-14f, BOUNDS_MOST = 1.1e18f;  // 2^-44, 2^60
 template <typename TX>
 __global__ __launch_bounds__(1024) void spread_kernel(const TX* __restrict__ X_t, const TX* __restrict__ centroids_t,
                                                       const uint32_t* __restrict__ labels,
                                                       const kmx_lloyd_status* __restrict__ status,
+                                                      const unsigned int* __restrict__ absmax,
                                                       unsigned long long* __restrict__ out, int64_t n, int d, int k) {
     if (status->state != KMX_RUNNING) return;
+    unsigned int most = (int)threadIdx.x < d ? absmax[threadIdx.x] : 0u;  // (d <= 64: the first wave)
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) most = max(most, (unsigned int)__shfl_xor((int)most, off, 64));
+    const bool within = __uint_as_float(most) >= BOUNDS_LEAST && __uint_as_float(most) <= BOUNDS_MOST;
     __shared__ double scratch[16];
     const int64_t place = (int64_t)(threadIdx.x >> 6) * n / 16 + (threadIdx.x & 63);
     const int64_t i = place < n ? place : n - 1;
@@ -785,8 +804,8 @@ __global__ __launch_bounds__(1024) void spread_kernel(const TX* __restrict__ X_t
     }
     const double total = kmx_block_sum<double>(sq, scratch);
     if (threadIdx.x == 0)
-        __hip_atomic_store(out, (unsigned long long)__double_as_longlong(sqrt(total / 1024.0)), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(out, (unsigned long long)__double_as_longlong(within ? sqrt(total / 1024.0) : 0.0),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <typename TX, int NK>
@@ -879,13 +898,13 @@ int32_t kmx_lloyd_iter_bounds(const LloydLayout& L, bool enter, char* area, int 
 }
 
 int32_t kmx_bounds_spread(const void* X_t, const void* centroids_t, const uint32_t* labels, const kmx_lloyd_status* status,
-                          unsigned long long* out, int64_t n, int d, int k, int dtype, hipStream_t stream) {
+                          const unsigned int* absmax, unsigned long long* out, int64_t n, int d, int k, int dtype, hipStream_t stream) {
     if (dtype == KMX_F32)
         hipLaunchKernelGGL((spread_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)X_t, (const float*)centroids_t,
-                           labels, status, out, n, d, k);
+                           labels, status, absmax, out, n, d, k);
     else
         hipLaunchKernelGGL((spread_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)X_t,
-                           (const double*)centroids_t, labels, status, out, n, d, k);
+                           (const double*)centroids_t, labels, status, absmax, out, n, d, k);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }

@@ -430,7 +430,7 @@ int32_t kmx_lloyd_iter_fewk(const LloydLayout& L, const void* X_t, const void* X
 // iterations of the screened steps that look only at samples whose label can have changed (lloyd_bounds.hip)
 size_t kmx_bounds_bytes(int64_t n, int d, int k);
 int32_t kmx_bounds_spread(const void* X_t, const void* centroids_t, const uint32_t* labels, const kmx_lloyd_status* status,
-                          unsigned long long* out, int64_t n, int d, int k, int dtype, hipStream_t stream);
+                          const unsigned int* absmax, unsigned long long* out, int64_t n, int d, int k, int dtype, hipStream_t stream);
 int32_t kmx_lloyd_iter_bounds(const LloydLayout& L, bool enter, char* area, int parity, const void* X_t, const void* w,
                               const void* centroids_t, void* new_centroids_t, uint32_t* labels_a, uint32_t* labels_b,
                               void* sizes, uint32_t* empty_clusters, char* ws, int64_t n, int d, int k, int dtype,

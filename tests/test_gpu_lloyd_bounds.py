@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 MARK = 0xFF
 
 
-def _run(X_t, w, init_t, max_iter, with_bounds):
+def _run(X_t, w, init_t, max_iter, with_bounds, must_enter=True):
     import torch
 
     from sklearn_numba_dpex_amd import _capi
@@ -32,20 +32,25 @@ def _run(X_t, w, init_t, max_iter, with_bounds):
     check(lib.kmx_lloyd_run(plan, ptr(X_t), None, ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]), ptr(labels[1]),
                             ptr(sizes), ptr(empty), ptr(ws), ws.numel(), ptr(area), need, 0, max_iter, status, stream), "run")
     torch.cuda.synchronize()
-    if with_bounds:
+    # (conditions first: pytest iterates over the tensors of a comparison that an assert contains)
+    if with_bounds and not must_enter:
+        untouched = bool((area == MARK).all())
+        assert untouched
+    elif with_bounds:
         # drift of the labels (two copies), then a word per sample: every one has been written, and some
         # samples were passed over at least once (what they have seen of the drift is behind it by then)
         words = area[(2 * k * 4 + 255) // 256 * 256:][: 4 * n].view(torch.int32)
-        assert bool((words != -1).all()), "no bounded iteration has run"
-        assert bool(((words & 0x7FF) < k).all())
+        written, labels_fit = bool((words != -1).all()), bool(((words & 0x7FF) < k).all())
+        assert written and labels_fit, "no bounded iteration has run"
     at = status.n_iter % 2
-    return dict(n_iter=status.n_iter, state=status.state, labels=labels[at], cent=cent[at], sizes=sizes)
+    return dict(n_iter=status.n_iter, state=status.state, labels=labels[at], cent=cent[at], sizes=sizes,
+                before=cent[at ^ 1])
 
 
 def _same(a, b):
     assert (a["n_iter"], a["state"]) == (b["n_iter"], b["state"])
-    for name in ("labels", "sizes", "cent"):
-        assert bool((a[name] == b[name]).all()), name
+    differ = [name for name in ("labels", "sizes", "cent") if not bool((a[name] == b[name]).all())]
+    assert not differ
 
 
 def _blobs(n, d, k, dtype, seed, cuda, spread=5.0):
@@ -133,3 +138,23 @@ def test_run_with_relocated_clusters(dtype, cuda, monkeypatch):
     without = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
     assert with_bounds[3] == without[3] and with_bounds[1] == without[1]
     assert bool((with_bounds[0] == without[0]).all()) and bool((with_bounds[2] == without[2]).all())
+
+
+# from 6e-14 to 1e18 (the data are about 15 wide) labels are those of bounded iterations; beyond, an fp32 chain loses
+# products that the screen keeps (7e-22: other labels than those of the screened step), and they are not entered
+@pytest.mark.parametrize("scale, dtype, entered", [
+    (1e-25, "float64", False), (1e-16, "float64", False), (1e-14, "float64", True), (3e16, "float64", True),
+    (2e17, "float64", False), (1e25, "float64", False),
+    (1e-22, "float32", False), (7e-22, "float32", False), (1e-16, "float32", False), (1e-14, "float32", True),
+    (3e16, "float32", True), (2e17, "float32", False),
+])
+def test_data_of_any_magnitude(scale, dtype, entered, cuda):
+    import torch
+
+    n, d, k = 1_200_001, 14, 64
+    X_t, w, init = _blobs(n, d, k, torch.float64, 11, cuda, spread=10.0)
+    X_t, w, init = ((scale * X_t).to(getattr(torch, dtype)), w.to(getattr(torch, dtype)),
+                    (scale * init).to(getattr(torch, dtype)))
+    a = _run(X_t, w, init, 30, False)
+    b = _run(X_t, w, init, 30, True, entered)
+    _same(a, b)
