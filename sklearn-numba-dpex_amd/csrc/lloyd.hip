@@ -353,23 +353,23 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
     unsigned long long* __restrict__ progress, KmxKept kept, int rest) {
     if (status->state != KMX_RUNNING) return;
     const int items = (d + 1) * k;
-    if (kept.hi != nullptr) {
+    if (kept.header != nullptr) {
         // The sums that a run keeps (lloyd_moves.hip): converted with one rounding, and left as they are.  The first
         // workgroup takes the sizes and, if one is zero, the list below, a thread what it has written itself; the others
         // take the sums.  None waits for another, so none may write the state that all of them ask for on entry:
         // the finalisation behind this launch stops the run.  With a ticket and fences at the end of each of
         // 128 workgroups, and the list always, 1 024 clusters of 256 features took 22 us, 100 of 100 (fp64) 9, now 5 both.
-        const bool odd = kept.header[KMX_TH_FINITE] == 0u || kept.header[KMX_TH_ODD] != 0u;
+        const bool fixed = kept.header[KMX_TH_FIXED] != 0u;
         auto converted = [&](const int item, const int q) __attribute__((always_inline)) {
+            const long long top = (long long)kept.sums[0][item];
+            if (!fixed) return (T)__longlong_as_double(top);
             const double unit = __hiloint2double((1023 - q) << 20, 0);  // 2^-q
-            const long long hi = (long long)kept.hi[item];
-            const double a = (double)hi;
-            double v = a * unit;
-            if (sizeof(T) == 8) {
-                const double small = (double)(long long)kept.lo[item] * __hiloint2double((1023 - q - rest) << 20, 0);
-                v += (double)(hi - (long long)a) * unit + small;
-            }
-            return (T)(odd ? v + kept.odd[item] : v);
+            const double a = (double)top;
+            double below = (double)(top - (long long)a) * unit;
+#pragma unroll
+            for (int i = 2; i > 0; --i)
+                if (i < kept.words) below += (double)(long long)kept.sums[i][item] * __hiloint2double((1023 - q - i * rest) << 20, 0);
+            return (T)(a * unit + below);
         };
         if (blockIdx.x != 0) {
             const int stride = ((int)gridDim.x - 1) * 256;
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
     // ---- last block: empty-cluster list + heaviest cluster (left to the one-workgroup
     // finalisation kernel when that one follows)
     if (!with_tail) return;
-    if (kept.hi == nullptr) {
+    if (kept.header == nullptr) {
         __shared__ unsigned int is_last;
         __threadfence();
         __syncthreads();
@@ -512,7 +512,7 @@ __global__ __launch_bounds__(256) void lloyd_reduce_kernel(
         status->reserved[0] = bidx;
         status->n_empty = base;
         status->ticket = 0;
-        if (base > 0 && kept.hi == nullptr) {  // (the last workgroup: all have asked for the state)
+        if (base > 0 && kept.header == nullptr) {  // (the last workgroup: all have asked for the state)
             status->state = KMX_NEED_RELOCATION;
             lloyd_publish(progress, status, status->n_iter, KMX_NEED_RELOCATION, base, status->shift_sum);
         }
@@ -855,13 +855,13 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         // labels from the half-precision copy, and sums that are corrected for the samples that move (their rows
         // are read four features at a time: narrower ones are summed as without the copy, below)
         const unsigned int* absmax = reinterpret_cast<const unsigned int*>(ws + L.off_scales);
-        kept = kmx_tiles_kept(L.tiles, absmax, n, d, k);
+        const bool wide = L.variant == KMX_VARIANT_MFMA_WIDE;
+        kept = kmx_tiles_kept(L.tiles, absmax, n, d, k, kmx_kept_words((int)sizeof(T), wide));
         constexpr int32_t dtype = sizeof(T) == 8 ? KMX_F64 : KMX_F32;
-        unsigned int* const listed = L.variant == KMX_VARIANT_MFMA_WIDE
-                                         ? const_cast<unsigned int*>(kmx_wide_screen_counter(ws + L.off_wscreen))
-                                         : nullptr;
+        unsigned int* const listed =
+            wide ? const_cast<unsigned int*>(kmx_wide_screen_counter(ws + L.off_wscreen)) : nullptr;
         int32_t rc = kmx_tiles_labels(X_t, X_rowmajor, centroids_t, cpack, half_norms, L.tiles, status, labels, n, d, L.dpad,
-                                      k, dtype, stream, listed, labels_prev, absmax);
+                                      k, dtype, stream, listed, labels_prev, absmax, kmx_kept_span(n, (int)sizeof(T), wide));
         if (rc != KMX_OK) return rc;
         rc = kmx_lloyd_kept_sums(X_rowmajor, w, labels_prev, labels, kept, status, ws + L.off_bucket, n, d, k, dtype, stream);
         if (rc != KMX_OK) return rc;
@@ -936,7 +936,7 @@ int32_t lloyd_iter_impl(const LloydLayout& L, const void* X_t, const void* X_row
         }
     }
     const int64_t kept_grid = 1 + (kmx_cdiv((int64_t)d * k, 256) < 1024 ? kmx_cdiv((int64_t)d * k, 256) : 1024);
-    const int64_t reduce_grid = kept.hi != nullptr ? kept_grid
+    const int64_t reduce_grid = kept.header != nullptr ? kept_grid
                                 : (gsum != nullptr || n_partials_used == 1)
                                     ? (kmx_cdiv(items, 256) < 128 ? kmx_cdiv(items, 256) : 128)
                                     : kmx_cdiv(items, RED_ITEMS);
@@ -1090,7 +1090,9 @@ int32_t kmx_lloyd_plan_reads_rowmajor(const kmx_lloyd_plan* plan) {
 size_t kmx_lloyd_resident_bytes(const kmx_lloyd_plan* plan) {
     if (plan_validate(plan) != KMX_OK) return 0;
     const LloydLayout L = lloyd_layout(plan->n, plan->d, plan->k, plan->dtype, plan->flags);
-    return lloyd_tiles_wanted(L, plan->n, plan->d, plan->k, plan->dtype) ? kmx_tiles_bytes(plan->n, plan->d, plan->k) : 0;
+    if (!lloyd_tiles_wanted(L, plan->n, plan->d, plan->k, plan->dtype)) return 0;
+    return kmx_tiles_bytes(plan->n, plan->d, plan->k,
+                           kmx_kept_words((int)kmx_dtype_size(plan->dtype), L.variant == KMX_VARIANT_MFMA_WIDE));
 }
 
 size_t kmx_lloyd_bounds_bytes(const kmx_lloyd_plan* plan) {
@@ -1186,7 +1188,7 @@ static int32_t lloyd_init_impl(const kmx_lloyd_plan* plan, void* workspace, size
         // (for the screened tiled product: max|x| per feature, from which its scale is taken)
         // (the pass over X that makes the resident copies takes the maxima along)
         if (resident != nullptr) {
-            const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, centroids_t, resident, absmax, n, d, k, dtype, stream);
+            const int32_t rc = kmx_tiles_prepare(X_t, X_rowmajor, sample_weight, centroids_t, resident, absmax, n, d, k, dtype, stream);
             if (rc != KMX_OK) return rc;
         }
         const int32_t rc = kmx_lloyd_mfma_prepare(L, resident != nullptr ? nullptr : X_t, sample_weight, ws, n, d, dtype, stream);

@@ -83,44 +83,86 @@ constexpr int KMX_TH_REST = 2;     // samples left to the tiled product
 constexpr int KMX_TH_MOVED = 3;    // samples with a certificate whose label is another one than before
 constexpr int KMX_TH_ENTRIES = 4;  // two for every sample that moved
 constexpr int KMX_TH_KEEP = 5;     // whether the kept sums are those of the labels before
-constexpr int KMX_TH_FINITE = 6;   // no NaN or infinity, no maximum past fp32's largest, not all of them below its smallest
+constexpr int KMX_TH_FIXED = 6;    // whether the sums are fixed point (kmx_kept_fixed), else fp64 additions
 constexpr int KMX_TH_SUMS = 7;     // iterations behind the kept sums (0: none)
-constexpr int KMX_TH_ODD = 8;      // NaN or infinity seen: among the samples (preparation), among the weights (sums)
+constexpr int KMX_TH_ODD = 8;      // NaN or infinity (past fp32's largest) seen among the samples or the weights
 constexpr int KMX_TH_WORDS = 64;
+// 64-bit words of a sum: the first holds a term to 41 binary places below its feature's largest (1e6 samples), every
+// further one 39 more.  A term then keeps its type's digits down to 2^-54 (fp32) and 2^-64 (fp64) of the largest.  The wide
+// fp32 step: one, as its own sums have.
+constexpr int kmx_kept_words(int esize, bool wide) { return esize == 8 ? 3 : wide ? 1 : 2; }
 struct KmxKept {
     unsigned int* header = nullptr;
     const unsigned int* absmax = nullptr;  // bits of max |x| per feature and of max |w|, in fp32
     int64_t n = 0;
-    unsigned long long* hi = nullptr;   // (d + 1, k) sums, 64-bit fixed point (kmx_kept_exponent)
-    unsigned long long* lo = nullptr;   // fp64: what the terms of `hi` leave out, kmx_kept_rest more binary places
-    double* odd = nullptr;              // values that are not finite
-    uint32_t* entry = nullptr;          // samples that moved, twice, and their clusters
+    int words = 0;
+    unsigned long long* sums[3] = {nullptr, nullptr, nullptr};  // (d + 1, k) each: word 0 in units of 2^-kmx_kept_exponent, word i
+                                                                // of 2^-(i kmx_kept_rest) of that; not fixed point: fp64 in the first
+    uint32_t* entry = nullptr;             // samples that moved, twice, and their clusters
     uint32_t* entry_cluster = nullptr;
 };
-// the rests of n terms, each at most half a unit of `hi`, stay within 2^59
+// the rests of n terms, each at most half a unit of the word before, stay within 2^59
 __host__ __device__ inline int kmx_kept_rest(int64_t n) {
     int en = 9;
     while (((int64_t)1 << en) < n && en < 31) ++en;  // n <= 2^en
     return 59 - en;
 }
-// Exponent of the sums of feature f (f = d: of the weights): n terms stay within 2^61, one within 2^50.  No clamp,
-// unlike the fused steps' (they scale in fp32): -226 to 346 are exponents that fp64 has, so data of any
-// magnitude keep their digits.  A maximum of zero may be fp64 values below fp32's smallest.
-__device__ inline int kmx_kept_exponent(const unsigned int* __restrict__ absmax, int64_t n, int d, int f) {
+// binary places of a term in the first word: n terms stay within 2^61, one within 2^50
+__host__ __device__ inline int kmx_kept_places(int64_t n) {
+    int en = 1;
+    while (((int64_t)1 << en) < n && en < 31) ++en;  // n <= 2^en
+    return 61 - en < 50 ? 61 - en : 50;
+}
+// Binary places by which a term may be smaller than the largest of its feature could be, so that its error stays below 2^-27
+// (fp32; 2^-25 of a term that the first word holds to 24 digits or more) or 2^-56 of itself: the rounding of its type.  Any for
+// the wide step, whose sums are fixed point whatever the range.
+constexpr int KMX_KEPT_ANY_SPAN = 1 << 20;
+inline int kmx_kept_span(int64_t n, int esize, bool wide) {
+    if (wide) return KMX_KEPT_ANY_SPAN;
+    return kmx_kept_places(n) + (kmx_kept_words(esize, wide) - 1) * kmx_kept_rest(n) - (esize == 8 ? 55 : 26);
+}
+// Exponent of the first word of feature f (f = d: of the weights).  No clamp,
+// unlike the fused steps' (they scale in fp32): -226 to 346 are exponents that fp64 has, so a factor common to all
+// data costs no digits.
+__device__ inline int kmx_kept_most(const unsigned int* __restrict__ absmax, int d, int f) {
     const float w = __uint_as_float(absmax[d]), x = f < d ? __uint_as_float(absmax[f]) : 1.0f;
     int e = kmx_not_finite(w) ? 0 : w > 0.0f ? ilogbf(w) + 1 : -149;
     if (f < d) e += kmx_not_finite(x) ? 0 : x > 0.0f ? ilogbf(x) + 1 : -149;
-    const int en = n > 2 ? 64 - __clzll(n - 1) : 1;  // n <= 2^en
-    return (61 - en < 50 ? 61 - en : 50) - e;
+    return e;
 }
-KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k);
+__device__ inline int kmx_kept_exponent(const unsigned int* __restrict__ absmax, int64_t n, int d, int f) {
+    const int en = n > 2 ? 64 - __clzll(n - 1) : 1;  // n <= 2^en
+    return (61 - en < 50 ? 61 - en : 50) - kmx_kept_most(absmax, d, f);
+}
+// The smallest magnitude but zero of a feature, for kmx_kept_fixed: the smallest of its values' bits without the sign less one,
+// which zero, then the largest, is out of (fp64: of the upper word's bits, and whether the lower one has any).
+__device__ __forceinline__ unsigned int kmx_least_word(float v) { return (__float_as_uint(v) << 1) - 1u; }
+__device__ __forceinline__ unsigned int kmx_least_word(double v) {
+    const unsigned int lo = (unsigned int)__double2loint(v);
+    return ((unsigned int)__double2hiint(v) << 1 | (lo < 1u ? lo : 1u)) - 1u;
+}
+// Whether the terms of feature f (f = d: the weights) have fixed point: finite, and none further than `span` below the largest.
+// least[f]: all bits of the smallest kmx_least_word flipped, so that zero stands for no value but zero.
+template <typename T>
+__device__ inline bool kmx_kept_fixed(const unsigned int* __restrict__ absmax, const unsigned int* __restrict__ least, int d, int f,
+                                      int span) {
+    const float x_most = __uint_as_float(absmax[f]), w_most = __uint_as_float(absmax[d]);
+    if (kmx_not_finite(x_most)) return false;
+    if (span >= KMX_KEPT_ANY_SPAN || least[f] == 0u) return true;
+    // (exponents of normal numbers; the maxima are fp32)
+    constexpr int SHIFT = sizeof(T) == 8 ? 21 : 24, BIAS = sizeof(T) == 8 ? 1023 : 127;
+    const int x = (int)((0u - least[f]) >> SHIFT), w = (int)((0u - least[d]) >> SHIFT);
+    if (x == 0 || w == 0 || x_most < 1.1754944e-38f || w_most < 1.1754944e-38f) return false;
+    return kmx_kept_most(absmax, d, f) - (f < d ? x - BIAS : 0) - (w - BIAS) <= span;
+}
+KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k, int words);
 int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_t* labels_prev, const uint32_t* labels,
                             const KmxKept& kept, kmx_lloyd_status* status, char* bucket, int64_t n, int d, int k,
                             int32_t dtype, hipStream_t stream);
 bool kmx_tiles_fit(int64_t n, int d, int k);
-size_t kmx_tiles_bytes(int64_t n, int d, int k);
-int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
-                          int64_t n, int d, int k, int dtype, hipStream_t stream);
+size_t kmx_tiles_bytes(int64_t n, int d, int k, int words);
+int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* w, const void* centroids_t, char* area,
+                          unsigned int* absmax, int64_t n, int d, int k, int dtype, hipStream_t stream);
 // the samples' tiles alone, for kmeans++: fragments, |x'|^2 and |e_x| per sample (scaled), the scale
 struct KmxTiles {
     const uint4* xt;
@@ -142,7 +184,7 @@ char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k);  // room for k 
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out = nullptr,
-                         const uint32_t* labels_prev = nullptr, const unsigned int* absmax = nullptr);
+                         const uint32_t* labels_prev = nullptr, const unsigned int* absmax = nullptr, int span = 0);
 // bucketed sums (lloyd_bucket.hip)
 size_t kmx_bucket_bytes(int64_t n, int k);
 int32_t kmx_bucket_offsets(const int* counts, int* offsets, const kmx_lloyd_status* status, int k, hipStream_t stream);

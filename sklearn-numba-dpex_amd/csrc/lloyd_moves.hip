@@ -5,14 +5,16 @@
 // added up in registers, one atomic per feature, stretch and cluster.  Few labels change after the first
 // iterations (1e6 x 256, 1 024 clusters within 3.5 standard deviations: 28, 7, 2 and 0.5 % in the second
 // to fifth), so an iteration sorts only the samples that moved, twice each, taken off the old cluster and added to
-// the new one.  That has to be exact, so the sums are integers: term = round(x w 2^q) in 64 bits, and for fp64 the
-// rest round((x w - term 2^-q) 2^p) in another 64, which leaves out 2^-80 of the largest term; sums
-// and corrections of the same labels are then the same bits in any order, and the
-// sum that an iteration divides has one rounding (fp64 additions in an order of their own before).
+// the new one.  That has to come to the same sums, so these are integers: round(x w 2^q) in 64 bits, what that leaves out,
+// 2^p as fine, in another 64 and, in fp64, the rest of that in a third; sums and corrections of the same labels are then
+// the same bits in any order.
 //
-// Values that are not finite, and those of a feature whose largest fp32 does not hold, have no such terms.  They are
-// added up as they are, in sums of their own that join in the end, and a run with any among its data rebuilds every
-// iteration (of fp64 features below fp32's smallest only where there are no others: beside those they are good to 2^-240).
+// Such a term is rounded at a place that the largest of its feature sets, 80 binary places below it for 1e6 samples in
+// fp32 and 119 in fp64.  So this is for data whose smallest |x| |w| but zero keep their digits (kmx_kept_fixed: 2^-54 and 2^-64
+// of the largest; the smallest of 1e9 normal values is 2^-33 of the largest, an outlier of 1e11 among values of
+// about 1 leaves them their digits).  Other runs, and those with NaN, infinities or fp64 values beyond fp32's range, add up in fp64 and
+// rebuild every iteration, as all did before.  The wide fp32 step's own sums are fixed point of one word, whatever the
+// range: so are these.
 //
 // Bound by the read of rows (a rebuild: 4.8 TB/s) or by a chain of trips to memory (corrections).  moves_sum_kernel, every
 // iteration a rebuild before: 1e6 x 256 fp32, 1 024 clusters 216 us, now 215 / 112 / 45 / 27 / 22 in the first five
@@ -38,6 +40,7 @@ __device__ __forceinline__ bool sums_corrected(const unsigned int* __restrict__ 
     return header[KMX_TH_KEEP] != 0u && listed <= (n >> 3) && 5 * moved <= 2 * n;
 }
 
+__device__ __forceinline__ float read_lane(float v, int src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); }
 __device__ __forceinline__ double read_lane(double v, int src) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src), __builtin_amdgcn_readlane(__double2loint(v), src));
 }
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(256) void moves_count_kernel(const uint32_t* __rest
 // The order: samples (rebuild; the kept sums are cleared) or entries by cluster.
 __global__ __launch_bounds__(256) void moves_scatter_kernel(const uint32_t* __restrict__ labels, KmxKept kept,
                                                             const int* __restrict__ offsets, const int* __restrict__ ranks,
-                                                            uint32_t* __restrict__ order, int64_t n, int items, bool two,
+                                                            uint32_t* __restrict__ order, int64_t n, int items,
                                                             const kmx_lloyd_status* __restrict__ status) {
     // (an iteration behind the end of the run: its labels may never have been written)
     if (status->state != KMX_RUNNING) return;
@@ -137,28 +140,28 @@ __global__ __launch_bounds__(256) void moves_scatter_kernel(const uint32_t* __re
     }
     for (int64_t i = first; i < n; i += stride) order[offsets[labels[i]] + ranks[i]] = (uint32_t)i;
     for (int64_t i = first; i < items; i += stride) {
-        kept.hi[i] = 0ull;
-        kept.odd[i] = 0.0;
-        if (two) kept.lo[i] = 0ull;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < kept.words) kept.sums[j][i] = 0ull;
     }
 }
 
 // LPR lanes take a row, 16 bytes each (RPW = 64 / LPR rows per wave and load); the features past LPR * V on the second
 // grid dimension.  A workgroup per stretch of the order, its four waves the rows in turn.  Clears counts
 // for the next iteration.
-template <typename T, int LPR>
-__global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_rm, const T* __restrict__ sample_weight,
+template <typename T, int LPR, int WORDS>
+__global__ __launch_bounds__(256, 4) void moves_sum_kernel(const T* __restrict__ X_rm, const T* __restrict__ sample_weight,
                                                         const uint32_t* __restrict__ order, const int* __restrict__ offsets,
                                                         int* __restrict__ counts, KmxKept kept,
                                                         const kmx_lloyd_status* __restrict__ status, int64_t n, int d, int k) {
     if (status->state != KMX_RUNNING) return;
-    constexpr bool TWO = sizeof(T) == 8;
     constexpr int V = 16 / (int)sizeof(T), RPW = 64 / LPR, FB = LPR * V, U = 4;  // (eight rows in flight: 272 for 216 us, half the waves)
     using Vec = typename KmxVec<T, V>::type;
-    __shared__ unsigned long long red_hi[4][FB + 1], red_lo[TWO ? 4 : 1][TWO ? FB + 1 : 1];
+    constexpr int REG = WORDS > 1 ? WORDS - 1 : 1;  // words of a feature in registers; the last one is in LDS
+    __shared__ unsigned long long red[REG][4][FB], red_w[WORDS][4], last[FB];
     __shared__ int c_first;
     const bool corrected = sums_corrected(kept.header, n);
-    const bool finite = kept.header[KMX_TH_FINITE] != 0u;
+    const bool fixed = kept.header[KMX_TH_FIXED] != 0u;
     const int total = offsets[k];
     int chunk = CHUNK;
     if (corrected) {
@@ -171,6 +174,8 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
     if (P0_64 >= total) return;
     const int P0 = (int)P0_64, P1 = total - P0 < chunk ? total : P0 + chunk;
     if (threadIdx.x == 0) c_first = k;
+    if (WORDS > 1)
+        for (int s = threadIdx.x; s < FB; s += 256) last[s] = 0ull;
     __syncthreads();
     // the (non-empty) cluster that holds position P0
     for (int c = threadIdx.x; c < k; c += 256)
@@ -185,29 +190,37 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
     const int fl = f0 + V <= d ? f0 : d - V;
     const bool lane_on = f0 < d;
     const int rest = kmx_kept_rest(n);
-    double m_hi[V], m_lo[V];
-    auto out_of_range = [&](const int f) __attribute__((always_inline)) {
-        const unsigned int bits = kept.absmax[f];
-        return kmx_not_finite(__uint_as_float(bits)) || (TWO && bits == 0u);
-    };
-    const bool w_as_is = out_of_range(d);
-    unsigned int as_is = 0u;  // bit j: the values of the lane's feature j are added up as they are
+    double magic[V], magic_w = 0.0;  // of the first word
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-        const int q = kmx_kept_exponent(kept.absmax, n, d, fl + j);
-        if (w_as_is || out_of_range(fl + j)) as_is |= 1u << j;
-        m_hi[j] = fix_magic(q);
-        m_lo[j] = fix_magic(q + rest);
-    }
-    const int q_w = kmx_kept_exponent(kept.absmax, n, d, d);
-    const double mw_hi = fix_magic(q_w), mw_lo = fix_magic(q_w + rest);
+    for (int j = 0; j < V; ++j) magic[j] = fixed ? fix_magic(kmx_kept_exponent(kept.absmax, n, d, fl + j)) : 0.0;
+    if (fixed) magic_w = fix_magic(kmx_kept_exponent(kept.absmax, n, d, d));
+    // (its binary point `rest` places further down per word)
+    auto magic_of = [&](const double first, const int word) __attribute__((always_inline)) {
+        return __hiloint2double(__double2hiint(first) - ((word * rest) << 20), 0);
+    };
     const T* __restrict__ col = X_rm + fl;
 
-    auto stretch = [&](auto finite_tag, const int p0, const int p1, const int c) __attribute__((always_inline)) {
-        constexpr bool FINITE = decltype(finite_tag)::value;
-        unsigned long long hi[V], lo[V], w_hi = 0ull, w_lo = 0ull;
+    auto stretch = [&](auto fixed_tag, const int p0, const int p1, const int c) __attribute__((always_inline)) {
+        constexpr bool FIXED = decltype(fixed_tag)::value;
+        unsigned long long sum[REG][V], w_sum[WORDS];
+        double plain[V], w_plain = 0.0;
 #pragma unroll
-        for (int j = 0; j < V; ++j) hi[j] = lo[j] = 0ull;
+        for (int i = 0; i < WORDS; ++i) w_sum[i] = 0ull;
+#pragma unroll
+        for (int i = 0; i < REG; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j) sum[i][j] = 0ull;
+#pragma unroll
+        for (int j = 0; j < V; ++j) plain[j] = 0.0;
+        // Terms x w: what a word leaves out, which has no error in fp32 and 2^-54 of itself in fp64, goes to the next; to the
+        // last one only of a term that the others hold to less than 24 (fp32) or 55 digits, one in ten thousand of
+        // normal values and next to none.  Those are read again and added to LDS: with the last word of all terms, in
+        // registers, the first iteration's sums took 235 us instead of 182 (1e6 x 100, 100 clusters fp64) and 8 us more in
+        // all iterations of 1e6 x 100, 128 clusters fp32 (one word 112, so 121).
+        const unsigned long long digits = 1ull << (WORDS == 3 ? 55 - rest : 24);  // (in units of the first word)
+        auto small = [&](const unsigned long long term) __attribute__((always_inline)) {  // |term| < digits
+            return term + (digits - 1ull) < 2ull * digits - 1ull;
+        };
         // each lane fetches one entry and its weight (a coalesced load and a gather per 64 entries), one group ahead of
         // the rows; lanes past the end hold the last one, weight 0
         auto fetch = [&](const int base, int& idx_out, T& w_out) __attribute__((always_inline)) {
@@ -222,91 +235,147 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
         fetch(p0, my_idx, my_w);
         for (int base = p0; base < p1; base += 64) {
             if (base + 64 < p1) fetch(base + 64, next_idx, next_w);
+            // (the weights: each lane the one that it holds, a wave every fourth group; beside the rows they cost half as
+            // much again as two fp64 features)
+            if ((((base - p0) >> 6) & 3) == wave) {
+                if constexpr (FIXED) {
+                    double left = (double)my_w;
+#pragma unroll
+                    for (int i = 0; i < WORDS; ++i) {
+                        const double m = magic_of(magic_w, i), t = left + m;
+                        w_sum[i] += to_fixed_q(t, m);
+                        left -= t - m;
+                    }
+                } else {
+                    w_plain += (double)my_w;
+                }
+            }
             const int n_here = p1 - base < 64 ? p1 - base : 64;
             for (int r0 = wave * RPW; r0 < n_here; r0 += 4 * RPW * U) {
                 Vec xv[U];
-                double wv[U];
+                T wv[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int src = r0 + 4 * RPW * u + sub;
                     const int idx = RPW == 1 ? __builtin_amdgcn_readlane(my_idx, src & 63) : __shfl(my_idx, src & 63, 64);
                     // (by all lanes, whichever of them have a row)
-                    const double w_at = RPW == 1 ? read_lane((double)my_w, src & 63) : (double)__shfl(my_w, src & 63, 64);
-                    wv[u] = src < n_here ? w_at : 0.0;
+                    const T w_at = RPW == 1 ? read_lane(my_w, src & 63) : __shfl(my_w, src & 63, 64);
+                    wv[u] = src < n_here ? w_at : T(0);
                     xv[u] = *reinterpret_cast<const Vec*>(col + (size_t)idx * (size_t)d);
                 }
+                unsigned int redo = 0u;  // bit u: some term of row u needs the last word (the same in all lanes)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const bool there = r0 + 4 * RPW * u + sub < n_here;
-                    if (!(fabs(wv[u]) < kmx_inf<double>())) {
-                        // (a weight that is not finite: its terms as they are; from the next iteration on FINITE is false)
-                        if (lane_on) {
-                            kept.header[KMX_TH_ODD] = 1u;
+                    if constexpr (FIXED) {
+                        bool more = false;
 #pragma unroll
-                            for (int j = 0; j < V; ++j)
-                                if (fl + j >= f0) kmx_atomic_add(kept.odd + (size_t)(fl + j) * k + c, (double)xv[u][j] * wv[u]);
-                            if (f0 == 0) kmx_atomic_add(kept.odd + (size_t)d * k + c, wv[u]);
+                        for (int j = 0; j < V; ++j) {
+                            const double x = (double)xv[u][j], w = (double)wv[u], first = magic[j], t = fma(x, w, first);
+                            const unsigned long long term = to_fixed_q(t, first);
+                            sum[0][j] += term;
+                            if constexpr (WORDS == 3) {
+                                const double m = magic_of(first, 1);
+                                sum[1][j] += to_fixed_q(fma(x, w, first - t) + m, m);
+                            }
+                            if constexpr (WORDS > 1) more |= small(term) && x != 0.0;
                         }
-                        continue;
+                        if (WORDS > 1 && __any(more && wv[u] != T(0))) redo |= 1u << u;
+                    } else if (r0 + 4 * RPW * u + sub < n_here) {  // (what is read twice may be infinite)
+#pragma unroll
+                        for (int j = 0; j < V; ++j) plain[j] = fma((double)xv[u][j], (double)wv[u], plain[j]);
                     }
+                }
+                while (FIXED && WORDS > 1 && redo != 0u) {
+                    const int u = __builtin_ctz(redo), src = r0 + 4 * RPW * u + sub;
+                    redo &= redo - 1u;
+                    const int idx = __shfl(my_idx, src & 63, 64);
+                    const T w_at = __shfl(my_w, src & 63, 64);
+                    const double w = src < n_here ? (double)w_at : 0.0;
+                    const Vec row = *reinterpret_cast<const Vec*>(col + (size_t)idx * (size_t)d);
+                    int down = rest;
+                    asm volatile("" : "+s"(down));  // (what is made of it stays in here)
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
-                        const double x = (double)xv[u][j];
-                        if (!FINITE && (((as_is >> j) & 1u) != 0u || !(fabs(x) < kmx_inf<double>()))) {
-                            if (lane_on && fl + j >= f0 && there && x != 0.0) kmx_atomic_add(kept.odd + (size_t)(fl + j) * k + c, x * wv[u]);
-                            continue;
+                        const double x = (double)row[j], first = magic[j], t = fma(x, w, first);
+                        double left = fma(x, w, first - t);
+                        if constexpr (WORDS == 3) {
+                            const double m = magic_of(first, 1);
+                            left -= (left + m) - m;
                         }
-                        const double t = fma(x, wv[u], m_hi[j]);
-                        hi[j] += to_fixed_q(t, m_hi[j]);
-                        if constexpr (TWO) lo[j] += to_fixed_q(fma(x, wv[u], m_hi[j] - t) + m_lo[j], m_lo[j]);
+                        const double m = __hiloint2double(__double2hiint(first) - (((WORDS - 1) * down) << 20), 0);
+                        if (lane_on && fl + j >= f0 && small(to_fixed_q(t, first)) && left != 0.0)
+                            atomicAdd(&last[fl + j - fb], to_fixed_q(left + m, m));
                     }
-                    if (!FINITE && w_as_is) {
-                        if (lane_on && f0 == 0 && there) kmx_atomic_add(kept.odd + (size_t)d * k + c, wv[u]);
-                        continue;
-                    }
-                    const double t = wv[u] + mw_hi;
-                    w_hi += to_fixed_q(t, mw_hi);
-                    if constexpr (TWO) w_lo += to_fixed_q((wv[u] + (mw_hi - t)) + mw_lo, mw_lo);
                 }
             }
             my_idx = next_idx;
             my_w = next_w;
         }
-        // the rows of a wave, then the waves in LDS; one global atomic per feature and stretch
+        if constexpr (!FIXED) {
+            // (their bits take the way of the first word)
 #pragma unroll
-        for (int off = LPR; off < 64; off <<= 1) {
+            for (int off = LPR; off < 64; off <<= 1) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) {
-                hi[j] += (unsigned long long)__shfl_xor((long long)hi[j], off, 64);
-                if constexpr (TWO) lo[j] += (unsigned long long)__shfl_xor((long long)lo[j], off, 64);
+                for (int j = 0; j < V; ++j) plain[j] += __shfl_xor(plain[j], off, 64);
             }
-            w_hi += (unsigned long long)__shfl_xor((long long)w_hi, off, 64);
-            if constexpr (TWO) w_lo += (unsigned long long)__shfl_xor((long long)w_lo, off, 64);
-        }
-        if (sub == 0 && lane_on) {
+            w_plain = kmx_wave_sum(w_plain);
 #pragma unroll
-            for (int j = 0; j < V; ++j)
-                if (fl + j >= f0) {
-                    red_hi[wave][fl + j - fb] = hi[j];
-                    if constexpr (TWO) red_lo[wave][fl + j - fb] = lo[j];
-                }
+            for (int j = 0; j < V; ++j) sum[0][j] = (unsigned long long)__double_as_longlong(plain[j]);
+            w_sum[0] = (unsigned long long)__double_as_longlong(w_plain);
         }
-        if (lane == 0) {
-            red_hi[wave][FB] = w_hi;
-            if constexpr (TWO) red_lo[wave][FB] = w_lo;
+        // the rows of a wave, then the waves in LDS; one global atomic per feature and stretch
+        constexpr int USED = FIXED ? REG : 1;
+#pragma unroll
+        for (int i = 0; i < USED; ++i) {
+            if constexpr (FIXED) {
+#pragma unroll
+                for (int off = LPR; off < 64; off <<= 1)
+#pragma unroll
+                    for (int j = 0; j < V; ++j) sum[i][j] += (unsigned long long)__shfl_xor((long long)sum[i][j], off, 64);
+            }
+            if (sub == 0 && lane_on) {
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (fl + j >= f0) red[i][wave][fl + j - fb] = sum[i][j];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < (FIXED ? WORDS : 1); ++i) {
+            if (FIXED && __any(w_sum[i] != 0ull)) w_sum[i] = kmx_wave_sum(w_sum[i]);
+            if (lane == 0) red_w[i][wave] = w_sum[i];
         }
         __syncthreads();
         const int here = d - fb < FB ? d - fb : FB;  // features of this part of the grid
-        for (int s = threadIdx.x; s <= here; s += 256) {
-            const bool weight = s == here;
-            if (weight && blockIdx.y != 0) continue;
-            const int slot = weight ? FB : s;
-            const size_t at = (size_t)(weight ? d : fb + s) * k + c;
-            const unsigned long long th = red_hi[0][slot] + red_hi[1][slot] + red_hi[2][slot] + red_hi[3][slot];
-            if (th != 0ull) atomicAdd(kept.hi + at, th);
-            if constexpr (TWO) {
-                const unsigned long long tl = red_lo[0][slot] + red_lo[1][slot] + red_lo[2][slot] + red_lo[3][slot];
-                if (tl != 0ull) atomicAdd(kept.lo + at, tl);
+        auto of = [&](const unsigned long long v) __attribute__((always_inline)) { return __longlong_as_double((long long)v); };
+        for (int s = threadIdx.x; s < here; s += 256) {
+            const size_t at = (size_t)(fb + s) * k + c;
+            if constexpr (FIXED) {
+#pragma unroll
+                for (int i = 0; i < REG; ++i) {
+                    const unsigned long long tot = red[i][0][s] + red[i][1][s] + red[i][2][s] + red[i][3][s];
+                    if (tot != 0ull) atomicAdd(kept.sums[i] + at, tot);
+                }
+                if constexpr (WORDS > 1) {
+                    const unsigned long long tot = last[s];
+                    if (tot != 0ull) {
+                        atomicAdd(kept.sums[WORDS - 1] + at, tot);
+                        last[s] = 0ull;
+                    }
+                }
+            } else {
+                const double tot = (of(red[0][0][s]) + of(red[0][1][s])) + (of(red[0][2][s]) + of(red[0][3][s]));
+                if (tot != 0.0) kmx_atomic_add(reinterpret_cast<double*>(kept.sums[0]) + at, tot);
+            }
+        }
+        if (blockIdx.y == 0 && wave == 3 && lane < (FIXED ? WORDS : 1)) {
+            const size_t at = (size_t)d * k + c;
+            const unsigned long long* part = red_w[lane];
+            if constexpr (FIXED) {
+                const unsigned long long tot = part[0] + part[1] + part[2] + part[3];
+                if (tot != 0ull) atomicAdd((lane == 0 ? kept.sums[0] : lane == 1 ? kept.sums[1] : kept.sums[2]) + at, tot);
+            } else {
+                const double tot = (of(part[0]) + of(part[1])) + (of(part[2]) + of(part[3]));
+                if (tot != 0.0) kmx_atomic_add(reinterpret_cast<double*>(kept.sums[0]) + at, tot);
             }
         }
         __syncthreads();
@@ -317,7 +386,7 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
         const int c_end = offsets[c + 1];  // wave-uniform
         const int p1 = c_end < P1 ? c_end : P1;
         if (p1 > pos) {
-            if (finite) stretch(std::true_type{}, pos, p1, c);
+            if (fixed) stretch(std::true_type{}, pos, p1, c);
             else stretch(std::false_type{}, pos, p1, c);
             pos = p1;
         }
@@ -325,14 +394,14 @@ __global__ __launch_bounds__(256) void moves_sum_kernel(const T* __restrict__ X_
     }
 }
 
-template <typename T>
+template <typename T, int WORDS>
 int32_t launch_sums(const void* X_rm, const void* w, const uint32_t* order, const int* offsets, int* counts, const KmxKept& kept,
                     const kmx_lloyd_status* status, int64_t n, int d, int k, hipStream_t stream) {
     constexpr int V = 16 / (int)sizeof(T);
     // workgroups: a chunk each, or about four per compute unit where there are fewer chunks
     const unsigned gx = (unsigned)kmx_cdiv(n, CHUNK);
 #define KMX_MOVES_SUM(LPR_)                                                                                                  \
-    hipLaunchKernelGGL((moves_sum_kernel<T, LPR_>), dim3(gx, (unsigned)kmx_cdiv(d, LPR_ * V)), dim3(256), 0, stream, (const T*)X_rm, \
+    hipLaunchKernelGGL((moves_sum_kernel<T, LPR_, WORDS>), dim3(gx, (unsigned)kmx_cdiv(d, LPR_ * V)), dim3(256), 0, stream, (const T*)X_rm, \
                        (const T*)w, order, offsets, counts, kept, status, n, d, k)
     if (d <= 16 * V) KMX_MOVES_SUM(16);
     else if (d <= 32 * V) KMX_MOVES_SUM(32);
@@ -363,8 +432,12 @@ int32_t kmx_lloyd_kept_sums(const void* X_rowmajor, const void* w, const uint32_
     int64_t sg = kmx_cdiv(n, 256 * 4);
     if (sg > 2048) sg = 2048;
     hipLaunchKernelGGL(moves_scatter_kernel, dim3((unsigned)sg), dim3(256), 0, stream, labels, kept, offsets, ranks, order, n,
-                       (d + 1) * k, dtype == KMX_F64, status);
+                       (d + 1) * k, status);
     KMX_LAUNCH_CHECK();
-    return dtype == KMX_F32 ? launch_sums<float>(X_rowmajor, w, order, offsets, counts, kept, status, n, d, k, stream)
-                            : launch_sums<double>(X_rowmajor, w, order, offsets, counts, kept, status, n, d, k, stream);
+#define KMX_SUMS(T, WORDS_) \
+    return launch_sums<T, WORDS_>(X_rowmajor, w, order, offsets, counts, kept, status, n, d, k, stream)
+    if (dtype == KMX_F64) KMX_SUMS(double, 3);
+    if (kept.words == 1) KMX_SUMS(float, 1);
+    KMX_SUMS(float, 2);
+#undef KMX_SUMS
 }

@@ -55,10 +55,10 @@ struct TileArea {
     int S;              // steps of 16 features
     int n_blocks;       // blocks of 32 centroids
     int64_t n_tiles;    // tiles of 32 samples (even)
-    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_half, off_list, off_thr, off_rest, off_hi, off_lo, off_odd, total;
+    size_t off_xt, off_norm, off_err, off_ct, off_hneg, off_cmax, off_half, off_list, off_thr, off_rest, off_least, off_sums, sums_bytes, total;
 };
 
-inline TileArea tile_area(int64_t n, int d, int k) {
+inline TileArea tile_area(int64_t n, int d, int k, int words = 0) {  // (words of the kept sums, at the end)
     TileArea a;
     a.S = (d + 15) / 16;
     a.n_blocks = (k + 31) / 32;
@@ -73,10 +73,10 @@ inline TileArea tile_area(int64_t n, int d, int k) {
     a.off_list = a.off_half + kmx_align256((size_t)k * sizeof(double));
     a.off_thr = a.off_list + kmx_align256((size_t)n * sizeof(int));
     a.off_rest = a.off_thr + kmx_align256((size_t)n * sizeof(float));
-    a.off_hi = a.off_rest + kmx_align256((size_t)n * sizeof(int));
-    a.off_lo = a.off_hi + kmx_align256((size_t)(d + 1) * k * 8);
-    a.off_odd = a.off_lo + kmx_align256((size_t)(d + 1) * k * 8);
-    a.total = a.off_odd + kmx_align256((size_t)(d + 1) * k * 8);
+    a.off_least = a.off_rest + kmx_align256((size_t)n * sizeof(int));
+    a.off_sums = a.off_least + kmx_align256((size_t)(d + 1) * sizeof(unsigned int));
+    a.sums_bytes = kmx_align256((size_t)(d + 1) * k * 8);
+    a.total = a.off_sums + words * a.sums_bytes;
     return a;
 }
 
@@ -143,9 +143,11 @@ __device__ __forceinline__ float sampled_max(const T* __restrict__ X_t, int64_t 
 
 template <typename T>
 __global__ __launch_bounds__(1024) void tiles_scale_kernel(const T* __restrict__ centroids_t, const T* __restrict__ X_t,
-                                                           unsigned int* __restrict__ header, int items, int64_t n, int d) {
+                                                           unsigned int* __restrict__ header, unsigned int* __restrict__ least,
+                                                           int items, int64_t n, int d) {
     __shared__ float m_s[2][16];
     float m = 0.0f;
+    if ((int)threadIdx.x <= d) least[threadIdx.x] = 0u;  // (d <= 256; for the pass that follows)
     for (int i0 = threadIdx.x; i0 < items; i0 += 16 * 1024) {
         float v[16];
 #pragma unroll
@@ -165,27 +167,38 @@ __global__ __launch_bounds__(1024) void tiles_sample_scale_kernel(const T* __res
 }
 
 // The tiles, |x'|^2 and |e_x| per sample, the row-major copy of X and (absmax not null) the bits of
-// max |x| per feature, in one pass: 128 samples per workgroup and pass, 32 features at a time through LDS.  Bound by memory: (2 + 2 sizeof(T)) bytes
-// per value.
+// max |x| per feature, the smallest |x| per feature and |w| (kmx_least_word) and whether all are finite, in one pass:
+// 128 samples per workgroup and pass, 32 features at a time through LDS.  Bound by memory: (2 + 2 sizeof(T)) bytes
+// per value.  A row's extremes meet over its lanes only where one of them exceeds what the workgroup has seen: of the few
+// tiles that a workgroup takes about the first two.
 template <typename T>
 __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict__ X_t, T* __restrict__ X_rm,
-                                                            uint4* __restrict__ xt, float* __restrict__ norm,
-                                                            float* __restrict__ err, unsigned int* __restrict__ header,
-                                                            unsigned int* __restrict__ absmax, int64_t n, int d, int S,
-                                                            int64_t n_pad) {
+                                                            const T* __restrict__ sample_weight, uint4* __restrict__ xt,
+                                                            float* __restrict__ norm, float* __restrict__ err,
+                                                            unsigned int* __restrict__ header,
+                                                            unsigned int* __restrict__ absmax, unsigned int* __restrict__ least,
+                                                            int64_t n, int d, int S, int64_t n_pad) {
     constexpr int NS = 128, NF = 32;
     constexpr int W = 16 / (int)sizeof(T);      // samples per 128-bit load
     constexpr int TPR = NS / W;                 // threads per row of 128 samples
     constexpr int RPP = 256 / TPR;              // rows per pass
     __shared__ T tile[NF][NS + 1];
     __shared__ float part[2][2][NS];
-    __shared__ unsigned int amax[TILE_D_MAX];
-    for (int f = threadIdx.x; f < TILE_D_MAX; f += 256) amax[f] = 0u;
+    __shared__ uint2 extremes[TILE_D_MAX];  // bits of the largest, flipped word of the smallest
+    __shared__ unsigned int w_min;
+    for (int f = threadIdx.x; f < TILE_D_MAX; f += 256) extremes[f] = make_uint2(0u, 0u);
+    if (threadIdx.x == 0) w_min = 0u;
     const float xs = __uint_as_float(header[KMX_TH_SCALE]);
     const int s = threadIdx.x & (NS - 1), g2 = threadIdx.x >> 7;   // sample, pair of groups of 8 features
     float odd = 0.0f;  // (NaN once a value is NaN or infinite; the maxima leave NaN out)
+    unsigned int w_least = ~0u;
     for (int64_t i0 = (int64_t)blockIdx.x * NS; i0 < n_pad; i0 += (int64_t)gridDim.x * NS) {
         float sq = 0.0f, e2 = 0.0f;
+        if (absmax != nullptr && g2 == 0 && i0 + s < n) {
+            const T w = sample_weight[i0 + s];
+            w_least = min(w_least, kmx_least_word(w));
+            odd = fmaf((float)w, 0.0f, odd);
+        }
         for (int f0 = 0; f0 < 16 * S; f0 += NF) {
             {
                 const int col = (threadIdx.x % TPR) * W, row0 = threadIdx.x / TPR;
@@ -210,13 +223,26 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
                 if (absmax != nullptr) {
 #pragma unroll
                     for (int p = 0; p < NF / RPP; ++p) {
+                        const int f = f0 + row0 + p * RPP;  // (below TILE_D_MAX)
                         float m = 0.0f;
+                        unsigned int low = ~0u;
 #pragma unroll
-                        for (int e = 0; e < W; ++e) m = fmaxf(m, fabsf((float)v[p][e]));
+                        for (int e = 0; e < W; ++e) {
+                            m = fmaxf(m, fabsf((float)v[p][e]));
+                            low = min(low, kmx_least_word(v[p][e]));
+                        }
+                        const uint2 seen = extremes[f];
+                        if (__any(__float_as_uint(m) > seen.x || ~low > seen.y)) {
 #pragma unroll
-                        for (int off = 1; off < TPR; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-                        const int f = f0 + row0 + p * RPP;
-                        if (col == 0 && f < d) atomicMax(&amax[f], __float_as_uint(m));
+                            for (int off = 1; off < TPR; off <<= 1) {
+                                m = fmaxf(m, __shfl_xor(m, off, 64));
+                                low = min(low, (unsigned int)__shfl_xor((int)low, off, 64));
+                            }
+                            if (col == 0) {
+                                atomicMax(&extremes[f].x, __float_as_uint(m));
+                                atomicMax(&extremes[f].y, ~low);
+                            }
+                        }
                     }
                 }
 #pragma unroll
@@ -268,8 +294,14 @@ __global__ __launch_bounds__(256) void tiles_prepare_kernel(const T* __restrict_
     }
     if (absmax != nullptr) {
         __syncthreads();
-        for (int f = threadIdx.x; f < d; f += 256) atomicMax(absmax + f, amax[f]);
+        for (int f = threadIdx.x; f < d; f += 256) {
+            atomicMax(absmax + f, extremes[f].x);
+            atomicMax(least + f, extremes[f].y);
+        }
+        if (w_least != ~0u) atomicMax(&w_min, ~w_least);
         if (odd != 0.0f) header[KMX_TH_ODD] = 1u;  // (true for NaN)
+        __syncthreads();
+        if (threadIdx.x == 0) atomicMax(least + d, w_min);
     }
 }
 
@@ -283,7 +315,8 @@ __global__ __launch_bounds__(64 * CENT_WAVES) void tiles_centroids_kernel(const 
                                                               float* __restrict__ hneg, float2* __restrict__ cmax,
                                                               unsigned int* __restrict__ header,
                                                               const kmx_lloyd_status* __restrict__ status,
-                                                              const unsigned int* __restrict__ absmax, int d, int k, int S) {
+                                                              const unsigned int* __restrict__ absmax,
+                                                              const unsigned int* __restrict__ least, int d, int k, int S, int span) {
     if (status != nullptr && status->state != KMX_RUNNING) return;
     __shared__ double part[2][CENT_WAVES][64];
     const float xs = __uint_as_float(header[KMX_TH_SCALE]);
@@ -339,17 +372,13 @@ __global__ __launch_bounds__(64 * CENT_WAVES) void tiles_centroids_kernel(const 
             }
         }
     }
-    // (an iteration: whether the sums kept from the one before can be corrected)
+    // (an iteration: whether the sums have fixed point, and whether those kept from the one before can be corrected)
     if (blockIdx.x == 0 && absmax != nullptr) {
-        bool finite = header[KMX_TH_ODD] == 0u && absmax[d] != 0u, some = false;
-        for (int f = threadIdx.x; f <= d; f += 64 * CENT_WAVES) {
-            finite &= !kmx_not_finite(__uint_as_float(absmax[f]));
-            some |= f < d && absmax[f] != 0u;
-        }
-        const bool any = __syncthreads_or(some ? 1 : 0) != 0;
-        const bool all = __syncthreads_and(finite && any ? 1 : 0) != 0;
+        bool fixed = header[KMX_TH_ODD] == 0u;
+        for (int f = threadIdx.x; f <= d; f += 64 * CENT_WAVES) fixed &= kmx_kept_fixed<T>(absmax, least, d, f, span);
+        const bool all = __syncthreads_and(fixed ? 1 : 0) != 0;
         if (threadIdx.x == 0) {
-            header[KMX_TH_FINITE] = all ? 1u : 0u;
+            header[KMX_TH_FIXED] = all ? 1u : 0u;
             header[KMX_TH_KEEP] = all && status->n_iter > 0 && header[KMX_TH_SUMS] == (unsigned int)status->n_iter ? 1u : 0u;
         }
     }
@@ -904,10 +933,10 @@ bool kmx_tiles_fit(int64_t n, int d, int k) {
     return d <= TILE_D_MAX && n <= INT32_MAX - 64 && k <= 8192;
 }
 
-size_t kmx_tiles_bytes(int64_t n, int d, int k) { return tile_area(n, d, k).total; }
+size_t kmx_tiles_bytes(int64_t n, int d, int k, int words) { return tile_area(n, d, k, words).total; }
 
-static void tiles_copy(const void* X_t, void* X_rowmajor, char* area, unsigned int* absmax, int64_t n, int d, int dtype,
-                       hipStream_t stream) {
+static void tiles_copy(const void* X_t, void* X_rowmajor, const void* w, char* area, unsigned int* absmax, unsigned int* least,
+                       int64_t n, int d, int dtype, hipStream_t stream) {
     const TileArea a = tile_area(n, d, 0);  // (the samples' part depends on n and d alone)
     unsigned int* header = (unsigned int*)area;
     const int64_t n_pad = a.n_tiles * 32;
@@ -917,24 +946,25 @@ static void tiles_copy(const void* X_t, void* X_rowmajor, char* area, unsigned i
 #define KMX_TILES_COPY(T)                                                                                                 \
     do {                                                                                                                  \
         hipLaunchKernelGGL((tiles_prepare_kernel<T>), dim3((unsigned)grid), dim3(256), 0, stream, (const T*)X_t,          \
-                           (T*)X_rowmajor, (uint4*)(area + a.off_xt), (float*)(area + a.off_norm),                        \
-                           (float*)(area + a.off_err), header, absmax, n, d, a.S, n_pad);                          \
+                           (T*)X_rowmajor, (const T*)w, (uint4*)(area + a.off_xt), (float*)(area + a.off_norm),           \
+                           (float*)(area + a.off_err), header, absmax, least, n, d, a.S, n_pad);                          \
     } while (0)
     if (dtype == KMX_F32) KMX_TILES_COPY(float); else KMX_TILES_COPY(double);
 #undef KMX_TILES_COPY
 }
 
 // Scale, tiles and norms of X, and its row-major copy; `centroids_t`: the initial centroids.
-int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* centroids_t, char* area, unsigned int* absmax,
-                          int64_t n, int d, int k, int dtype, hipStream_t stream) {
+int32_t kmx_tiles_prepare(const void* X_t, void* X_rowmajor, const void* w, const void* centroids_t, char* area,
+                          unsigned int* absmax, int64_t n, int d, int k, int dtype, hipStream_t stream) {
     unsigned int* header = (unsigned int*)area;
+    unsigned int* least = (unsigned int*)(area + tile_area(n, d, k).off_least);
     if (dtype == KMX_F32)
         hipLaunchKernelGGL((tiles_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)centroids_t,
-                           (const float*)X_t, header, d * k, n, d);
+                           (const float*)X_t, header, least, d * k, n, d);
     else
         hipLaunchKernelGGL((tiles_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)centroids_t,
-                           (const double*)X_t, header, d * k, n, d);
-    tiles_copy(X_t, X_rowmajor, area, absmax, n, d, dtype, stream);
+                           (const double*)X_t, header, least, d * k, n, d);
+    tiles_copy(X_t, X_rowmajor, w, area, absmax, least, n, d, dtype, stream);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
@@ -949,7 +979,7 @@ int32_t kmx_tiles_prepare_samples(const void* X_t, void* X_rowmajor, char* area,
         hipLaunchKernelGGL((tiles_sample_scale_kernel<float>), dim3(1), dim3(1024), 0, stream, (const float*)X_t, header, n, d);
     else
         hipLaunchKernelGGL((tiles_sample_scale_kernel<double>), dim3(1), dim3(1024), 0, stream, (const double*)X_t, header, n, d);
-    tiles_copy(X_t, X_rowmajor, area, nullptr, n, d, dtype, stream);
+    tiles_copy(X_t, X_rowmajor, nullptr, area, nullptr, nullptr, n, d, dtype, stream);
     KMX_LAUNCH_CHECK();
     return KMX_OK;
 }
@@ -960,15 +990,14 @@ KmxTiles kmx_tiles_view(char* area, int64_t n, int d) {
             (const float*)area + KMX_TH_SCALE, a.S};
 }
 
-KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k) {
-    const TileArea a = tile_area(n, d, k);
+KmxKept kmx_tiles_kept(char* area, const unsigned int* absmax, int64_t n, int d, int k, int words) {
+    const TileArea a = tile_area(n, d, k, words);
     KmxKept kept;
     kept.header = (unsigned int*)area;
     kept.absmax = absmax;
     kept.n = n;
-    kept.hi = (unsigned long long*)(area + a.off_hi);
-    kept.lo = (unsigned long long*)(area + a.off_lo);
-    kept.odd = (double*)(area + a.off_odd);
+    kept.words = words;
+    for (int i = 0; i < words; ++i) kept.sums[i] = (unsigned long long*)(area + a.off_sums + i * a.sums_bytes);
     // (the lists of a labelling, which is over when the sums begin)
     kept.entry = (uint32_t*)(area + a.off_list);
     kept.entry_cluster = (uint32_t*)(area + a.off_thr);
@@ -980,22 +1009,23 @@ char* kmx_tiles_half_norms(char* area, int64_t n, int d, int k) { return area + 
 // Labels of all samples for `centroids_t` (their packed copy `cpack` and half norms as the workspace
 // holds them).  `status` null: labels whatever the state, those of kmx_assign_labels, whose half norms
 // `half_norms` are then.  listed_out (or null): the number of samples without a certificate.  An iteration whose
-// sums are kept hands over the labels before and the bits of max |x| per feature and max |w| (else null).
+// sums are kept hands over the labels before, the bits of max |x| per feature and max |w| (else null) and kmx_kept_span.
 int32_t kmx_tiles_labels(const void* X_t, const void* X_rowmajor, const void* centroids_t, const void* cpack,
                          const void* half_norms, char* area, kmx_lloyd_status* status, uint32_t* labels, int64_t n,
                          int d, int dpad, int k, int dtype, hipStream_t stream, unsigned int* listed_out,
-                         const uint32_t* labels_prev, const unsigned int* absmax) {
+                         const uint32_t* labels_prev, const unsigned int* absmax, int span) {
     const TileArea a = tile_area(n, d, k);
     unsigned int* header = (unsigned int*)area;
     uint4* ct = (uint4*)(area + a.off_ct);
     float* hneg = (float*)(area + a.off_hneg);
     float2* cmax = (float2*)(area + a.off_cmax);
+    const unsigned int* least = (const unsigned int*)(area + a.off_least);
     if (dtype == KMX_F32)
         hipLaunchKernelGGL((tiles_centroids_kernel<float>), dim3((unsigned)a.n_blocks), dim3(64 * CENT_WAVES), 0, stream,
-                           (const float*)centroids_t, ct, hneg, cmax, header, status, absmax, d, k, a.S);
+                           (const float*)centroids_t, ct, hneg, cmax, header, status, absmax, least, d, k, a.S, span);
     else
         hipLaunchKernelGGL((tiles_centroids_kernel<double>), dim3((unsigned)a.n_blocks), dim3(64 * CENT_WAVES), 0, stream,
-                           (const double*)centroids_t, ct, hneg, cmax, header, status, absmax, d, k, a.S);
+                           (const double*)centroids_t, ct, hneg, cmax, header, status, absmax, least, d, k, a.S, span);
     // (an fp32 score: d + 1 roundings of partial sums, as many of the half norm)
     const bool match = status == nullptr && dtype == KMX_F32;
     const float prod_rho = match ? ULP * (float)(d + 8) : 0.0f;

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 HEADER_SUMS = 7  # word of the copy's header: iterations behind the kept sums
 HEADER_KEEP = 5  # whether the last iteration had sums to correct
 HEADER_ENTRIES = 4
+HEADER_FIXED = 6  # whether the sums are fixed point
 KMX_NEED_RELOCATION = 4
 
 
@@ -155,3 +156,93 @@ def test_all_sums_are_converted_when_the_gpu_is_busy(cuda):
                 want = np.bincount(lab, weights=X[:, f].astype(np.float64) * w, minlength=k)
                 np.testing.assert_allclose(sums[f], want, rtol=1e-6, atol=1e-6 * np.abs(X[:, f]).max())
         np.testing.assert_array_equal(sums, expected)
+
+
+def _check_means(run, X, w, k, features, tol):
+    """Centroids of the clusters that hold samples of some weight against fp64 means, relative to the mean magnitude of their
+    terms; cluster sizes likewise."""
+    lab = run.labels[run.n_done % 2].cpu().numpy()
+    w64 = w.astype(np.float64)
+    sizes = np.bincount(lab, weights=w64, minlength=k)
+    full = sizes > 0
+    np.testing.assert_allclose(run.sizes.cpu().numpy().astype(np.float64), sizes, rtol=tol)
+    c = run.cent[run.n_done % 2].cpu().numpy().astype(np.float64)
+    for f in features:
+        x = X[:, f].astype(np.float64)
+        want = np.bincount(lab, weights=x * w64, minlength=k)[full] / sizes[full]
+        size_of = np.bincount(lab, weights=np.abs(x) * w64, minlength=k)[full] / sizes[full]
+        assert np.abs((c[f][full] - want) / np.maximum(size_of, np.finfo(np.float64).tiny)).max() < tol
+
+
+# a copy whose sums were fp64 additions before they were kept: the tiled product in fp32, all of fp64.  An outlier within
+# the words of a sum and one beyond them; a cluster whose weights are that far below the others'
+@pytest.mark.parametrize("outlier,weight,fixed", [
+    (1e9, 1.0, True), (1e11, 1.0, True), (1e25, 1.0, False), (1.0, 1e-10, True), (1.0, 1e-30, False), (1e9, 1e-30, False),
+])
+@pytest.mark.parametrize("n,d,k,dtype", [(100_003, 129, 128, np.float32), (65_603, 100, 100, np.float64)])
+def test_sums_beside_much_larger_ones(cuda, n, d, k, dtype, outlier, weight, fixed):
+    X, w, init = _blobs(n, d, k, dtype, 8)
+    X += np.sign(X) * 0.1  # (smallest magnitude 0.1: the line is that of the outlier and the weights)
+    X[n // 2, 5] = 3.0 * outlier
+    w[w > 0] = 1.0
+    lightest = np.arange(n) % (k * 3 // 4) == 7
+    w[lightest] = weight
+    X = X.astype(dtype)
+    # (samples of that blob stand apart, so that clusters are of one weight)
+    X[lightest] += dtype(30.0)
+    init = X[:k].copy()
+    run = _ResidentRun(cuda, X, w, init, 3)
+    for step in (1, 2):
+        run.run(step)
+        if step > 1 and run.n_done < step:
+            break  # (the outlier's score is no number in fp32: a cluster is empty)
+        assert run.n_done == step and run.status.state in (0, 3)
+        assert int(_words(run)[HEADER_FIXED]) == int(fixed)
+        assert int(_words(run)[HEADER_KEEP]) == int(fixed and step > 1)
+        # (a term's own rounding, fp64 additions in some order and the result's)
+        _check_means(run, X, w, k, (0, 5, d - 1), 4 * np.finfo(dtype).eps if dtype == np.float32 else 1e-13)
+
+
+@pytest.mark.parametrize("n,d,k,dtype", [(20_001, 100, 300, np.float32), (100_003, 129, 128, np.float32),
+                                         (65_603, 100, 100, np.float64)])
+def test_sums_corrected_behind_a_relocation(cuda, n, d, k, dtype):
+    """The iterations behind a relocation, which has moved samples between sums but not between the kept ones: the same
+    bits as with sums rebuilt in every iteration; the run goes on without a look at its state."""
+    import torch
+
+    from sklearn_numba_dpex_amd._capi import check, lib, ptr
+    from sklearn_numba_dpex_amd.kmeans import drivers
+
+    X, w, init = _blobs(n, d, k, dtype, 9)
+    w[w == 0] = 1.0
+    init[[2, k // 2, k - 1]] = 1e4
+    steps, seen = 6, {}
+    for rebuilt in (False, True):
+        run = _ResidentRun(cuda, X, w, init, steps)
+        results, kept = [], []
+        relocations, until = 0, 1
+        while until <= steps:
+            if rebuilt:
+                _words(run)[HEADER_SUMS] = 0
+            run.run(until)
+            if run.status.state == KMX_NEED_RELOCATION:
+                relocations += 1
+                j = run.status.n_iter
+                a, b = j % 2, (j + 1) % 2
+                drivers._relocate_empty_clusters(run.status.n_empty, run.X_t, run.w, run.cent[b], run.sizes, run.labels[b],
+                                                 run.empty, run.cent[a])
+                check(lib.kmx_lloyd_finalize(run.plan, ptr(run.cent[a]), ptr(run.cent[b]), ptr(run.sizes), ptr(run.ws),
+                                             run.ws_bytes, run.stream), "kmx_lloyd_finalize")
+                run.n_done = j + 1
+            kept.append(int(_words(run)[HEADER_KEEP]))
+            results.append((run.cent[run.n_done % 2].clone(), run.labels[run.n_done % 2].clone(), run.sizes.clone()))
+            until = run.n_done + 1
+            if run.status.state not in (0, 3, KMX_NEED_RELOCATION):
+                break
+        assert relocations >= 1 and len(results) >= 4
+        assert kept[1:] == [0 if rebuilt else 1] * (len(kept) - 1)
+        seen[rebuilt] = results
+    assert len(seen[False]) == len(seen[True])
+    for step, (one, other) in enumerate(zip(seen[False], seen[True])):
+        differ = [i for i in range(3) if not torch.equal(one[i], other[i])]
+        assert not differ, step
