@@ -56,6 +56,23 @@ constexpr int QUEUE_MAX = 24576, UNSURE_MAX = 640, MOVED_MAX = 512;
 
 constexpr int bounds_waves(int esize, int nk) { return esize == 8 && nk > 2 ? 8 : 16; }
 
+// Workgroups: one per compute unit, or fewer with a load of words for each wave.
+constexpr int64_t bounds_grid(int64_t n, int waves, int cus) {
+    const int64_t g = (n + (int64_t)UNIT * waves - 1) / ((int64_t)UNIT * waves);
+    return g < cus ? g : cus;
+}
+// Whether the number of a sample within its workgroup's units, past the last of them included (the waves
+// take the same number of units), fits an entry of the queue beside its label.  A partition of the GPU has fewer compute
+// units, and more samples for each.
+constexpr bool bounds_entries_fit(int64_t n, int waves, int cus) {
+    const int64_t units = (n + UNIT - 1) / UNIT, per_step = bounds_grid(n, waves, cus) * waves;
+    return (units + per_step - 1) / per_step * waves * UNIT <= (int64_t)1 << (32 - LABEL_BITS);
+}
+static_assert(bounds_entries_fit(((int64_t)1 << 29) - 1, 16, 256) && bounds_entries_fit((int64_t)1 << 29, 8, 256));
+static_assert(!bounds_entries_fit(((int64_t)1 << 29) + 1, 16, 256));
+static_assert(bounds_entries_fit((int64_t)1 << 26, 16, 32) && !bounds_entries_fit(((int64_t)1 << 26) + 1, 16, 32));
+static_assert(bounds_entries_fit(1, 16, 1) && !bounds_entries_fit(((int64_t)1 << 21) + 1, 8, 1));
+
 struct BoundsLds {
     size_t off_hi, off_lo, off_hneg, off_frag, off_half, off_drift, off_part, off_moved, off_unsure, off_queue, total;
     int kp, q_cap;
@@ -149,8 +166,7 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     uint32_t* moved = reinterpret_cast<uint32_t*>(bounds_raw + lay.off_moved);     // [MOVED_MAX][2]: sample; old and new label
     uint32_t* u_index = reinterpret_cast<uint32_t*>(bounds_raw + lay.off_unsure);  // samples without a certificate
     uint16_t* u_label = reinterpret_cast<uint16_t*>(u_index + UNSURE_MAX);
-    // samples to look at: number within the workgroup's units (below 2^21: n < 2^29 and a workgroup per compute
-    // unit, or fewer samples each), then the label
+    // samples to look at: number within the workgroup's units (bounds_entries_fit), then the label
     uint32_t* queue = reinterpret_cast<uint32_t*>(bounds_raw + lay.off_queue);
     __shared__ unsigned int queued, unsure_count, moved_count, changed_s;
     __shared__ int q_s[65];
@@ -818,8 +834,7 @@ int32_t launch_bounds(const LloydLayout& L, bool enter, char* area, int parity, 
     float* drift = reinterpret_cast<float*>(area + a.off_drift);
     const size_t lds = bounds_lds(d, k, NK, (int)sizeof(TX)).total;
     constexpr int THREADS = 64 * bounds_waves((int)sizeof(TX), NK);
-    int64_t grid = kmx_cdiv(n, (int64_t)UNIT * THREADS / 64);
-    if (grid > kmx_num_cus()) grid = kmx_num_cus();
+    const int64_t grid = bounds_grid(n, THREADS / 64, kmx_num_cus());
 #define KMX_BOUNDS(ENTER_)                                                                                              \
     do {                                                                                                                \
         if (lds > 64 * 1024) {                                                                                          \
@@ -876,7 +891,8 @@ int32_t iter_bounds(const LloydLayout& L, bool enter, char* area, int parity, co
 
 bool kmx_bounds_fit(int64_t n, int d, int k, int dtype) {
     const int esize = dtype == KMX_F64 ? 8 : 4, nk = (d + 15) / 16;
-    if (d > 64 || k > (int)LABEL_MASK || n >= ((int64_t)1 << 29)) return false;
+    if (d > 64 || k > (int)LABEL_MASK || n >= ((int64_t)1 << 29)) return false;  // (as the screened steps)
+    if (!bounds_entries_fit(n, bounds_waves(esize, nk), kmx_num_cus())) return false;
     // (one load of words by every wave must fit the queue)
     return bounds_lds(d, k, nk, esize).q_cap >= UNIT * bounds_waves(esize, nk);
 }
