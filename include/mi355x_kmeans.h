@@ -265,8 +265,8 @@ int32_t kmx_lloyd_status_read(const void* workspace, kmx_lloyd_status* status_ho
 
 /* Where labels are screened on the fp16 matrix cores (kernel variants 61, 71 and 42, the last also in a
  * run with a half-precision copy): number of samples whose label the screen of the last completed
- * iteration could not certify and that were evaluated more precisely instead; 0 for the other
- * variants.  Synchronises the stream.
+ * iteration could not certify and that were evaluated more precisely instead (of those that it looked at,
+ * where it passed samples over: kmx_lloyd_bounds_bytes); 0 for the other variants.  Synchronises the stream.
  * It has no counterpart in the reference (diagnostics). */
 int32_t kmx_lloyd_recheck_count(const kmx_lloyd_plan* plan, const void* workspace,
                                 uint32_t* count_host, void* stream);

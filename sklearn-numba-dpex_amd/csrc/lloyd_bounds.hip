@@ -147,8 +147,7 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     const TX* __restrict__ centroids_t, const TX* __restrict__ before_t, uint32_t* __restrict__ labels_a,
     uint32_t* __restrict__ labels_b, uint32_t* __restrict__ words, const float* __restrict__ drift_in,
     float* __restrict__ drift_out, kmx_lloyd_status* __restrict__ status, const unsigned int* __restrict__ absmax,
-    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum, uint32_t* __restrict__ looked_at,
-    int64_t n, int d, int k, int ds, const LloydTail<TX> tail) {
+    const int* __restrict__ q_exp, unsigned long long* __restrict__ gsum, int64_t n, int d, int k, int ds, const LloydTail<TX> tail) {
     constexpr bool F64 = sizeof(TX) == 8;
     constexpr int WAVES = bounds_waves((int)sizeof(TX), NK), THREADS = 64 * WAVES;
     extern __shared__ __align__(16) unsigned char bounds_raw[];
@@ -769,8 +768,9 @@ __global__ __launch_bounds__(64 * bounds_waves((int)sizeof(TX), NK)) void bounds
     __syncthreads();
     if (threadIdx.x == 0) {
         if (changed_s) atomicAdd(&status->n_changed, changed_s);
-        if (!ENTER && looked) atomicAdd(looked_at, looked);
-        if (ENTER && blockIdx.x == 0) atomicAdd(looked_at, (unsigned int)n);
+        if (unsure_count) atomicAdd(tail.clear_word, unsure_count);
+        if (!ENTER && looked) atomicAdd(tail.looked_word, looked);
+        if (ENTER && blockIdx.x == 0) atomicAdd(tail.looked_word, (unsigned int)n);
     }
     // (every workgroup starts at another word: they finish together)
     const int n_out = (d + 1) * k;
@@ -846,7 +846,7 @@ int32_t launch_bounds(const LloydLayout& L, bool enter, char* area, int parity, 
                            (const TX*)X_t, (float*)(area + a.off_rows), (const TX*)w, (const TX*)centroids_t,              \
                            (const TX*)before_t, labels_a, labels_b, (uint32_t*)(area + a.off_words),                    \
                            drift + (size_t)parity * k, drift + (size_t)(parity ^ 1) * k, tail.status, absmax, q_exp,    \
-                           (unsigned long long*)(ws + L.off_gsum), tail.clear_word, n, d, k, a.ds, tail);               \
+                           (unsigned long long*)(ws + L.off_gsum), n, d, k, a.ds, tail);               \
     } while (0)
     if (enter) KMX_BOUNDS(true); else KMX_BOUNDS(false);
 #undef KMX_BOUNDS
@@ -870,7 +870,8 @@ int32_t iter_bounds(const LloydLayout& L, bool enter, char* area, int parity, co
     tail.k = k;
     tail.dpad = L.dpad;
     tail.progress = L.progress;
-    tail.clear_word = reinterpret_cast<uint32_t*>(ws + L.off_bucket);
+    tail.clear_word = reinterpret_cast<uint32_t*>(ws + L.off_bucket);  // (the screened steps' counter block)
+    tail.looked_word = tail.clear_word + 3;
     tail.n_samples = n;
     tail.delta_divisor = 3;  // (as the screened steps)
     tail.list_divisor = 24;

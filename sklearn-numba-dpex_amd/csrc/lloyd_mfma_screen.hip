@@ -70,6 +70,7 @@ constexpr int SCR_REDO_COLUMN = 3;  // uncertain samples from which a 32-sample 
 // fp32 by the running iteration, the same of the last finished one, and how the next step is
 // to bring the sums up to date (written by the finalisation): 0 rebuild them, 1 correct them for
 // the samples that change cluster, collected in the workgroup's list, 2 correct them tile by tile.
+// The word behind these counts the samples that a bounded iteration (lloyd_bounds.hip) looks at.
 constexpr int SCR_WORD_DELTA = 2;
 // Waves per workgroup (one workgroup per compute unit, or two of four waves).
 #ifndef KMX_SCR_WAVES

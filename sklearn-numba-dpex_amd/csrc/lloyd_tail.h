@@ -53,6 +53,7 @@ struct LloydTail {
     int64_t n_samples = 0;
     int delta_divisor = 0;
     int list_divisor = 0;
+    uint32_t* looked_word = nullptr;  // bounded iterations: how many samples this one has looked at, to announce and zero, or null
 };
 
 // Empty-cluster list (ascending) and heaviest cluster; one workgroup of up to 1024 threads, all
@@ -223,6 +224,9 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
     if (a.clear_word != nullptr && threadIdx.x == 0)
         counter_word = COHERENT ? __hip_atomic_load(&a.clear_word[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                                 : a.clear_word[0];
+    unsigned int hint_word = 0u;
+    if (a.looked_word != nullptr && threadIdx.x == 0)
+        hint_word = __hip_atomic_load(a.looked_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned int n_changed =
         COHERENT ? __hip_atomic_load(&a.status->n_changed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                  : a.status->n_changed;
@@ -230,6 +234,8 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
         a.clear_word[1] = counter_word;  // kept for kmx_lloyd_recheck_count
         a.clear_word[0] = 0u;
     }
+    if (a.looked_word != nullptr && threadIdx.x == 0) *a.looked_word = 0u;
+    else hint_word = counter_word;
     const T* sizes_s = vals + dk;  // vals: [(d + 1) * k], sums, then sizes
     T* __restrict__ out_t = a.sums_t;
     const T* __restrict__ old_t = a.old_centroids_t;
@@ -409,7 +415,7 @@ __device__ inline void lloyd_small_finalize_body(unsigned long long* __restrict_
     const double total = kmx_block_sum<double>(shift, scratch);
     if (threadIdx.x == 0) {
         if (a.progress != nullptr && a.clear_word != nullptr)
-            __hip_atomic_store(&a.progress[KMX_PROGRESS_HINT], (unsigned long long)n_changed | (unsigned long long)counter_word << 32,
+            __hip_atomic_store(&a.progress[KMX_PROGRESS_HINT], (unsigned long long)n_changed | (unsigned long long)hint_word << 32,
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         lloyd_update_status(a.status, WIDE ? lloyd_before(a.status) : was, total, n_changed, a.progress);
     }

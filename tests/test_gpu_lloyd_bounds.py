@@ -4,6 +4,8 @@ iteration read all of X.  Labels, centroids, cluster sizes and the number of ite
 for bit: sums are integers, and what is passed over is proven unchanged.  The screened steps
 themselves are compared with the oracle in test_gpu_lloyd_screen.py."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -32,19 +34,27 @@ def _run(X_t, w, init_t, max_iter, with_bounds, must_enter=True):
     check(lib.kmx_lloyd_run(plan, ptr(X_t), None, ptr(w), ptr(cent[0]), ptr(cent[1]), ptr(labels[0]), ptr(labels[1]),
                             ptr(sizes), ptr(empty), ptr(ws), ws.numel(), ptr(area), need, 0, max_iter, status, stream), "run")
     torch.cuda.synchronize()
+    uncertain = ctypes.c_uint32(0)
+    check(lib.kmx_lloyd_recheck_count(plan, ptr(ws), ctypes.byref(uncertain), stream), "recheck")
     # (conditions first: pytest iterates over the tensors of a comparison that an assert contains)
     if with_bounds and not must_enter:
         untouched = bool((area == MARK).all())
         assert untouched
     elif with_bounds:
-        # drift of the labels (two copies), then a word per sample: every one has been written, and some
-        # samples were passed over at least once (what they have seen of the drift is behind it by then)
+        # drift of the labels (two copies), then a word per sample.  Every word has been written, by the iteration that
+        # enters; a drift above zero comes from one behind it; and words with a margin above the drift by now are
+        # of samples that the next iteration passes over
+        drift = area[:2 * k * 4].view(torch.float32).view(2, k)
         words = area[(2 * k * 4 + 255) // 256 * 256:][: 4 * n].view(torch.int32)
         written, labels_fit = bool((words != -1).all()), bool(((words & 0x7FF) < k).all())
         assert written and labels_fit, "no bounded iteration has run"
+        by_now = drift.max(0).values
+        assert float(by_now.min()) > 0.0, "no iteration behind the entering one has run"
+        passed = float(((words & ~0x7FF).view(torch.float32) > by_now[(words & 0x7FF).long()]).double().mean())
+        assert passed > 0.5
     at = status.n_iter % 2
     return dict(n_iter=status.n_iter, state=status.state, labels=labels[at], cent=cent[at], sizes=sizes,
-                before=cent[at ^ 1])
+                uncertain=uncertain.value)
 
 
 def _same(a, b):
@@ -84,6 +94,8 @@ def test_same_as_iterations_over_all_samples(n, d, k, dtype, cuda):
     b = _run(X_t, w, init, 40, True)
     assert a["n_iter"] > 10
     _same(a, b)
+    # samples without a certificate: a few of those looked at, none of the others (the bounds are nearly the same)
+    assert b["uncertain"] <= 2 * a["uncertain"] + 16 and a["uncertain"] < n // 20
 
 
 def test_samples_on_the_bisector_and_more_of_them_than_the_list_holds(cuda):
