@@ -511,7 +511,8 @@ def test_finite_input_whose_sum_overflows_is_accepted(cuda):
 @pytest.mark.parametrize("dtype", DTYPES)
 # (not to convergence: in fp32 the iteration at which the last near tie is settled is not the oracle's)
 @pytest.mark.parametrize("max_iter,tol", [(1, 0.0), (5, 1e30), (2, 0.0), (4, 0.0)])
-@pytest.mark.parametrize("n,d,k", [(500, 3, 9), (30_000, 80, 70)])
+# (the last with a half-precision copy; its data are such that the oracle comes to the same centroids in fp32 and fp64)
+@pytest.mark.parametrize("n,d,k", [(500, 3, 9), (30_000, 80, 70), (61_000, 160, 170)])
 def test_a_run_that_ends_with_its_relocation(cuda, dtype, max_iter, tol, n, d, k):
     """The finalisation of a relocation reaches the last iteration or the tolerance, or the run goes on: iterations and
     centroids of the oracle."""

@@ -14,6 +14,24 @@ pytestmark = pytest.mark.gpu
 MARK = 0xFF
 
 
+def _drift_and_words(area, n, k):
+    import torch
+
+    # drift of the labels (two copies), then a word per sample
+    return (area[:2 * k * 4].view(torch.float32).view(2, k),
+            area[(2 * k * 4 + 255) // 256 * 256:][: 4 * n].view(torch.int32))
+
+
+def _entered(area, n, k):
+    """Whether a bounded iteration has written the area (all of its words: the entering one does), or none has."""
+    # (conditions first: pytest iterates over the tensors of a comparison that an assert contains)
+    _, words = _drift_and_words(area, n, k)
+    written, labels_fit = bool((words != -1).all()), bool(((words & 0x7FF) < k).all())
+    untouched = bool((area == MARK).all())
+    assert untouched or (written and labels_fit)
+    return not untouched
+
+
 def _run(X_t, w, init_t, max_iter, with_bounds, must_enter=True):
     import torch
 
@@ -36,18 +54,12 @@ def _run(X_t, w, init_t, max_iter, with_bounds, must_enter=True):
     torch.cuda.synchronize()
     uncertain = ctypes.c_uint32(0)
     check(lib.kmx_lloyd_recheck_count(plan, ptr(ws), ctypes.byref(uncertain), stream), "recheck")
-    # (conditions first: pytest iterates over the tensors of a comparison that an assert contains)
-    if with_bounds and not must_enter:
-        untouched = bool((area == MARK).all())
-        assert untouched
-    elif with_bounds:
-        # drift of the labels (two copies), then a word per sample.  Every word has been written, by the iteration that
-        # enters; a drift above zero comes from one behind it; and words with a margin above the drift by now are
-        # of samples that the next iteration passes over
-        drift = area[:2 * k * 4].view(torch.float32).view(2, k)
-        words = area[(2 * k * 4 + 255) // 256 * 256:][: 4 * n].view(torch.int32)
-        written, labels_fit = bool((words != -1).all()), bool(((words & 0x7FF) < k).all())
-        assert written and labels_fit, "no bounded iteration has run"
+    if with_bounds and must_enter is not None:
+        assert _entered(area, n, k) == must_enter
+    if with_bounds and must_enter:
+        drift, words = _drift_and_words(area, n, k)
+        # a drift above zero comes from an iteration behind the entering one; and words with a margin above the drift by now
+        # are of samples that the next iteration passes over
         by_now = drift.max(0).values
         assert float(by_now.min()) > 0.0, "no iteration behind the entering one has run"
         passed = float(((words & ~0x7FF).view(torch.float32) > by_now[(words & 0x7FF).long()]).double().mean())
@@ -123,6 +135,7 @@ def test_samples_on_the_bisector_and_more_of_them_than_the_list_holds(cuda):
     a = _run(X_t, w, init, 24, False)
     b = _run(X_t, w, init, 24, True)
     _same(a, b)
+    assert b["uncertain"] > 640 * torch.cuda.get_device_properties(cuda).multi_processor_count  # (some list is too short)
     tied = (X_t[0] == 0.0) & (w == 0.0)
     assert int(tied.sum()) == on_plane
     assert float(a["cent"][0, 3]) == -float(a["cent"][0, 11])  # the ties are exact
@@ -134,22 +147,93 @@ def test_run_with_relocated_clusters(dtype, cuda, monkeypatch):
     """Through the driver: relocations end a call to the library, and the run goes on with another."""
     import torch
 
+    from sklearn_numba_dpex_amd import _capi
     from sklearn_numba_dpex_amd.kmeans import drivers
 
-    X_t, w, init = _blobs(420_001, 32, 64, getattr(torch, dtype), 5, cuda)
+    n, k, seen = 600_001, 64, dict(areas=[], relocations=0)
+    X_t, w, init = _blobs(n, 32, k, getattr(torch, dtype), 5, cuda)
     for j in range(8):
         init[:, 63 - j] = 1e3 * (1 + j * 1e-3)
-    with_bounds = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
-
-    class NoBounds:
-        def __getattr__(self, name):
-            return (lambda plan: 0) if name == "kmx_lloyd_bounds_bytes" else getattr(lib, name)
-
     lib = drivers.lib
-    monkeypatch.setattr(drivers, "lib", NoBounds())
+
+    class Torch:
+        def __getattr__(self, name):
+            return getattr(torch, name)
+
+        def empty(self, *args, **kwargs):
+            out = torch.empty(*args, **kwargs)
+            if kwargs.get("dtype") is torch.uint8 and out.numel() > n:
+                seen["areas"].append(out.fill_(MARK))
+            return out
+
+    class Lib:
+        def __init__(self, with_bounds):
+            self.with_bounds = with_bounds
+
+        def __getattr__(self, name):
+            if name == "kmx_lloyd_bounds_bytes" and not self.with_bounds:
+                return lambda plan: 0
+            return self.run if name == "kmx_lloyd_run" else getattr(lib, name)
+
+        def run(self, *args):
+            rc = lib.kmx_lloyd_run(*args)
+            if args[-2].state == _capi.KMX_NEED_RELOCATION:
+                seen["relocations"] += 1
+                for area in seen["areas"]:  # (used within a call only: what is written from here on comes behind)
+                    area.fill_(MARK)
+            return rc
+
+    monkeypatch.setattr(drivers, "torch", Torch())
+    monkeypatch.setattr(drivers, "lib", Lib(True))
+    with_bounds = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
+    assert seen["relocations"] >= 1 and len(seen["areas"]) == 1 and _entered(seen["areas"][0], n, k)
+    monkeypatch.setattr(drivers, "lib", Lib(False))
     without = drivers.lloyd(X_t, w, init, False, 25, False, 0.0)
+    assert len(seen["areas"]) == 1
     assert with_bounds[3] == without[3] and with_bounds[1] == without[1]
-    assert bool((with_bounds[0] == without[0]).all()) and bool((with_bounds[2] == without[2]).all())
+    same = bool((with_bounds[0] == without[0]).all()), bool((with_bounds[2] == without[2]).all())
+    assert same == (True, True)
+
+
+@pytest.mark.parametrize("d, k, dtype", [(49, 133, "float32"), (49, 105, "float64")])
+def test_queue_that_holds_one_load_of_words(d, k, dtype, cuda):
+    """The largest operands that leave room for it: 2 048 and 1 024 entries, emptied behind every load of a workgroup's
+    3 900 samples."""
+    import torch
+
+    from sklearn_numba_dpex_amd import _capi
+    from sklearn_numba_dpex_amd._capi import lib
+
+    n, code = 1_000_003, _capi.dtype_code(getattr(torch, dtype))
+    assert lib.kmx_lloyd_bounds_bytes(_capi.lloyd_plan(n, d, k, code, 0)) > 0
+    assert lib.kmx_lloyd_bounds_bytes(_capi.lloyd_plan(n, d, k + 1, code, 0)) == 0
+    X_t, w, init = _blobs(n, d, k, getattr(torch, dtype), 13, cuda)
+    _same(_run(X_t, w, init, 30, False), _run(X_t, w, init, 30, True))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_runs_of_every_length(dtype, cuda):
+    import torch
+
+    X_t, w, init = _blobs(800_001, 20, 48, getattr(torch, dtype), 17, cuda)
+    for max_iter in range(4, 24):
+        _same(_run(X_t, w, init, max_iter, False), _run(X_t, w, init, max_iter, True, max_iter > 20 or None))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_a_sample_that_is_no_number(dtype, cuda):
+    """Its scores compare with none, which gives it the first label in every iteration, and no margin."""
+    import torch
+
+    X_t, w, init = _blobs(1_200_001, 14, 64, getattr(torch, dtype), 19, cuda)
+    at = 777_777
+    X_t[3, at] = float("nan")
+    w[at] = 0.0
+    a, b = _run(X_t, w, init, 30, False), _run(X_t, w, init, 30, True, None)
+    for run in (a, b):
+        assert int(run["labels"][at]) == 0
+    a["cent"], b["cent"] = (run["cent"].nan_to_num(nan=-1e30) for run in (a, b))
+    _same(a, b)
 
 
 # from 6e-14 to 1e18 (the data are about 15 wide) labels are those of bounded iterations; beyond, an fp32 chain loses
