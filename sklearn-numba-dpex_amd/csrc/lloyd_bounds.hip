@@ -28,11 +28,11 @@
 // of the workgroup, and its waves screen the queue by 32.  The few samples that the screen cannot tell, or that
 // move, are read from X_t.
 //
-// Bound by trips to memory and barriers, one after the other: 5e6 x 14 fp32 with 127 clusters, 5 % looked at, 45 us of
-// which the centroids' preparation takes 7, the words 7, the screen 7, the chain 3, the end of the
-// iteration 14 (a screened step 107, the iteration that enters 196: 680 MB); 2e6 x 32 fp64 with 64 clusters, 10 % looked
-// at, 47 (132, 209).  Runs of 20 and 12 iterations: 2 431 -> 2 069 us, 2 653 -> 2 385 (three relocations and the
-// iterations behind them included).
+// Bound by trips to memory and barriers, one after the other: 5e6 x 14 fp32 with 127 clusters, 4 to 7 % looked at, 46 to
+// 54 us, of which the centroids' preparation takes 7, the words 7, the screen 7, the chain 3, the end of the
+// iteration 14 (a screened step 104 to 112, the iteration that enters 192: 680 MB); 2e6 x 32 fp64 with 64 clusters, 10 %
+// looked at, 48 to 56 (134, 195).  Runs of 20 and 12 iterations by this step alone: 2 431 -> 2 069 us, 2 653 -> 2 385 (with
+// relocations and the iterations behind them).
 #include "lloyd_layout.h"
 #include "lloyd_screen.h"
 

@@ -17,8 +17,8 @@
 // range: so are these.
 //
 // Bound by the read of rows (a rebuild: 4.8 TB/s) or by a chain of trips to memory (corrections).  moves_sum_kernel, every
-// iteration a rebuild before: 1e6 x 256 fp32, 1 024 clusters 216 us, now 215 / 112 / 45 / 27 / 22 in the first five
-// iterations; 1e6 x 100 fp64, 100 clusters 177, now 180 / 165 / 47 / 27.  Runs 5 801 -> 5 220, 2 152 -> 1 920 us.
+// iteration a rebuild before: 1e6 x 256 fp32, 1 024 clusters 216 us, now 211 / 114 / 45 / 29 / 24 in the first five
+// iterations; 1e6 x 100 fp64, 100 clusters 177, now 181 / 170 / 59 / 38.  Runs by this step alone 6 106 -> 5 390, 2 168 -> 1 926 us.
 #include "lloyd_layout.h"
 #include "lloyd_screen.h"
 
