@@ -18,9 +18,9 @@
 // other are further apart than two errors E of the chain: with r of the margin left and D the distance to the
 // own centroid those scores are at least r D + r^2 / 2 apart, and D is still at least D0 - (margin - r); the word
 // leaves out as much of the margin as makes that exceed 2 E, with E for the largest centroid that means of the
-// data can be.  Scores, margins and drift are those of scaled values (the largest coordinate in
-// [2^12, 2^13)): squares of the data themselves leave fp32 from 1e-19 and 1e19 on, with the bounds made of them.  The sums are fixed point: a sample that moves is taken off its old cluster and added to the new
-// one, exactly.
+// data can be.  Scores, margins and drift are those of scaled values (the largest coordinate in [2^12, 2^13)): squares of
+// the data themselves leave fp32 from 1e-19 and 1e19 on, with the bounds made of them.  The sums are fixed point: a
+// sample that moves is taken off its old cluster and added to the new one, exactly.
 //
 // bounds_kernel<ENTER> is an iteration over all samples that also writes the words and, in fp32, the rows of X side
 // by side (samples here and there read feature by feature cost a 64-byte sector per value);

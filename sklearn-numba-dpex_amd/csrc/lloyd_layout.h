@@ -121,9 +121,9 @@ inline int kmx_kept_span(int64_t n, int esize, bool wide) {
     if (wide) return KMX_KEPT_ANY_SPAN;
     return kmx_kept_places(n) + (kmx_kept_words(esize, wide) - 1) * kmx_kept_rest(n) - (esize == 8 ? 55 : 26);
 }
-// Exponent of the first word of feature f (f = d: of the weights).  No clamp,
-// unlike the fused steps' (they scale in fp32): -226 to 346 are exponents that fp64 has, so a factor common to all
-// data costs no digits.
+// What the largest term of feature f (f = d: the largest weight) stays below, as a power of two, and the exponent of the first
+// word.  No clamp, unlike the fused steps' (they scale in fp32): -226 to 348, and 100 more for a third word, are
+// exponents that fp64 has, so a factor common to all data costs no digits.
 __device__ inline int kmx_kept_most(const unsigned int* __restrict__ absmax, int d, int f) {
     const float w = __uint_as_float(absmax[d]), x = f < d ? __uint_as_float(absmax[f]) : 1.0f;
     int e = kmx_not_finite(w) ? 0 : w > 0.0f ? ilogbf(w) + 1 : -149;
